@@ -42,20 +42,19 @@ struct Table {
 // the layer fields of one member in the ensemble's arithmetic type
 template <typename T>
 struct Layers {
-    T *u, *v, *h, *h0, *htmp, *up, *vp, *uh, *vh, *u_cor, *bt_h_u, *hx, *v_cor, *bt_h_v, *del2u, *del2v;
+    T *u, *v, *h, *h0, *htmp, *up, *vp, *uh, *vh, *u_cor, *bt_h_u, *hx, *v_cor, *bt_h_v;
 };
 
 Layers<float> layers_f32(mom6h_model *m)
 {
     auto &f = m->f;
-    return {f.u, f.v, f.h, f.h0, f.htmp, f.up, f.vp, f.uh, f.vh, f.u_cor, f.bt_h_u, f.hx, f.v_cor, f.bt_h_v,
-            f.del2u, f.del2v};
+    return {f.u, f.v, f.h, f.h0, f.htmp, f.up, f.vp, f.uh, f.vh, f.u_cor, f.bt_h_u, f.hx, f.v_cor, f.bt_h_v};
 }
 
 Layers<double> layers_f64(mom6h_model *m)
 {
     return {m->u, m->v, m->h, m->h0, m->htmp, m->up, m->vp, m->uh, m->vh, m->u_cor, m->bt.h_u, m->hx, m->v_cor,
-            m->bt_v.h_u, m->del2u, m->del2v};
+            m->bt_v.h_u};
 }
 
 template <typename T>
@@ -85,7 +84,7 @@ struct mom6h_ensemble {
     hipGraphExec_t gexec = nullptr;      // one 3D step of every member (stream s0)
     hipGraph_t graph_bt = nullptr;       // one barotropic step of every member (stream s1)
     hipGraphExec_t gexec_bt = nullptr;
-    int momentum_tile = 8;
+    int momentum_tile = 0, momentum_splits = 0;   // options of the momentum march (march_rows); 0: not set
     int bt_tile = 4;         // rows of the barotropic substep tile (4, 8 or 16)
     int bt_substeps = 5;     // barotropic substeps per blocked launch (1 = one launch per substep)
     long long max_lds = 0;
@@ -118,10 +117,9 @@ int build_tables(mom6h_ensemble *e, StepTables<T> &t, Layers<T> (*layers)(mom6h_
         const int nk = m->c.nk;
         MomArgsT<T> a{};
         a.d = m->d; a.g = m->ug; a.Kh = (T)m->c.Kh; a.h_neglect = (T)1.0e-3; a.no_slip = m->c.no_slip;
-        a.mask2dT = m->mask2dT; a.mask2dBu = m->mask2dBu; a.CoriolisBu = m->CoriolisBu;
+        a.mask = m->mask_bits; a.CoriolisBu = m->CoriolisBu;
         a.bu = L.u; a.bv = L.v;
-        a.Ah = (T)m->c.Ah; a.del2u = m->c.biharmonic ? L.del2u : nullptr; a.del2v = m->c.biharmonic ? L.del2v : nullptr;
-        a.nkz = 1;
+        a.Ah = (T)m->c.Ah; a.bih = m->c.biharmonic;
         // predictor: u, v, h0 -> up, vp; corrector: up, vp, htmp -> u, v (rk2_serial_driver.F90:236-350)
         a.u = L.u; a.v = L.v; a.h = L.h0; a.ou = L.up; a.ov = L.vp; a.fdt = (T)dt;
         t.mom_pred.h.push_back(a);
@@ -153,7 +151,10 @@ int build_tables(mom6h_ensemble *e, StepTables<T> &t, Layers<T> (*layers)(mom6h_
         t.h_htmp.h.push_back(job(m, L.htmp, nk));
         for (T *x : {L.u, L.v, L.h}) t.h_uvh.h.push_back(job(m, x, nk));
     }
-    for (auto *x : {&t.mom_pred, &t.mom_corr}) RC(x->upload());
+    for (auto *x : {&t.mom_pred, &t.mom_corr}) {
+        RC(plan_momentum_batch<T>(x->h.data(), x->n(), march_rows(e->momentum_tile, e->momentum_splits)));
+        RC(x->upload());
+    }
     for (auto *x : {&t.vv_pred, &t.vv_corr}) RC(x->upload());
     for (auto *x : {&t.cx_pred, &t.cx_corr, &t.cy_pred, &t.cy_corr}) RC(x->upload());
     for (auto *x : {&t.h_upvp, &t.h_htmp, &t.h_uvh, &t.h_hx}) RC(x->upload());
@@ -172,9 +173,8 @@ int enqueue_3d(mom6h_ensemble *e, StepTables<T> &t)
 {
     hipStream_t s = e->s0;
     const int n = (int)e->members.size();
-    const int ty = e->momentum_tile;
     // predictor
-    RC(launch_momentum_batch<T>(t.mom_pred.d, t.mom_pred.h.data(), n, s, ty));
+    RC(launch_momentum_batch<T>(t.mom_pred.d, t.mom_pred.h.data(), n, s));
     RC(vert_visc_batch<T>(t.vv_pred.d, t.vv_pred.h.data(), n, e->max_lds, s));
     RC(halo(t.h_upvp, s));
     RC(continuity_batch<T>(t.cx_pred.d, t.cx_pred.h.data(), n, false, true, e->max_lds, s));
@@ -184,7 +184,7 @@ int enqueue_3d(mom6h_ensemble *e, StepTables<T> &t)
     }
     RC(halo(t.h_htmp, s));
     // corrector
-    RC(launch_momentum_batch<T>(t.mom_corr.d, t.mom_corr.h.data(), n, s, ty));
+    RC(launch_momentum_batch<T>(t.mom_corr.d, t.mom_corr.h.data(), n, s));
     RC(vert_visc_batch<T>(t.vv_corr.d, t.vv_corr.h.data(), n, e->max_lds, s));
     RC(continuity_batch<T>(t.cx_corr.d, t.cx_corr.h.data(), n, false, true, e->max_lds, s));
     if (e->meridional) {
@@ -228,15 +228,21 @@ int capture_on(mom6h_ensemble *e, hipStream_t s, int (*enq)(mom6h_ensemble *), h
     return MOM6H_OK;
 }
 
-// layer splits of every member's momentum launch (capped at its nk), both phases
+// the march of every member's momentum launch, both phases
 template <typename T>
-int set_splits(StepTables<T> &t, int nkz)
+int set_march(StepTables<T> &t, int rows)
 {
     for (auto *x : {&t.mom_pred, &t.mom_corr}) {
-        for (auto &a : x->h) a.nkz = nkz < a.d.nk ? nkz : a.d.nk;
+        RC(plan_momentum_batch<T>(x->h.data(), x->n(), rows));
         if (x->d) MOM6H_CHECK(hipMemcpy(x->d, x->h.data(), x->h.size() * sizeof(x->h[0]), hipMemcpyHostToDevice));
     }
     return MOM6H_OK;
+}
+
+int set_march(mom6h_ensemble *e)
+{
+    const int rows = march_rows(e->momentum_tile, e->momentum_splits);
+    return e->mixed ? set_march<float>(e->tf, rows) : set_march<double>(e->td, rows);
 }
 
 void drop_graph(mom6h_ensemble *e)
@@ -251,17 +257,17 @@ void drop_graph(mom6h_ensemble *e)
     e->graph_bt = nullptr;
 }
 
-// mean time (ms) of reps predictor momentum launches with tile height ty
+// mean time (ms) of reps predictor momentum launches
 template <typename T>
-int time_momentum(mom6h_ensemble *e, StepTables<T> &t, int ty, int reps, float *ms)
+int time_momentum(mom6h_ensemble *e, StepTables<T> &t, int reps, float *ms)
 {
     const int n = (int)e->members.size();
     hipEvent_t a, b;
     MOM6H_CHECK(hipEventCreate(&a));
     MOM6H_CHECK(hipEventCreate(&b));
-    int rc = launch_momentum_batch<T>(t.mom_pred.d, t.mom_pred.h.data(), n, e->s0, ty);   // warm
+    int rc = launch_momentum_batch<T>(t.mom_pred.d, t.mom_pred.h.data(), n, e->s0);   // warm
     if (!rc && hipEventRecord(a, e->s0) != hipSuccess) rc = set_error(MOM6H_ESTATE, "event record failed");
-    for (int r = 0; r < reps && !rc; ++r) rc = launch_momentum_batch<T>(t.mom_pred.d, t.mom_pred.h.data(), n, e->s0, ty);
+    for (int r = 0; r < reps && !rc; ++r) rc = launch_momentum_batch<T>(t.mom_pred.d, t.mom_pred.h.data(), n, e->s0);
     if (!rc && hipEventRecord(b, e->s0) != hipSuccess) rc = set_error(MOM6H_ESTATE, "event record failed");
     if (!rc && hipEventSynchronize(b) != hipSuccess) rc = set_error(MOM6H_ESTATE, "event wait failed");
     float x = 0.f;
@@ -406,6 +412,7 @@ int mom6h_ensemble_set_option(mom6h_ensemble *e, const char *key, double value)
         const int ty = (int)value;
         MOM6H_REQUIRE(ty == 4 || ty == 8 || ty == 16, "mom6h_ensemble_set_option: momentum_tile must be 4, 8 or 16");
         e->momentum_tile = ty;
+        if (e->prepared) RC(set_march(e));
         drop_graph(e);
     } else if (k == "bt_tile") {
         MOM6H_REQUIRE(value == 4.0 || value == 8.0 || value == 16.0, "mom6h_ensemble_set_option: bt_tile must be 4, 8 or 16");
@@ -420,7 +427,8 @@ int mom6h_ensemble_set_option(mom6h_ensemble *e, const char *key, double value)
         MOM6H_REQUIRE(e->prepared, "mom6h_ensemble_set_option: momentum_splits after prepare");
         const int v = (int)value;
         MOM6H_REQUIRE(v >= 1, "mom6h_ensemble_set_option: momentum_splits >= 1");
-        RC(e->mixed ? set_splits<float>(e->tf, v) : set_splits<double>(e->td, v));
+        e->momentum_splits = v;
+        RC(set_march(e));
         drop_graph(e);
     } else {
         return set_error(MOM6H_EINVAL, "mom6h_ensemble_set_option: unknown option '%s'", key);
@@ -433,28 +441,31 @@ int mom6h_ensemble_autotune(mom6h_ensemble *e, int reps, char *report, int nbyte
     MOM6H_REQUIRE(e != nullptr, "mom6h_ensemble_autotune: NULL ensemble");
     MOM6H_REQUIRE(e->prepared, "mom6h_ensemble_autotune: call mom6h_ensemble_prepare first");
     MOM6H_CHECK(hipDeviceSynchronize());
-    const int rows[3] = {4, 8, 16}, splits[4] = {1, 2, 4, 8};
+    // marches of 128, 64, 32, 16, 8 and 4 rows
+    const int tiles[6] = {16, 8, 4, 4, 4, 4}, splits[6] = {1, 1, 1, 2, 4, 8};
     float best = 0.f;
     int pick = 8, pick_s = 1;
-    std::string rep = "momentum tile rows x layer splits (ms):";
-    for (int q = 0; q < 12; ++q) {
+    std::string rep = "momentum march rows (ms):";
+    for (int q = 0; q < 6; ++q) {
         float ms = 0.f;
-        RC(e->mixed ? set_splits<float>(e->tf, splits[q % 4]) : set_splits<double>(e->td, splits[q % 4]));
-        RC(e->mixed ? time_momentum<float>(e, e->tf, rows[q / 4], reps, &ms)
-                    : time_momentum<double>(e, e->td, rows[q / 4], reps, &ms));
+        e->momentum_tile = tiles[q];
+        e->momentum_splits = splits[q];
+        RC(set_march(e));
+        RC(e->mixed ? time_momentum<float>(e, e->tf, reps, &ms) : time_momentum<double>(e, e->td, reps, &ms));
         char buf[64];
-        snprintf(buf, sizeof(buf), " %dx%d %.4f;", rows[q / 4], splits[q % 4], ms);
+        snprintf(buf, sizeof(buf), " %d %.4f;", march_rows(tiles[q], splits[q]), ms);
         rep += buf;
         if (q == 0 || ms < best) {
             best = ms;
-            pick = rows[q / 4];
-            pick_s = splits[q % 4];
+            pick = tiles[q];
+            pick_s = splits[q];
         }
     }
     e->momentum_tile = pick;
-    RC(e->mixed ? set_splits<float>(e->tf, pick_s) : set_splits<double>(e->td, pick_s));
+    e->momentum_splits = pick_s;
+    RC(set_march(e));
     drop_graph(e);
-    rep += " chosen " + std::to_string(pick) + "x" + std::to_string(pick_s);
+    rep += " chosen " + std::to_string(march_rows(pick, pick_s));
     if (report && nbytes > 0) snprintf(report, (size_t)nbytes, "%s", rep.c_str());
     return MOM6H_OK;
 }

@@ -36,7 +36,7 @@ struct UMetT {
 
 // Arguments of the fused momentum stencil.  T is the type of the 3D layer
 // fields and of the stencil arithmetic (double: the reference's FP64; float:
-// the mixed-precision form); 2D masks and Coriolis stay FP64 in memory.
+// the mixed-precision form); Coriolis stays FP64 in memory.
 template <typename T>
 struct MomArgsT {
     Dims d;
@@ -46,21 +46,32 @@ struct MomArgsT {
     const T *u, *v, *h;               // stencil inputs
     const T *bu, *bv;                 // bases of the update (may alias ou/ov)
     T *ou, *ov;
-    const double *mask2dT, *mask2dBu, *CoriolisBu;
-    // biharmonic viscosity: Ah and the Del2 scratch (NULL: Laplacian only)
+    const unsigned char *mask;        // the 0/1 masks per point: bit 0 mask2dT, bit 1 mask2dBu
+    const double *CoriolisBu;         // constant along every row
     T Ah;
-    T *del2u, *del2v;
-    int nkz;   // the layers split over this many blocks per tile (1..nk)
+    int bih;                          // biharmonic viscosity beside the Laplacian (Ah)
+    int march;                        // rows a wave marches through (0: chosen from the grid)
 };
 using MomArgs = MomArgsT<double>;
 
-// One grid (tile height ty = 4, 8 or 16 rows), or every member of an ensemble
-// in one launch per kernel (d_args: the members' arguments on the device,
-// h_args: the same on the host)
+// One grid, or every member of an ensemble in one launch (d_args: the members'
+// arguments on the device, h_args: the same on the host, their march set by
+// plan_momentum_batch: `rows`, or with 0 chosen from all members' grids)
 template <typename T>
-int launch_momentum(const MomArgsT<T> &a, hipStream_t s, int ty = 8);
+int launch_momentum(const MomArgsT<T> &a, hipStream_t s);
 template <typename T>
-int launch_momentum_batch(const MomArgsT<T> *d_args, const MomArgsT<T> *h_args, int n, hipStream_t s, int ty = 8);
+int plan_momentum_batch(MomArgsT<T> *h_args, int n, int rows);
+template <typename T>
+int launch_momentum_batch(const MomArgsT<T> *d_args, const MomArgsT<T> *h_args, int n, hipStream_t s);
+
+// Rows a wave of the momentum stencil marches through for the options
+// momentum_tile and momentum_splits (0 while neither is set: chosen from the grid)
+inline int march_rows(int tile, int splits)
+{
+    if (!tile && !splits) return 0;
+    const int rows = 8 * (tile ? tile : 8) / (splits ? splits : 1);
+    return rows < 4 ? 4 : rows;
+}
 
 // true and the common value when every element of a[0..n) is identical
 inline bool uniform_value(const double *a, size_t n, double *v)
@@ -72,7 +83,7 @@ inline bool uniform_value(const double *a, size_t n, double *v)
 }
 
 // true when every element of a[0..n) is 0 or 1 (a land/sea mask the fused
-// momentum stencil can stage as bytes)
+// momentum stencil can read as a bit)
 inline bool binary_mask(const double *a, size_t n)
 {
     for (size_t q = 0; q < n; ++q)
@@ -81,7 +92,7 @@ inline bool binary_mask(const double *a, size_t n)
 }
 
 // true when the 2D field a (ni x nj, i fastest) is constant along every row
-// j (f-plane and beta-plane Coriolis: the fused momentum stencil stages one
+// j (f-plane and beta-plane Coriolis: the fused momentum stencil reads one
 // value per row)
 inline bool rows_uniform(const double *a, size_t ni, size_t nj)
 {

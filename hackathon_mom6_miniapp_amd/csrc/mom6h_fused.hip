@@ -3,13 +3,11 @@
 // One launch performs, for every layer, what the reference does in four
 // module calls (app/rk2_serial_driver.F90:236-270 and :316-350):
 //   compute_transports (:544-561) -> hor_visc (src/serial/mom6_hor_visc_serial.F90,
-//   Laplacian) -> CorAdCalc (src/serial/mom6_coriolis_serial.F90, Sadourny
-//   energy scheme) -> velocity update  ou = base + fdt*(CA + diff)
-// The transports, tendencies and potential vorticity never leave the chip: a
-// block stages u, v, h of its tile plus a one-cell ring in LDS for one layer,
-// forms q, KE and the viscous stresses on the staged q/h points (each once),
-// then every thread finishes its velocity points.  It walks all layers, so the 2D masks and Coriolis
-// parameter stay in L1/L2 for the whole layer walk.
+//   Laplacian, with or without the biharmonic term) -> CorAdCalc
+//   (src/serial/mom6_coriolis_serial.F90, Sadourny energy scheme) -> velocity
+//   update  ou = base + fdt*(CA + diff)
+// The transports, tendencies, strains, Del2 fields and potential vorticity
+// never leave the registers (the march below).
 //
 // On a uniform grid every metric array holds one value; the kernels take those
 // values (read from the arrays at set-up) and keep the reference's operation
@@ -18,66 +16,11 @@
 // matter for diffu/diffv/CAu/CAv outside the velocity-update ranges; inside
 // them the q values on row js-1 and column is-1 still see the zero hArea the
 // reference reads, exactly as here.
+#include <algorithm>
+
 #include "mom6h_fused.h"
 
 namespace mom6h {
-
-// Output tile MT_X x TY (TY = 4, 8 or 16 rows, chosen at launch); the staged
-// region is [i0-1, i1+1] x [j0-1, j1+1]
-constexpr int MT_X = 64;
-constexpr int MW = MT_X + 2;
-
-// Biharmonic viscosity, first half: Del2u on u points I = is-1..ie,
-// j = js..je and Del2v on v points i = is..ie, J = js-1..je
-// (mom6_hor_visc_serial.F90:587-607, uniform metrics).  The arrays are zero
-// at allocation and never written outside those ranges, which is what the
-// reference's second half reads there.
-template <typename T>
-__device__ __forceinline__ void del2_body(const MomArgsT<T> &a, int bx, int by, int bz)
-{
-    const Dims &d = a.d;
-    const UMetT<T> g(a.g);
-    const int i = d.isc - 1 + bx * 64 + (threadIdx.x & 63);
-    const int j = d.jsc - 1 + by * 4 + (threadIdx.x >> 6);
-    const int k = 1 + bz;
-    if (i > d.iec || j > d.jec) return;
-    auto U = [&](int ii, int jj) -> T { return a.u[IX3(d, ii, jj, k)]; };
-    auto V = [&](int ii, int jj) -> T { return a.v[IX3(d, ii, jj, k)]; };
-    auto sh_xx = [&](int ii, int jj) -> T {   // h point (:503-510)
-        const T dudx = g.DY_dxT * ((g.IdyCu * U(ii, jj)) - (g.IdyCu * U(ii - 1, jj)));
-        const T dvdy = g.DX_dyT * ((g.IdxCv * V(ii, jj)) - (g.IdxCv * V(ii, jj - 1)));
-        return dudx - dvdy;
-    };
-    auto sh_xy = [&](int I, int J) -> T {    // q point (:513-547)
-        const T dvdx = g.DY_dxBu * ((V(I + 1, J) * g.IdyCv) - (V(I, J) * g.IdyCv));
-        const T dudy = g.DX_dyBu * ((U(I, J + 1) * g.IdxCu) - (U(I, J) * g.IdxCu));
-        const T m = (T)a.mask2dBu[IX2(d, I, J)];
-        return (a.no_slip ? (T(2.0) - m) : m) * (dvdx + dudy);
-    };
-    const long long c = IX3(d, i, j, k);
-    if (j >= d.jsc)
-        a.del2u[c] = g.Idx2dyCu * ((g.dx2q * sh_xy(i, j)) - (g.dx2q * sh_xy(i, j - 1))) +
-                     g.Idxdy2u * ((g.dy2h * sh_xx(i + 1, j)) - (g.dy2h * sh_xx(i, j)));
-    if (i >= d.isc)
-        a.del2v[c] = g.Idxdy2v * ((g.dy2q * sh_xy(i, j)) - (g.dy2q * sh_xy(i - 1, j))) -
-                     g.Idx2dyCv * ((g.dx2h * sh_xx(i, j + 1)) - (g.dx2h * sh_xx(i, j)));
-}
-
-template <typename T>
-__global__ void __launch_bounds__(256) k_del2(MomArgsT<T> a)
-{
-    del2_body(a, blockIdx.x, blockIdx.y, blockIdx.z);
-}
-
-template <typename T>
-__global__ void __launch_bounds__(256) k_del2_batch(const MomArgsT<T> *__restrict__ args, BatchMap mp)
-{
-    int m, local;
-    batch_locate(mp, blockIdx.x, m, local);
-    const int r = local / mp.nbx[m];
-    const MomArgsT<T> a = args[m];
-    del2_body(a, local % mp.nbx[m], r % mp.nby[m], r / mp.nby[m]);
-}
 
 // Division in the stencil's type: exact in FP64 (the reference's arithmetic);
 // in the FP32 form a product with the hardware reciprocal (about 1 ulp, the
@@ -89,289 +32,352 @@ __device__ __forceinline__ T sdiv(T num, T den)
     else return num / den;
 }
 
-// The tile (tile_x, tile_y) of one grid.  BIH: the biharmonic stress of the
-// Del2 fields staged like u and v, added to the Laplacian stress
-// (:824-886, :979-1036).
-template <typename T, bool BIH, int TY>
-__device__ __forceinline__ void momentum_body(const MomArgsT<T> &a, int tile_x, int tile_y, int k_first, int k_last)
+// The value of the lane to the west (lane - 1) and to the east (lane + 1): DPP
+// wave shifts, one VALU move per 32 bits.  Lane 0 (63) gets zero; every lane
+// of the wave must be active.
+constexpr int kWaveShl1 = 0x130, kWaveShr1 = 0x138;
+template <int CTRL>
+__device__ __forceinline__ int dpp32(int x)
 {
-    constexpr int MH = TY + 2, RPT = TY / 4;   // staged rows; output rows per thread
-    __shared__ T s_u[MH][MW], s_v[MH][MW], s_h[MH][MW];
-    __shared__ T s_q[MH][MW], s_KE[MH][MW];
-    // the Laplacian (+ biharmonic) stresses str_xx*h at the staged h points and
-    // str_xy*hq at the staged q points, formed once per point (each is read by
-    // up to three output points)
-    __shared__ T s_sxx[MH][MW], s_sxy[MH][MW];
-    __shared__ T s_d2u[BIH ? MH : 1][BIH ? MW : 1], s_d2v[BIH ? MH : 1][BIH ? MW : 1];
-    // the 2D masks and Coriolis of the staged region, the same for every
-    // layer: the masks as bytes (the host checks that they hold 0 or 1) and
-    // Coriolis as one value per row (the host checks that CoriolisBu is
-    // constant along every row), which leaves a 64 x 8 tile in FP64 38 KB of
-    // LDS, four blocks per CU instead of three
-    __shared__ unsigned char s_mT[MH][MW], s_mBu[MH][MW];
-    __shared__ T s_cor[MH];
+    return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp(float x)
+{
+    return __int_as_float(dpp32<CTRL>(__float_as_int(x)));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp(double x)
+{
+    return __hiloint2double(dpp32<CTRL>(__double2hiint(x)), dpp32<CTRL>(__double2loint(x)));
+}
+template <typename T>
+__device__ __forceinline__ T west(T x)
+{
+    return dpp<kWaveShr1>(x);
+}
+template <typename T>
+__device__ __forceinline__ T east(T x)
+{
+    return dpp<kWaveShl1>(x);
+}
+
+// One wave marches along j through rows ja..jb of one layer, lane l holding
+// column i0 + l: the i neighbours come from the neighbouring lanes (DPP), the
+// j neighbours are the values kept from the rows before.  So every strain, q,
+// KE, transport and stress is formed once per point, no LDS, no barrier and no
+// index arithmetic beyond a row pointer; the outermost LM lanes on either side
+// only lend their values (the next strip's wave computes them).  At step r the
+// row r arrives (its loads were issued a step before); the h-point terms of
+// row r and the q-point terms of row p = r - 1 follow, and with them the
+// outputs of row p.  BIH: Del2u and Del2v of row p come next, then the stresses
+// of h row p and q row p - 1, and the outputs are those of row p - 1 (its
+// Coriolis terms kept for one step).
+//
+// What bounds it: 225 VALU instructions per row of 62 points (FP64, Laplacian)
+// against the 370 of a 64 x 8 tile staged in LDS with its recomputed ring, 38
+// KB of LDS and two barriers per layer, which was VALU-bound.  At 720x720x75
+// the predictor now takes 0.40 ms and the corrector 0.49 ms (0.61-0.69 ms
+// before): 1.68 and 2.35 GB of memory traffic at 4.2 and 4.8 TB/s, the rate of
+// a plain copy.  FP32: 0.22 ms (0.34), its memory and VALU time about equal; with
+// the biharmonic term 0.26 ms, which took 0.70 ms with Del2 formed by a launch
+// of its own (0.30 ms) and read back.
+template <typename T, bool BIH>
+struct March {
+    static constexpr int LM = BIH ? 2 : 1;          // lent lanes on either side
+    static constexpr int OUT = 64 - 2 * LM;         // columns a wave updates
+    static constexpr int LAG = BIH ? 2 : 1;         // rows between the newest row and the outputs
+};
+
+// SAME: the base of the update is the stencil's own input (the predictor), so
+// its row is at hand; otherwise (the corrector) it is loaded
+template <typename T, bool BIH, bool SAME>
+__device__ __forceinline__ void march(const MomArgsT<T> &a, int strip, int ja, int jb, int k)
+{
+    using M = March<T, BIH>;
     const Dims &d = a.d;
     const UMetT<T> g(a.g);
     const int is = d.isc, ie = d.iec, js = d.jsc, je = d.jec;
-    const int i0 = is + tile_x * MT_X, j0 = js + tile_y * TY;
-    const int bi = i0 - 1, bj = j0 - 1;
-    const int tid = threadIdx.x;
-    const int tx = tid % MT_X, ty = tid / MT_X;          // 64 x 4 threads, RPT rows each
+    const int lane = threadIdx.x & 63;
+    const int i = is + strip * M::OUT - M::LM + lane;
+    const unsigned col = (unsigned)((i <= d.ied ? i : d.ied) - d.isd);   // clamped: such lanes only lend
+    const bool mine = lane >= M::LM && lane < 64 - M::LM;
+    const bool out_u = mine && i <= ie - 1, out_v = mine && i <= ie;
+    const bool west_edge = i < is;
+    const bool del2u_col = i >= is - 1 && i <= ie, del2v_col = i >= is && i <= ie;
+    const long long n1 = d.n1, layer = (long long)(k - 1) * d.s2;
+    const T slip_a = a.no_slip ? T(2.0) : T(0.0), slip_b = a.no_slip ? T(-1.0) : T(1.0);
 
-    // u, v, h of the staged region [i0-1, i1+1] x [j0-1, j1+1] of one layer go
-    // through registers: the next layer's loads are issued before the current
-    // layer is computed (NS points per thread), and so are the base velocities
-    // of the thread's output rows
-    constexpr int NS = (MW * MH + 255) / 256;
-    T pu[NS], pv[NS], ph[NS], pbu[RPT], pbv[RPT];
-    T p2u[BIH ? NS : 1], p2v[BIH ? NS : 1];
-    auto load_layer = [&](int k) {
-#pragma unroll
-        for (int r = 0; r < NS; ++r) {
-            const int t = tid + 256 * r;
-            const int li = t % MW, lj = t / MW, i = bi + li, j = bj + lj;
-            pu[r] = T(0.0); pv[r] = T(0.0); ph[r] = T(0.0);
-            if (BIH) { p2u[BIH ? r : 0] = T(0.0); p2v[BIH ? r : 0] = T(0.0); }
-            if (t < MW * MH && i <= d.ied && j <= d.jed) {
-                const long long c = IX3(d, i, j, k);
-                pu[r] = a.u[c]; pv[r] = a.v[c]; ph[r] = a.h[c];
-                if (BIH) { p2u[BIH ? r : 0] = a.del2u[c]; p2v[BIH ? r : 0] = a.del2v[c]; }
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < RPT; ++r) {
-            const int i = i0 + tx, j = j0 + ty + 4 * r;
-            pbu[r] = T(0.0); pbv[r] = T(0.0);
-            if (i <= ie && j <= je) {
-                const long long c = IX3(d, i, j, k);
-                pbu[r] = a.bu[c]; pbv[r] = a.bv[c];
+    // the newest row (in flight until its step)
+    T nu, nv, nh, ncor, nbu = T(0.0), nbv = T(0.0);
+    unsigned nm;
+    auto load = [&](int r) __attribute__((always_inline)) {
+        const long long row = (long long)(r - d.jsd) * n1, o = layer + row;
+        nu = (a.u + o)[col];
+        nv = (a.v + o)[col];
+        nh = (a.h + o)[col];
+        nm = (a.mask + row)[col];
+        ncor = (T)a.CoriolisBu[row];   // constant along the row
+        if (!SAME) {                   // the base of the row that step r finishes
+            const int b = r - M::LAG;
+            if (b >= ja) {
+                const long long ob = layer + (long long)(b - d.jsd) * n1;
+                nbu = (a.bu + ob)[col];
+                nbv = (a.bv + ob)[col];
             }
         }
     };
-    for (int t = tid; t < MW * MH; t += blockDim.x) {
-        const int li = t % MW, lj = t / MW, i = bi + li, j = bj + lj;
-        T mt = T(0.0), mb = T(0.0), cor = T(0.0);
-        if (i <= d.ied && j <= d.jed) {
-            const long long c2 = IX2(d, i, j);
-            mt = (T)a.mask2dT[c2];
-            mb = (T)a.mask2dBu[c2];
-            cor = (T)a.CoriolisBu[c2];
-        }
-        s_mT[lj][li] = (unsigned char)(mt != T(0.0));
-        s_mBu[lj][li] = (unsigned char)(mb != T(0.0));
-        if (li == 0) s_cor[lj] = cor;   // i = i0-1: inside the data domain
+
+    // kept from the row before (p): state, masked thickness, h-point terms
+    T u_p, v_p, ve_p, h_p, he_p, mh_p, mBu_p, cor_p, hAu_p;
+    T KE_p = T(0.0), KEe_p = T(0.0), uh_p = T(0.0), uhw_p = T(0.0);
+    T sxx_p = T(0.0), sxxe_p = T(0.0);              // stress*h (BIH: the strain sh_xx)
+    // kept from q row p - 1
+    T q_s = T(0.0), vhs_s = T(0.0), sxy_s = T(0.0); // (BIH: sxy_s is the strain sh_xy)
+    // BIH: kept for the outputs of row p - 1
+    T CAu_o = T(0.0), CAv_o = T(0.0), hu_o = T(1.0), hv_o = T(1.0), hqm_s = T(0.0), h_o = T(0.0);
+    T d2u_s = T(0.0), d2v_s = T(0.0);               // Del2 of row p - 1
+    T txx_o = T(0.0), txxe_o = T(0.0), txy_o = T(0.0);   // stress*h of h row p - 1, stress*hq of q row p - 2
+    T u_o = T(0.0), v_o = T(0.0);                   // SAME: the base of row p - 1
+
+    const int r0 = ja - M::LAG;
+    load(r0);
+    {
+        u_p = nu; v_p = nv; h_p = nh;
+        ve_p = east(nv); he_p = east(nh);
+        mh_p = (T)(nm & 1u) * nh;
+        mBu_p = (T)((nm >> 1) & 1u);
+        cor_p = ncor;
+        // never formed on row js-1 (mom6_coriolis_serial.F90:142-152): zero
+        hAu_p = r0 < js ? T(0.0) : T(0.5) * ((g.areaT * h_p) + (g.areaT * he_p));
     }
-    // Laplacian stress pieces (mom6_hor_visc_serial.F90:503-547, 807-1053)
-    auto str_xx = [&](int pi, int pj) -> T {   // LDS coords of an h point
-        const T dudx = g.DY_dxT * ((g.IdyCu * s_u[pj][pi]) - (g.IdyCu * s_u[pj][pi - 1]));
-        const T dvdy = g.DX_dyT * ((g.IdxCv * s_v[pj][pi]) - (g.IdxCv * s_v[pj - 1][pi]));
-        T str = -(a.Kh * (dudx - dvdy));
-        if (BIH) {
-            const int qi = BIH ? pi : 0, qj = BIH ? pj : 0;
-            const T d_del2u = (g.IdyCu * s_d2u[qj][qi]) - (g.IdyCu * s_d2u[qj][BIH ? qi - 1 : 0]);
-            const T d_del2v = (g.IdxCv * s_d2v[qj][qi]) - (g.IdxCv * s_d2v[BIH ? qj - 1 : 0][qi]);
-            str = str + a.Ah * ((g.DY_dxT * d_del2u) - (g.DX_dyT * d_del2v));
+    load(r0 + 1);
+    for (int r = r0 + 1; r <= jb + M::LAG; ++r) {
+        const T u = nu, v = nv, h = nh, cor = ncor, bu = nbu, bv = nbv;
+        const T mT = (T)(nm & 1u), mBu = (T)((nm >> 1) & 1u);
+        if (r < jb + M::LAG) load(r + 1);
+        const int p = r - 1;
+        const T uw = west(u), ve = east(v), he = east(h);
+        const T mh = mT * h;
+        // h points of row r: strain and KE (mom6_hor_visc_serial.F90:503-510,
+        // mom6_coriolis_serial.F90:196-203), transport uh
+        const T dudx = g.DY_dxT * ((g.IdyCu * u) - (g.IdyCu * uw));
+        const T dvdy = g.DX_dyT * ((g.IdxCv * v) - (g.IdxCv * v_p));
+        const T sh_xx = dudx - dvdy;
+        const T KE = sdiv(T(0.25) * ((g.dyCu * (u * u) + g.dyCu * (uw * uw)) +
+                                     (g.dxCv * (v * v) + g.dxCv * (v_p * v_p))), g.areaT);
+        const T KEe = east(KE);
+        const T uh = u * T(0.5) * (h + he) * g.dyCu;
+        const T uhw = west(uh);
+        // q points of row p: potential vorticity (:134-168), transport vh
+        const T hAu = T(0.5) * ((g.areaT * h) + (g.areaT * he));
+        const T hAv = T(0.5) * ((g.areaT * h_p) + (g.areaT * h));
+        const T hAve = T(0.5) * ((g.areaT * he_p) + (g.areaT * he));
+        const T rel_vort = mBu_p * (((ve_p * g.dyCv) - (v_p * g.dyCv)) - ((u * g.dxCu) - (u_p * g.dxCu))) * g.IareaBu;
+        const T hArea_q = (hAu_p + hAu) + ((west_edge ? T(0.0) : hAv) + hAve);
+        const T q = (cor_p + rel_vort) * sdiv(g.Area_q, hArea_q + T(1.0e-20));
+        const T qw = west(q);
+        const T vh = v_p * T(0.5) * (h_p + h) * g.dxCv;
+        const T vhs = east(vh) + vh;
+        // CAu and CAv of row p, Sadourny (:208-226)
+        const T CAu = T(0.25) * ((q * vhs) + (q_s * vhs_s)) * g.IdxCu - (KEe_p - KE_p) * g.IdxCu;
+        const T CAv = -(T(0.25) * ((qw * (uhw_p + uhw)) + (q * (uh_p + uh))) * g.IdyCv) - (KE - KE_p) * g.IdyCv;
+        // strain at the q points of row p (:513-547) and the thickness there
+        const T dvdx = g.DY_dxBu * ((ve_p * g.IdyCv) - (v_p * g.IdyCv));
+        const T dudy = g.DX_dyBu * ((u * g.IdxCu) - (u_p * g.IdxCu));
+        const T sh_xy = (slip_a + slip_b * mBu_p) * (dvdx + dudy);
+        const T hq = T(0.25) * ((h_p + he) + (he_p + h));
+        const T hqm = hq * (a.no_slip ? T(1.0) : mBu_p);
+        const T h_u = T(0.5) * (mh_p + east(mh_p)) + a.h_neglect, h_v = T(0.5) * (mh_p + mh) + a.h_neglect;
+
+        // outputs of row jo (diffu :1059-1067, diffv :1070-1078, velocity
+        // update): stresses xx of its h points (own and east) and of the row
+        // above, xy of its q points (own and west) and of the row below
+        auto finish = [&](int jo, T Cu, T Cv, T den_u, T den_v, T xx, T xxe, T xx_n, T xy, T xy_s, T b_u, T b_v)
+                          __attribute__((always_inline)) {
+            const T xyw = west(xy);
+            if (jo < ja) return;
+            const T diffu = sdiv((g.IdxCu * ((g.dx2q * xy_s) - (g.dx2q * xy)) +
+                                  g.IdyCu * ((g.dy2h * xx) - (g.dy2h * xxe))) * g.IareaCu, den_u);
+            const T diffv = sdiv((g.IdyCv * ((g.dy2q * xyw) - (g.dy2q * xy)) -
+                                  g.IdxCv * ((g.dx2h * xx) - (g.dx2h * xx_n))) * g.IareaCv, den_v);
+            const long long o = layer + (long long)(jo - d.jsd) * n1;
+            if (out_u) (a.ou + o)[col] = b_u + a.fdt * (Cu + diffu);
+            if (out_v && jo <= je - 1) (a.ov + o)[col] = b_v + a.fdt * (Cv + diffv);
+        };
+        if constexpr (!BIH) {
+            const T xx = -(a.Kh * sh_xx) * h, xxe = east(xx);
+            const T xy = -(a.Kh * sh_xy) * hqm;
+            finish(p, CAu, CAv, h_u, h_v, sxx_p, sxxe_p, xx, xy, sxy_s, SAME ? u_p : bu, SAME ? v_p : bv);
+            sxx_p = xx; sxxe_p = xxe;
+            sxy_s = xy;
+        } else {
+            // Del2u on u points I = is-1..ie, j = js..je and Del2v on v points
+            // i = is..ie, J = js-1..je of row p (:587-607), zero elsewhere
+            const T sh_xxe = east(sh_xx);
+            T d2u = g.Idx2dyCu * ((g.dx2q * sh_xy) - (g.dx2q * sxy_s)) +
+                    g.Idxdy2u * ((g.dy2h * sxxe_p) - (g.dy2h * sxx_p));
+            T d2v = g.Idxdy2v * ((g.dy2q * sh_xy) - (g.dy2q * west(sh_xy))) -
+                    g.Idx2dyCv * ((g.dx2h * sh_xx) - (g.dx2h * sxx_p));
+            if (!(del2u_col && p >= js && p <= je)) d2u = T(0.0);
+            if (!(del2v_col && p >= js - 1 && p <= je)) d2v = T(0.0);
+            // stress*h at the h points of row p (:824-886)
+            const T d_del2u = (g.IdyCu * d2u) - (g.IdyCu * west(d2u));
+            const T d_del2v = (g.IdxCv * d2v) - (g.IdxCv * d2v_s);
+            const T txx = (-(a.Kh * sxx_p) + a.Ah * ((g.DY_dxT * d_del2u) - (g.DX_dyT * d_del2v))) * h_p;
+            const T txxe = east(txx);
+            // stress*hq at the q points of row p - 1 (:979-1036)
+            const T txy = (-(a.Kh * sxy_s) +
+                           a.Ah * ((g.DY_dxBu * ((east(d2v_s) * g.IdyCv) - (d2v_s * g.IdyCv))) +
+                                   (g.DX_dyBu * ((d2u * g.IdxCu) - (d2u_s * g.IdxCu))))) * hqm_s;
+            finish(p - 1, CAu_o, CAv_o, hu_o, hv_o, txx_o, txxe_o, txx, txy, txy_o, SAME ? u_o : bu, SAME ? v_o : bv);
+            CAu_o = CAu; CAv_o = CAv; hu_o = h_u; hv_o = h_v; hqm_s = hqm;
+            txx_o = txx; txxe_o = txxe; txy_o = txy;
+            d2u_s = d2u; d2v_s = d2v;
+            sxx_p = sh_xx; sxxe_p = sh_xxe;
+            sxy_s = sh_xy;
+            u_o = u_p; v_o = v_p;
         }
-        return str * (s_h[pj][pi] * T(1.0));
-    };
-    auto str_xy = [&](int pi, int pj) -> T {   // q point at LDS (pi, pj)
-        const T dvdx = g.DY_dxBu * ((s_v[pj][pi + 1] * g.IdyCv) - (s_v[pj][pi] * g.IdyCv));
-        const T dudy = g.DX_dyBu * ((s_u[pj + 1][pi] * g.IdxCu) - (s_u[pj][pi] * g.IdxCu));
-        const T m = (T)s_mBu[pj][pi];
-        const T sh = (a.no_slip ? (T(2.0) - m) : m) * (dvdx + dudy);
-        const T hq = T(0.25) * ((s_h[pj][pi] + s_h[pj + 1][pi + 1]) + (s_h[pj][pi + 1] + s_h[pj + 1][pi]));
-        T str = -(a.Kh * sh);
-        if (BIH) {
-            const int qi = BIH ? pi : 0, qj = BIH ? pj : 0;
-            str = str + a.Ah * ((g.DY_dxBu * ((s_d2v[qj][BIH ? qi + 1 : 0] * g.IdyCv) - (s_d2v[qj][qi] * g.IdyCv))) +
-                                (g.DX_dyBu * ((s_d2u[BIH ? qj + 1 : 0][qi] * g.IdxCu) - (s_d2u[qj][qi] * g.IdxCu))));
-        }
-        return a.no_slip ? str * (hq * T(1.0)) : str * (hq * m * T(1.0));
-    };
-    load_layer(k_first);
-    for (int k = k_first; k <= k_last; ++k) {
-#pragma unroll
-        for (int r = 0; r < NS; ++r) {
-            const int t = tid + 256 * r;
-            if (t < MW * MH) {
-                const int li = t % MW, lj = t / MW;
-                s_u[lj][li] = pu[r]; s_v[lj][li] = pv[r]; s_h[lj][li] = ph[r];
-                if (BIH) { s_d2u[BIH ? lj : 0][BIH ? li : 0] = p2u[BIH ? r : 0]; s_d2v[BIH ? lj : 0][BIH ? li : 0] = p2v[BIH ? r : 0]; }
-            }
-        }
-        T bu_r[RPT], bv_r[RPT];
-#pragma unroll
-        for (int r = 0; r < RPT; ++r) { bu_r[r] = pbu[r]; bv_r[r] = pbv[r]; }
-        __syncthreads();
-        if (k < k_last) load_layer(k + 1);
-        // q on q points [i0-1, i1] x [j0-1, j1] (mom6_coriolis_serial.F90:134-168)
-        // and KE on h points [i0, i1+1] x [j0, j1+1] (:196-203)
-        for (int t = tid; t < MW * MH; t += blockDim.x) {
-            const int li = t % MW, lj = t / MW, i = bi + li, j = bj + lj;
-            if (li < MW - 1 && lj < MH - 1 && i <= ie && j <= je) {
-                const T dvdx = (s_v[lj][li + 1] * g.dyCv) - (s_v[lj][li] * g.dyCv);
-                const T dudy = (s_u[lj + 1][li] * g.dxCu) - (s_u[lj][li] * g.dxCu);
-                const T hAu0 = (j < js) ? T(0.0) : T(0.5) * ((g.areaT * s_h[lj][li]) + (g.areaT * s_h[lj][li + 1]));
-                const T hAu1 = T(0.5) * ((g.areaT * s_h[lj + 1][li]) + (g.areaT * s_h[lj + 1][li + 1]));
-                const T hAv0 = (i < is) ? T(0.0) : T(0.5) * ((g.areaT * s_h[lj][li]) + (g.areaT * s_h[lj + 1][li]));
-                const T hAv1 = T(0.5) * ((g.areaT * s_h[lj][li + 1]) + (g.areaT * s_h[lj + 1][li + 1]));
-                const T rel_vort = (T)s_mBu[lj][li] * (dvdx - dudy) * g.IareaBu;
-                const T abs_vort = s_cor[lj] + rel_vort;
-                const T hArea_q = (hAu0 + hAu1) + (hAv0 + hAv1);
-                s_q[lj][li] = abs_vort * sdiv(g.Area_q, hArea_q + T(1.0e-20));
-            }
-            if (li >= 1 && lj >= 1) s_sxx[lj][li] = str_xx(li, lj);
-            if (li < MW - 1 && lj < MH - 1) s_sxy[lj][li] = str_xy(li, lj);
-            if (li >= 1 && lj >= 1 && i <= ie && j <= je) {
-                const T uc = s_u[lj][li], uw = s_u[lj][li - 1], vc = s_v[lj][li], vs = s_v[lj - 1][li];
-                s_KE[lj][li] = sdiv(T(0.25) * ((g.dyCu * (uc * uc) + g.dyCu * (uw * uw)) +
-                                            (g.dxCv * (vc * vc) + g.dxCv * (vs * vs))), g.areaT);
-            }
-        }
-        __syncthreads();
-#pragma unroll 1
-        for (int r = 0; r < RPT; ++r) {
-            const int i = i0 + tx, j = j0 + ty + 4 * r;
-            if (i > ie || j > je) continue;
-            const int li = i - bi, lj = j - bj;
-            const long long c = IX3(d, i, j, k);
-            if (i <= ie - 1) {
-                // diffu (:1059-1067)
-                const T h_u = T(0.5) * ((T)s_mT[lj][li] * s_h[lj][li] + (T)s_mT[lj][li + 1] * s_h[lj][li + 1]);
-                const T diffu = sdiv((g.IdxCu * ((g.dx2q * s_sxy[lj - 1][li]) - (g.dx2q * s_sxy[lj][li])) +
-                                      g.IdyCu * ((g.dy2h * s_sxx[lj][li]) - (g.dy2h * s_sxx[lj][li + 1]))) *
-                                         g.IareaCu, h_u + a.h_neglect);
-                // CAu, Sadourny (:208-216); vh from compute_transports
-                auto vh = [&](int pi, int pj) { return s_v[pj][pi] * T(0.5) * (s_h[pj][pi] + s_h[pj + 1][pi]) * g.dxCv; };
-                const T KEx = (s_KE[lj][li + 1] - s_KE[lj][li]) * g.IdxCu;
-                const T CAu = T(0.25) * ((s_q[lj][li] * (vh(li + 1, lj) + vh(li, lj))) +
-                                           (s_q[lj - 1][li] * (vh(li, lj - 1) + vh(li + 1, lj - 1)))) * g.IdxCu - KEx;
-                a.ou[c] = bu_r[r] + a.fdt * (CAu + diffu);
-            }
-            if (j <= je - 1) {
-                // diffv (:1070-1078)
-                const T h_v = T(0.5) * ((T)s_mT[lj][li] * s_h[lj][li] + (T)s_mT[lj + 1][li] * s_h[lj + 1][li]);
-                const T diffv = sdiv((g.IdyCv * ((g.dy2q * s_sxy[lj][li - 1]) - (g.dy2q * s_sxy[lj][li])) -
-                                      g.IdxCv * ((g.dx2h * s_sxx[lj][li]) - (g.dx2h * s_sxx[lj + 1][li]))) *
-                                         g.IareaCv, h_v + a.h_neglect);
-                // CAv, Sadourny (:218-226); uh from compute_transports
-                auto uh = [&](int pi, int pj) { return s_u[pj][pi] * T(0.5) * (s_h[pj][pi] + s_h[pj][pi + 1]) * g.dyCu; };
-                const T KEy = (s_KE[lj + 1][li] - s_KE[lj][li]) * g.IdyCv;
-                const T CAv = -(T(0.25) * ((s_q[lj][li - 1] * (uh(li - 1, lj) + uh(li - 1, lj + 1))) +
-                                             (s_q[lj][li] * (uh(li, lj) + uh(li, lj + 1)))) * g.IdyCv) - KEy;
-                a.ov[c] = bv_r[r] + a.fdt * (CAv + diffv);
-            }
-        }
-        __syncthreads();
+        q_s = q; vhs_s = vhs;
+        u_p = u; v_p = v; ve_p = ve; h_p = h; he_p = he; mh_p = mh; mBu_p = mBu; cor_p = cor;
+        hAu_p = r < js ? T(0.0) : hAu;
+        KE_p = KE; KEe_p = KEe; uh_p = uh; uhw_p = uhw;
     }
 }
 
-// layers k_first..k_last of split kz of nkz (the layers are independent)
-__device__ inline void layer_range(int nk, int kz, int nkz, int &k_first, int &k_last)
+// Tasks of one grid: strips (fastest), row chunks of `rows` rows, layers; one
+// wave per task, four waves per block
+struct MarchPlan {
+    int strips, chunks, rows;
+    long long tasks;
+};
+
+inline MarchPlan march_plan(const Dims &d, bool bih, int rows)
 {
-    const int per = (nk + nkz - 1) / nkz;
-    k_first = 1 + kz * per;
-    k_last = k_first + per - 1 < nk ? k_first + per - 1 : nk;
+    MarchPlan m;
+    const int out = bih ? March<double, true>::OUT : March<double, false>::OUT, nj = d.jec - d.jsc + 1;
+    m.strips = (d.iec - d.isc + out) / out;
+    m.chunks = (nj + rows - 1) / rows;
+    m.rows = (nj + m.chunks - 1) / m.chunks;   // even chunks
+    m.chunks = (nj + m.rows - 1) / m.rows;
+    m.tasks = (long long)m.strips * m.chunks * d.nk;
+    return m;
 }
 
-// grid (tiles x, tiles y, layer splits); each block walks its split's layers
-template <typename T, bool BIH, int TY>
-__global__ void __launch_bounds__(256) k_momentum(MomArgsT<T> a)
+template <typename T, bool BIH, bool SAME>
+__device__ __forceinline__ void march_task(const MomArgsT<T> &a, int strips, int chunks, int rows, int block)
 {
-    const int nxy = gridDim.x * gridDim.y;
-    const int tile = xcd_tile(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), nxy * gridDim.z);
-    const int xy = tile % nxy;
-    int k0, k1;
-    layer_range(a.d.nk, tile / nxy, gridDim.z, k0, k1);
-    if (k0 > k1) return;
-    momentum_body<T, BIH, TY>(a, xy % gridDim.x, xy / gridDim.x, k0, k1);
+    const int t = block * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int per = strips * chunks, k = t / per, q = t % per;
+    if (k >= a.d.nk) return;
+    const int ja = a.d.jsc + (q / strips) * rows, jb = ja + rows - 1 < a.d.jec ? ja + rows - 1 : a.d.jec;
+    march<T, BIH, SAME>(a, q % strips, ja, jb, k + 1);
 }
 
-// every member's tiles in one launch, renumbered per XCD over the whole batch
-template <typename T, bool BIH, int TY>
+template <typename T, bool BIH, bool SAME>
+__global__ void __launch_bounds__(256) k_momentum(MomArgsT<T> a, int strips, int chunks, int rows)
+{
+    march_task<T, BIH, SAME>(a, strips, chunks, rows, xcd_tile(blockIdx.x, gridDim.x));
+}
+
+// every member of an ensemble in one launch, renumbered per XCD over the whole
+// batch; mp.nbx, mp.nby: strips and chunks, a.march the rows of a chunk
+template <typename T, bool BIH, bool SAME>
 __global__ void __launch_bounds__(256) k_momentum_batch(const MomArgsT<T> *__restrict__ args, BatchMap mp)
 {
     int m, local;
     batch_locate(mp, xcd_tile(blockIdx.x, gridDim.x), m, local);
     const MomArgsT<T> a = args[m];
-    const int nxy = mp.nbx[m] * mp.nby[m], xy = local % nxy;
-    int k0, k1;
-    layer_range(a.d.nk, local / nxy, a.nkz, k0, k1);
-    if (k0 > k1) return;
-    momentum_body<T, BIH, TY>(a, xy % mp.nbx[m], xy / mp.nbx[m], k0, k1);
+    march_task<T, BIH, SAME>(a, mp.nbx[m], mp.nby[m], a.march, local);
 }
 
-template <typename T, bool BIH>
-void momentum_launch_ty(const MomArgsT<T> &a, int ty, dim3 grid, hipStream_t s)
+template <typename T, bool BIH, bool SAME>
+void march_launch(const MomArgsT<T> &a, const MarchPlan &m, hipStream_t s)
 {
-    if (ty == 4) k_momentum<T, BIH, 4><<<grid, 256, 0, s>>>(a);
-    else if (ty == 16) k_momentum<T, BIH, 16><<<grid, 256, 0, s>>>(a);
-    else k_momentum<T, BIH, 8><<<grid, 256, 0, s>>>(a);
+    k_momentum<T, BIH, SAME><<<(unsigned)((m.tasks + 3) / 4), 256, 0, s>>>(a, m.strips, m.chunks, m.rows);
+}
+
+// Rows of a march when the caller sets none: a long march repeats less (each
+// starts LAG + 1 rows early), a short one gives more waves.  Four waves per SIMD
+// (4096) are worth shorter marches, down to 4 rows; beyond that 32 rows serve
+// every size.  FP64, us per launch at 128 / 64 / 32 / 16 / 8 / 4 rows:
+// 140x100x40: 67 / 36 / 26 / 15 / 13 / 11; 180x180x75: 79 / 56 / 39 / 31 / 27 /
+// 30; 720x720x75: 495 / 432 / 400 / 397 / 414 / 456; 1440x1440x75: 1702 / 1513 /
+// 1504 / 1534 / 1631 / 1775.
+constexpr long long kMarchWaves = 4096;
+inline int auto_rows(long long wave_rows)
+{
+    return (int)std::min(32LL, std::max(4LL, wave_rows / kMarchWaves));
+}
+inline long long wave_rows(const Dims &d, bool bih)
+{
+    return march_plan(d, bih, 1).tasks;
 }
 
 template <typename T>
-int launch_momentum(const MomArgsT<T> &a, hipStream_t s, int ty)
+int launch_momentum(const MomArgsT<T> &a, hipStream_t s)
 {
-    const Dims &d = a.d;
-    MOM6H_REQUIRE(ty == 4 || ty == 8 || ty == 16, "momentum: tile height %d not in {4, 8, 16}", ty);
-    if (a.del2u) {
-        dim3 g2((d.iec - d.isc + 2 + 63) / 64, (d.jec - d.jsc + 2 + 3) / 4, d.nk);
-        k_del2<T><<<g2, dim3(256), 0, s>>>(a);
-        MOM6H_LAUNCH_CHECK();
+    const bool same = a.u == a.bu && a.v == a.bv;
+    const MarchPlan m = march_plan(a.d, a.bih, a.march > 0 ? a.march : auto_rows(wave_rows(a.d, a.bih)));
+    if (a.bih) {
+        if (same) march_launch<T, true, true>(a, m, s);
+        else march_launch<T, true, false>(a, m, s);
+    } else {
+        if (same) march_launch<T, false, true>(a, m, s);
+        else march_launch<T, false, false>(a, m, s);
     }
-    const int nkz = a.nkz < 1 ? 1 : (a.nkz > d.nk ? d.nk : a.nkz);
-    dim3 grid((d.iec - d.isc + 1 + MT_X - 1) / MT_X, (d.jec - d.jsc + 1 + ty - 1) / ty, nkz);
-    if (a.del2u) momentum_launch_ty<T, true>(a, ty, grid, s);
-    else momentum_launch_ty<T, false>(a, ty, grid, s);
     MOM6H_LAUNCH_CHECK();
     return MOM6H_OK;
 }
 
-template <typename T, bool BIH>
-void momentum_batch_ty(const MomArgsT<T> *d_args, const BatchMap &mp, int ty, hipStream_t s)
-{
-    const unsigned nb = (unsigned)mp.first[mp.n];
-    if (ty == 4) k_momentum_batch<T, BIH, 4><<<nb, 256, 0, s>>>(d_args, mp);
-    else if (ty == 16) k_momentum_batch<T, BIH, 16><<<nb, 256, 0, s>>>(d_args, mp);
-    else k_momentum_batch<T, BIH, 8><<<nb, 256, 0, s>>>(d_args, mp);
-}
-
 template <typename T>
-int launch_momentum_batch(const MomArgsT<T> *d_args, const MomArgsT<T> *h_args, int n, hipStream_t s, int ty)
+int plan_momentum_batch(MomArgsT<T> *h_args, int n, int rows)
 {
     MOM6H_REQUIRE(n >= 1 && n <= kMaxMembers, "momentum batch: 1..%d members", kMaxMembers);
-    MOM6H_REQUIRE(ty == 4 || ty == 8 || ty == 16, "momentum: tile height %d not in {4, 8, 16}", ty);
-    const bool bih = h_args[0].del2u != nullptr;
-    for (int m = 1; m < n; ++m)
-        MOM6H_REQUIRE((h_args[m].del2u != nullptr) == bih, "momentum batch: members differ in biharmonic");
+    if (rows <= 0) {
+        long long all = 0;
+        for (int m = 0; m < n; ++m) all += wave_rows(h_args[m].d, h_args[m].bih);
+        rows = auto_rows(all);
+    }
+    for (int m = 0; m < n; ++m) h_args[m].march = march_plan(h_args[m].d, h_args[m].bih, rows).rows;
+    return MOM6H_OK;
+}
+
+template <typename T>
+int launch_momentum_batch(const MomArgsT<T> *d_args, const MomArgsT<T> *h_args, int n, hipStream_t s)
+{
+    MOM6H_REQUIRE(n >= 1 && n <= kMaxMembers, "momentum batch: 1..%d members", kMaxMembers);
+    const bool bih = h_args[0].bih, same = h_args[0].u == h_args[0].bu && h_args[0].v == h_args[0].bv;
     BatchMap mp{};
     mp.n = n;
-    if (bih) {
-        for (int m = 0; m < n; ++m) {
-            const Dims &d = h_args[m].d;
-            mp.nbx[m] = (d.iec - d.isc + 2 + 63) / 64;
-            mp.nby[m] = (d.jec - d.jsc + 2 + 3) / 4;
-            mp.first[m + 1] = mp.first[m] + mp.nbx[m] * mp.nby[m] * d.nk;
-        }
-        k_del2_batch<T><<<(unsigned)mp.first[n], 256, 0, s>>>(d_args, mp);
-        MOM6H_LAUNCH_CHECK();
-    }
     for (int m = 0; m < n; ++m) {
-        const Dims &d = h_args[m].d;
-        MOM6H_REQUIRE(h_args[m].nkz >= 1 && h_args[m].nkz <= d.nk, "momentum batch: layer splits 1..nk");
-        mp.nbx[m] = (d.iec - d.isc + 1 + MT_X - 1) / MT_X;
-        mp.nby[m] = (d.jec - d.jsc + 1 + ty - 1) / ty;
-        mp.first[m + 1] = mp.first[m] + mp.nbx[m] * mp.nby[m] * h_args[m].nkz;
+        const MomArgsT<T> &a = h_args[m];
+        MOM6H_REQUIRE((a.bih != 0) == bih, "momentum batch: members differ in biharmonic");
+        MOM6H_REQUIRE((a.u == a.bu && a.v == a.bv) == same, "momentum batch: members differ in their base fields");
+        MOM6H_REQUIRE(a.march >= 1, "momentum batch: members have no march plan");
+        const MarchPlan p = march_plan(a.d, bih, a.march);
+        MOM6H_REQUIRE(p.rows == a.march, "momentum batch: a member's march plan is not its launch's");
+        mp.nbx[m] = p.strips;
+        mp.nby[m] = p.chunks;
+        mp.first[m + 1] = mp.first[m] + (int)((p.tasks + 3) / 4);
     }
-    if (bih) momentum_batch_ty<T, true>(d_args, mp, ty, s);
-    else momentum_batch_ty<T, false>(d_args, mp, ty, s);
+    const unsigned nb = (unsigned)mp.first[n];
+    if (bih) {
+        if (same) k_momentum_batch<T, true, true><<<nb, 256, 0, s>>>(d_args, mp);
+        else k_momentum_batch<T, true, false><<<nb, 256, 0, s>>>(d_args, mp);
+    } else {
+        if (same) k_momentum_batch<T, false, true><<<nb, 256, 0, s>>>(d_args, mp);
+        else k_momentum_batch<T, false, false><<<nb, 256, 0, s>>>(d_args, mp);
+    }
     MOM6H_LAUNCH_CHECK();
     return MOM6H_OK;
 }
 
-template int launch_momentum<double>(const MomArgsT<double> &, hipStream_t, int);
-template int launch_momentum<float>(const MomArgsT<float> &, hipStream_t, int);
-template int launch_momentum_batch<double>(const MomArgsT<double> *, const MomArgsT<double> *, int, hipStream_t, int);
-template int launch_momentum_batch<float>(const MomArgsT<float> *, const MomArgsT<float> *, int, hipStream_t, int);
+template int launch_momentum<double>(const MomArgsT<double> &, hipStream_t);
+template int launch_momentum<float>(const MomArgsT<float> &, hipStream_t);
+template int plan_momentum_batch<double>(MomArgsT<double> *, int, int);
+template int plan_momentum_batch<float>(MomArgsT<float> *, int, int);
+template int launch_momentum_batch<double>(const MomArgsT<double> *, const MomArgsT<double> *, int, hipStream_t);
+template int launch_momentum_batch<float>(const MomArgsT<float> *, const MomArgsT<float> *, int, hipStream_t);
 
 }  // namespace mom6h

@@ -35,12 +35,13 @@ struct mom6h_model {
     Halo halo;
     bool prepared = false;
     int use_graph = 0, profile = 0;
-    int momentum_tile = 8;   // rows of the fused momentum tile (4, 8 or 16)
-    int momentum_splits = 1; // blocks per tile over the layers (1..nk)
+    // options of the fused momentum stencil's march (march_rows); 0: not set
+    int momentum_tile = 0, momentum_splits = 0;
     int serialize = 0;       // barotropic chain on the 3D stream (per-kernel timing without overlap)
     int fused = 1;           // fused momentum stencil (module-by-module when 0)
     bool uniform = false;    // every metric array constant (fused kernels allowed)
-    bool fused_rows = false; // masks 0/1 and Coriolis constant along rows (the fused stencil's staging)
+    bool fused_rows = false; // masks 0/1 and Coriolis constant along rows (what the fused stencil reads)
+    unsigned char *mask_bits = nullptr;   // those masks, one byte per point (MomArgsT::mask)
     UMetrics ug{};
     hipStream_t s0 = nullptr, s1 = nullptr;
     hipEvent_t e_start = nullptr, e_bt = nullptr;
@@ -57,9 +58,7 @@ struct mom6h_model {
     struct {
         float *u, *v, *h, *h0, *htmp, *uh, *vh, *up, *vp, *u_cor, *bt_h_u;
         float *hx, *v_cor, *bt_h_v;   // meridional pass
-        float *del2u, *del2v;         // biharmonic scratch of the fused stencil
     } f{};
-    double *del2u = nullptr, *del2v = nullptr;   // biharmonic scratch of the fused stencil (FP64)
     std::vector<Field> fields;
     // host copies of the uniform metrics (init_ocean_grid)
     std::vector<double> IareaT, areaT, dxT, dyT, IdxT, IdyT, dxCu, dyCu, dy_Cu, IdxCu, IdyCu;

@@ -201,9 +201,9 @@ int momentum_phase(mom6h_model *m, const double *u, const double *v, const doubl
         MomArgs a;
         a.d = d; a.g = m->ug; a.Kh = m->c.Kh; a.h_neglect = 1.0e-3; a.fdt = fdt; a.no_slip = m->c.no_slip;
         a.u = u; a.v = v; a.h = h; a.bu = m->u; a.bv = m->v; a.ou = ou; a.ov = ov;
-        a.mask2dT = m->mask2dT; a.mask2dBu = m->mask2dBu; a.CoriolisBu = m->CoriolisBu;
-        a.Ah = m->c.Ah; a.del2u = m->del2u; a.del2v = m->del2v; a.nkz = m->momentum_splits;
-        return launch_momentum(a, s0, m->momentum_tile);
+        a.mask = m->mask_bits; a.CoriolisBu = m->CoriolisBu;
+        a.Ah = m->c.Ah; a.bih = m->c.biharmonic; a.march = march_rows(m->momentum_tile, m->momentum_splits);
+        return launch_momentum(a, s0);
     }
     { StageTimer t(m, ST_TRANSPORTS, s0);
       RC(mom6h_transports(d.isd, d.ied, d.jsd, d.jed, nk, u, v, h, m->cor->dyCu, m->cor->dxCv, m->uh, m->vh, s0)); }
@@ -243,9 +243,9 @@ int momentum_phase_f32(mom6h_model *m, const float *u, const float *v, const flo
     a.d = m->d; a.g = m->ug; a.Kh = (float)m->c.Kh; a.h_neglect = 1.0e-3f; a.fdt = (float)fdt;
     a.no_slip = m->c.no_slip;
     a.u = u; a.v = v; a.h = h; a.bu = m->f.u; a.bv = m->f.v; a.ou = ou; a.ov = ov;
-    a.mask2dT = m->mask2dT; a.mask2dBu = m->mask2dBu; a.CoriolisBu = m->CoriolisBu;
-    a.Ah = (float)m->c.Ah; a.del2u = m->f.del2u; a.del2v = m->f.del2v; a.nkz = m->momentum_splits;
-    return launch_momentum(a, m->s0, m->momentum_tile);
+    a.mask = m->mask_bits; a.CoriolisBu = m->CoriolisBu;
+    a.Ah = (float)m->c.Ah; a.bih = m->c.biharmonic; a.march = march_rows(m->momentum_tile, m->momentum_splits);
+    return launch_momentum(a, m->s0);
 }
 
 int continuity_phase_f32(mom6h_model *m, const float *u, const float *v, const float *hin, float *hout, double dt)
@@ -396,15 +396,6 @@ int mom6h_model_create(mom6h_model **out, const mom6h_config *c)
         if (!m->mixed) m->fields.push_back(Field{names[6], (void **)&bt.h_u, n3, 8, false});
         else rc = add_field(m, names[6], h3_f32, n3, true);
     };
-    if (!rc && c->biharmonic) {   // zero outside the Del2 ranges, for good
-        if (!m->mixed) {
-            rc = add_field(m, "del2u", &m->del2u, n3, true);
-            rc = rc ? rc : add_field(m, "del2v", &m->del2v, n3, true);
-        } else {
-            rc = add_field(m, "del2u", &m->f.del2u, n3, true);
-            rc = rc ? rc : add_field(m, "del2v", &m->f.del2v, n3, true);
-        }
-    }
     static const char *const bt_u_names[7] = {"FA_u_EE", "FA_u_E0", "FA_u_W0", "FA_u_WW", "uBT_WW", "uBT_EE", "BT_h_u"};
     static const char *const bt_v_names[7] = {"FA_v_NN", "FA_v_N0", "FA_v_S0", "FA_v_SS", "vBT_SS", "vBT_NN", "BT_h_v"};
     bt_fields(m->bt, bt_u_names, &m->f.bt_h_u);
@@ -641,6 +632,12 @@ int mom6h_model_prepare(mom6h_model *m)
         m->uniform = ok;
         m->fused_rows = binary_mask(mT.data(), n) && binary_mask(mBu.data(), n) &&
                         rows_uniform(fq.data(), (size_t)d.n1, (size_t)d.n2);
+        if (m->fused_rows) {
+            std::vector<unsigned char> bits(n);
+            for (size_t q = 0; q < n; ++q) bits[q] = (unsigned char)((mT[q] != 0.0 ? 1 : 0) | (mBu[q] != 0.0 ? 2 : 0));
+            RC(dev_alloc_bytes((void **)&m->mask_bits, n, false));
+            MOM6H_CHECK(hipMemcpy(m->mask_bits, bits.data(), n, hipMemcpyHostToDevice));
+        }
     }
     MOM6H_REQUIRE(!m->mixed || (m->uniform && m->fused_rows),
                   "mom6h_model_prepare: the mixed-precision form needs a grid with uniform metrics, 0/1 masks "
@@ -910,13 +907,14 @@ int mom6h_model_autotune(mom6h_model *m, int reps, char *report, int nbytes)
     hipEvent_t a, b;
     MOM6H_CHECK(hipEventCreate(&a));
     MOM6H_CHECK(hipEventCreate(&b));
-    const int rows[3] = {4, 8, 16}, splits[4] = {1, 2, 4, 8};
+    // marches of 128, 64, 32, 16, 8 and 4 rows
+    const int tiles[6] = {16, 8, 4, 4, 4, 4}, splits[6] = {1, 1, 1, 2, 4, 8};
     float best = 0.f;
     int pick = 8, pick_s = 1, rc = 0;
-    std::string rep = "momentum tile rows x layer splits (ms):";
-    for (int q = 0; q < 12 && !rc; ++q) {
-        m->momentum_tile = rows[q / 4];
-        m->momentum_splits = splits[q % 4] < m->c.nk ? splits[q % 4] : m->c.nk;
+    std::string rep = "momentum march rows (ms):";
+    for (int q = 0; q < 6 && !rc; ++q) {
+        m->momentum_tile = tiles[q];
+        m->momentum_splits = splits[q];
         rc = launch();   // warm
         if (!rc && hipEventRecord(a, m->s0) != hipSuccess) rc = set_error(MOM6H_ESTATE, "event record failed");
         for (int r = 0; r < reps && !rc; ++r) rc = launch();
@@ -926,7 +924,7 @@ int mom6h_model_autotune(mom6h_model *m, int reps, char *report, int nbytes)
         if (!rc && hipEventElapsedTime(&ms, a, b) != hipSuccess) rc = set_error(MOM6H_ESTATE, "event timing failed");
         ms /= (float)(reps > 0 ? reps : 1);
         char buf[64];
-        snprintf(buf, sizeof(buf), " %dx%d %.4f;", m->momentum_tile, m->momentum_splits, ms);
+        snprintf(buf, sizeof(buf), " %d %.4f;", march_rows(m->momentum_tile, m->momentum_splits), ms);
         rep += buf;
         if (q == 0 || ms < best) {
             best = ms;
@@ -941,7 +939,7 @@ int mom6h_model_autotune(mom6h_model *m, int reps, char *report, int nbytes)
     m->momentum_splits = pick_s;
     drop_graphs(m);
     if (rc) return rc;
-    rep += " chosen " + std::to_string(pick) + "x" + std::to_string(pick_s);
+    rep += " chosen " + std::to_string(march_rows(pick, pick_s));
     if (report && nbytes > 0) snprintf(report, (size_t)nbytes, "%s", rep.c_str());
     return MOM6H_OK;
 }
@@ -961,6 +959,7 @@ int mom6h_model_destroy(mom6h_model *m)
     mom6h_bt_cont_free(&m->bt);
     mom6h_bt_cont_free(&m->bt_v);
     for (double *p : {m->diag_work2d, m->diag_ke, m->diag_mass, m->diag_red, m->diag_out}) dev_free(p);
+    if (m->mask_bits) (void)hipFree(m->mask_bits);
     drop_graphs(m);
     if (m->e_start) (void)hipEventDestroy(m->e_start);
     if (m->e_bt) (void)hipEventDestroy(m->e_bt);

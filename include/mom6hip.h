@@ -318,9 +318,10 @@ int mom6h_model_step(mom6h_model *m, int niter);
 int mom6h_model_synchronize(mom6h_model *m);
 /* Options: "graph" (1 = capture one step as two hipGraphs, the 3D chain on
  * the model's first stream and the barotropic chain on its second, and replay
- * them per step, joined once per call as the eager path is; default 0), "momentum_tile" (rows of the fused momentum
- * tile: 4, 8 or 16; default 8), "momentum_splits" (blocks per tile sharing its
- * layers, 1..nk; default 1), "bt_tile" (rows of the barotropic substep tile,
+ * them per step, joined once per call as the eager path is; default 0), "momentum_tile" (4, 8 or 16;
+ * default 8) and "momentum_splits" (1..nk; default 1): a wave of the fused
+ * momentum stencil marches through 8*tile/splits rows (at least 4), or through
+ * a number chosen from the grid while neither is set, "bt_tile" (rows of the barotropic substep tile,
  * 4, 8 or 16; after prepare; default 4), "bt_substeps" (barotropic substeps per
  * launch between the first and the last of a call: 1 = one launch per substep,
  * up to 5 = the blocked kernel; after prepare; default 5), "bt_rows" (1 = the
@@ -338,9 +339,9 @@ int mom6h_model_set_option(mom6h_model *m, const char *key, double value);
 int mom6h_model_stage_times(mom6h_model *m, double *ms, int max_stages, char *names, int nbytes);
 int mom6h_model_main_stream(mom6h_model *m, void **stream);
 /* Times the fused momentum stencil (reps launches of the predictor's, whose
- * outputs every step rewrites) for each launch shape -- tile rows 4, 8, 16 x
- * layer splits 1, 2, 4, 8 -- keeps the fastest as options "momentum_tile" and
- * "momentum_splits" and writes the timings into report. */
+ * outputs every step rewrites) for marches of 4 to 128 rows, keeps the fastest
+ * as options "momentum_tile" and "momentum_splits" and writes the timings into
+ * report. */
 int mom6h_model_autotune(mom6h_model *m, int reps, char *report, int nbytes);
 /* With option "diag" = 1 (FP64 form) every step posts the predictor's
  * diffu_sum and diffv_sum statistics; this call adds KE and mass of the
@@ -367,13 +368,12 @@ int mom6h_ensemble_prepare(mom6h_ensemble *e);
 int mom6h_ensemble_step(mom6h_ensemble *e, int niter);
 int mom6h_ensemble_synchronize(mom6h_ensemble *e);
 /* Options: "graph" (1 = capture one step, replay it per step), "momentum_tile"
- * (rows of the fused momentum tile: 4, 8 or 16; default 8), "momentum_splits"
- * (blocks per tile sharing its layers; after prepare; default 1), "bt_tile" (4, 8 or 16),
+ * (4, 8 or 16; default 8) and "momentum_splits" (after prepare; default 1): the
+ * rows of the momentum march as for the model, "bt_tile" (4, 8 or 16),
  * "bt_substeps" (barotropic substeps per blocked launch, 1-5; default 5). */
 int mom6h_ensemble_set_option(mom6h_ensemble *e, const char *key, double value);
-/* Times the fused momentum launch of the ensemble (reps launches) for every
- * launch shape (tile rows x layer splits), keeps the fastest and writes the
- * timings into report.  It runs
+/* Times the fused momentum launch of the ensemble (reps launches) for marches
+ * of 4 to 128 rows, keeps the fastest and writes the timings into report.  It runs
  * only the predictor's momentum stencil, whose outputs every step rewrites,
  * so the state is unchanged. */
 int mom6h_ensemble_autotune(mom6h_ensemble *e, int reps, char *report, int nbytes);
