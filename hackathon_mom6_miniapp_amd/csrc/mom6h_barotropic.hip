@@ -51,7 +51,8 @@ __global__ void k_bt_copy_in(Dims d, const double *eta_in, const double *ubt_in,
     }
 }
 
-// Output tile BT_TX x BT_TY (BT_TY = 4, 8 or 16 rows: the launch's choice),
+// The one-substep form, for grids whose coefficients vary and for single
+// substeps.  Output tile BT_TX x BT_TY (BT_TY = 4, 8 or 16 rows: the launch's choice),
 // 256 threads, BT_TY/4 outputs per thread.  Three LDS arrays hold eta, ubt
 // and vbt of the staged region and are updated in place: eta becomes the
 // predicted eta (each point reads only its own eta), each velocity update
@@ -257,323 +258,362 @@ __global__ void __launch_bounds__(256) k_bt_substep(BT p, M m, BTStep st)
 }
 
 // ---------------------------------------------------------------------------
-// Several substeps per launch (temporal blocking) for the substeps between the
-// first and the last of a call, on uniform grids.  The reference refills the
-// periodic halos after every substep but the last, so from the second substep
-// on a halo cell always holds the value of its periodic image: the substeps in
-// between run on a torus.  A block therefore stages the region its output tile
-// needs for ns substeps -- radius 2 to the west/south and 1 to the east/north
-// per substep -- and maps every staged position to its canonical cell (the
-// periodic image inside the compute domain; a position outside the arrays in
-// a wall direction holds zero and is never updated).  Each position is updated
-// as its canonical cell, with the state, Datv and f4 of the neighbouring
-// staged positions (the refilled images; Datv's halo rows equal their images,
-// which the host checks before it uses this kernel).  The region that holds
-// valid values shrinks by the stencil radius each substep and is the output
-// tile after the last.  The output tile is written whole, halo positions
-// included (their images), so the state after the launch is what the reference
-// holds after its refill.  The first substep of a call (which reads the halos
-// as stored) and the last (after which nothing is refilled) stay with the
-// one-substep kernel.
+// Several substeps per launch (temporal blocking), on uniform grids.  The
+// reference refills the periodic halos after every substep but the last, so
+// from the second substep on a halo cell always holds the value of its periodic
+// image: the substeps run on a torus.  A block therefore stages the region its
+// output tile needs for ns substeps -- radius 2 to the west/south and 1 to the
+// east/north per substep -- and maps every staged position to its canonical
+// cell (the periodic image inside the compute domain; a position outside the
+// arrays in a wall direction holds zero and is never updated).  Each position
+// is updated as its canonical cell, with the state, Datv and f4 of the
+// neighbouring staged positions (the refilled images; Datv's halo rows equal
+// their images, which the host checks before it uses this kernel).  The region
+// that holds valid values shrinks by the stencil radius each substep and is the
+// output tile after the last.
+//   The first substep of a call on a periodic grid reads the halos as the
+// caller stored them: a launch of its own, with every position its own cell
+// (wrap = 0; on other grids every launch is such a one).  The last substep has
+// no refill after it: its range tests take the positions themselves, so that
+// the halo positions keep what they held.  In between, the halo positions of
+// the state arrays in a periodic direction are written but never read.
 struct BTMulti {
     const double *eta_o, *ubt_o, *vbt_o;   // state before substep n0
     double *eta_n, *ubt_n, *vbt_n;         // state after substep n0 + ns - 1
-    int n0, ns;                            // first substep, number of substeps (1 .. TS)
+    double *out_u, *out_v, *out_eta;       // the call's outputs (written after substep nstep)
+    int n0, ns, wrap;                      // first substep, number of substeps, positions are canonical cells
 };
 
-// M(w) = ceil(2^20 / w) for widths w < 256, so that t / w = (t * M(w)) >> 20
-// exactly for t < 4096; read from constant memory with a uniform index (a
-// scalar load) instead of an integer division per call.
-struct MulShift {
-    unsigned v[256];
-};
-constexpr MulShift make_mulshift()
-{
-    MulShift t{};
-    for (unsigned w = 1; w < 256; ++w) t.v[w] = ((1u << 20) + w - 1) / w;
-    return t;
-}
-__constant__ MulShift kMulShift = make_mulshift();
+// The layout: a block stages kBTW columns x kBTH rows (64 x 64), lane l of a wave
+// holding column x0 + l and wave w the R rows from w*R on, all in registers: e,
+// u, v and the running averages.  i neighbours come by DPP wave shifts, j
+// neighbours from the wave's own rows; of the waves above and below a wave keeps
+// copies of the rows its updates reach (v two rows south; e, u, v one row south
+// and one north) and updates those it needs itself, so that the waves meet once
+// per substep: each leaves its outer rows in LDS (double buffered), one barrier.
+// Every position is updated in every substep, in the same place: the valid
+// region shrinks by the stencil radius, and what the rim holds then is never
+// read by a valid point.  ts substeps leave a tile of 64 - 3 ts in each
+// direction.
+//
+// What bounds it: VALU issue, 65 instructions per position and substep (76 in
+// waves that need the range selects), and about 8 us per launch for the launch
+// and the state's way in and out.  At 720x720 a launch of 6 substeps takes 26.7
+// us and a call of 100 substeps 413 us.  The form before kept the state in LDS,
+// mapped threads to the positions of a shrinking rectangle in each of four
+// phases (half of its instructions) and met at four barriers per substep: 36.6
+// us per 5 substeps, and a copy-in and two one-substep launches per call, 707 us.
+constexpr int kBTW = 64, kBTH = 64, kBTRows = 8, kBTWaves = kBTH / kBTRows;
 
-// Calls f(x0 + t % w, y0 + t / w) for the positions t < w*h of a rectangle of
-// width w >= 8 and at most NT*MAXI positions (<= 4096: t / w as an exact
-// multiply-shift), t spread over the block's NT threads.  The products fit in
-// 24-bit operands (t < 2^12, M <= 2^17, q < 2^9, w < 2^12), so they take the
-// full-rate 24-bit multiply rather than the quarter-rate 32-bit one.
-template <int NT, int MAXI, typename F>
-__device__ __forceinline__ void rect_each(int x0, int x1, int y0, int y1, int tid, F &&f)
+// the value of the lane to the west / east (DPP wave shift; 0 beyond the wave)
+template <int CTRL>
+__device__ __forceinline__ double bt_dpp(double x)
 {
-    static_assert(NT * MAXI <= 4096, "positions beyond the exact multiply-shift range");
-    const unsigned w = (unsigned)(x1 - x0 + 1), n = w * (unsigned)(y1 - y0 + 1);
-    const unsigned M = kMulShift.v[w];   // 8 <= w < 256
-#pragma unroll
-    for (int r = 0; r < MAXI; ++r) {
-        const unsigned t = (unsigned)tid + (unsigned)NT * r;
-        if (t < n) {
-            const unsigned q = __umul24(t, M) >> 20;
-            const int li = x0 + (int)(t - __umul24(q, w)), lj = y0 + (int)q;
-            // staged positions: small and non-negative, so that their LDS
-            // offsets take 24-bit multiplies
-            __builtin_assume(li >= 0 && li < 4096 && lj >= 0 && lj < 4096);
-            f(li, lj);
-        }
-    }
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xf, 0xf, true),
+                            __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xf, 0xf, true));
 }
+__device__ __forceinline__ double bt_west(double x) { return bt_dpp<0x138>(x); }
+__device__ __forceinline__ double bt_east(double x) { return bt_dpp<0x130>(x); }
 
 // ROW: Datv and f4 constant along each row of the compute domain (walls close
-// whole rows, f depends on latitude only; the host checks it): one staged value
-// per row, and the predicted eta goes to an array of its own (no barrier
-// between reading the old values and the predictor).
-template <int NT, int TX, int TY, int TS, bool ROW>
-__device__ __forceinline__ void bt_multi_body(const BT &p, const BTUniform &m, const BTMulti &st, int tile_x,
-                                              int tile_y)
+// whole rows, f depends on latitude only; the host checks it): one scalar per
+// row instead of one value per position.
+template <bool ROW>
+__device__ __forceinline__ void bt_multi_body(const BT &p, const BTUniform &m, const BTMulti &st, int tile_x, int tile_y)
 {
-    constexpr int RW = TX + 3 * TS, RH = TY + 3 * TS;   // staged region (LDS)
-    constexpr int NOUT = (TX * TY + NT - 1) / NT;       // output points per thread (t < TX*TY)
-    constexpr int NR = ((TX + 3 * (TS - 1)) * (TY + 3 * (TS - 1)) + NT - 1) / NT;          // valid region
-    constexpr int NP = ((TX + 3 * (TS - 1) + 2) * (TY + 3 * (TS - 1) + 2) + NT - 1) / NT;  // update regions
-    static_assert(RW * RH <= 4096 && RW + 2 < 256, "staged region too large for the multiply-shift index");
-    __shared__ double s_e[RH][RW], s_u[RH][RW], s_v[RH][RW];
-    __shared__ double s_dv[RH][ROW ? 1 : RW], s_f4[RH][ROW ? 1 : RW];
-    __shared__ double s_ep[ROW ? RH : 1][ROW ? RW : 1];   // ROW: the predicted eta
-    __shared__ int s_cx[RW], s_cy[RH];
-    // range tests of each staged column (x) and row (y) on its canonical
-    // index, one bit each, formed once per launch: bit 0 inside the compute
-    // domain (is..ie / js..je), bit 1 inside it but for the last face
-    // (..ie-1 / ..je-1: the u / v update ranges), bit 2 inside the u / v
-    // transport range (iu0..iu1 / jv0..jv1), bit 3 the same for the index - 1
-    __shared__ int s_fx[RW], s_fy[RH];
-    auto DV = [&](int lj, int li) -> double { return s_dv[lj][ROW ? 0 : li]; };
-    auto F4 = [&](int lj, int li) -> double { return s_f4[lj][ROW ? 0 : li]; };
-    auto EP = [&](int lj, int li) -> double { return ROW ? s_ep[ROW ? lj : 0][ROW ? li : 0] : s_e[lj][li]; };
+    constexpr int R = kBTRows, NW = kBTWaves;
+    // outer rows of each wave: row 0 (e, u, v), row R-1 (e, u, v), row R-2 (v)
+    __shared__ double s_out[2][NW][7][kBTW];
+    // ROW: Datv, f4 and the transport's Datv (0 outside its range) by row, from row -2 of wave 0
+    __shared__ double s_dv[ROW ? kBTH + 3 : 1], s_f4[ROW ? kBTH + 3 : 1], s_dt[ROW ? kBTH + 3 : 1];
     const Dims &d = p.d;
     const int is = d.isc, ie = d.iec, js = d.jsc, je = d.jec;
-    const int i0 = d.isd + tile_x * TX, j0 = d.jsd + tile_y * TY;
-    const int bi = i0 - 2 * TS, bj = j0 - 2 * TS;   // LDS origin
-    const int tid = threadIdx.x;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int ts = st.ns, TX = kBTW - 3 * ts, TY = kBTH - 3 * ts;
+    const bool wx = st.wrap && p.px, wy = st.wrap && p.py;
+    const int x = d.isd + tile_x * TX - 2 * ts + lane;           // this lane's column
+    const int y0 = d.jsd + tile_y * TY - 2 * ts + w * R;         // this wave's first row
     const double dtbt = p.dtbt;
     const int iu0 = p.extended ? is - 1 : is, iu1 = p.extended ? ie : ie - 1;
     const int jv0 = p.extended ? js - 1 : js, jv1 = p.extended ? je : je - 1;
-    auto flags = [](int c, int lo, int hi, int t0, int t1) -> int {
-        return ((c >= lo && c <= hi) ? 1 : 0) | ((c >= lo && c <= hi - 1) ? 2 : 0) |
-               ((c >= t0 && c <= t1) ? 4 : 0) | ((c - 1 >= t0 && c - 1 <= t1) ? 8 : 0);
-    };
-    // canonical index of each staged column and row, and its range bits
-    for (int t = tid; t < RW + RH; t += NT) {
-        if (t < RW) {
-            const int x = bi + t, P = ie - is + 1;
-            const int c = p.px ? is + ((x - is) % P + P) % P : x;
-            s_cx[t] = c;
-            s_fx[t] = flags(c, is, ie, iu0, iu1);
-        } else {
-            const int y = bj + (t - RW), Q = je - js + 1;
-            const int c = p.py ? js + ((y - js) % Q + Q) % Q : y;
-            s_cy[t - RW] = c;
-            s_fy[t - RW] = flags(c, js, je, jv0, jv1);
-        }
-    }
-    __syncthreads();
-    rect_each<NT, (RW * RH + NT - 1) / NT>(0, RW - 1, 0, RH - 1, tid, [&](int li, int lj) {
-        const int i = s_cx[li], j = s_cy[lj];
-        double e = 0.0, uu = 0.0, vv = 0.0, dv = 0.0, f4 = 0.0;
-        if (i >= d.isd && i <= d.ied && j >= d.jsd && j <= d.jed) {
-            const long long c = IX2(d, i, j);
-            e = st.eta_o[c]; uu = st.ubt_o[c]; vv = st.vbt_o[c];
-            if (!ROW) { dv = m.Datv[c]; f4 = m.f4[c]; }
-        }
-        s_e[lj][li] = e; s_u[lj][li] = uu; s_v[lj][li] = vv;
-        if (!ROW) { s_dv[lj][ROW ? 0 : li] = dv; s_f4[lj][ROW ? 0 : li] = f4; }
-    });
+    // the canonical column, and whether it lies in the compute domain, in the u
+    // update range (is..ie-1) and in the u transport range
+    const int P = ie - is + 1, Q = je - js + 1;
+    const int ci = wx ? is + ((x - is) % P + P) % P : x;
+    const bool col = ci >= d.isd && ci <= d.ied;
+    bool x_in = ci >= is && ci <= ie, x_u = ci >= is && ci <= ie - 1;
+    const bool x_t = ci >= iu0 && ci <= iu1;
+    const double Datu_t = x_t ? m.Datu : 0.0;   // the transport's Datu
+    // the same for the rows -2..R (bit r + 2), wave-uniform
+    unsigned y_in = 0, y_v = 0, y_t = 0;
+    double e[R + 3], u[R + 3], v[R + 3];                          // index r + 2: rows -2..R
+    double dvp[ROW ? 1 : R + 3], f4p[ROW ? 1 : R + 3];            // !ROW: per position
     if (ROW) {
-        for (int t = tid; t < RH; t += NT) {
-            const int j = s_cy[t];
-            const bool in = j >= d.jsd && j <= d.jed;
-            s_dv[t][0] = in ? m.Datv_row[j - d.jsd] : 0.0;
-            s_f4[t][0] = in ? m.f4_row[j - d.jsd] : 0.0;
+        for (int t = threadIdx.x; t < kBTH + 3; t += 64 * NW) {
+            const int y = d.jsd + tile_y * TY - 2 * ts + t - 2, cj = wy ? js + ((y - js) % Q + Q) % Q : y;
+            const bool row = cj >= d.jsd && cj <= d.jed;
+            const double dv = row ? m.Datv_row[cj - d.jsd] : 0.0;
+            s_dv[t] = dv;
+            s_dt[t] = cj >= jv0 && cj <= jv1 ? dv : 0.0;
+            s_f4[t] = row ? m.f4_row[cj - d.jsd] : 0.0;
         }
     }
-    // running averages of this thread's output points (the array positions)
-    double ua_r[NOUT], va_r[NOUT];
 #pragma unroll
-    for (int r = 0; r < NOUT; ++r) {
-        const int t = tid + NT * r;
-        const int i = i0 + t % TX, j = j0 + t / TX;
-        ua_r[r] = 0.0; va_r[r] = 0.0;
-        if (t < TX * TY && i <= d.ied && j <= d.jed) {
-            ua_r[r] = p.ubt_av[IX2(d, i, j)];
-            va_r[r] = p.vbt_av[IX2(d, i, j)];
+    for (int q = 0; q < R + 3; ++q) {
+        const int y = y0 + q - 2;
+        const int cj = wy ? js + ((y - js) % Q + Q) % Q : y;
+        const bool row = cj >= d.jsd && cj <= d.jed;
+        y_in |= (cj >= js && cj <= je ? 1u : 0u) << q;
+        y_v |= (cj >= js && cj <= je - 1 ? 1u : 0u) << q;
+        y_t |= (cj >= jv0 && cj <= jv1 ? 1u : 0u) << q;
+        e[q] = u[q] = v[q] = 0.0;
+        if (!ROW) dvp[ROW ? 0 : q] = f4p[ROW ? 0 : q] = 0.0;
+        if (row && col) {
+            const long long c = IX2(d, ci, cj);
+            if (q >= 1) { e[q] = st.eta_o[c]; u[q] = st.ubt_o[c]; }
+            v[q] = st.vbt_o[c];
+            if (!ROW) { dvp[ROW ? 0 : q] = m.Datv[c]; f4p[ROW ? 0 : q] = m.f4[c]; }
         }
     }
-    __syncthreads();
-    // pressure forces and the velocity updates (:234-260) of the canonical
-    // cell (i, j) at staged position (li, lj); the coefficients are uniform
-    // but for Datv and f4
-    auto new_v = [&](int lj, int li) -> double {
-        double vn = s_v[lj][li];
-        if ((s_fx[li] & 1) && (s_fy[lj] & 2)) {   // is..ie x js..je-1
-            const double f4 = F4(lj, li);
-            const double Cor = -1.0 * (((f4 * s_u[lj][li - 1]) + (f4 * s_u[lj + 1][li])) +
-                                       ((f4 * s_u[lj][li]) + (f4 * s_u[lj + 1][li - 1])));
-            const double pf = ((EP(lj, li) * m.gtot) - (EP(lj + 1, li) * m.gtot)) * p.dgeo_de * m.IdyCv;
-            vn = m.bt_rem_v * (vn + dtbt * (Cor + pf));
+    // every position this wave updates inside every range: no selects needed
+    constexpr unsigned kRows = (1u << (R + 3)) - 2;                // rows -1..R
+    auto all_in = [&]() { return (y_in & y_v & kRows) == kRows && (ROW || (y_t & kRows) == kRows) && __all(x_u); };
+    bool inner = all_in();
+    // running averages of this wave's output positions (array positions)
+    const bool out_x = lane >= 2 * ts && lane < 2 * ts + TX && x <= d.ied;
+    const int out0 = 2 * ts - w * R, out1 = out0 + TY;             // rows [out0, out1) of this wave
+    auto out_row = [&](int r) { return r >= out0 && r < out1 && y0 + r <= d.jed; };
+    const bool first = st.n0 == 1, last = st.n0 + st.ns - 1 == p.nstep;
+    double ua[R], va[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        ua[r] = va[r] = 0.0;
+        if (!first && out_x && out_row(r)) {
+            ua[r] = p.ubt_av[IX2(d, x, y0 + r)];
+            va[r] = p.vbt_av[IX2(d, x, y0 + r)];
         }
-        return vn;
-    };
-    auto new_u = [&](int lj, int li) -> double {
-        double un = s_u[lj][li];
-        if ((s_fx[li] & 2) && (s_fy[lj] & 1)) {   // is..ie-1 x js..je
-            const double f4 = F4(lj, li);
-            const double Cor = (((f4 * s_v[lj][li + 1]) + (f4 * s_v[lj - 1][li])) +
-                                ((f4 * s_v[lj][li]) + (f4 * s_v[lj - 1][li + 1])));
-            const double pf = ((EP(lj, li) * m.gtot) - (EP(lj, li + 1) * m.gtot)) * p.dgeo_de * m.IdxCu;
-            un = m.bt_rem_u * (un + dtbt * (Cor + pf));
-        }
-        return un;
-    };
+    }
+    const bool av_u = x >= is && x <= ie - 1, av_v = x >= is && x <= ie;
     const double trans_wt1 = 1.0 + p.bebt, trans_wt2 = -p.bebt;
     const double inv_nstep = 1.0 / (double)p.nstep;
-    for (int s = 0; s < st.ns; ++s) {
-        const int n = st.n0 + s;
-        const int k = st.ns - 1 - s;   // substeps of this launch after this one
-        // R = [A0, A1] x [B0, B1]: the positions this substep leaves valid
-        const int A0 = 2 * TS - 2 * k, A1 = 2 * TS + TX - 1 + k;
-        const int B0 = 2 * TS - 2 * k, B1 = 2 * TS + TY - 1 + k;
-        const bool v_first = ((n + p.first_direction) % 2) == 1;
-        // this thread's points of R: t = tid + NT r, (A0 + t % rw, B0 + t / rw)
-        const unsigned rw = (unsigned)(A1 - A0 + 1), nR = rw * (unsigned)(B1 - B0 + 1);
-        const unsigned Mr = kMulShift.v[rw];
-        auto r_pos = [&](int r, int &li, int &lj) -> bool {
-            const unsigned t = (unsigned)tid + (unsigned)NT * r, q = __umul24(t, Mr) >> 20;
-            li = A0 + (int)(t - __umul24(q, rw));
-            lj = B0 + (int)q;
-            __builtin_assume(li >= 0 && li < 4096 && lj >= 0 && lj < 4096);
-            return t < nR;
+    const double dtI = dtbt * m.IareaT;
+
+    // dgeo_de is 1 (barotropic_init), so folding it into the metric is exact
+    const double idx = p.dgeo_de * m.IdxCu, idy = p.dgeo_de * m.IdyCv;
+    if (ROW) __syncthreads();   // s_dv, s_f4
+
+    // one substep of this wave's rows; q = r + 2 throughout.  INNER: without
+    // the range selects.  VF: v before u.
+    auto substep = [&](auto inner_c, auto vf_c) __attribute__((always_inline)) {
+        constexpr bool INNER = decltype(inner_c)::value, VF = decltype(vf_c)::value;
+        auto DV = [&](int q) __attribute__((always_inline)) -> double { return ROW ? s_dv[w * R + q] : dvp[ROW ? 0 : q]; };
+        auto F4 = [&](int q) __attribute__((always_inline)) -> double { return ROW ? s_f4[w * R + q] : f4p[ROW ? 0 : q]; };
+        // a value on its range, the old one elsewhere: a select, not a branch
+        // around the value (the empty asm keeps it so)
+        auto pick = [&](bool lane_ok, unsigned rows, int q, double val, double old) __attribute__((always_inline)) -> double {
+            if (INNER) return val;
+            asm("" : "+v"(val));
+            return lane_ok && ((rows >> q) & 1u) ? val : old;
         };
-        // old values the transports of these points need
-        double e_old[NR], u_old[NR], uw_old[NR], v_old[NR], vs_old[NR];
+        double dv_s = DV(0) * v[0];            // Datv*v of the row below
+        // eta predictor (:224-231) of row r (its west u given), times gtot
+        auto predict = [&](int q, double uw) __attribute__((always_inline)) -> double {
+            const double dvv = DV(q) * v[q];
+            const double ep = e[q] + dtI * (((m.Datu * uw) - (m.Datu * u[q])) + (dv_s - dvv));
+            dv_s = dvv;
+            return pick(x_in, y_in, q, ep, e[q]) * m.gtot;
+        };
+        // velocity updates (:234-260) of row r from the predicted eta of the row
+        // and its neighbour, and the other component as it stands
+        auto new_v = [&](int q, double g0, double g1, double u0, double u0w, double u1, double u1w)
+                         __attribute__((always_inline)) -> double {
+            const double f = F4(q);
+            const double Cor = -1.0 * (((f * u0w) + (f * u1)) + ((f * u0) + (f * u1w)));
+            const double vn = m.bt_rem_v * (v[q] + dtbt * (Cor + (g0 - g1) * idy));
+            return pick(x_in, y_v, q, vn, v[q]);
+        };
+        auto new_u = [&](int q, double g0, double v0, double v0e, double vs, double vse)
+                         __attribute__((always_inline)) -> double {
+            const double f = F4(q);
+            const double Cor = (((f * v0e) + (f * vs)) + ((f * v0) + (f * vse)));
+            const double un = m.bt_rem_u * (u[q] + dtbt * (Cor + (g0 - bt_east(g0)) * idx));
+            return pick(x_u, y_in, q, un, u[q]);
+        };
+        // transports (:262-272), free surface (:274-279) and averages
+        // (:281-291) of row r >= 0; vh_s: the transport of row r - 1
+        auto vtrans = [&](int q, double vn) __attribute__((always_inline)) -> double {
+            if (ROW) return s_dt[w * R + q] * (trans_wt1 * vn + trans_wt2 * v[q]);
+            return pick(true, y_t, q, DV(q) * (trans_wt1 * vn + trans_wt2 * v[q]), 0.0);
+        };
+        auto surface = [&](int q, double un, double vn, double vh, double vh_s) __attribute__((always_inline)) {
+            const double uh = Datu_t * (trans_wt1 * un + trans_wt2 * u[q]);
+            e[q] = pick(x_in, y_in, q, e[q] - dtI * ((uh - bt_west(uh)) + (vh - vh_s)), e[q]);
+            u[q] = un;
+            v[q] = vn;
+            ua[q - 2] = ua[q - 2] + un * inv_nstep;
+            va[q - 2] = va[q - 2] + vn * inv_nstep;
+        };
+        // rows upwards, each as soon as the row above has what it needs; row -1
+        // (q = 1) is formed for its new v and transport, row R (q = R + 2) for
+        // its predicted eta (and, u first, its new u)
+        double uw = bt_west(u[1]), g1 = predict(1, uw), vh_s = 0.0;
+        if constexpr (VF) {
+            double u1 = u[1], vs = 0.0, vse = 0.0;
 #pragma unroll
-        for (int r = 0; r < NR; ++r) {
-            int li, lj;
-            if (r_pos(r, li, lj)) {
-                e_old[r] = s_e[lj][li];
-                u_old[r] = s_u[lj][li]; uw_old[r] = s_u[lj][li - 1];
-                v_old[r] = s_v[lj][li]; vs_old[r] = s_v[lj - 1][li];
+            for (int q = 1; q <= R + 1; ++q) {
+                const double g0 = g1, u0 = u1, u0w = uw;
+                u1 = u[q + 1];
+                uw = bt_west(u1);
+                g1 = predict(q + 1, uw);
+                const double vn = new_v(q, g0, g1, u0, u0w, u1, uw);
+                const double vne = bt_east(vn), vh = vtrans(q, vn);
+                if (q >= 2) surface(q, new_u(q, g0, vn, vne, vs, vse), vn, vh, vh_s);
+                vs = vn; vse = vne; vh_s = vh;
+            }
+        } else {
+            double v0 = v[0], v0e = bt_east(v[0]), v1 = v[1], v1e = bt_east(v[1]);
+            double u1 = new_u(1, g1, v1, v1e, v0, v0e), u1w = bt_west(u1);
+#pragma unroll
+            for (int q = 1; q <= R + 1; ++q) {
+                const double g0 = g1, u0 = u1, u0w = u1w;
+                v0 = v1; v0e = v1e;
+                g1 = predict(q + 1, bt_west(u[q + 1]));
+                v1 = v[q + 1];
+                v1e = bt_east(v1);
+                u1 = new_u(q + 1, g1, v1, v1e, v0, v0e);
+                u1w = bt_west(u1);
+                const double vn = new_v(q, g0, g1, u0, u0w, u1, u1w);
+                const double vh = vtrans(q, vn);
+                if (q >= 2) surface(q, u0, vn, vh, vh_s);
+                vh_s = vh;
             }
         }
-        if (!ROW) __syncthreads();   // the predictor below overwrites s_e in place
-        // eta predictor (:224-231): in place, or (ROW) into s_ep, which then
-        // holds eta itself where no prediction applies
-        rect_each<NT, NP>(A0 - 1, A1 + 1, B0 - 1, B1 + 1, tid, [&](int li, int lj) {
-            const bool in = (s_fx[li] & s_fy[lj] & 1) != 0;
-            if (!ROW && !in) return;
-            const double e0 = s_e[lj][li];
-            const double ep = in ? e0 + (dtbt * m.IareaT) *
-                                            (((m.Datu * s_u[lj][li - 1]) - (m.Datu * s_u[lj][li])) +
-                                             ((DV(lj - 1, li) * s_v[lj - 1][li]) - (DV(lj, li) * s_v[lj][li])))
-                                 : e0;
-            if (ROW) s_ep[ROW ? lj : 0][ROW ? li : 0] = ep;
-            else s_e[lj][li] = ep;
-        });
-        __syncthreads();
-        // the first velocity update
-        if (v_first)
-            rect_each<NT, NP>(A0 - 1, A1 + 1, B0 - 1, B1, tid, [&](int li, int lj) {
-                s_v[lj][li] = new_v(lj, li);
-            });
-        else
-            rect_each<NT, NP>(A0 - 1, A1, B0 - 1, B1 + 1, tid, [&](int li, int lj) {
-                s_u[lj][li] = new_u(lj, li);
-            });
-        __syncthreads();
-        // the second velocity update
-        if (v_first)
-            rect_each<NT, NP>(A0 - 1, A1, B0, B1, tid, [&](int li, int lj) {
-                s_u[lj][li] = new_u(lj, li);
-            });
-        else
-            rect_each<NT, NP>(A0, A1, B0 - 1, B1, tid, [&](int li, int lj) {
-                s_v[lj][li] = new_v(lj, li);
-            });
-        __syncthreads();
-        // time averages (:281-291) of the output points: the array faces
-        // inside the update ranges
-#pragma unroll
-        for (int r = 0; r < NOUT; ++r) {
-            const int t = tid + NT * r;
-            const int i = i0 + t % TX, j = j0 + t / TX;
-            const int li = 2 * TS + t % TX, lj = 2 * TS + t / TX;
-            if (t >= TX * TY) continue;
-            if (i >= is && i <= ie - 1 && j >= js && j <= je) ua_r[r] = ua_r[r] + s_u[lj][li] * inv_nstep;
-            if (i >= is && i <= ie && j >= js && j <= je - 1) va_r[r] = va_r[r] + s_v[lj][li] * inv_nstep;
+    };
+    y_in = __builtin_amdgcn_readfirstlane(y_in);
+    y_v = __builtin_amdgcn_readfirstlane(y_v);
+    y_t = __builtin_amdgcn_readfirstlane(y_t);
+    for (int s = 0; s < st.ns; ++s) {
+        if (last && s + 1 == st.ns && (wx || wy)) {   // no refill follows: the positions themselves
+            x_in = x >= is && x <= ie;
+            x_u = x >= is && x <= ie - 1;
+            y_in = y_v = 0;
+            for (int q = 0; q < R + 3; ++q) {
+                const int y = y0 + q - 2;
+                y_in |= (y >= js && y <= je ? 1u : 0u) << q;
+                y_v |= (y >= js && y <= je - 1 ? 1u : 0u) << q;
+            }
+            y_in = __builtin_amdgcn_readfirstlane(y_in);
+            y_v = __builtin_amdgcn_readfirstlane(y_v);
+            inner = all_in();
         }
-        // transports (:262-272) and the free surface (:274-279) on R, in place
-#pragma unroll
-        for (int r = 0; r < NR; ++r) {
-            int li, lj;
-            if (!r_pos(r, li, lj)) continue;
-            const int fx = s_fx[li], fy = s_fy[lj];
-            if (!(fx & fy & 1)) continue;   // outside is..ie x js..je
-            const double un = s_u[lj][li], uw = s_u[lj][li - 1], vn = s_v[lj][li], vs = s_v[lj - 1][li];
-            const double uh_e = (fx & 4) ? m.Datu * (trans_wt1 * un + trans_wt2 * u_old[r]) : 0.0;
-            const double uh_w = (fx & 8) ? m.Datu * (trans_wt1 * uw + trans_wt2 * uw_old[r]) : 0.0;
-            const double vh_n = (fy & 4) ? DV(lj, li) * (trans_wt1 * vn + trans_wt2 * v_old[r]) : 0.0;
-            const double vh_s = (fy & 8) ? DV(lj - 1, li) * (trans_wt1 * vs + trans_wt2 * vs_old[r]) : 0.0;
-            s_e[lj][li] = e_old[r] - dtbt * m.IareaT * ((uh_e - uh_w) + (vh_n - vh_s));
+        const bool v_first = ((st.n0 + s + p.first_direction) % 2) == 1;
+        // opaque in every substep, so that no select mask is formed ahead for
+        // every row and kept over the loop (they would not fit the scalar registers)
+        asm volatile("" : "+s"(y_in), "+s"(y_v), "+s"(y_t));
+        using Yes = std::true_type;
+        using No = std::false_type;
+        if (inner) {
+            if (v_first) substep(Yes{}, Yes{});
+            else substep(Yes{}, No{});
+        } else {
+            if (v_first) substep(No{}, Yes{});
+            else substep(No{}, No{});
         }
+        if (s + 1 == st.ns) break;
+        // the outer rows to the neighbouring waves
+        double (*mine)[kBTW] = s_out[s & 1][w];
+        mine[0][lane] = e[2]; mine[1][lane] = u[2]; mine[2][lane] = v[2];
+        mine[3][lane] = e[R + 1]; mine[4][lane] = u[R + 1]; mine[5][lane] = v[R + 1];
+        mine[6][lane] = v[R];
         __syncthreads();
+        if (w > 0) {
+            double (*south)[kBTW] = s_out[s & 1][w - 1];
+            e[1] = south[3][lane]; u[1] = south[4][lane]; v[1] = south[5][lane];
+            v[0] = south[6][lane];
+        }
+        if (w < NW - 1) {
+            double (*north)[kBTW] = s_out[s & 1][w + 1];
+            e[R + 2] = north[0][lane]; u[R + 2] = north[1][lane]; v[R + 2] = north[2][lane];
+        }
     }
-    // the state after the launch on the output tile, halo positions included
+    // the state after the launch on the output tile, or after the call's last
+    // substep its outputs (:296-302; the averages are zero outside their ranges)
 #pragma unroll
-    for (int r = 0; r < NOUT; ++r) {
-        const int t = tid + NT * r;
-        const int i = i0 + t % TX, j = j0 + t / TX;
-        if (t >= TX * TY || i > d.ied || j > d.jed) continue;
-        const int li = 2 * TS + t % TX, lj = 2 * TS + t / TX;
-        const long long c = IX2(d, i, j);
-        st.eta_n[c] = s_e[lj][li]; st.ubt_n[c] = s_u[lj][li]; st.vbt_n[c] = s_v[lj][li];
-        if (i >= is && i <= ie - 1 && j >= js && j <= je) p.ubt_av[c] = ua_r[r];
-        if (i >= is && i <= ie && j >= js && j <= je - 1) p.vbt_av[c] = va_r[r];
+    for (int r = 0; r < R; ++r) {
+        if (!(out_x && out_row(r))) continue;
+        const int y = y0 + r;
+        const long long c = IX2(d, x, y);
+        const bool in_u = av_u && y >= js && y <= je, in_v = av_v && y >= js && y <= je - 1;
+        if (last) {
+            st.out_u[c] = in_u ? ua[r] : 0.0;
+            st.out_v[c] = in_v ? va[r] : 0.0;
+            st.out_eta[c] = e[r + 2];
+        } else {
+            st.eta_n[c] = e[r + 2]; st.ubt_n[c] = u[r + 2]; st.vbt_n[c] = v[r + 2];
+            p.ubt_av[c] = in_u ? ua[r] : 0.0;
+            p.vbt_av[c] = in_v ? va[r] : 0.0;
+        }
     }
 }
 
-// Tile and block of the blocked kernel for TS substeps per launch.  66 x 16
-// (512 threads) covers a 720-wide grid and its halos in 11 x 46 tiles, one
-// round of two blocks per CU; 4 substeps take 66 x 32 tiles of 1024 threads
-// (one block per CU, 11 x 23 tiles), which recompute less of their halo.
-template <int TS>
-struct BTMShape {
-    static constexpr int TX = 66, TY = 16, NT = 512;
-};
-template <>
-struct BTMShape<4> {
-    static constexpr int TX = 66, TY = 32, NT = 1024;
-};
-template <>
-struct BTMShape<5> : BTMShape<4> {};
+constexpr int kBTThreads = 64 * kBTWaves;
 
-inline dim3 bt_multi_grid(const Dims &d, int ts)
+inline dim3 bt_multi_grid(const Dims &d, int ns)
 {
-    const int tx = ts >= 4 ? BTMShape<4>::TX : BTMShape<3>::TX, ty = ts >= 4 ? BTMShape<4>::TY : BTMShape<3>::TY;
+    const int tx = kBTW - 3 * ns, ty = kBTH - 3 * ns;
     return dim3((d.n1 + tx - 1) / tx, (d.n2 + ty - 1) / ty);
-}
-inline int bt_multi_threads(int ts) { return ts >= 4 ? BTMShape<4>::NT : BTMShape<3>::NT; }
-
-template <int TS, bool ROW>
-__global__ void __launch_bounds__(BTMShape<TS>::NT) k_bt_multi(BT p, BTUniform m, BTMulti st)
-{
-    using S = BTMShape<TS>;
-    const int tile = xcd_tile(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
-    bt_multi_body<S::NT, S::TX, S::TY, TS, ROW>(p, m, st, tile % gridDim.x, tile / gridDim.x);
 }
 
 template <bool ROW>
-void launch_bt_multi(int ts, dim3 g, const BT &p, const BTUniform &m, const BTMulti &st, hipStream_t s)
+__global__ void __launch_bounds__(kBTThreads) k_bt_multi(BT p, BTUniform m, BTMulti st)
 {
-    const dim3 b(bt_multi_threads(ts));
-    if (ts == 2) k_bt_multi<2, ROW><<<g, b, 0, s>>>(p, m, st);
-    else if (ts == 3) k_bt_multi<3, ROW><<<g, b, 0, s>>>(p, m, st);
-    else if (ts == 4) k_bt_multi<4, ROW><<<g, b, 0, s>>>(p, m, st);
-    else k_bt_multi<5, ROW><<<g, b, 0, s>>>(p, m, st);
+    const int tile = xcd_tile(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
+    bt_multi_body<ROW>(p, m, st, tile % gridDim.x, tile / gridDim.x);
+}
+
+// Substeps of each launch of a call: on periodic grids the first alone, the
+// rest spread evenly over launches of up to ts.  At least two launches: the
+// outputs may alias the inputs, which only the first launch reads.
+inline std::vector<int> bt_split(int nstep, bool periodic, int ts)
+{
+    std::vector<int> ns;
+    int rest = nstep;
+    if (periodic) {
+        ns.push_back(1);
+        --rest;
+    }
+    int launches = (rest + ts - 1) / ts;
+    if (!periodic && launches < 2) launches = 2;
+    for (int q = 0; q < launches; ++q) ns.push_back(rest / launches + (q < rest % launches ? 1 : 0));
+    return ns;
+}
+
+// Substeps per launch when the caller sets none.  A launch costs about 6 us and
+// the state's way through memory, a substep about 3 us per round of blocks, and
+// every block takes a CU that the layers' kernels beside it could use; longer
+// launches mean fewer of the first, smaller tiles and so more of the others.
+// us per call at 4 / 5 / 6 / 8 / 10 / 14 substeps (alone): 28x20, 20 substeps:
+// 82 / 78 / 74 / 74 / 71 / 71; 180x180, 30: 140 / 133 / 125 / 118 / 111 / 105;
+// 720x720, 50: 279 / 264 / 250 / 357 / 364 / 724 (two rounds from 7 on).
+constexpr int kBTMost = 16;
+inline int bt_auto_substeps(const std::vector<Dims> &grids, int nstep, bool periodic)
+{
+    double points = 0.0, best = 0.0;
+    for (const Dims &d : grids) points += (double)d.s2;
+    int pick = 5;
+    for (int ts = 2; ts <= kBTMost; ++ts) {
+        double cost = 0.0;
+        for (int ns : bt_split(nstep, periodic, ts)) {
+            long long blocks = 0;
+            for (const Dims &d : grids) blocks += (long long)bt_multi_grid(d, ns).x * bt_multi_grid(d, ns).y;
+            cost += 6.0 + 1.0e-5 * points + 3.0 * ns * ((double)((blocks + 255) / 256) + blocks / 256.0);
+        }
+        if (ts == 2 || cost < best) {
+            best = cost;
+            pick = ts;
+        }
+    }
+    return pick;
 }
 
 // ---- the ensemble form: every member's substep n (or substeps n0 ..
@@ -608,78 +648,84 @@ __global__ void __launch_bounds__(256) k_bt_substep_batch(const BTMember *__rest
     bt_body<BTUniform, TY>(a.p, a.m, st, local % mp.nbx[m], local / mp.nbx[m]);
 }
 
-template <int TS, bool ROW>
-__global__ void __launch_bounds__(BTMShape<TS>::NT) k_bt_multi_batch(const BTMember *__restrict__ args, BatchMap mp, int n0,
-                                                            int ns, int from_a)
+// src: the set a launch reads (0: the call's inputs, 1: A, 2: B); it writes
+// the other one (A after the inputs)
+template <bool ROW>
+__global__ void __launch_bounds__(kBTThreads) k_bt_multi_batch(const BTMember *__restrict__ args, BatchMap mp, int n0,
+                                                               int ns, int wrap, int src)
 {
     int m, local;
     batch_locate(mp, xcd_tile(blockIdx.x, gridDim.x), m, local);
     const BTMember a = args[m];
     BTMulti st;
-    st.eta_o = from_a ? a.A[0] : a.B[0]; st.ubt_o = from_a ? a.A[1] : a.B[1]; st.vbt_o = from_a ? a.A[2] : a.B[2];
-    st.eta_n = from_a ? a.B[0] : a.A[0]; st.ubt_n = from_a ? a.B[1] : a.A[1]; st.vbt_n = from_a ? a.B[2] : a.A[2];
+    st.eta_o = src == 0 ? a.in[0] : src == 1 ? a.A[0] : a.B[0];
+    st.ubt_o = src == 0 ? a.in[1] : src == 1 ? a.A[1] : a.B[1];
+    st.vbt_o = src == 0 ? a.in[2] : src == 1 ? a.A[2] : a.B[2];
+    st.eta_n = src == 1 ? a.B[0] : a.A[0]; st.ubt_n = src == 1 ? a.B[1] : a.A[1]; st.vbt_n = src == 1 ? a.B[2] : a.A[2];
+    st.out_u = a.out[0]; st.out_v = a.out[1]; st.out_eta = a.out[2];
     st.n0 = n0;
     st.ns = ns;
-    using S = BTMShape<TS>;
-    bt_multi_body<S::NT, S::TX, S::TY, TS, ROW>(a.p, a.m, st, local % mp.nbx[m], local / mp.nbx[m]);
+    st.wrap = wrap;
+    bt_multi_body<ROW>(a.p, a.m, st, local % mp.nbx[m], local / mp.nbx[m]);
 }
 
-// btstep of every member (all with nstep substeps and uniform coefficients);
-// substeps 2 .. nstep-1 in blocked launches of up to per_launch when every
-// member allows it
+// btstep of every member (all with nstep substeps and uniform coefficients), in
+// blocked launches of up to per_launch substeps (0: chosen from the grids) when
+// every member allows it
 int btstep_batch(const BTMember *d_args, const BTMember *h_args, int n, hipStream_t s, int ty, int per_launch)
 {
     MOM6H_REQUIRE(ty == 4 || ty == 8 || ty == 16, "btstep batch: tile rows must be 4, 8 or 16");
-    MOM6H_REQUIRE(per_launch >= 1 && per_launch <= 5, "btstep batch: 1..5 substeps per launch");
+    MOM6H_REQUIRE(per_launch >= 0 && per_launch <= 5, "btstep batch: 1..5 substeps per launch, or 0");
     const int BT_TY = ty;
     MOM6H_REQUIRE(n >= 1 && n <= kMaxMembers, "btstep batch: 1..%d members", kMaxMembers);
     const int nstep = h_args[0].p.nstep;
-    BatchMap mc{}, mt{}, mm{};
-    mc.n = mt.n = mm.n = n;
-    bool blocked = per_launch > 1, rowwise = true;
+    bool blocked = per_launch != 1 && nstep >= 2, rowwise = true, periodic = false;
+    std::vector<Dims> grids;
     for (int m = 0; m < n; ++m) {
-        const Dims &d = h_args[m].p.d;
         MOM6H_REQUIRE(h_args[m].p.nstep == nstep, "btstep batch: members differ in bt_nsteps");
+        grids.push_back(h_args[m].p.d);
+        blocked = blocked && h_args[m].blocked_ok;
+        rowwise = rowwise && h_args[m].m.Datv_row != nullptr;
+        periodic = periodic || h_args[m].p.px || h_args[m].p.py;
+    }
+    if (blocked) {
+        const int ts = per_launch ? per_launch : bt_auto_substeps(grids, nstep, periodic);
+        int n0 = 1, src = 0;
+        for (int ns : bt_split(nstep, periodic, ts)) {
+            BatchMap mm{};
+            mm.n = n;
+            for (int m = 0; m < n; ++m) {
+                const dim3 g = bt_multi_grid(grids[m], ns);
+                mm.nbx[m] = (int)g.x;
+                mm.nby[m] = (int)g.y;
+                mm.first[m + 1] = mm.first[m] + mm.nbx[m] * mm.nby[m];
+            }
+            const unsigned nb = (unsigned)mm.first[n];
+            if (rowwise) k_bt_multi_batch<true><<<nb, kBTThreads, 0, s>>>(d_args, mm, n0, ns, n0 > 1, src);
+            else k_bt_multi_batch<false><<<nb, kBTThreads, 0, s>>>(d_args, mm, n0, ns, n0 > 1, src);
+            MOM6H_LAUNCH_CHECK();
+            n0 += ns;
+            src = src == 1 ? 2 : 1;
+        }
+        return MOM6H_OK;
+    }
+    BatchMap mc{}, mt{};
+    mc.n = mt.n = n;
+    for (int m = 0; m < n; ++m) {
+        const Dims &d = grids[m];
         mc.nbx[m] = (int)((d.s2 + 255) / 256);
         mc.first[m + 1] = mc.first[m] + mc.nbx[m];
         mt.nbx[m] = (d.n1 + BT_TX - 1) / BT_TX;
         mt.nby[m] = (d.n2 + BT_TY - 1) / BT_TY;
         mt.first[m + 1] = mt.first[m] + mt.nbx[m] * mt.nby[m];
-        const dim3 gm = bt_multi_grid(d, per_launch);
-        mm.nbx[m] = (int)gm.x;
-        mm.nby[m] = (int)gm.y;
-        mm.first[m + 1] = mm.first[m] + mm.nbx[m] * mm.nby[m];
-        blocked = blocked && h_args[m].blocked_ok;
-        rowwise = rowwise && h_args[m].m.Datv_row != nullptr;
     }
     k_bt_copy_in_batch<<<(unsigned)mc.first[n], 256, 0, s>>>(d_args, mc);
     MOM6H_LAUNCH_CHECK();
-    int from_a = 1;
-    for (int q = 1; q <= nstep;) {
-        if (blocked && q >= 2 && q <= nstep - 1) {
-            const int ns = std::min(per_launch, nstep - q);
-            const unsigned nb = (unsigned)mm.first[n], nt = (unsigned)bt_multi_threads(per_launch);
-            if (rowwise) {
-                if (per_launch == 2) k_bt_multi_batch<2, true><<<nb, nt, 0, s>>>(d_args, mm, q, ns, from_a);
-                else if (per_launch == 3) k_bt_multi_batch<3, true><<<nb, nt, 0, s>>>(d_args, mm, q, ns, from_a);
-                else if (per_launch == 4) k_bt_multi_batch<4, true><<<nb, nt, 0, s>>>(d_args, mm, q, ns, from_a);
-                else k_bt_multi_batch<5, true><<<nb, nt, 0, s>>>(d_args, mm, q, ns, from_a);
-            } else {
-                if (per_launch == 2) k_bt_multi_batch<2, false><<<nb, nt, 0, s>>>(d_args, mm, q, ns, from_a);
-                else if (per_launch == 3) k_bt_multi_batch<3, false><<<nb, nt, 0, s>>>(d_args, mm, q, ns, from_a);
-                else if (per_launch == 4) k_bt_multi_batch<4, false><<<nb, nt, 0, s>>>(d_args, mm, q, ns, from_a);
-                else k_bt_multi_batch<5, false><<<nb, nt, 0, s>>>(d_args, mm, q, ns, from_a);
-            }
-            MOM6H_LAUNCH_CHECK();
-            q += ns;
-        } else {
-            if (ty == 4) k_bt_substep_batch<4><<<(unsigned)mt.first[n], 256, 0, s>>>(d_args, mt, q, from_a);
-            else if (ty == 16) k_bt_substep_batch<16><<<(unsigned)mt.first[n], 256, 0, s>>>(d_args, mt, q, from_a);
-            else k_bt_substep_batch<8><<<(unsigned)mt.first[n], 256, 0, s>>>(d_args, mt, q, from_a);
-            MOM6H_LAUNCH_CHECK();
-            ++q;
-        }
-        from_a = !from_a;
+    for (int q = 1, from_a = 1; q <= nstep; ++q, from_a = !from_a) {
+        if (ty == 4) k_bt_substep_batch<4><<<(unsigned)mt.first[n], 256, 0, s>>>(d_args, mt, q, from_a);
+        else if (ty == 16) k_bt_substep_batch<16><<<(unsigned)mt.first[n], 256, 0, s>>>(d_args, mt, q, from_a);
+        else k_bt_substep_batch<8><<<(unsigned)mt.first[n], 256, 0, s>>>(d_args, mt, q, from_a);
+        MOM6H_LAUNCH_CHECK();
     }
     return MOM6H_OK;
 }
@@ -736,11 +782,12 @@ int mom6h_barotropic_init(mom6h_barotropic_cs **out, int isd, int ied, int jsd, 
                   "mom6h_barotropic_init: NULL array");
     auto *cs = new mom6h_barotropic_cs();
     cs->tile_rows = 4;
-    cs->substeps = 5;
+    cs->substeps = 0;
     cs->use_rows = 1;
     cs->d = make_dims(isd, ied, jsd, jed, isc, iec, jsc, jec, 1);
     cs->halo = Halo{periodic_x, periodic_y};
     cs->nstep = nstep;
+    cs->auto_substeps = bt_auto_substeps({cs->d}, nstep, periodic_x || periodic_y);
     cs->first_direction = first_direction;
     cs->dtbt = dt / (double)nstep;   // barotropic_init (:72-75)
     cs->bebt = bebt;
@@ -863,8 +910,35 @@ static int btstep_run(mom6h_barotropic_cs *cs, double *const w[8], bool zero_b, 
     p.extended = (p.px || p.py) ? 1 : 0;
     p.dtbt = cs->dtbt; p.bebt = cs->bebt; p.dgeo_de = cs->dgeo_de;
     p.ubt_av = w[6]; p.vbt_av = w[7];
-    // copy-in, then one launch per substep ping-ponging between the two state sets
     const Dims &d = cs->d;
+    double *A[3] = {w[0], w[1], w[2]}, *B[3] = {w[3], w[4], w[5]};
+    if (cs->substeps != 1 && cs->blocked_ok && cs->nstep >= 2) {   // blocked launches
+        BTUniform m{cs->u_Datu, cs->u_gtot, cs->u_rem_u, cs->u_rem_v, cs->u_IareaT, cs->u_IdxCu, cs->u_IdyCv,
+                    cs->Datv, cs->f4};
+        const bool periodic = p.px || p.py, rows = cs->Datv_row && cs->use_rows;
+        if (rows) {
+            m.Datv_row = cs->Datv_row;
+            m.f4_row = cs->f4_row;
+        }
+        const int ts = cs->substeps ? cs->substeps : cs->auto_substeps;
+        BTMulti st;
+        st.eta_o = eta_in; st.ubt_o = ubt_in; st.vbt_o = vbt_in;
+        st.out_u = u_av; st.out_v = v_av; st.out_eta = eta_av;
+        st.n0 = 1;
+        for (int ns : bt_split(cs->nstep, periodic, ts)) {
+            st.eta_n = A[0]; st.ubt_n = A[1]; st.vbt_n = A[2];
+            st.ns = ns;
+            st.wrap = st.n0 > 1;
+            if (rows) k_bt_multi<true><<<bt_multi_grid(d, ns), kBTThreads, 0, strm>>>(p, m, st);
+            else k_bt_multi<false><<<bt_multi_grid(d, ns), kBTThreads, 0, strm>>>(p, m, st);
+            MOM6H_LAUNCH_CHECK();
+            st.n0 += ns;
+            st.eta_o = A[0]; st.ubt_o = A[1]; st.vbt_o = A[2];
+            for (int q = 0; q < 3; ++q) std::swap(A[q], B[q]);
+        }
+        return MOM6H_OK;
+    }
+    // copy-in, then one launch per substep ping-ponging between the two state sets
     {
         const int bs = 256;
         k_bt_copy_in<<<(unsigned)((d.s2 + bs - 1) / bs), bs, 0, strm>>>(
@@ -874,31 +948,7 @@ static int btstep_run(mom6h_barotropic_cs *cs, double *const w[8], bool zero_b, 
     }
     const int BT_TY = cs->tile_rows;
     dim3 grid((d.n1 + BT_TX - 1) / BT_TX, (d.n2 + BT_TY - 1) / BT_TY), block(256);
-    const dim3 grid_m = bt_multi_grid(d, cs->substeps);
-    const int per_launch = cs->substeps;
-    double *A[3] = {w[0], w[1], w[2]}, *B[3] = {w[3], w[4], w[5]};
-    for (int n = 1; n <= cs->nstep;) {
-        // substeps 2 .. nstep-1 in blocks of up to per_launch
-        if (per_launch > 1 && cs->blocked_ok && n >= 2 && n <= cs->nstep - 1) {
-            BTMulti st;
-            st.eta_o = A[0]; st.ubt_o = A[1]; st.vbt_o = A[2];
-            st.eta_n = B[0]; st.ubt_n = B[1]; st.vbt_n = B[2];
-            st.n0 = n;
-            st.ns = std::min(per_launch, cs->nstep - n);
-            BTUniform m{cs->u_Datu, cs->u_gtot, cs->u_rem_u, cs->u_rem_v, cs->u_IareaT, cs->u_IdxCu,
-                        cs->u_IdyCv, cs->Datv, cs->f4};
-            if (cs->Datv_row && cs->use_rows) {
-                m.Datv_row = cs->Datv_row;
-                m.f4_row = cs->f4_row;
-                launch_bt_multi<true>(per_launch, grid_m, p, m, st, strm);
-            } else {
-                launch_bt_multi<false>(per_launch, grid_m, p, m, st, strm);
-            }
-            MOM6H_LAUNCH_CHECK();
-            for (int q = 0; q < 3; ++q) std::swap(A[q], B[q]);
-            n += st.ns;
-            continue;
-        }
+    for (int n = 1; n <= cs->nstep; ++n) {
         BTStep st;
         st.eta_o = A[0]; st.ubt_o = A[1]; st.vbt_o = A[2];
         st.eta_n = B[0]; st.ubt_n = B[1]; st.vbt_n = B[2];
@@ -919,7 +969,6 @@ static int btstep_run(mom6h_barotropic_cs *cs, double *const w[8], bool zero_b, 
         }
         MOM6H_LAUNCH_CHECK();
         for (int q = 0; q < 3; ++q) std::swap(A[q], B[q]);
-        ++n;
     }
     return MOM6H_OK;
 }

@@ -86,7 +86,7 @@ struct mom6h_ensemble {
     hipGraphExec_t gexec_bt = nullptr;
     int momentum_tile = 0, momentum_splits = 0;   // options of the momentum march (march_rows); 0: not set
     int bt_tile = 4;         // rows of the barotropic substep tile (4, 8 or 16)
-    int bt_substeps = 5;     // barotropic substeps per blocked launch (1 = one launch per substep)
+    int bt_substeps = 0;     // barotropic substeps per blocked launch (1 = one launch per substep, 0 = chosen from the grids)
     long long max_lds = 0;
     StepTables<float> tf;
     StepTables<double> td;

@@ -326,7 +326,8 @@ struct mom6h_barotropic_cs {
     double u_Datu, u_gtot, u_rem_u, u_rem_v, u_IareaT, u_IdxCu, u_IdyCv;
     double *f4;
     int tile_rows;           // rows of the substep tile (4, 8 or 16)
-    int substeps;            // substeps per launch of the blocked kernel (1: one launch per substep)
+    int substeps;            // substeps per launch of the blocked kernel (1: one launch per substep, 0: auto_substeps)
+    int auto_substeps;       // the number chosen from the grid at init
     int blocked_ok;          // uniform coefficients whose periodic Datv halo rows equal their images
     double *Datv_row, *f4_row;   // Datv and f4 per row when constant along the compute rows (else NULL)
     int use_rows;                // stage Datv and f4 per row when the grid allows (1, the default) or as 2D fields

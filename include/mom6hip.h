@@ -118,8 +118,8 @@ int mom6h_coriolis_end(mom6h_coriolis_cs *cs);
  * src/serial/mom6_barotropic_serial.F90:178-356.  Each substep is ONE launch
  * of an LDS-tiled kernel (eta predictor, pressure forces, both velocity
  * updates, transports, free surface, time averages on a tile plus its halo)
- * instead of ~9 dependent launches; grids whose coefficients are uniform take
- * a variant that holds them as values.  periodic_x/periodic_y select the
+ * instead of ~9 dependent launches; grids whose coefficients are uniform run
+ * several substeps per launch in registers.  periodic_x/periodic_y select the
  * split-API ranges (btstep_do_step, :379-474) with a halo refill of
  * ubt, vbt, eta after every substep but the last. */
 typedef struct mom6h_barotropic_cs mom6h_barotropic_cs;
@@ -323,11 +323,11 @@ int mom6h_model_synchronize(mom6h_model *m);
  * momentum stencil marches through 8*tile/splits rows (at least 4), or through
  * a number chosen from the grid while neither is set, "bt_tile" (rows of the barotropic substep tile,
  * 4, 8 or 16; after prepare; default 4), "bt_substeps" (barotropic substeps per
- * launch between the first and the last of a call: 1 = one launch per substep,
- * up to 5 = the blocked kernel; after prepare; default 5), "bt_rows" (1 = the
- * blocked kernel stages Datv and the Coriolis factor per row when both are
- * constant along the compute rows, 0 = always as 2D fields; after prepare;
- * default 1), "fused" (1 = fused momentum stencil and
+ * launch: 1 = one launch per substep, 2-5 = the blocked kernel with at most so
+ * many; after prepare; by default the blocked kernel with a number chosen from
+ * the grid), "bt_rows" (1 = the blocked kernel takes Datv and the Coriolis factor
+ * per row when both are constant along the compute rows, 0 = always as 2D
+ * fields; after prepare; default 1), "fused" (1 = fused momentum stencil and
  * on-chip vert_visc coefficients where the grid allows, default 1; 0 = the
  * module-by-module path), "profile" (1 = record per-stage HIP events; the
  * graph is not used while profiling), "serialize" (1 = run the barotropic
@@ -370,7 +370,8 @@ int mom6h_ensemble_synchronize(mom6h_ensemble *e);
 /* Options: "graph" (1 = capture one step, replay it per step), "momentum_tile"
  * (4, 8 or 16; default 8) and "momentum_splits" (after prepare; default 1): the
  * rows of the momentum march as for the model, "bt_tile" (4, 8 or 16),
- * "bt_substeps" (barotropic substeps per blocked launch, 1-5; default 5). */
+ * "bt_substeps" (barotropic substeps per blocked launch, 1-5; by default chosen
+ * from the members' grids). */
 int mom6h_ensemble_set_option(mom6h_ensemble *e, const char *key, double value);
 /* Times the fused momentum launch of the ensemble (reps launches) for marches
  * of 4 to 128 rows, keeps the fastest and writes the timings into report.  It runs
