@@ -305,16 +305,6 @@ struct BTMulti {
 // us per 5 substeps, and a copy-in and two one-substep launches per call, 707 us.
 constexpr int kBTW = 64, kBTH = 64, kBTRows = 8, kBTWaves = kBTH / kBTRows;
 
-// the value of the lane to the west / east (DPP wave shift; 0 beyond the wave)
-template <int CTRL>
-__device__ __forceinline__ double bt_dpp(double x)
-{
-    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xf, 0xf, true),
-                            __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xf, 0xf, true));
-}
-__device__ __forceinline__ double bt_west(double x) { return bt_dpp<0x138>(x); }
-__device__ __forceinline__ double bt_east(double x) { return bt_dpp<0x130>(x); }
-
 // ROW: Datv and f4 constant along each row of the compute domain (walls close
 // whole rows, f depends on latitude only; the host checks it): one scalar per
 // row instead of one value per position.
@@ -436,7 +426,7 @@ __device__ __forceinline__ void bt_multi_body(const BT &p, const BTUniform &m, c
                          __attribute__((always_inline)) -> double {
             const double f = F4(q);
             const double Cor = (((f * v0e) + (f * vs)) + ((f * v0) + (f * vse)));
-            const double un = m.bt_rem_u * (u[q] + dtbt * (Cor + (g0 - bt_east(g0)) * idx));
+            const double un = m.bt_rem_u * (u[q] + dtbt * (Cor + (g0 - east(g0)) * idx));
             return pick(x_u, y_in, q, un, u[q]);
         };
         // transports (:262-272), free surface (:274-279) and averages
@@ -447,7 +437,7 @@ __device__ __forceinline__ void bt_multi_body(const BT &p, const BTUniform &m, c
         };
         auto surface = [&](int q, double un, double vn, double vh, double vh_s) __attribute__((always_inline)) {
             const double uh = Datu_t * (trans_wt1 * un + trans_wt2 * u[q]);
-            e[q] = pick(x_in, y_in, q, e[q] - dtI * ((uh - bt_west(uh)) + (vh - vh_s)), e[q]);
+            e[q] = pick(x_in, y_in, q, e[q] - dtI * ((uh - west(uh)) + (vh - vh_s)), e[q]);
             u[q] = un;
             v[q] = vn;
             ua[q - 2] = ua[q - 2] + un * inv_nstep;
@@ -456,32 +446,32 @@ __device__ __forceinline__ void bt_multi_body(const BT &p, const BTUniform &m, c
         // rows upwards, each as soon as the row above has what it needs; row -1
         // (q = 1) is formed for its new v and transport, row R (q = R + 2) for
         // its predicted eta (and, u first, its new u)
-        double uw = bt_west(u[1]), g1 = predict(1, uw), vh_s = 0.0;
+        double uw = west(u[1]), g1 = predict(1, uw), vh_s = 0.0;
         if constexpr (VF) {
             double u1 = u[1], vs = 0.0, vse = 0.0;
 #pragma unroll
             for (int q = 1; q <= R + 1; ++q) {
                 const double g0 = g1, u0 = u1, u0w = uw;
                 u1 = u[q + 1];
-                uw = bt_west(u1);
+                uw = west(u1);
                 g1 = predict(q + 1, uw);
                 const double vn = new_v(q, g0, g1, u0, u0w, u1, uw);
-                const double vne = bt_east(vn), vh = vtrans(q, vn);
+                const double vne = east(vn), vh = vtrans(q, vn);
                 if (q >= 2) surface(q, new_u(q, g0, vn, vne, vs, vse), vn, vh, vh_s);
                 vs = vn; vse = vne; vh_s = vh;
             }
         } else {
-            double v0 = v[0], v0e = bt_east(v[0]), v1 = v[1], v1e = bt_east(v[1]);
-            double u1 = new_u(1, g1, v1, v1e, v0, v0e), u1w = bt_west(u1);
+            double v0 = v[0], v0e = east(v[0]), v1 = v[1], v1e = east(v[1]);
+            double u1 = new_u(1, g1, v1, v1e, v0, v0e), u1w = west(u1);
 #pragma unroll
             for (int q = 1; q <= R + 1; ++q) {
                 const double g0 = g1, u0 = u1, u0w = u1w;
                 v0 = v1; v0e = v1e;
-                g1 = predict(q + 1, bt_west(u[q + 1]));
+                g1 = predict(q + 1, west(u[q + 1]));
                 v1 = v[q + 1];
-                v1e = bt_east(v1);
+                v1e = east(v1);
                 u1 = new_u(q + 1, g1, v1, v1e, v0, v0e);
-                u1w = bt_west(u1);
+                u1w = west(u1);
                 const double vn = new_v(q, g0, g1, u0, u0w, u1, u1w);
                 const double vh = vtrans(q, vn);
                 if (q >= 2) surface(q, u0, vn, vh, vh_s);

@@ -32,36 +32,6 @@ __device__ __forceinline__ T sdiv(T num, T den)
     else return num / den;
 }
 
-// The value of the lane to the west (lane - 1) and to the east (lane + 1): DPP
-// wave shifts, one VALU move per 32 bits.  Lane 0 (63) gets zero; every lane
-// of the wave must be active.
-constexpr int kWaveShl1 = 0x130, kWaveShr1 = 0x138;
-template <int CTRL>
-__device__ __forceinline__ int dpp32(int x)
-{
-    return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, true);
-}
-template <int CTRL>
-__device__ __forceinline__ float dpp(float x)
-{
-    return __int_as_float(dpp32<CTRL>(__float_as_int(x)));
-}
-template <int CTRL>
-__device__ __forceinline__ double dpp(double x)
-{
-    return __hiloint2double(dpp32<CTRL>(__double2hiint(x)), dpp32<CTRL>(__double2loint(x)));
-}
-template <typename T>
-__device__ __forceinline__ T west(T x)
-{
-    return dpp<kWaveShr1>(x);
-}
-template <typename T>
-__device__ __forceinline__ T east(T x)
-{
-    return dpp<kWaveShl1>(x);
-}
-
 // One wave marches along j through rows ja..jb of one layer, lane l holding
 // column i0 + l: the i neighbours come from the neighbouring lanes (DPP), the
 // j neighbours are the values kept from the rows before.  So every strain, q,

@@ -6,8 +6,8 @@
 // viscosities with the thickness-aware bounds.  One 3D launch computes every layer: each thread forms the
 // strain/stress values its diffu/diffv stencil needs directly from u, v, h
 // (no 2D work arrays, no per-layer launches).  On grids whose metric arrays
-// are constant the constant-coefficient operator runs as a tiled layer walk
-// with LDS staging instead (k_hv_tile), bit-identical to the general kernel.
+// are constant every operator runs as a march of waves along j instead
+// (k_hv_march), bit-identical to the general kernels.
 //
 // The serial code keeps ONE 2D array for Kh (and Ah) at h- and q-points: the
 // h-point pass writes is..ie x js..je but the stress uses is-1..ie+1 x
@@ -19,6 +19,7 @@
 // (biharmonic: also the first interior column/row), and are reproduced here.
 #include "mom6h_internal.h"
 
+#include <algorithm>
 #include <initializer_list>
 #include <utility>
 
@@ -167,146 +168,6 @@ __global__ void k_hv_main(HV p, const double *__restrict__ u, const double *__re
     }
     diffu[c] = du;
     diffv[c] = dv;
-}
-
-// ---------------------------------------------------------------------------
-// The constant-coefficient operator on a grid whose metric arrays are constant
-// (over is-2..ie+2 x js-2..je+2, every point the stencil reads): a tiled layer
-// walk.  A block owns HT_X x TY points of the data domain and walks a range of
-// layers.  Per layer it stages u, v, h (and Del2u, Del2v) of the tile and a
-// one-cell ring in LDS, forms str_xx*h at every staged h point and str_xy*hq
-// at every staged q point once, then diffu and diffv of its points (zero
-// outside their ranges).  The masks stay in LDS for the whole walk, and the
-// next layer's loads are in flight while the current one is computed.  The
-// expressions are k_hv_main's with the constant metric values, so the results
-// are bit-identical to it.
-constexpr int HT_X = 64, HW = HT_X + 2;
-
-template <bool BIH, int TY>
-__global__ void __launch_bounds__(256) k_hv_tile(HV p, HVUniform g, const double *__restrict__ u,
-                                                 const double *__restrict__ v, const double *__restrict__ h,
-                                                 double *__restrict__ diffu, double *__restrict__ diffv)
-{
-    constexpr int MH = TY + 2, RPT = TY / 4, NS = (HW * MH + 255) / 256;
-    __shared__ double s_u[MH][HW], s_v[MH][HW], s_h[MH][HW], s_mT[MH][HW], s_mBu[MH][HW];
-    __shared__ double s_xx[MH][HW], s_xy[MH][HW];
-    __shared__ double s_2u[BIH ? MH : 1][BIH ? HW : 1], s_2v[BIH ? MH : 1][BIH ? HW : 1];
-    const Dims &d = p.d;
-    const int nxy = gridDim.x * gridDim.y;
-    const int tile = xcd_tile(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), nxy * gridDim.z);
-    const int xy = tile % nxy, kz = tile / nxy;
-    const int per = (d.nk + (int)gridDim.z - 1) / (int)gridDim.z;
-    const int k0 = 1 + kz * per, k1 = k0 + per - 1 < d.nk ? k0 + per - 1 : d.nk;
-    if (k0 > k1) return;
-    const int i0 = d.isd + (xy % (int)gridDim.x) * HT_X, j0 = d.jsd + (xy / (int)gridDim.x) * TY;
-    const int bi = i0 - 1, bj = j0 - 1;
-    const int tid = threadIdx.x, tx = tid % HT_X, ty = tid / HT_X;
-
-    double pu[NS], pv[NS], ph[NS], p2u[BIH ? NS : 1], p2v[BIH ? NS : 1];
-    auto load_layer = [&](int k) {
-#pragma unroll
-        for (int r = 0; r < NS; ++r) {
-            const int t = tid + 256 * r, li = t % HW, lj = t / HW, i = bi + li, j = bj + lj;
-            pu[r] = 0.0; pv[r] = 0.0; ph[r] = 0.0;
-            if (BIH) { p2u[BIH ? r : 0] = 0.0; p2v[BIH ? r : 0] = 0.0; }
-            if (t < HW * MH && i >= d.isd && i <= d.ied && j >= d.jsd && j <= d.jed) {
-                const long long c = IX3(d, i, j, k);
-                pu[r] = u[c]; pv[r] = v[c]; ph[r] = h[c];
-                if (BIH) { p2u[BIH ? r : 0] = p.Del2u[c]; p2v[BIH ? r : 0] = p.Del2v[c]; }
-            }
-        }
-    };
-    for (int t = tid; t < HW * MH; t += 256) {
-        const int li = t % HW, lj = t / HW, i = bi + li, j = bj + lj;
-        double mt = 0.0, mb = 0.0;
-        if (i >= d.isd && i <= d.ied && j >= d.jsd && j <= d.jed) {
-            mt = p.mask2dT[IX2(d, i, j)];
-            mb = p.mask2dBu[IX2(d, i, j)];
-        }
-        s_mT[lj][li] = mt;
-        s_mBu[lj][li] = mb;
-    }
-    const int is = d.isc, ie = d.iec, js = d.jsc, je = d.jec;
-    load_layer(k0);
-    for (int k = k0; k <= k1; ++k) {
-#pragma unroll
-        for (int r = 0; r < NS; ++r) {
-            const int t = tid + 256 * r;
-            if (t < HW * MH) {
-                const int li = t % HW, lj = t / HW;
-                s_u[lj][li] = pu[r]; s_v[lj][li] = pv[r]; s_h[lj][li] = ph[r];
-                if (BIH) { s_2u[BIH ? lj : 0][BIH ? li : 0] = p2u[BIH ? r : 0]; s_2v[BIH ? lj : 0][BIH ? li : 0] = p2v[BIH ? r : 0]; }
-            }
-        }
-        __syncthreads();
-        if (k < k1) load_layer(k + 1);
-        // Kh and Ah at the h points of the stress ring: what the previous
-        // layer's q-point pass left there, zero on the first layer of the
-        // first call (visc_h)
-        const bool ring_zero = k == 1 && p.first_call;
-        for (int t = tid; t < HW * MH; t += 256) {
-            const int li = t % HW, lj = t / HW, i = bi + li, j = bj + lj;
-            if (li >= 1 && lj >= 1) {   // str_xx * h at h point (i, j) (:807-895)
-                const double dudx = g.DY_dxT * ((g.IdyCu * s_u[lj][li]) - (g.IdyCu * s_u[lj][li - 1]));
-                const double dvdy = g.DX_dyT * ((g.IdxCv * s_v[lj][li]) - (g.IdxCv * s_v[lj - 1][li]));
-                const double sh = dudx - dvdy;
-                const bool in = i >= is && i <= ie && j >= js && j <= je;
-                const bool ring = !in && i >= is - 1 && i <= ie && j >= js - 1 && j <= je;
-                const bool on = in || (ring && !ring_zero);
-                const double Kh = on ? p.Kh : 0.0;
-                double str = p.laplacian ? -(Kh * sh) : 0.0;
-                if (BIH) {
-                    const int qi = BIH ? li : 0, qj = BIH ? lj : 0;
-                    const double d_del2u = (g.IdyCu * s_2u[qj][qi]) - (g.IdyCu * s_2u[qj][BIH ? qi - 1 : 0]);
-                    const double d_del2v = (g.IdxCv * s_2v[qj][qi]) - (g.IdxCv * s_2v[BIH ? qj - 1 : 0][qi]);
-                    const double Ah = on ? p.Ah : 0.0;
-                    const double d_str = Ah * ((g.DY_dxT * d_del2u) - (g.DX_dyT * d_del2v));
-                    str = str + d_str;
-                }
-                s_xx[lj][li] = str * (s_h[lj][li] * g.red_xx);
-            }
-            if (li < HW - 1 && lj < MH - 1) {   // str_xy * hq at q point (i, j) (:954-1053)
-                const double dvdx = g.DY_dxBu * ((s_v[lj][li + 1] * g.IdyCv) - (s_v[lj][li] * g.IdyCv));
-                const double dudy = g.DX_dyBu * ((s_u[lj + 1][li] * g.IdxCu) - (s_u[lj][li] * g.IdxCu));
-                const double m = s_mBu[lj][li];
-                const double sh = (p.no_slip ? (2.0 - m) : m) * (dvdx + dudy);
-                double str = p.laplacian ? -(p.Kh * sh) : 0.0;
-                if (BIH) {
-                    const int qi = BIH ? li : 0, qj = BIH ? lj : 0;
-                    const double d_str =
-                        p.Ah * ((g.DY_dxBu * ((s_2v[qj][BIH ? qi + 1 : 0] * g.IdyCv) - (s_2v[qj][qi] * g.IdyCv))) +
-                                (g.DX_dyBu * ((s_2u[BIH ? qj + 1 : 0][qi] * g.IdxCu) - (s_2u[qj][qi] * g.IdxCu))));
-                    str = str + d_str;
-                }
-                const double hq = 0.25 * ((s_h[lj][li] + s_h[lj + 1][li + 1]) + (s_h[lj][li + 1] + s_h[lj + 1][li]));
-                s_xy[lj][li] = p.no_slip ? str * (hq * g.red_xy) : str * (hq * m * g.red_xy);
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < RPT; ++r) {
-            const int i = i0 + tx, j = j0 + ty + 4 * r;
-            if (i > d.ied || j > d.jed) continue;
-            const int li = tx + 1, lj = ty + 4 * r + 1;
-            double du = 0.0, dv = 0.0;
-            if (i >= is - 1 && i <= ie && j >= js && j <= je) {   // (:1059-1067)
-                const double h_u = 0.5 * (s_mT[lj][li] * s_h[lj][li] + s_mT[lj][li + 1] * s_h[lj][li + 1]);
-                du = ((g.IdxCu * ((g.dx2q * s_xy[lj - 1][li]) - (g.dx2q * s_xy[lj][li])) +
-                       g.IdyCu * ((g.dy2h * s_xx[lj][li]) - (g.dy2h * s_xx[lj][li + 1]))) *
-                      g.IareaCu) / (h_u + p.h_neglect);
-            }
-            if (i >= is && i <= ie && j >= js - 1 && j <= je) {   // (:1070-1078)
-                const double h_v = 0.5 * (s_mT[lj][li] * s_h[lj][li] + s_mT[lj + 1][li] * s_h[lj + 1][li]);
-                dv = ((g.IdyCv * ((g.dy2q * s_xy[lj][li - 1]) - (g.dy2q * s_xy[lj][li])) -
-                       g.IdxCv * ((g.dx2h * s_xx[lj][li]) - (g.dx2h * s_xx[lj + 1][li]))) *
-                      g.IareaCv) / (h_v + p.h_neglect);
-            }
-            const long long c = IX3(d, i, j, k);
-            diffu[c] = du;
-            diffv[c] = dv;
-        }
-        __syncthreads();
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -590,6 +451,268 @@ __global__ void k_hv_keep_ring(HV p, const double *__restrict__ u, const double 
     p.ring_Ah[IX2(d, I, J)] = p.biharmonic ? visc_q_point(p, u, v, h, I, J, d.nk, 1) : 0.0;
 }
 
+// ---------------------------------------------------------------------------
+// Grids whose metric arrays are constant (over is-2..ie+2 x js-2..je+2, every
+// point the stencil reads): every operator -- constant Kh and Ah, Smagorinsky,
+// Leith, the bounds -- as one march, as the fused momentum stencil does it.  A
+// wave holds 64 columns of one layer and walks along j: i neighbours by lane
+// shifts, j neighbours kept from the rows before, so each strain, vorticity and
+// its derivatives, thickness ratio, viscosity, Del2 and stress is formed once per
+// point.  At step r row r arrives; suffix 0 marks its h points, 1 the q and h
+// points of row r - 1, and so on.  The expressions are the general kernels' with
+// the constant metric values, so the results are bit-identical to theirs.
+//
+// The stress at the h points of the ring (is-1 or js-1) reads Kh and Ah of the
+// previous layer's q points: k_hv_ring forms those for every layer beforehand
+// (a few thousand points), and the march loads them with the row.
+//
+// What bounds it: VALU issue with the closures, memory without.  360x283x50 with
+// Smagorinsky, the bounds and the biharmonic term: 116 us per call (march 98, ring
+// 11) against 3240 us when one thread per point evaluated every work value it
+// needed from u, v and h (and Del2 in a launch of its own, 214 us of them).
+// 471x363x50 Laplacian: 107 us, the time of the 64 x 8 tile staged in LDS that it
+// replaces (108 us); with the biharmonic term it saves the Del2 launch and arrays.
+template <bool SMAG, bool LEITH, bool BOUND, bool BIH>
+struct HVMarch {
+    static constexpr bool CL = SMAG || LEITH || BOUND;
+    static constexpr int LM = CL || BIH ? 2 : 1;                       // lanes that only lend, west
+    static constexpr int RM = LEITH ? 3 : CL || BIH ? 2 : 1;           // and east
+    static constexpr int OUT = 64 - LM - RM;
+};
+
+// compact index of a ring point: (is-1, js-1..je), then (is..ie, js-1)
+__device__ inline int ring_index(const Dims &d, int I, int J)
+{
+    return I == d.isc - 1 ? J - (d.jsc - 1) : d.jec - d.jsc + 2 + (I - d.isc);
+}
+__host__ __device__ inline int ring_points(const Dims &d)
+{
+    return (d.jec - d.jsc + 2) + (d.iec - d.isc + 1);
+}
+
+// Kh (ring_q[0 ..]) and Ah (ring_q[nk*points ..]) of every layer at the ring points
+__global__ void __launch_bounds__(64) k_hv_ring(HV p, const double *__restrict__ u, const double *__restrict__ v,
+                                                const double *__restrict__ h, double *__restrict__ ring_q)
+{
+    const Dims &d = p.d;
+    const int q = blockIdx.x * 64 + threadIdx.x, n = ring_points(d), k = 1 + blockIdx.y;
+    if (q >= n) return;
+    const int ncol = d.jec - d.jsc + 2;
+    const int I = q < ncol ? d.isc - 1 : d.isc + (q - ncol);
+    const int J = q < ncol ? d.jsc - 1 + q : d.jsc - 1;
+    ring_q[(long long)(k - 1) * n + q] = p.laplacian ? visc_q_point(p, u, v, h, I, J, k, 0) : 0.0;
+    ring_q[(long long)(d.nk + k - 1) * n + q] = p.biharmonic ? visc_q_point(p, u, v, h, I, J, k, 1) : 0.0;
+}
+
+// After the call: the last layer's, for the next call's first layer
+__global__ void __launch_bounds__(64) k_hv_keep_last(HV p, const double *__restrict__ ring_q)
+{
+    const Dims &d = p.d;
+    const int q = blockIdx.x * 64 + threadIdx.x, n = ring_points(d);
+    if (q >= n) return;
+    const int ncol = d.jec - d.jsc + 2;
+    const long long c = IX2(d, q < ncol ? d.isc - 1 : d.isc + (q - ncol), q < ncol ? d.jsc - 1 + q : d.jsc - 1);
+    p.ring_Kh[c] = ring_q[(long long)(d.nk - 1) * n + q];
+    p.ring_Ah[c] = ring_q[(long long)(2 * d.nk - 1) * n + q];
+}
+
+template <bool SMAG, bool LEITH, bool BOUND, bool BIH>
+__global__ void __launch_bounds__(256) k_hv_march(HV p, HVUniform g, const double *__restrict__ u,
+                                                  const double *__restrict__ v, const double *__restrict__ h,
+                                                  const double *__restrict__ ring_q, double *__restrict__ diffu,
+                                                  double *__restrict__ diffv, int strips, int chunks, int rows)
+{
+    using M = HVMarch<SMAG, LEITH, BOUND, BIH>;
+    const Dims &d = p.d;
+    const int is = d.isc, ie = d.iec, js = d.jsc, je = d.jec;
+    const int t = xcd_tile(blockIdx.x, gridDim.x) * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int per = strips * chunks, k = t / per + 1, tq = t % per, strip = tq % strips;
+    if (k > d.nk) return;
+    const int ja = d.jsd + (tq / strips) * rows, jb = ja + rows - 1 < d.jed ? ja + rows - 1 : d.jed;
+    const int lane = threadIdx.x & 63;
+    const int i = d.isd + strip * M::OUT - M::LM + lane;
+    const unsigned col = (unsigned)((i < d.isd ? d.isd : i > d.ied ? d.ied : i) - d.isd);   // clamped: such lanes only lend
+    const bool mine = lane >= M::LM && lane < 64 - M::RM && i <= d.ied;
+    const bool in_i = i >= is && i <= ie, in_I = i >= is - 1 && i <= ie;
+    const long long n1 = d.n1, layer = (long long)(k - 1) * d.s2;
+    auto row_of = [&](int j) -> long long { return (long long)((j < d.jsd ? d.jsd : j > d.jed ? d.jed : j) - d.jsd) * n1; };
+    auto in_j = [&](int j) { return j >= js && j <= je; };       // h rows
+    auto in_J = [&](int j) { return j >= js - 1 && j <= je; };   // q rows
+    // the ring's viscosities: of the previous layer (the first layer: of the
+    // previous call), or the constants (zero in the first layer of the first call)
+    const bool ring_strip = strip * M::OUT - M::LM + d.isd <= is - 1;
+    const int nring = ring_points(d);
+    const double ring_c = k == 1 && p.first_call ? 0.0 : 1.0;
+    const double Kh_c = ring_c * p.Kh, Ah_c = ring_c * p.Ah;
+    const double area = g.areaT, h3 = sqrt(area) * area;
+    const bool lap = p.laplacian;
+    const double smag_K = p.smag_Kh ? 0.15 * 0.15 * area : 0.0, smag_A = 0.06 * 0.06 * (area * area);
+
+    double nu, nv, nh, nmT, nmB, nrK = 0.0, nrA = 0.0;   // the newest row, in flight until its step
+    auto load = [&](int r) __attribute__((always_inline)) {
+        const long long row = row_of(r), o = layer + row;
+        nu = (u + o)[col];
+        nv = (v + o)[col];
+        nh = (h + o)[col];
+        nmT = (p.mask2dT + row)[col];
+        nmB = (p.mask2dBu + row)[col];
+        if (M::CL) {   // the ring's Kh and Ah for the stress of h row r - 2
+            const int J = r - 2;
+            if (in_J(J) && (ring_strip || J == js - 1)) {
+                const bool on = i == is - 1 || (J == js - 1 && in_i);
+                if (on) {
+                    const int q = ring_index(d, i, J);
+                    if (k > 1) {
+                        nrK = ring_q[(long long)(k - 2) * nring + q];
+                        nrA = ring_q[(long long)(d.nk + k - 2) * nring + q];
+                    } else {
+                        nrK = p.ring_Kh[IX2(d, i, J)];
+                        nrA = p.ring_Ah[IX2(d, i, J)];
+                    }
+                }
+            }
+        }
+    };
+    double u1, v1, ve1, h1, he1, mh1, mB1;                                     // row r - 1
+    double xx1 = 0.0, xx1e = 0.0, xx2 = 0.0, xy2 = 0.0, hq2 = 0.0, h2 = 0.0, hu2 = 0.0, hv2 = 0.0, hv3 = 0.0, mB2 = 0.0;
+    double sxx1 = 0.0, sxx1e = 0.0, sxy2 = 0.0, sxy2w = 0.0, shear_h2 = 0.0, shear_q2 = 0.0;      // SMAG
+    double vort2 = 0.0, vdx2 = 0.0, vdy2 = 0.0, vvm2 = 0.0, d2v3_ = 0.0;                          // LEITH (d2v3_: row r - 3)
+    double hrat2 = 1.0;                                                                           // BOUND
+    double d2u2 = 0.0, d2v2 = 0.0, d2v3 = 0.0;                                                    // BIH
+    double tx3 = 0.0, ty3 = 0.0;                                               // stresses of row r - 3
+    load(ja - 2);
+    u1 = nu; v1 = nv; h1 = nh; ve1 = east(nv); he1 = east(nh); mh1 = nmT * nh; mB1 = nmB;
+    load(ja - 1);
+    for (int r = ja - 1; r <= jb + 3; ++r) {
+        const double u0 = nu, v0 = nv, h0 = nh, mT0 = nmT, mB0 = nmB, rK = nrK, rA = nrA;
+        if (r < jb + 3) load(r + 1);
+        const double ve0 = east(v0), he0 = east(h0), mh0 = mT0 * h0;
+        // tension at the h points of row r (:503-530)
+        const double dudx = g.DY_dxT * ((g.IdyCu * u0) - (g.IdyCu * west(u0)));
+        const double dvdy = g.DX_dyT * ((g.IdxCv * v0) - (g.IdxCv * v1));
+        const double xx0 = dudx - dvdy, xx0e = east(xx0);
+        // row r - 1: shearing strain (:513-547), thicknesses (:551-562)
+        const double dvdx = g.DY_dxBu * ((ve1 * g.IdyCv) - (v1 * g.IdyCv));
+        const double dudy = g.DX_dyBu * ((u0 * g.IdxCu) - (u1 * g.IdxCu));
+        const double slip = p.no_slip ? (2.0 - mB1) : mB1;
+        const double xy1 = slip * (dvdx + dudy);
+        const double hq1 = 0.25 * ((h1 + he0) + (he1 + h0));
+        const double hu1 = 0.5 * (mh1 + east(mh1)), hv1 = 0.5 * (mh1 + mh0);
+        const bool in1 = in_i && in_j(r - 1), in2 = in_i && in_j(r - 2);
+        double hrat1 = 1.0;
+        if (BOUND) {   // hrat_min (:730-737)
+            const double h_min = fmin(fmin(fmin(hu1, west(hu1)), hv1), hv2);
+            const double x = fmin(1.0, h_min / (h1 + p.h_neglect));
+            hrat1 = in1 ? x : 1.0;
+        }
+        double sxx0 = 0.0, sxx0e = 0.0, sxy1 = 0.0, sxy1w = 0.0, shear_h1 = 0.0, shear_q1 = 0.0;
+        if (SMAG) {    // Shear_mag at h (:710-720) and q points
+            sxx0 = sq(xx0); sxx0e = east(sxx0);
+            sxy1 = sq(xy1); sxy1w = west(sxy1);
+            shear_h1 = sqrt(sxx1 + 0.25 * ((sxy2w + sxy1) + (sxy1w + sxy2)));
+            shear_q1 = sqrt(0.25 * ((sxx1 + sxx0e) + (sxx1e + sxx0)) + sxy1);
+        }
+        double vort1 = 0.0, vdx1 = 0.0, vdy1 = 0.0, vvm1 = 0.0, d2_2 = 0.0, d2h2 = 0.0, gq2 = 0.0;
+        if (LEITH) {   // vorticity (:612-626), its gradients (:629-645) and Laplacian (:648-659)
+            vort1 = slip * (dvdx - dudy);
+            const double vx = g.DY_dxBu_v * ((vort1 * g.IdyCu) - (west(vort1) * g.IdyCu));
+            const double vy = g.DX_dyBu_v * ((vort1 * g.IdxCv) - (vort2 * g.IdxCv));
+            vdx1 = in1 ? vx : 0.0;
+            vdy1 = in_I && in_j(r - 1) ? vy : 0.0;
+            vvm1 = sqrt(sq(0.5 * (vdx1 + vdx2)) + sq(0.5 * (vdy1 + west(vdy1)))) + 0.0;
+            const double vdx2e = east(vdx2);
+            gq2 = sqrt(sq(0.5 * (vdx2 + vdx2e)) + sq(0.5 * (vdy2 + vdy1)));
+            const double x = g.DY_dxBu * ((vdx2e * g.IdyCv) - (vdx2 * g.IdyCv)) +
+                             g.DX_dyBu * ((vdy1 * g.IdxCu) - (vdy2 * g.IdxCu));
+            d2_2 = in_I && in_J(r - 2) ? x : 0.0;
+            d2h2 = 0.25 * ((d2_2 + west(d2v3_)) + (west(d2_2) + d2v3_));
+        }
+        double d2u1 = 0.0, d2v1 = 0.0;
+        if (BIH) {     // Del2u, Del2v of row r - 1 (:587-607), zero outside their ranges
+            const double x = g.Idx2dyCu * ((g.dx2q * xy1) - (g.dx2q * xy2)) +
+                             g.Idxdy2u * ((g.dy2h * xx1e) - (g.dy2h * xx1));
+            const double y = g.Idxdy2v * ((g.dy2q * xy1) - (g.dy2q * west(xy1))) -
+                             g.Idx2dyCv * ((g.dx2h * xx0) - (g.dx2h * xx1));
+            d2u1 = in_I && in_j(r - 1) ? x : 0.0;
+            d2v1 = in_i && in_J(r - 1) ? y : 0.0;
+        }
+        // row r - 2: viscosities at h (:743-863) and q points (:897-1023)
+        double Kh = p.Kh, Ah = p.Ah, Kq = p.Kh, Aq = p.Ah;
+        if (M::CL) {
+            double rem = 1.0;
+            const double Kh_top = hrat2 * (0.25 * area / 1.0), Ah_top = 0.0625 * (area * area) / 1.0;
+            if (SMAG && p.smag_Kh) {
+                Kh = fmax(Kh, smag_K * shear_h2);
+                Kq = fmax(Kq, smag_K * shear_q2);
+            }
+            if (LEITH) {
+                Kh = fmax(Kh, 1.0 * h3 * vvm2 * HV_INV_PI3);
+                Kq = fmax(Kq, 1.0 * h3 * gq2 * HV_INV_PI3);
+            }
+            Kh = fmax(Kh, 0.0);
+            Kq = fmax(Kq, 0.0);
+            double hmin_q = 1.0;
+            if (BOUND) {
+                hmin_q = 0.25 * ((hrat2 + east(hrat1)) + (east(hrat2) + hrat1));
+                if (lap) {
+                    const double part = 1.0 - Kh / Kh_top;
+                    rem = Kh >= Kh_top ? 0.0 : (Kh > 0.0 ? part : 1.0);
+                    Kh = Kh >= Kh_top ? Kh_top : Kh;
+                }
+                Kq = fmin(Kq, hmin_q * (0.25 * area / 1.0));
+            }
+            if (BIH) {
+                if (SMAG) {
+                    Ah = fmax(Ah, smag_A * shear_h2);
+                    Aq = fmax(Aq, smag_A * shear_q2);
+                }
+                if (LEITH) {
+                    Ah = fmax(Ah, 1.0 * h3 * h3 * fabs(d2h2) * HV_INV_PI6);
+                    Aq = fmax(Aq, 1.0 * h3 * h3 * fabs(d2_2) * HV_INV_PI6);
+                }
+                if (BOUND) {
+                    Ah = fmin(Ah, rem * hrat2 * Ah_top);
+                    Aq = fmin(Aq, hmin_q * Ah_top);
+                }
+            }
+        }
+        const bool ring2 = in_I && in_J(r - 2);   // and not in2
+        Kh = in2 ? Kh : (ring2 ? (M::CL ? rK : Kh_c) : 0.0);
+        if (BIH) Ah = in2 ? Ah : (ring2 ? (M::CL ? rA : Ah_c) : 0.0);
+        // its stresses times thickness (:807-895, :954-1053)
+        double tx2 = lap ? -(Kh * xx2) : 0.0, ty2 = lap ? -(Kq * xy2) : 0.0;
+        if (BIH) {
+            const double d_del2u = (g.IdyCu * d2u2) - (g.IdyCu * west(d2u2));
+            const double d_del2v = (g.IdxCv * d2v2) - (g.IdxCv * d2v3);
+            tx2 = tx2 + Ah * ((g.DY_dxT * d_del2u) - (g.DX_dyT * d_del2v));
+            ty2 = ty2 + Aq * ((g.DY_dxBu * ((east(d2v2) * g.IdyCv) - (d2v2 * g.IdyCv))) +
+                              (g.DX_dyBu * ((d2u1 * g.IdxCu) - (d2u2 * g.IdxCu))));
+        }
+        tx2 = tx2 * (h2 * g.red_xx);
+        ty2 = p.no_slip ? ty2 * (hq2 * g.red_xy) : ty2 * (hq2 * mB2 * g.red_xy);
+        // diffu of row r - 2 and diffv of row r - 3 (:1059-1078), zero outside their ranges
+        const double tx2e = east(tx2), ty3w = west(ty3);
+        if (r - 2 >= ja && r - 2 <= jb) {
+            const double x = ((g.IdxCu * ((g.dx2q * ty3) - (g.dx2q * ty2)) + g.IdyCu * ((g.dy2h * tx2) - (g.dy2h * tx2e))) *
+                              g.IareaCu) / (hu2 + p.h_neglect);
+            if (mine) (diffu + layer + row_of(r - 2))[col] = in_I && in_j(r - 2) ? x : 0.0;
+        }
+        if (r - 3 >= ja) {
+            const double x = ((g.IdyCv * ((g.dy2q * ty3w) - (g.dy2q * ty3)) - g.IdxCv * ((g.dx2h * tx3) - (g.dx2h * tx2))) *
+                              g.IareaCv) / (hv3 + p.h_neglect);
+            if (mine) (diffv + layer + row_of(r - 3))[col] = in_i && in_J(r - 3) ? x : 0.0;
+        }
+        tx3 = tx2; ty3 = ty2;
+        hv3 = hv2; hv2 = hv1; hu2 = hu1; hq2 = hq1; h2 = h1; mB2 = mB1;
+        xx2 = xx1; xx1 = xx0; xx1e = xx0e; xy2 = xy1;
+        if (SMAG) { sxx1 = sxx0; sxx1e = sxx0e; sxy2 = sxy1; sxy2w = sxy1w; shear_h2 = shear_h1; shear_q2 = shear_q1; }
+        if (LEITH) { vort2 = vort1; vdx2 = vdx1; vdy2 = vdy1; vvm2 = vvm1; d2v3_ = d2_2; }
+        if (BOUND) hrat2 = hrat1;
+        if (BIH) { d2v3 = d2v2; d2u2 = d2u1; d2v2 = d2v1; }
+        u1 = u0; v1 = v0; ve1 = ve0; h1 = h0; he1 = he0; mh1 = mh0; mB1 = mB0;
+    }
+}
+
 static HV make_hv(const mom6h_hor_visc_cs *cs)
 {
     HV p;
@@ -616,17 +739,43 @@ static HV make_hv(const mom6h_hor_visc_cs *cs)
 
 static bool closures_on(const mom6h_hor_visc_cs *cs) { return cs->smagorinsky || cs->leith || cs->better_bound; }
 
-// the tiled kernel's launch: 8-row tiles over the data domain, the layers
-// split so that a block walks about 15 of them
-static void launch_tile(const mom6h_hor_visc_cs *cs, const HV &p, const double *u, const double *v,
-                        const double *h, double *diffu, double *diffv, hipStream_t s)
+// the march's launch over the data domain: chunks of rows that leave about
+// four waves per SIMD, at least 8 (a chunk walks five rows more than it writes)
+template <bool SMAG, bool LEITH, bool BOUND, bool BIH>
+static void launch_march(const mom6h_hor_visc_cs *cs, const HV &p, const double *u, const double *v, const double *h,
+                         double *diffu, double *diffv, hipStream_t s)
 {
     const Dims &d = cs->d;
-    constexpr int TY = 8;
-    const int nkz = (d.nk + 14) / 15;
-    const dim3 grid((unsigned)((d.n1 + HT_X - 1) / HT_X), (unsigned)((d.n2 + TY - 1) / TY), (unsigned)nkz);
-    if (cs->biharmonic) k_hv_tile<true, TY><<<grid, 256, 0, s>>>(p, cs->g, u, v, h, diffu, diffv);
-    else k_hv_tile<false, TY><<<grid, 256, 0, s>>>(p, cs->g, u, v, h, diffu, diffv);
+    constexpr int OUT = HVMarch<SMAG, LEITH, BOUND, BIH>::OUT;
+    const int strips = (d.n1 + OUT - 1) / OUT;
+    int rows = (int)std::min(48LL, std::max(8LL, (long long)strips * d.n2 * d.nk / 4096));
+    int chunks = (d.n2 + rows - 1) / rows;
+    rows = (d.n2 + chunks - 1) / chunks;
+    chunks = (d.n2 + rows - 1) / rows;
+    const long long tasks = (long long)strips * chunks * d.nk;
+    k_hv_march<SMAG, LEITH, BOUND, BIH><<<(unsigned)((tasks + 3) / 4), 256, 0, s>>>(
+        p, cs->g, u, v, h, cs->ring_q, diffu, diffv, strips, chunks, rows);
+}
+
+template <bool SMAG, bool LEITH, bool BOUND>
+static void launch_march(const mom6h_hor_visc_cs *cs, const HV &p, const double *u, const double *v, const double *h,
+                         double *diffu, double *diffv, hipStream_t s)
+{
+    if (cs->biharmonic) launch_march<SMAG, LEITH, BOUND, true>(cs, p, u, v, h, diffu, diffv, s);
+    else launch_march<SMAG, LEITH, BOUND, false>(cs, p, u, v, h, diffu, diffv, s);
+}
+
+template <bool SMAG>
+static void launch_march(const mom6h_hor_visc_cs *cs, const HV &p, const double *u, const double *v, const double *h,
+                         double *diffu, double *diffv, hipStream_t s)
+{
+    if (cs->leith) {
+        if (cs->better_bound) launch_march<SMAG, true, true>(cs, p, u, v, h, diffu, diffv, s);
+        else launch_march<SMAG, true, false>(cs, p, u, v, h, diffu, diffv, s);
+    } else {
+        if (cs->better_bound) launch_march<SMAG, false, true>(cs, p, u, v, h, diffu, diffv, s);
+        else launch_march<SMAG, false, false>(cs, p, u, v, h, diffu, diffv, s);
+    }
 }
 
 // every metric the stencil reads constant over is-2..ie+2 x js-2..je+2
@@ -728,6 +877,22 @@ int mom6h_hor_visc(mom6h_hor_visc_cs *cs, const double *u, const double *v, cons
     const Dims &d = cs->d;
     hipStream_t s = (hipStream_t)stream;
     HV p = make_hv(cs);
+    if (cs->uniform && (!cs->biharmonic || cs->bih_uniform) && (!closures_on(cs) || cs->closure_uniform) && !cs->general) {
+        const unsigned nring = (unsigned)((ring_points(d) + 63) / 64);
+        if (closures_on(cs)) {
+            k_hv_ring<<<dim3(nring, d.nk), 64, 0, s>>>(p, u, v, h, cs->ring_q);
+            MOM6H_LAUNCH_CHECK();
+        }
+        if (cs->smagorinsky) launch_march<true>(cs, p, u, v, h, diffu, diffv, s);
+        else launch_march<false>(cs, p, u, v, h, diffu, diffv, s);
+        MOM6H_LAUNCH_CHECK();
+        if (closures_on(cs)) {
+            k_hv_keep_last<<<nring, 64, 0, s>>>(p, cs->ring_q);
+            MOM6H_LAUNCH_CHECK();
+        }
+        cs->calls++;
+        return MOM6H_OK;
+    }
     if (cs->biharmonic) {
         const int ni = d.iec - (d.isc - 1) + 1, nj = d.jec - (d.jsc - 1) + 1;
         dim3 b(64), g((ni + 63) / 64, nj, d.nk);
@@ -738,10 +903,7 @@ int mom6h_hor_visc(mom6h_hor_visc_cs *cs, const double *u, const double *v, cons
     if (closures_on(cs)) {
         k_hv_closures<<<g, b, 0, s>>>(p, u, v, h, diffu, diffv);
         MOM6H_LAUNCH_CHECK();
-        const int nring = (d.jec - d.jsc + 2) + (d.iec - d.isc + 1);
-        k_hv_keep_ring<<<(nring + 63) / 64, 64, 0, s>>>(p, u, v, h);
-    } else if (cs->uniform && (!cs->biharmonic || cs->bih_uniform) && !cs->general) {
-        launch_tile(cs, p, u, v, h, diffu, diffv, s);
+        k_hv_keep_ring<<<(ring_points(d) + 63) / 64, 64, 0, s>>>(p, u, v, h);
     } else {
         k_hv_main<<<g, b, 0, s>>>(p, u, v, h, diffu, diffv);
     }
@@ -764,6 +926,16 @@ int mom6h_hor_visc_set_closures(mom6h_hor_visc_cs *cs, int smagorinsky, int leit
         if (!cs->areaT) rc = dev_upload(&cs->areaT, areaT, n2);
         if (!rc && !cs->ring_Kh) rc = dev_alloc(&cs->ring_Kh, n2, true);
         if (!rc && !cs->ring_Ah) rc = dev_alloc(&cs->ring_Ah, n2, true);
+        if (!rc && !cs->ring_q) rc = dev_alloc(&cs->ring_q, (size_t)2 * cs->d.nk * ring_points(cs->d), false);
+        HVUniform &g = cs->g;
+        cs->closure_uniform = hv_uniform(cs->d, {{areaT, &g.areaT}});
+        if (leith) {
+            double dx = 0.0, dy = 0.0, idx = 0.0, idy = 0.0;
+            cs->closure_uniform = cs->closure_uniform &&
+                                  hv_uniform(cs->d, {{dxBu, &dx}, {dyBu, &dy}, {IdxBu, &idx}, {IdyBu, &idy}});
+            g.DY_dxBu_v = dy * idx;
+            g.DX_dyBu_v = dx * idy;
+        }
     }
     if (!rc && leith && !cs->dxBu) {
         rc = dev_upload(&cs->dxBu, dxBu, n2);
@@ -785,7 +957,7 @@ int mom6h_hor_visc_end(mom6h_hor_visc_cs *cs)
                       cs->IdyCv, cs->IdxCv, cs->IareaCu, cs->IareaCv, cs->mask2dT, cs->mask2dBu,
                       cs->reduction_xx, cs->reduction_xy, cs->dy2h, cs->dx2h, cs->dy2q, cs->dx2q,
                       cs->Idx2dyCu, cs->Idxdy2u, cs->Idx2dyCv, cs->Idxdy2v, cs->Del2u, cs->Del2v,
-                      cs->areaT, cs->dxBu, cs->dyBu, cs->IdxBu, cs->IdyBu, cs->ring_Kh, cs->ring_Ah})
+                      cs->areaT, cs->dxBu, cs->dyBu, cs->IdxBu, cs->IdyBu, cs->ring_Kh, cs->ring_Ah, cs->ring_q})
         dev_free(p);
     delete cs;
     return MOM6H_OK;

@@ -88,6 +88,35 @@ __device__ inline void batch_locate(const BatchMap &mp, int b, int &m, int &loca
     local = b - mp.first[q];
 }
 
+// The value of the lane to the west (lane - 1) and to the east (lane + 1): DPP
+// wave shifts, one VALU move per 32 bits.  Lane 0 (63) gets zero; every lane of
+// the wave must be active.
+template <int CTRL>
+__device__ __forceinline__ int lane_shift(int x)
+{
+    return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ __forceinline__ float lane_shift(float x)
+{
+    return __int_as_float(lane_shift<CTRL>(__float_as_int(x)));
+}
+template <int CTRL>
+__device__ __forceinline__ double lane_shift(double x)
+{
+    return __hiloint2double(lane_shift<CTRL>(__double2hiint(x)), lane_shift<CTRL>(__double2loint(x)));
+}
+template <typename T>
+__device__ __forceinline__ T west(T x)
+{
+    return lane_shift<0x138>(x);   // wave_shr:1
+}
+template <typename T>
+__device__ __forceinline__ T east(T x)
+{
+    return lane_shift<0x130>(x);   // wave_shl:1
+}
+
 __device__ inline double dmax(double a, double b) { return a > b ? a : b; }
 __device__ inline double dmin(double a, double b) { return a < b ? a : b; }
 
@@ -354,6 +383,7 @@ struct HVUniform {
     double DY_dxT, DX_dyT, DY_dxBu, DX_dyBu, IdyCu, IdxCu, IdyCv, IdxCv, IareaCu, IareaCv;
     double red_xx, red_xy, dy2h, dx2h, dy2q, dx2q;
     double Idx2dyCu, Idxdy2u, Idx2dyCv, Idxdy2v;
+    double areaT, DY_dxBu_v, DX_dyBu_v;   // the closures: areaT, and Leith's dyBu*IdxBu and dxBu*IdyBu
 };
 }  // namespace mom6h
 
@@ -372,12 +402,13 @@ struct mom6h_hor_visc_cs {
     int smagorinsky = 0, leith = 0, better_bound = 0;
     double *areaT = nullptr, *dxBu = nullptr, *dyBu = nullptr, *IdxBu = nullptr, *IdyBu = nullptr;
     // q-point Kh and Ah of the last layer of the previous call, read by the
-    // first layer's stress ring (zero before the first call)
-    double *ring_Kh = nullptr, *ring_Ah = nullptr;
+    // first layer's stress ring (zero before the first call); and, for the
+    // march, those of every layer of the call at the ring points (compact)
+    double *ring_Kh = nullptr, *ring_Ah = nullptr, *ring_q = nullptr;
     // every metric constant over the points the stencil reads (is-2..ie+2 x
-    // js-2..je+2): the values, for the tiled kernel; bih_uniform likewise for
-    // the four biharmonic metrics
-    int uniform = 0, bih_uniform = 0;
+    // js-2..je+2): the values, for the march; bih_uniform likewise for the four
+    // biharmonic metrics, closure_uniform for the closures'
+    int uniform = 0, bih_uniform = 0, closure_uniform = 0;
     int general = 0;         // use the general kernel even on a uniform grid
     mom6h::HVUniform g{};
 };
