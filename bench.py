@@ -78,7 +78,7 @@ STAGE_CALLS = {"transports": 2, "hor_visc": 2, "coriolis": 2, "vel_update": 2, "
 # and that kernel.  The barotropic stage brackets bt_nsteps+1 launches on the
 # second stream, so its events do not time a single kernel; it is reported in
 # "stages" only.
-ROOFLINE_KERNELS = {"momentum": "k_momentum", "vert_visc": "k_vert_visc_chunked",
+ROOFLINE_KERNELS = {"momentum": "k_momentum", "vert_visc": "k_vert_visc_split",
                     "continuity": "k_continuity_blk"}
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic_720x720x75.md")
 COUNTERS_FILE = os.path.join(ROOT, "profiles", "counters_720x720x75.md")
@@ -88,8 +88,8 @@ ROOFLINE_LIMIT = {
     "k_continuity_blk": "latency: one 12-wave block per CU, its set-up waiting on its loads, "
                         "serial k-order column folds and the barriers around them",
     "k_momentum": "VALU issue (bit-exact FP64 divisions)",
-    "k_vert_visc_chunked": "forward-sweep VALU issue and the memory queueing of the load-heavy "
-                           "sweeps at one wave per SIMD",
+    "k_vert_visc_split": "VALU issue (four exact divisions per level) and the tridiagonal recurrence's "
+                         "latency at three waves per SIMD",
 }
 
 

@@ -587,18 +587,6 @@ __device__ __forceinline__ void lds_walk(const T (*col)[FW], int nk, int lane, S
     for (; k0 < nk; ++k0) step(col[k0][lane]);
 }
 
-// Barrier of the block column path.  The waves of a block exchange data
-// through LDS only (nothing a block stores to global memory is read back by
-// it), so the barrier orders LDS operations alone: __syncthreads' workgroup
-// fence would also wait for every global store still in flight, a memory
-// round trip at the first barrier after the output stores.
-__device__ __forceinline__ void lds_barrier()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // Block-wide "any face has pred", for the predicates of the Newton iteration
 // and of BT_cont: every wave holds all the block's faces (FW = 32: twice) and
 // evaluates pred for each from the same operands (the column sums and parked

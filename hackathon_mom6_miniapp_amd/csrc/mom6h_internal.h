@@ -69,6 +69,18 @@ __device__ inline int xcd_tile(int b, int nb)
     return x < r ? x * (m + 1) + q : r * (m + 1) + (x - r) * m + q;
 }
 
+// Barrier of a block whose waves exchange data through LDS only (nothing that
+// one of them stores to global memory is read back by another): it orders LDS
+// operations alone.  __syncthreads' workgroup fence would also wait for every
+// global store still in flight, a memory round trip at the first barrier after
+// the output stores.
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Several grids (the members of an ensemble) in one launch: the blocks of
 // member m are first[m] .. first[m+1]-1, laid out as that member's own
 // launch would be (nbx x nby tiles, x fastest, then any further dimension).

@@ -167,7 +167,8 @@ __global__ void k_vert_visc(Dims d, double *__restrict__ u, double *__restrict__
 }
 
 
-// Chunked variant.  One thread per column; the only per-column scratch is one
+// Chunked variant (columns the level-split variant below does not take).  One
+// thread per column; the only per-column scratch is one
 // LDS slot per level, holding z_i(k) after sweep A and c1(k) after sweep B
 // (slot nk+1 holds z_i(nk+1) = 0).  Sweep B re-derives hvel from h and the input
 // velocity (reloaded) and leaves the forward-eliminated velocity in the
@@ -545,6 +546,373 @@ __device__ __forceinline__ void vv_body(const VVArgs<T> &p, int bx, int row, VVS
     if (act) *tb_out = t;
 }
 
+// Level-split variant, for columns of up to VV_SPLIT_MAX levels.  A block of
+// four waves owns 64 columns of one row; wave w holds a quarter of the levels
+// in registers (L slots, n of them in use) and reads them once, so nothing but
+// the state goes through memory and every division off the tridiagonal
+// recurrence runs in four waves side by side.  The two running sums (z_i from
+// the bottom, z_top from the top) go through LDS in the serial order: each wave
+// adds up the levels before its own again (a chain of adds costs less than
+// handing the sum on from wave to wave).  The recurrence passes from wave to
+// wave, down and back up, behind one barrier each, while the other blocks of
+// the CU (3 in FP64, 5 in FP32 at 75 levels) load and form their coefficients.
+//
+// The chunked kernel (one wave per SIMD, held there by its LDS column, and the
+// eliminated velocity written and read back: 2.8 GB a call) took 756 us per
+// FP64 call at 720x720x75 and 396 us in the FP32 form; this one 450 and 285 us
+// (1.6 GB, 3.5 TB/s, VALU 60% busy; FP32 73%): VALU issue and the recurrence's
+// latency at three waves per SIMD.  180x180x75: 76 -> 43 us, 471x363x50: 180 ->
+// 109, 300x260x25: 52 -> 31, 200x100x12: 21 -> 15; with drag at every level
+// 347x188x75 269 -> 97 (289 -> 122 with the coefficients stored).  Faster at every depth it takes; the chunked kernel
+// keeps the deeper columns (more slots would spill) and planes whose level
+// offsets pass 4 GiB.  One spilled value per level made it slower than the
+// chunked kernel (1170 us), hence the pins and fences below.
+constexpr int VV_W = 4;                       // waves (level groups) of a block
+constexpr int VV_SPLIT_MAX = 80;              // VV_W * the largest slot class
+constexpr int VV_HAND = 4;                    // LDS rows of the hand-over between waves
+constexpr int VV_G = 6;                       // levels whose divisions are interleaved (2 and 4 measured 1-3% slower)
+
+// slot classes (L slots, up to VV_W*L levels): few unused slots at any depth
+__host__ __device__ constexpr int vv_class(int nk)
+{
+    return nk <= 16 ? 4 : nk <= 28 ? 7 : nk <= 40 ? 10 : nk <= 52 ? 13 : nk <= 64 ? 16 : nk <= 76 ? 19 : 20;
+}
+constexpr int vv_nmin(int L) { return L == 4 ? 0 : L == 20 ? 19 : L - 3; }   // slots in use in every wave
+
+// columns the level-split kernel takes: its level offsets are 32-bit bytes
+inline bool vv_split_fits(const Dims &d)
+{
+    return d.nk <= VV_SPLIT_MAX && VV_SPLIT_MAX / VV_W * d.s2 * (long long)sizeof(double) < (1LL << 32);
+}
+
+template <typename T>
+__host__ __device__ constexpr size_t vv_split_lds(int nk)   // columns, rows that unused slots read, hand-over
+{
+    return (size_t)(nk + 4) * 64 * sizeof(VVSlot<T>) + (size_t)VV_HAND * 64 * sizeof(double);
+}
+
+// waves per SIMD that the registers of L slots leave room for without a spill
+template <typename T, bool RAY3>
+constexpr int vv_waves(int L)
+{
+    if (sizeof(T) == 4) return L > 16 ? 5 : L > 13 ? 6 : L > 10 ? 7 : 8;
+    if (RAY3) return L > 16 ? 2 : L > 10 ? 3 : L > 7 ? 4 : L > 4 ? 5 : 8;
+    return L > 13 ? 3 : L > 7 ? 4 : L > 4 ? 6 : 8;
+}
+
+// An array from a uniform address on, for accesses at a lane's byte offset plus
+// a uniform one (each below 4 GiB)
+template <typename T>
+struct LevelBuf {
+    __amdgpu_buffer_rsrc_t r;
+    using V = std::remove_const_t<T>;
+    using B = std::conditional_t<sizeof(V) == 8, unsigned __attribute__((ext_vector_type(2))), unsigned>;
+    __device__ __forceinline__ explicit LevelBuf(T *base)
+        : r(__builtin_amdgcn_make_buffer_rsrc((void *)base, 0, 0xffffffffu, 0x00027000))
+    {
+    }
+    __device__ __forceinline__ V load(unsigned lane_off, unsigned off) const
+    {
+        if constexpr (sizeof(V) == 8)
+            return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(r, lane_off, off, 0));
+        else
+            return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(r, lane_off, off, 0));
+    }
+    __device__ __forceinline__ void store(V x, unsigned lane_off, unsigned off) const
+    {
+        if constexpr (sizeof(V) == 8)
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(B, x), r, lane_off, off, 0);
+        else
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(B, x), r, lane_off, off, 0);
+    }
+};
+
+template <typename T, bool KEEP, bool RAY3, int L>
+__device__ __forceinline__ void vv_split(const VVArgs<T> &p, int bx, int row, double *lds)
+{
+    using C = T;                 // arithmetic of the coefficients (as in vv_body)
+    using ZT = VVSlot<T>;
+    constexpr int NMIN = vv_nmin(L);
+    const Dims &d = p.d;
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nk = d.nk;
+    const long long s = d.s2;
+    const bool is_u = (row & 1) != 0;
+    const int i = d.isc - (is_u ? 1 : 0) + bx * 64 + lane;
+    const int j = is_u ? d.jsc + (row - 1) / 2 : d.jsc - 1 + row / 2;
+    if (i > d.iec) return;       // the same lanes in every wave
+    const long long c2 = IX2(d, i, j);
+    const int q = nk / VV_W, r = nk % VV_W;
+    const int n = q + (w < r ? 1 : 0);                 // this wave's levels k1 .. k1+n-1
+    const int k1 = w * q + (w < r ? w : r) + 1;
+    double *Hs = lds + lane;                           // hand-over rows
+    ZT *Zs = reinterpret_cast<ZT *>(lds + VV_HAND * 64) + lane;
+    // slot c's level in memory (unused slots re-read the last level) and in LDS
+    // (unused slots read what is there and write nothing)
+    auto used = [&](int c) { return c < NMIN || c < n; };
+    auto kmem = [&](int c) { return used(c) ? k1 + c : nk; };
+    auto Z = [&](int k) -> ZT & { return Zs[(k - 1) * 64]; };
+    ZT *Zw = &Z(k1);
+    // An empty asm on a value keeps its computation where it stands: moved to
+    // its use, behind a barrier, it would hold its operands' registers instead.
+    // A fence after every VV_G levels bounds what is interleaved.
+    auto fence = [](int c) __attribute__((always_inline)) { if (c % VV_G == 0) __builtin_amdgcn_sched_barrier(0); };
+    auto pin = [](auto &x) __attribute__((always_inline)) { asm volatile("" : "+v"(x)); };
+
+    // buffer loads and stores: the column is one 32-bit offset, the level a
+    // scalar one (flat addresses would be kept in registers from the loads of
+    // a velocity to its store)
+    const int kb = k1 < nk ? k1 : nk;                  // level of the buffers' first plane
+    const unsigned oT = (unsigned)(c2 * sizeof(T));
+    const unsigned oN = (unsigned)((is_u ? c2 + 1 : c2 + d.n1) * sizeof(T));
+    auto plane = [&](int c, size_t size) { return (unsigned)((kmem(c) - kb) * s * size); };
+    const LevelBuf<const T> h(p.h + (kb - 1) * s);
+    const LevelBuf<T> vel((is_u ? p.u : p.v) + (kb - 1) * s);
+    T v[L];
+    C ha[L], hb[L];
+#pragma unroll
+    for (int c = 0; c < L; ++c) {
+        ha[c] = h.load(oT, plane(c, sizeof(T)));
+        hb[c] = h.load(oN, plane(c, sizeof(T)));
+        v[c] = vel.load(oT, plane(c, sizeof(T)));
+    }
+    const double m = (is_u ? p.mask2dCu : p.mask2dCv)[c2];
+    const double *tau = is_u ? p.taux : p.tauy, *rayb = is_u ? p.ray_u : p.ray_v;
+    const double sfc = tau ? p.dt / 1035.0 * tau[c2] * m : 0.0;
+    const double Ray_bot = rayb ? rayb[c2] : 0.0;
+    const double h_neglect = 1.0e-10;
+    const C hn = (C)h_neglect;
+    const C Kv = (C)p.Kv, Kv_ml = (C)p.Kv_ml, Kv_extra_bbl = (C)p.Kv_extra_bbl, Hmix = (C)p.Hmix;
+    const double dt = p.dt;
+    const C I_Hbbl = C(1.0) / ((C)p.Hbbl + hn);
+    auto cdiv = [](C num, C den) __attribute__((always_inline)) -> C {   // as in vv_body
+        if constexpr (sizeof(C) == 4) return num * __builtin_amdgcn_rcpf(den);
+        else return num / den;
+    };
+
+    // harmonic-mean thickness into LDS; the arithmetic mean and the upwind
+    // choice (:165-176) stay in registers
+    C hv[L];
+    unsigned upw = 0;
+#pragma unroll
+    for (int c = 0; c < L; ++c) {
+        hv[c] = C(0.5) * (hb[c] + ha[c]);
+        const C h_delta = hb[c] - ha[c];
+        upw |= (v[c] * h_delta < C(0.0)) ? 1u << c : 0u;
+        const C hh = cdiv(C(2.0) * ha[c] * hb[c], ha[c] + hb[c] + hn);
+        if (used(c)) Zw[c * 64] = hh;
+        pin(upw);
+        pin(hv[c]);
+        fence(c);
+    }
+    lds_barrier();
+    // z_i(k+1) (bottom-up sum), the bottom taper botfn(z_i(k+1)) and hvel(k)
+    C bf[L];
+    {
+        C zi = C(0.0);
+#pragma unroll 8
+        for (int k = nk; k >= k1 + n; --k) zi = zi + Z(k) * I_Hbbl;
+#pragma unroll
+        for (int c = L - 1; c >= 0; --c) {
+            const C hh = Zw[c * 64];
+            bf[c] = cdiv(C(1.0), C(1.0) + C(0.09) * zi * zi * zi * zi * zi * zi);
+            if (used(c)) zi = zi + hh * I_Hbbl;
+            const C blend = (C(1.0) - bf[c]) * hh + bf[c] * hv[c];
+            hv[c] = (upw >> c & 1u) ? blend : hh;
+            fence(c);
+        }
+    }
+    lds_barrier();               // every wave has read the harmonic means
+#pragma unroll
+    for (int c = 0; c < L; ++c)
+        if (used(c)) Zw[c * 64] = hv[c];
+    lds_barrier();
+    // coupling coefficient a(k+1) (:184-202) from z_top (top-down sum through
+    // level k), botfn(z_i(k+1)), hvel(k) and hvel(k+1); replaces bf
+    {
+        C z_top = C(0.0);
+#pragma unroll 8
+        for (int k = 1; k < k1; ++k) z_top = z_top + Z(k);
+        const C hv_below = Z(k1 + n <= nk ? k1 + n : nk);
+        // in groups of VV_G levels: the mixed-layer taper's divisions (:188-192)
+        // only in a group where some column has a level above Hmix, then the
+        // group's couplings side by side
+#pragma unroll
+        for (int c0 = 0; c0 < L; c0 += VV_G) {
+            C kvt[VV_G], zt[VV_G];
+            bool taper = false;
+#pragma unroll
+            for (int g = 0; g < VV_G; ++g) {
+                if (c0 + g < L) z_top = z_top + hv[c0 + g];
+                zt[g] = z_top;
+                taper = taper || (z_top < Hmix);
+                kvt[g] = Kv;
+            }
+            if (__any(taper)) {
+#pragma unroll
+                for (int g = 0; g < VV_G; ++g) {
+                    C t = Kv + (Kv_ml - Kv) * (C(1.0) - zt[g] / Hmix);
+                    pin(t);      // a select, not a branch per level
+                    kvt[g] = (zt[g] < Hmix) ? t : Kv;
+                }
+            }
+#pragma unroll
+            for (int g = 0; g < VV_G; ++g) {
+                const int c = c0 + g;
+                if (c >= L) break;
+                const C hvn = (c == L - 1 || (c >= NMIN - 1 && c + 1 >= n)) ? hv_below : hv[c < L - 1 ? c + 1 : c];
+                bf[c] = cdiv(kvt[g] + Kv_extra_bbl * bf[c], C(0.5) * (hvn + hv[c] + hn));
+            }
+#pragma unroll
+            for (int c = c0; c < (c0 + VV_G < L ? c0 + VV_G : L); ++c) pin(bf[c]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (n > 0 && k1 + n - 1 == nk) {   // a(nk+1) (:205-206)
+#pragma unroll
+            for (int c = (NMIN > 0 ? NMIN - 1 : 0); c < L; ++c)
+                if (c == n - 1) bf[c] = (Kv + Kv_extra_bbl) / (C(0.5) * hv[c] + hn);
+        }
+    }
+    C *an = bf;                  // a(k+1)
+    const bool act = m > 0.0;
+    if (KEEP) {
+        const LevelBuf<double> a_out((is_u ? p.a_u : p.a_v) + kb * s);
+        const LevelBuf<double> hu_out((is_u ? p.h_u : p.h_v) + (kb - 1) * s);
+        const unsigned oD = (unsigned)(c2 * sizeof(double));
+        if (w == 0) (is_u ? p.a_u : p.a_v)[c2] = 0.0;
+#pragma unroll
+        for (int c = 0; c < L; ++c) {
+            if (used(c)) {
+                a_out.store(act ? (double)an[c] : 0.0, oD, plane(c, sizeof(double)));
+                hu_out.store(act ? (double)hv[c] + h_neglect : h_neglect, oD, plane(c, sizeof(double)));
+            }
+        }
+    }
+    double ray[RAY3 ? L : 1];
+    if constexpr (RAY3) {
+        const LevelBuf<const double> ray3((is_u ? p.ray_u3 : p.ray_v3) + (kb - 1) * s);
+#pragma unroll
+        for (int c = 0; c < L; ++c)
+            ray[c] = ray3.load((unsigned)(c2 * sizeof(double)), plane(c, sizeof(double)));
+    }
+
+    // ---- forward elimination, top-down (:430-444), wave after wave ----
+    for (int t = 0; t < w; ++t) lds_barrier();
+    double vbot = 0.0, abot = 0.0;
+    {
+        double d1 = 0.0, b1 = 0.0, vprev = sfc, a_k = 0.0, dta = 1.0;   // level 1: dta*vprev is the surface stress
+        if (w > 0) {
+            d1 = Hs[0]; b1 = Hs[64]; vprev = Hs[128]; a_k = Hs[192];
+            dta = dt * a_k;
+        }
+#pragma unroll
+        for (int c = 0; c < L; ++c) {
+            C ax = an[c], hx = hv[c];
+            T vx = v[c];
+            pin(ax);
+            pin(hx);
+            pin(vx);
+            if (used(c)) {
+                const double hu_k = (double)hx + h_neglect;
+                const double a_n = (double)ax;
+                double t = a_k * d1;
+                if constexpr (RAY3) t = ray[c] + t;
+                else if (c >= NMIN - 1 && k1 + c == nk) t = Ray_bot + t;
+                const double b_denom_1 = hu_k + dt * t;
+                ax = (C)(dta * b1);                 // c1(k)
+                const double dtan = dt * a_n;
+                b1 = 1.0 / (b_denom_1 + dtan);
+                d1 = b_denom_1 * b1;
+                vprev = (hu_k * (double)vx + dta * vprev) * b1;
+                vx = (T)vprev;
+                a_k = a_n;
+                dta = dtan;
+            }
+            pin(ax);
+            pin(vx);
+            an[c] = ax;
+            v[c] = vx;
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        vbot = vprev;
+        abot = a_k;
+        if (w < VV_W - 1) { Hs[0] = d1; Hs[64] = b1; Hs[128] = vprev; Hs[192] = a_k; }
+    }
+    for (int t = w; t < 2 * (VV_W - 1) - w; ++t) lds_barrier();
+    // ---- back substitution, bottom-up (:447-449) ----
+    {
+        const bool bottom = n > 0 && k1 + n - 1 == nk;
+        double vnext = vbot, c1n = 0.0;
+        if (!bottom) { vnext = Hs[0]; c1n = Hs[64]; }
+#pragma unroll
+        for (int c = L - 1; c >= 0; --c) {
+            T vx = v[c];
+            if (used(c)) {
+                if (!(c >= NMIN - 1 && k1 + c == nk)) vnext = (double)vx + c1n * vnext;
+                c1n = (double)an[c];
+                vx = (T)vnext;
+            }
+            v[c] = vx;
+        }
+        if (w > 0 && n > 0) { Hs[0] = vnext; Hs[64] = c1n; }
+        if (act) {
+#pragma unroll
+            for (int c = 0; c < L; ++c) {
+                const T vx = v[c];
+                if (used(c)) vel.store(vx, oT, plane(c, sizeof(T)));
+            }
+        }
+        // bottom stress (:452-458)
+        const double RHO_0 = 1035.0;
+        double *tb = is_u ? p.taux_bot : p.tauy_bot;
+        if (bottom) {
+            const double t = RHO_0 * vbot * abot;
+            if (RAY3) Hs[128] = t;
+            else if (act) tb[c2] = t + RHO_0 * Ray_bot * vbot;
+        }
+        for (int t = 0; t < w; ++t) lds_barrier();
+        if constexpr (RAY3) {   // + sum_k RHO_0*Ray(k)*u(k) of the solved column, in k order
+#pragma unroll
+            for (int c = 0; c < L; ++c)
+                if (used(c)) Zw[c * 64] = RHO_0 * ray[c] * (double)v[c];
+            lds_barrier();
+            if (w == 0) {
+                double t = Hs[128];
+#pragma unroll 8
+                for (int k = 1; k <= nk; ++k) t = t + Z(k);
+                if (act) tb[c2] = t;
+            }
+        }
+    }
+}
+
+// one grid, tiles renumbered per XCD
+template <typename T, bool KEEP, bool RAY3, int L>
+__global__ void __launch_bounds__(64 * VV_W) __attribute__((amdgpu_waves_per_eu(vv_waves<T, RAY3>(L))))
+k_vert_visc_split(VVArgs<T> p)
+{
+    extern __shared__ double Zs_raw[];
+    const int tile = xcd_tile(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
+    vv_split<T, KEEP, RAY3, L>(p, tile % gridDim.x, tile / gridDim.x, Zs_raw);
+}
+
+template <typename T, bool KEEP, bool RAY3>
+void vv_split_launch(const VVArgs<T> &p, dim3 g, hipStream_t s)
+{
+    const size_t lds = vv_split_lds<T>(p.d.nk);
+    const dim3 b(64 * VV_W);
+    switch (vv_class(p.d.nk)) {
+    case 4: k_vert_visc_split<T, KEEP, RAY3, 4><<<g, b, lds, s>>>(p); break;
+    case 7: k_vert_visc_split<T, KEEP, RAY3, 7><<<g, b, lds, s>>>(p); break;
+    case 10: k_vert_visc_split<T, KEEP, RAY3, 10><<<g, b, lds, s>>>(p); break;
+    case 13: k_vert_visc_split<T, KEEP, RAY3, 13><<<g, b, lds, s>>>(p); break;
+    case 16: k_vert_visc_split<T, KEEP, RAY3, 16><<<g, b, lds, s>>>(p); break;
+    case 19: k_vert_visc_split<T, KEEP, RAY3, 19><<<g, b, lds, s>>>(p); break;
+    default: k_vert_visc_split<T, KEEP, RAY3, 20><<<g, b, lds, s>>>(p); break;
+    }
+}
+
 // one grid, tiles renumbered per XCD
 template <typename T, bool KEEP, bool RAY3 = false>
 // FP64: one wave per SIMD (the LDS column), registers up to 512 with AGPRs;
@@ -571,6 +939,27 @@ k_vert_visc_batch(const VVArgs<T> *__restrict__ args, BatchMap mp)
     vv_body<T, false>(p, local % mp.nbx[m], local / mp.nbx[m], Zs);
 }
 
+// the same with level-split members only
+template <typename T>
+__global__ void __launch_bounds__(64 * VV_W) __attribute__((amdgpu_waves_per_eu(vv_waves<T, false>(20))))
+k_vert_visc_split_batch(const VVArgs<T> *__restrict__ args, BatchMap mp)
+{
+    extern __shared__ double Zs_raw[];
+    int m, local;
+    batch_locate(mp, xcd_tile(blockIdx.x, gridDim.x), m, local);
+    const VVArgs<T> p = args[m];
+    const int bx = local % mp.nbx[m], row = local / mp.nbx[m];
+    switch (vv_class(p.d.nk)) {
+    case 4: vv_split<T, false, false, 4>(p, bx, row, Zs_raw); break;
+    case 7: vv_split<T, false, false, 7>(p, bx, row, Zs_raw); break;
+    case 10: vv_split<T, false, false, 10>(p, bx, row, Zs_raw); break;
+    case 13: vv_split<T, false, false, 13>(p, bx, row, Zs_raw); break;
+    case 16: vv_split<T, false, false, 16>(p, bx, row, Zs_raw); break;
+    case 19: vv_split<T, false, false, 19>(p, bx, row, Zs_raw); break;
+    default: vv_split<T, false, false, 20>(p, bx, row, Zs_raw); break;
+    }
+}
+
 // The mixed-precision form: FP32 u, v, h in memory, FP64 solve; the
 // coefficients stay on chip (the LDS kernel only).
 int vert_visc_f32(mom6h_vert_visc_cs *cs, float *u, float *v, const float *h, double dt, const double *taux,
@@ -580,12 +969,16 @@ int vert_visc_f32(mom6h_vert_visc_cs *cs, float *u, float *v, const float *h, do
     const int ni = d.iec - d.isc + 2;
     const int rows = (d.jec - d.jsc + 1) + (d.jec - d.jsc + 2);
     const size_t lds = (size_t)(d.nk + 1) * 64 * sizeof(VVSlot<float>);
+    const dim3 g((ni + 63) / 64, rows);
     MOM6H_REQUIRE((long long)lds <= cs->max_lds, "vert_visc (FP32 state): nk = %d exceeds the LDS column (%lld B)",
                   d.nk, cs->max_lds);
     VVArgs<float> p{d, u, v, h, dt, taux, tauy, ray_u_bot, ray_v_bot, cs->mask2dCu, cs->mask2dCv,
                     cs->a_u, cs->a_v, cs->h_u, cs->h_v, cs->taux_bot, cs->tauy_bot, cs->Kv, cs->Kv_ml,
                     cs->Kv_extra_bbl, cs->Hmix, cs->Hbbl};
-    k_vert_visc_chunked<float, false><<<dim3((ni + 63) / 64, rows), dim3(64), lds, stream>>>(p);
+    if (vv_split_fits(d))
+        vv_split_launch<float, false, false>(p, g, stream);
+    else
+        k_vert_visc_chunked<float, false><<<g, dim3(64), lds, stream>>>(p);
     MOM6H_LAUNCH_CHECK();
     return MOM6H_OK;
 }
@@ -597,8 +990,10 @@ int vert_visc_batch(const VVArgs<T> *d_args, const VVArgs<T> *h_args, int n, lon
     BatchMap mp{};
     mp.n = n;
     int nk_max = 1;
+    bool split = true;
     for (int m = 0; m < n; ++m) {
         const Dims &d = h_args[m].d;
+        split = split && vv_split_fits(d);
         mp.nbx[m] = (d.iec - d.isc + 2 + 63) / 64;
         mp.nby[m] = (d.jec - d.jsc + 1) + (d.jec - d.jsc + 2);
         mp.first[m + 1] = mp.first[m] + mp.nbx[m] * mp.nby[m];
@@ -606,7 +1001,10 @@ int vert_visc_batch(const VVArgs<T> *d_args, const VVArgs<T> *h_args, int n, lon
     }
     const size_t lds = (size_t)(nk_max + 1) * 64 * sizeof(VVSlot<T>);
     MOM6H_REQUIRE((long long)lds <= max_lds, "vert_visc batch: nk = %d exceeds the LDS column", nk_max);
-    k_vert_visc_batch<T><<<(unsigned)mp.first[n], 64, lds, s>>>(d_args, mp);
+    if (split)
+        k_vert_visc_split_batch<T><<<(unsigned)mp.first[n], 64 * VV_W, vv_split_lds<T>(nk_max), s>>>(d_args, mp);
+    else
+        k_vert_visc_batch<T><<<(unsigned)mp.first[n], 64, lds, s>>>(d_args, mp);
     MOM6H_LAUNCH_CHECK();
     return MOM6H_OK;
 }
@@ -673,7 +1071,11 @@ int mom6h_vert_visc(mom6h_vert_visc_cs *cs, double *u, double *v, const double *
                  cs->a_u, cs->a_v, cs->h_u, cs->h_v, cs->taux_bot, cs->tauy_bot, cs->Kv, cs->Kv_ml,
                  cs->Kv_extra_bbl, cs->Hmix, cs->Hbbl};
         const dim3 g((ni + 63) / 64, rows);
-        if (cs->keep_coefs)
+        if (vv_split_fits(d) && cs->keep_coefs)
+            vv_split_launch<double, true, false>(p, g, (hipStream_t)stream);
+        else if (vv_split_fits(d))
+            vv_split_launch<double, false, false>(p, g, (hipStream_t)stream);
+        else if (cs->keep_coefs)
             k_vert_visc_chunked<double, true><<<g, dim3(64), lds, (hipStream_t)stream>>>(p);
         else
             k_vert_visc_chunked<double, false><<<g, dim3(64), lds, (hipStream_t)stream>>>(p);
@@ -707,7 +1109,11 @@ int mom6h_vert_visc_ray3d(mom6h_vert_visc_cs *cs, double *u, double *v, const do
                      cs->a_u, cs->a_v, cs->h_u, cs->h_v, cs->taux_bot, cs->tauy_bot, cs->Kv, cs->Kv_ml,
                      cs->Kv_extra_bbl, cs->Hmix, cs->Hbbl, ray_u, ray_v};
     const dim3 g((ni + 63) / 64, rows);
-    if (cs->keep_coefs)
+    if (vv_split_fits(d) && cs->keep_coefs)
+        vv_split_launch<double, true, true>(p, g, (hipStream_t)stream);
+    else if (vv_split_fits(d))
+        vv_split_launch<double, false, true>(p, g, (hipStream_t)stream);
+    else if (cs->keep_coefs)
         k_vert_visc_chunked<double, true, true><<<g, dim3(64), lds, (hipStream_t)stream>>>(p);
     else
         k_vert_visc_chunked<double, false, true><<<g, dim3(64), lds, (hipStream_t)stream>>>(p);
