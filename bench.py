@@ -79,14 +79,14 @@ STAGE_CALLS = {"transports": 2, "hor_visc": 2, "coriolis": 2, "vel_update": 2, "
 # second stream, so its events do not time a single kernel; it is reported in
 # "stages" only.
 ROOFLINE_KERNELS = {"momentum": "k_momentum", "vert_visc": "k_vert_visc_split",
-                    "continuity": "k_continuity_blk"}
+                    "continuity": "k_continuity_split"}
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic_720x720x75.md")
 COUNTERS_FILE = os.path.join(ROOT, "profiles", "counters_720x720x75.md")
 FP64_PEAK_TFLOPS = 78.6   # MI355X FP64 vector
 # what binds each roofline kernel (from its counters and per-wave time stamps)
 ROOFLINE_LIMIT = {
-    "k_continuity_blk": "latency: one 12-wave block per CU, its set-up waiting on its loads, "
-                        "serial k-order column folds and the barriers around them",
+    "k_continuity_split": "VALU issue and, at two waves per SIMD, the latency of dependent FP64 "
+                          "operations (k-order column sums handed from wave to wave)",
     "k_momentum": "VALU issue (bit-exact FP64 divisions)",
     "k_vert_visc_split": "VALU issue (four exact divisions per level) and the tridiagonal recurrence's "
                          "latency at three waves per SIMD",

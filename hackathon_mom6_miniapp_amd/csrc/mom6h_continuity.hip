@@ -330,8 +330,8 @@ __global__ void k_mass_flux(Dims d, const double *__restrict__ u, const double *
 }
 
 // ----------------------------------------------------- block column path ---
-// A block of CW wavefronts owns CF = 64 consecutive faces I0-1 .. I0+62
-// (one face per lane, the same face in every wavefront) and all their levels:
+// The meridional pass.  A block of CW wavefronts owns CF = 64 consecutive faces
+// of a row (one face per lane, the same face in every wavefront) and all their levels:
 // wavefront w holds levels w*K+1 .. w*K+K of its lane's face in registers (u,
 // the PPM edges and thickness of both neighbouring cells, the layer transport
 // and marginal thickness of the last evaluation).  Every pass over the columns
@@ -341,10 +341,7 @@ __global__ void k_mass_flux(Dims d, const double *__restrict__ u, const double *
 // one lane per face -- a sequential sum costs 64 faces one add per level.
 // The Newton logic of a face runs redundantly in every wavefront on the same
 // values, so all copies agree; the block keeps iterating while any face
-// needs another evaluation.  The block updates the 63 cells I0 .. I0+62, whose
-// convergence needs the transport at the face to the west (the neighbouring
-// lane); neighbouring blocks overlap by one face, which both evaluate
-// identically and only one writes.
+// needs another evaluation.
 constexpr int CF = 64;
 
 
@@ -352,6 +349,8 @@ __device__ __forceinline__ double vabs(double x) { return fabs(x); }
 __device__ __forceinline__ float vabs(float x) { return fabsf(x); }
 __device__ __forceinline__ double vsign1(double s) { return copysign(1.0, s); }
 __device__ __forceinline__ float vsign1(float s) { return copysignf(1.0f, s); }
+__device__ __forceinline__ double vfma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float vfma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 template <typename T>
 __device__ __forceinline__ T vmax(T a, T b) { return a > b ? a : b; }
 template <typename T>
@@ -428,6 +427,25 @@ __device__ __forceinline__ void ppm_limit(int monotonic, double hi, double h_min
             }
         }
     }
+}
+
+// whether the limiter changes the cell's edges (straight-line, so that a group
+// of levels takes the limiter in one branch; CW84's always runs)
+__device__ __forceinline__ bool ppm_limits(int monotonic, double hi, double h_min, double hl, double hr)
+{
+    const float curv = (float)(3.0 * ((hl + hr) - 2.0 * hi));
+    const float dh = (float)(hr - hl);
+    const double lhs = (double)(12.0f * curv) * (hi - h_min);
+    const float rhs = curv * curv + 3.0f * (dh * dh);
+    return monotonic || ((curv > 0.0f) & (fabsf(dh) < curv) & ((hi <= h_min) | (lhs < (double)rhs)));
+}
+__device__ __forceinline__ bool ppm_limits(int monotonic, float hi, float h_min, float hl, float hr)
+{
+    const float curv = 3.0f * ((hl + hr) - 2.0f * hi);
+    const float dh = hr - hl;
+    const float lhs = (12.0f * curv) * (hi - h_min);
+    const float rhs = curv * curv + 3.0f * (dh * dh);
+    return monotonic || ((curv > 0.0f) & (fabsf(dh) < curv) & ((hi <= h_min) | (lhs < rhs)));
 }
 
 // The same limiters entirely in FP32 (the mixed-precision form)
@@ -528,15 +546,12 @@ struct ColRegs {
 // Newton iteration's starting point for a second iteration).
 template <typename T>
 constexpr int walk_batch = 4;   // rows per batch of a column walk (two batches in flight)
-// FW = faces per block (64: one level group per wave; 32: two, lanes 0-31
-// and 32-63 holding the same faces at different levels).
-template <typename T, int CW, int K, int FW = CF>
+template <typename T, int CW, int K>
 struct ContShared {
-    static constexpr int L = CW * (64 / FW) * K;
+    static constexpr int L = CW * K, FW = CF;
     T U[L][FW], S0[L][FW], S1[L][FW], R[9][FW];
     // per-face 2D values, loaded with the block's set-up loads and parked here
-    // until they are used rather than held in registers: P[0] = dt*IareaT of
-    // the lane's cell (x), P[1] = dxCu of its face, P[2] = its barotropic
+    // until they are used rather than held in registers: P[1] = dxCu of its face, P[2] = its barotropic
     // transport target, P[3] = dt*min(IareaT) of its two cells, P[4], P[5] =
     // dxT of cells 0 and 1; P[6], P[7] = du_eval and sum_dyhm of the face's
     // Newton iteration, kept over the output stores for BT_cont
@@ -588,7 +603,7 @@ __device__ __forceinline__ void lds_walk(const T (*col)[FW], int nk, int lane, S
 }
 
 // Block-wide "any face has pred", for the predicates of the Newton iteration
-// and of BT_cont: every wave holds all the block's faces (FW = 32: twice) and
+// and of BT_cont: every wave holds all the block's faces and
 // evaluates pred for each from the same operands (the column sums and parked
 // 2D values in LDS, and what every wave derives from them by the same
 // instructions), so one wave's vote is the block's and needs no barrier (an
@@ -637,49 +652,63 @@ __device__ __forceinline__ float col_sum(const float (*col)[FW], int nk, int lan
     return acc;
 }
 
-// Y = false: the zonal pass.  A block covers the faces I0-1 .. I0+62 of row j
-// and also updates the thickness of cells I0 .. I0+62 (the convergence needs
-// the neighbouring lane's transport).  Y = true: the meridional pass, the same
-// algorithm across the rows: a block covers the faces (i, J), i = i0 .. i0+63,
-// of one face row J (lanes still run along i, so every load stays coalesced);
-// its convergence is a separate kernel (the faces J-1 belong to another block).
-//
-// FW = 32: a block covers 32 faces and each wave two level groups (lanes
-// 0-31 and 32-63), so a block needs half the registers and LDS of FW = 64 and
-// two blocks share a CU: one block's loads, folds and barriers overlap the
-// other's flux passes.  Both halves of a wave run the Newton logic of the same
-// face (the same inputs, so the same decisions); the column folds are done by
-// whole waves, both halves folding the same column (no divergence) and
-// storing the same value.
+// Face areas and limiting transports of set_zonal_BT_cont (:1064-1121) at one
+// face, from the sums at du0, duL and duR
+template <typename T>
+__device__ __forceinline__ void bt_cont_store(const ContArgsT<T> &a, long long c2, T du0, T FAmt_0, T duL, T uhtot_L,
+                                              T FAmt_L, T duR, T uhtot_R, T FAmt_R)
+{
+    T FA_0 = FAmt_0, FA_avg = FAmt_0;
+    if ((duL - du0) != T(0.0)) FA_avg = uhtot_L / (duL - du0);
+    if (FA_avg > vmax(FA_0, FAmt_L)) FA_avg = vmax(FA_0, FAmt_L);
+    else if (FA_avg < vmin(FA_0, FAmt_L)) FA_0 = FA_avg;
+    a.FA_u_W0[c2] = (double)FA_0;
+    a.FA_u_WW[c2] = (double)FAmt_L;
+    a.uBT_WW[c2] = (double)((vabs(FA_0 - FAmt_L) <= (T)1e-12f * FA_0)
+                                ? T(0.0)
+                                : (T(1.5) * (duL - du0)) * ((FAmt_L - FA_avg) / (FAmt_L - FA_0)));
+    FA_0 = FAmt_0;
+    FA_avg = FAmt_0;
+    if ((duR - du0) != T(0.0)) FA_avg = uhtot_R / (duR - du0);
+    if (FA_avg > vmax(FA_0, FAmt_R)) FA_avg = vmax(FA_0, FAmt_R);
+    else if (FA_avg < vmin(FA_0, FAmt_R)) FA_0 = FA_avg;
+    a.FA_u_E0[c2] = (double)FA_0;
+    a.FA_u_EE[c2] = (double)FAmt_R;
+    a.uBT_EE[c2] = (double)((vabs(FAmt_R - FA_0) <= (T)1e-12f * FA_0)
+                                ? T(0.0)
+                                : (T(1.5) * (duR - du0)) * ((FAmt_R - FA_avg) / (FAmt_R - FA_0)));
+}
+
+// The meridional pass: a block covers the faces (i, J), i = i0 .. i0+63, of one
+// face row J (lanes run along i, so every load stays coalesced); its
+// convergence is a separate kernel (the faces J-1 belong to another block).
+// The cell across the face is another row's, so each lane keeps both cells'
+// terms of every level, and the levels spread over 8 or 12 waves.
 //
 // FP32 form: the Newton stopping test of zonal_flux_adjust also accepts a
 // residual at the rounding level of the layer fluxes (4 ulp of sum |uh_k| of
 // the first pass); the FP64 tolerance of 1e-12 m lies below what FP32 sums
 // resolve, and the iteration would otherwise run to its 20-pass limit.
-template <typename T, bool Y, int CW, int K, int FW, bool EVEN>
-__device__ __forceinline__ void continuity_body(const ContArgsT<T> &a, int monotonic, unsigned bx, unsigned by,
-                                                bool pf_on = false)
+template <typename T, int CW, int K, bool EVEN>
+__device__ __forceinline__ void continuity_body(const ContArgsT<T> &a, int monotonic, unsigned bx, unsigned by)
 {
     extern __shared__ double smem_raw[];
     constexpr bool F32 = sizeof(T) == 4;
-    constexpr int L = ContShared<T, CW, K, FW>::L;
-    ContShared<T, CW, K, FW> &S = *reinterpret_cast<ContShared<T, CW, K, FW> *>(smem_raw);
+    constexpr int FW = CF;
+    constexpr int L = ContShared<T, CW, K>::L;
+    ContShared<T, CW, K> &S = *reinterpret_cast<ContShared<T, CW, K> *>(smem_raw);
     const Dims &d = a.d;
     const int w = threadIdx.x >> 6;
     const int lane = threadIdx.x & (FW - 1);                  // the face of the block this thread works on
-    const int grp = w * (64 / FW) + (int)((threadIdx.x & 63) / FW);   // its level group
-    // face (fi, fj) between cell 0 = (fi, fj) and cell 1 = (fi+1, fj) [x] or (fi, fj+1) [y]
-    // x: a block advances by FW-2 faces (its last face lane only lends its cell
-    // to the lane below; its first lane's face feeds the convergence of the second)
-    const int f_raw = Y ? d.isc + bx * FW + lane : d.isc - 1 + bx * (FW - 2) + lane;
+    // face (fi, fj) between cell 0 = (fi, fj) and cell 1 = (fi, fj+1)
+    const int f_raw = d.isc + bx * FW + lane;
     const int f_max = d.iec;
     const int fi = f_raw > f_max ? f_max : f_raw;           // clamped: evaluated, never written
-    const int fj = Y ? d.jsc - 1 + (int)by : d.jsc + (int)by;
+    const int fj = d.jsc - 1 + (int)by;
     const bool live = f_raw <= f_max;
     auto cell = [&](int q) __attribute__((always_inline)) -> long long {   // q-th cell of the stencil, q = 2: cell 0
-        return Y ? IX2(d, fi, fj - 2 + q) : IX2(d, fi - 2 + q, fj);
+        return IX2(d, fi, fj - 2 + q);
     };
-    const int i = fi, j = fj;
     const int nk = d.nk;
     const long long s = d.s2;
     // my levels.  EVEN = false: k0+1 .. k0+K, every slot evaluated (a slot
@@ -694,13 +723,12 @@ __device__ __forceinline__ void continuity_body(const ContArgsT<T> &a, int monot
     int k0;
     bool tail = true;
     if constexpr (EVEN) {
-        static_assert(FW == 64, "one level group per wave");
-        const int g = __builtin_amdgcn_readfirstlane(grp);
+        const int g = __builtin_amdgcn_readfirstlane(w);
         const int full = nk - CW * (K - 1);   // waves with K levels
         tail = g < full;
         k0 = g * (K - 1) + (tail ? g : full);
     } else {
-        k0 = grp * K;
+        k0 = w * K;
     }
     auto valid = [&](int kk) __attribute__((always_inline)) {
         if constexpr (EVEN) return kk < K - 1 || tail;
@@ -713,17 +741,8 @@ __device__ __forceinline__ void continuity_body(const ContArgsT<T> &a, int monot
     col.dt = (T)a.dt;
     const long long c2 = IX2(d, fi, fj);
     col.dy = (T)a.dy_Cu[c2];
-    if constexpr (!Y && FW == 64) {
-        // cell 1's IdxT is the next lane's cell 0's, read at cell
-        // min(f_raw, iec+1): the lane after the last live one holds cell
-        // iec+1 (a lane past iec evaluates values that are never written)
-        const int ci0 = f_raw < d.iec + 1 ? f_raw : d.iec + 1;
-        col.IdxT0 = (T)a.IdxT[IX2(d, ci0, fj)];
-        col.IdxT1 = __shfl_down(col.IdxT0, 1, FW);
-    } else {
-        col.IdxT0 = (T)a.IdxT[cell(2)];
-        col.IdxT1 = (T)a.IdxT[cell(3)];
-    }
+    col.IdxT0 = (T)a.IdxT[cell(2)];
+    col.IdxT1 = (T)a.IdxT[cell(3)];
     T mCu = T(0.0);   // read by the CFL folds of waves 2 and 3 only
     if (w == 2 || w == 3) mCu = (T)a.mask2dCu[c2];
     const long long cu = IX3(d, fi, fj, 1);
@@ -742,7 +761,6 @@ __device__ __forceinline__ void continuity_body(const ContArgsT<T> &a, int monot
     }
     auto park = [&]() __attribute__((always_inline)) {
         if (w == 0) {
-            if (!Y) S.P[0][lane] = (T)(a.dt * IareaT0);
             S.P[1][lane] = (T)dxCu_f;
             S.P[2][lane] = (T)uhbt_f;
             S.P[3][lane] = (T)(a.dt * dmin(IareaT0, IareaT1));
@@ -750,133 +768,10 @@ __device__ __forceinline__ void continuity_body(const ContArgsT<T> &a, int monot
             S.P[5][lane] = (T)dxT1;
         }
     };
-    // PPM edges of cells 0 and 1 (zonal_edge_thickness :185-207); the loads
-    // of a slot past the lane's levels read level min(k, nk) (in bounds) and
-    // nothing is formed from them.  x: each lane reconstructs its own cell 0 from the
-    // 5-cell stencil and takes cell 1 from the next lane (whose cell 0 it is),
-    // so every cell is reconstructed once.  y: both cells from the 6-cell
-    // stencil along j.
-    if (!Y) {
-        const int ci = f_raw < d.iec + 1 ? f_raw : d.iec + 1;   // this lane's cell (in bounds)
-        auto ccell = [&](int q) __attribute__((always_inline)) -> long long { return IX2(d, ci - 2 + q, fj); };
-        // STAGE: each level's row of thicknesses is loaded once, the lanes'
-        // own cells (position t = lane holds cell f_raw(lane 0) - 2 + t) and
-        // the four beyond the last lane (t = 64..67, those of all the wave's
-        // levels in one load), and each lane reads its 5-cell stencil t =
-        // lane .. lane+4 back from LDS: one load per level and lane instead
-        // of five (a load with few active lanes costs about what a full one
-        // does, so the extensions share one).  The rows are
-        // staged in the wave's own rows of S0 (levels 0..KA-1) and S1 (the
-        // rest), which no other wave touches before the first pass's barrier
-        // and this wave's first pass overwrites only after these reads.  A
-        // cell index past iec+3 (the last one the lanes of the unstaged form
-        // read) is clamped there: only lanes past iec+1, which are evaluated
-        // and never written, read a clamped cell.  STAGE_M: the row of masks
-        // likewise, after the thickness rows in S1 where they fit.
-        constexpr bool STAGE = FW == 64 && K >= 3;
-        constexpr int KA = K / 2, RL = FW + 4;
-        static_assert(!STAGE || (KA * RL <= (K - 1) * FW && (K - KA) * RL <= K * FW &&
-                                 (K - 1 - KA) * RL <= (K - 1) * FW),
-                      "staged rows exceed the wave's own rows");
-        constexpr bool STAGE_M = STAGE && (K - KA + 1) * RL <= (K - 1) * FW;
-        T m5[5], hs[K][5], us[K];
-        if constexpr (!STAGE_M) {
-#pragma unroll
-            for (int q = 0; q < 5; ++q) m5[q] = (T)a.mask2dT[ccell(q)];
-        }
-        if constexpr (STAGE) {
-            const int c_lo = f_raw - 2, c_hi = d.iec + 3;
-            const long long rA = IX2(d, c_lo < c_hi ? c_lo : c_hi, fj);
-            const long long rB = IX2(d, c_lo + FW < c_hi ? c_lo + FW : c_hi, fj);
-            T mA = T(0.0), mB = T(0.0);
-            if constexpr (STAGE_M) {
-                mA = (T)a.mask2dT[rA];
-                if (lane < 4) mB = (T)a.mask2dT[rB];
-            }
-            T hA[K], hX = T(0.0);
-            // the four cells past the last lane of every level in one load:
-            // lane 4*kk + x holds cell 64 + x of slot kk
-            const int xk = lane >> 2;
-            const int cx = f_raw - lane - 2 + FW + (lane & 3);
-            const long long rX = IX2(d, cx < c_hi ? cx : c_hi, fj);
-#pragma unroll
-            for (int kk = 0; kk < K; ++kk) {
-                const int kr = k0 + kk + 1;
-                const int k = kr < nk ? kr : nk;
-                const long long o = (long long)(k - 1) * s;
-                us[kk] = a.u[cu + o];
-                if (!formed(kk)) continue;
-                hA[kk] = a.hin[rA + o];
-            }
-            if (lane < 4 * K) {
-                const int kr = k0 + xk + 1;
-                hX = a.hin[rX + (long long)((kr < nk ? kr : nk) - 1) * s];
-            }
-            park();
-            auto row = [&](int kk) __attribute__((always_inline)) -> T * {
-                return kk < KA ? &S.S0[k0][0] + kk * RL : &S.S1[k0][0] + (kk - KA) * RL;
-            };
-            T *const mrow = &S.S1[k0][0] + (K - KA) * RL;
-            if constexpr (STAGE_M) {
-                mrow[lane] = mA;
-                if (lane < 4) mrow[FW + lane] = mB;
-            }
-#pragma unroll
-            for (int kk = 0; kk < K; ++kk) {
-                if (!formed(kk)) continue;
-                row(kk)[lane] = hA[kk];
-            }
-            if (lane < 4 * K && formed(xk)) {
-                T *const r = xk < KA ? &S.S0[k0][0] + xk * RL : &S.S1[k0][0] + (xk - KA) * RL;
-                r[FW + (lane & 3)] = hX;
-            }
-            // one wave's LDS operations complete in order: the fences only
-            // keep the compiler from moving the reads above the stores
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
-            if constexpr (STAGE_M) {
-#pragma unroll
-                for (int q = 0; q < 5; ++q) m5[q] = mrow[lane + q];
-            }
-#pragma unroll
-            for (int kk = 0; kk < K; ++kk) {
-                if (!formed(kk)) continue;
-#pragma unroll
-                for (int q = 0; q < 5; ++q) hs[kk][q] = row(kk)[lane + q];
-            }
-        } else {
-#pragma unroll
-            for (int kk = 0; kk < K; ++kk) {
-                const int kr = k0 + kk + 1;
-                const int k = kr < nk ? kr : nk;
-                const long long o = (long long)(k - 1) * s;
-                us[kk] = a.u[cu + o];
-#pragma unroll
-                for (int q = 0; q < 5; ++q) hs[kk][q] = a.hin[ccell(q) + o];
-            }
-            park();
-        }
-        T wW[K], wE[K], w0[K];
-#pragma unroll
-        for (int kk = 0; kk < K; ++kk) {
-            if (!formed(kk)) continue;
-            S.U[k0 + kk][lane] = us[kk];
-            const T *h5 = hs[kk];
-            T sl[3];
-#pragma unroll
-            for (int q = 0; q < 3; ++q) sl[q] = ppm_slope_v(m5[q], m5[q + 1], m5[q + 2], h5[q], h5[q + 1], h5[q + 2]);
-            ppm_edges_v(m5, h5, sl, 2, wW[kk], wE[kk]);
-            w0[kk] = h5[2];
-        }
-#pragma unroll
-        for (int kk = 0; kk < K; ++kk) {
-            if (!formed(kk)) continue;
-            ppm_limit(monotonic, w0[kk], (T)a.h_min, wW[kk], wE[kk]);
-            col.set(kk, wW[kk], wE[kk], w0[kk], __shfl_down(wW[kk], 1, FW), __shfl_down(wE[kk], 1, FW),
-                    __shfl_down(w0[kk], 1, FW));
-        }
-    } else {
+    // PPM edges of cells 0 and 1 (zonal_edge_thickness :185-207), both from the
+    // 6-cell stencil along j; the loads of a slot past the lane's levels read
+    // level min(k, nk) (in bounds) and nothing is formed from them
+    {
         T m6[6], hs[K][6], us[K];
 #pragma unroll
         for (int q = 0; q < 6; ++q) m6[q] = (T)a.mask2dT[cell(q)];
@@ -953,43 +848,6 @@ __device__ __forceinline__ void continuity_body(const ContArgsT<T> &a, int monot
     const T CFL_dt = (T)a.CFL_limit_adjust / (T)a.dt;
     eval_pass(T(0.0), true);
     lds_barrier();
-    // Prefetch (pf_on: the single-model launch, whose blocks are dispatched
-    // in blockIdx order, round-robin over the 8 XCDs): the u and h rows of
-    // block b + 256, which runs on this block's XCD (256 is a multiple of 8)
-    // about one block lifetime later at one block per CU.  One 4-byte load per
-    // lane touches one 128-byte line of a row (9 lines per level in FP64, 5 in
-    // FP32, as many levels as the block's lanes cover).  A block's set-up
-    // waits on its own loads (the last wave of each SIMD receives its rows
-    // about 14 K cycles after the block starts); lines this prefetch brought
-    // in arrive sooner (0.98 against 1.017 ms per FP64 launch at
-    // 720x720x75; the FP32 launch gains 4%, and a distance of 512 measured no
-    // better for it).  The loads are issued after this block's first pass,
-    // their value is consumed by an empty asm at the end so that they are
-    // kept, and they read inside the arrays, at indices that the block they
-    // prefetch for reads.
-    int pf = 0;
-    if constexpr (!Y && FW == 64) {
-        const unsigned gx = gridDim.x, b2 = bx + gx * by + 256;
-        if (pf_on && b2 < gx * gridDim.y) {
-            constexpr int LU = (64 * (int)sizeof(T) + 127) / 128, LH = (68 * (int)sizeof(T) + 127) / 128;
-            constexpr int ST = 128 / (int)sizeof(T);
-            const int bx2 = (int)(b2 % gx), by2 = (int)(b2 / gx);
-            const int q = w * 64 + (int)(threadIdx.x & 63);
-            const int lvl = q / (LU + LH), part = q % (LU + LH);
-            if (lvl < nk) {
-                const int f0 = d.isc - 1 + bx2 * (FW - 2), fj2 = d.jsc + by2;
-                const int *pp;
-                if (part < LU) {
-                    const int f = f0 + part * ST;
-                    pp = (const int *)(a.u + IX3(d, f < d.iec ? f : d.iec, fj2, lvl + 1));
-                } else {
-                    const int c = f0 - 2 + (part - LU) * ST;
-                    pp = (const int *)(a.hin + IX2(d, c < d.iec + 3 ? c : d.iec + 3, fj2) + (long long)lvl * s);
-                }
-                pf = *pp;
-            }
-        }
-    }
     const T dx_W = S.P[4][lane], dx_E = S.P[5][lane];
     if (w < 2) {
         S.R[w][lane] = (w == 0) ? col_sum<L>(S.S0, nk, lane, T(0.0)) : sum_dy(T(0.0));
@@ -1033,9 +891,7 @@ __device__ __forceinline__ void continuity_body(const ContArgsT<T> &a, int monot
         T du = T(0.0), du_max = st.du_max_CFL, du_min = st.du_min_CFL;
         T uh_err = st.uh_tot_0 - uhbt, duhdu_tot = st.duhdu_tot_0;
         T uh_err_best = vabs(uh_err);
-        // x: lanes past the last face and the block's last lane (no cell 1 of
-        // its own) take no Newton passes
-        bool do_I = Y || (live && lane < FW - 1);
+        bool do_I = true;
         *du_eval = T(0.0);   // the first pass evaluated at du = 0
         for (int itt = 1; itt <= max_itts; ++itt) {
             if (do_I) {
@@ -1099,24 +955,11 @@ __device__ __forceinline__ void continuity_body(const ContArgsT<T> &a, int monot
     // reads back what it stored whether or not a barrier lies between
     S.P[6][lane] = du_eval;
     S.P[7][lane] = sum_dyhm;
-    // the convergence's cell thicknesses (cell I = I0 + lane, every level of
-    // the lane's group; clamped levels repeat nk), issued before the face
-    // stores so that one round trip covers all levels
-    T hc[K];
-    if (!Y) {
-#pragma unroll
-        for (int kk = 0; kk < K; ++kk) {
-            const int kr = k0 + kk + 1;
-            hc[kk] = a.hin[IX3(d, i, j, kr < nk ? kr : nk)];
-        }
-    }
-
-    // outputs at the face: uh, u_cor, du_cor; a face shared with the western
-    // neighbour block is written by that block.  u_cor = u + du needs only u
+    // outputs at the face: uh, u_cor, du_cor.  u_cor = u + du needs only u
     // (in LDS to the end) and du: with the BT_cont outputs its stores wait for
     // the CFL folds of BT_cont, where the other waves are idle, instead of
     // joining the burst of the other outputs (1.8% of the kernel)
-    const bool writes_face = live && (Y || ((lane > 0 || bx == 0) && lane < FW - 1));
+    const bool writes_face = live;
     auto store_u_cor = [&]() __attribute__((always_inline)) {
         if (a.u_cor && writes_face) {
 #pragma unroll
@@ -1129,27 +972,10 @@ __device__ __forceinline__ void continuity_body(const ContArgsT<T> &a, int monot
         for (int kk = 0; kk < K; ++kk) {
             if (valid(kk)) a.uh[cu + (long long)(k0 + kk) * s] = S.S0[k0 + kk][lane];
         }
-        if (a.du_cor && grp == 0) a.du_cor[c2] = (double)du;
+        if (a.du_cor && w == 0) a.du_cor[c2] = (double)du;
     }
     if (!a.bt_h_u) store_u_cor();
-    // continuity_zonal_convergence (:148-176) for cell i = I (faces I-1 and I)
-    if (!Y) {
-        const T dtIareaT = S.P[0][lane];   // dt*IareaT(i, j): cell 0 of the face
-        const bool writes_cell = live && lane > 0 && lane < FW - 1 && i >= d.isc;
-#pragma unroll
-        for (int kk = 0; kk < K; ++kk) {
-            if (writes_cell && valid(kk)) {
-                const long long c3 = IX3(d, i, j, k0 + kk + 1);
-                const T fw = S.S0[k0 + kk][lane - 1];   // face I-1 (the lane to the west), same level
-                const T v = hc[kk] - dtIareaT * (S.S0[k0 + kk][lane] - fw);
-                a.h[c3] = vmax(v, T(0.0));
-            }
-        }
-    }
-    if (!a.bt_h_u) {   // block-uniform
-        asm volatile("" ::"v"(pf));
-        return;
-    }
+    if (!a.bt_h_u) return;   // block-uniform
 
     // h_u = marginal thickness at u_cor = u + du (zonal_flux_thickness :602-735):
     // the last Newton pass's (in S1, each wave's own rows) when that was at
@@ -1225,35 +1051,612 @@ __device__ __forceinline__ void continuity_body(const ContArgsT<T> &a, int monot
     eval_pass(duR, true);
     sum_pass(T(0.0), T(0.0), true);
     const T uhtot_R = S.R[0][lane], FAmt_R = S.R[1][lane];
-    asm volatile("" ::"v"(pf));
-    if (!writes_face || grp != 0) return;
-    T FA_0 = FAmt_0, FA_avg = FAmt_0;
-    if ((duL - du0) != T(0.0)) FA_avg = uhtot_L / (duL - du0);
-    if (FA_avg > vmax(FA_0, FAmt_L)) FA_avg = vmax(FA_0, FAmt_L);
-    else if (FA_avg < vmin(FA_0, FAmt_L)) FA_0 = FA_avg;
-    a.FA_u_W0[c2] = (double)FA_0;
-    a.FA_u_WW[c2] = (double)FAmt_L;
-    a.uBT_WW[c2] = (double)((vabs(FA_0 - FAmt_L) <= (T)1e-12f * FA_0)
-                                ? T(0.0)
-                                : (T(1.5) * (duL - du0)) * ((FAmt_L - FA_avg) / (FAmt_L - FA_0)));
-    FA_0 = FAmt_0;
-    FA_avg = FAmt_0;
-    if ((duR - du0) != T(0.0)) FA_avg = uhtot_R / (duR - du0);
-    if (FA_avg > vmax(FA_0, FAmt_R)) FA_avg = vmax(FA_0, FAmt_R);
-    else if (FA_avg < vmin(FA_0, FAmt_R)) FA_0 = FA_avg;
-    a.FA_u_E0[c2] = (double)FA_0;
-    a.FA_u_EE[c2] = (double)FAmt_R;
-    a.uBT_EE[c2] = (double)((vabs(FAmt_R - FA_0) <= (T)1e-12f * FA_0)
-                                ? T(0.0)
-                                : (T(1.5) * (duR - du0)) * ((FAmt_R - FA_avg) / (FAmt_R - FA_0)));
+    if (!writes_face || w != 0) return;
+    bt_cont_store(a, c2, du0, FAmt_0, duL, uhtot_L, FAmt_L, duR, uhtot_R, FAmt_R);
 }
 
-template <typename T, bool Y, int CW, int K, int FW = CF, bool EVEN = false>
+// The zonal pass with a column's levels split over four waves (columns of up
+// to kSplitMax levels).  Wave w holds a quarter of the levels: per level the
+// two PPM edges and the thickness of the lane's own cell (the cell across the
+// face is the next lane's: a DPP shift), and the layer transport and marginal
+// thickness of the last pass.  Nothing but u sits in LDS.  A pass evaluates all
+// levels side by side; its column sums then go from wave to wave in the
+// reference's k order, each wave adding its own levels (a turn and a barrier
+// per wave).  The Newton logic of a face runs redundantly in every wave on the
+// same values.
+//
+// The zonal form of the block kernel above held both cells' terms of a level
+// (84 registers for 7 levels) and the terms of a pass in LDS (134 KB): one
+// 12-wave block per CU, so nothing covered its loads, folds and barriers.  Here
+// two blocks share a CU at 75 levels in FP64, three in FP32.  Per call at
+// 720x720x75, FP64: 976 -> 705 us (reads 1.9 -> 0.9 GB: the convergence keeps
+// its thicknesses), FP32 465 -> 393; 471x363x50 352 -> 187 and 154 -> 94;
+// 140x100x40 57 -> 31; 300x260x25 72 -> 48; 180x180x75 88 -> 78.  Faster at
+// every depth, so it replaced the zonal form.  What bounds it: VALU issue (55%
+// busy at 75 levels FP64) and, at two waves per SIMD, the latency of dependent
+// FP64 operations.  Groups of 3 levels measured the same as 4.
+template <typename T, int K>
+struct ContCols {
+    T hW[K], hE[K], h0[K];   // west and east edge and mean thickness of the lane's cell
+    T f[K], hm[K];           // layer transport and marginal thickness of the last pass
+    T dt, dy, IdxT0, IdxT1;
+    // zonal_flux_layer (:516-598) at velocity u; every lane of the wave active.
+    // As ColRegs::eval, with the far edge minus the near one formed here;
+    // true where u is zero (or NaN), whose values eval_zero gives
+    __device__ __forceinline__ bool eval(int kk, T u, T &uh, T &h_marg) const
+    {
+        const T hW1 = east(hW[kk]), hE1 = east(hE[kk]), h1 = east(h0[kk]);
+        const bool pos = u > T(0.0);
+        const T A = pos ? hE[kk] : hW1, B = pos ? hW[kk] : hE1;
+        const T D = B - A;
+        const T curv_3 = vfma(T(-2.0), pos ? h0[kk] : h1, A + B);   // 2 h is exact: (A + B) - 2 h
+        const T c = u * dt * (pos ? IdxT0 : IdxT1);
+        const T CFL = vabs(c);
+        uh = (dy * u) * (A + CFL * (T(0.5) * D + curv_3 * (CFL - T(1.5))));
+        h_marg = A + CFL * (D + T(3.0) * curv_3 * (CFL - T(1.0)));
+        return !(u > T(0.0)) && !(u < T(0.0));
+    }
+    __device__ __forceinline__ void eval_zero(int kk, T u, T &uh, T &h_marg) const
+    {
+        const T hW1 = east(hW[kk]);
+        if (!(u > T(0.0)) && !(u < T(0.0))) {
+            uh = T(0.0);
+            h_marg = T(0.5) * (hW1 + hE[kk]);
+        }
+    }
+};
+
+constexpr int CX_RL = CF + 4;   // cells staged per level: the lanes' own and two on each side
+// LDS rows of CF values ahead of u: sums handed from wave to wave, results,
+// the Newton iteration's starting point, the parked 2D values (dt*IareaT of the
+// lane's cell, dxCu of its face, its barotropic transport target, dt*min(IareaT)
+// of its two cells), BT_cont's running minima and maxima and a flag
+constexpr int CX_PAR = 0, CX_FIN = 7, CX_START = 14, CX_P = 18, CX_BT = 22, CX_ROWS = 31;
+// Levels from one buffer base on: 8, or 1 where 8 levels' byte offsets pass 32
+// bits (a base per level costs 4-8% of the kernel)
+constexpr int CX_BASE = 8;
+template <typename T>
+bool cont_split_wide(const Dims &d)
+{
+    return CX_BASE * d.s2 * (long long)sizeof(T) >= (1LL << 32);
+}
+template <typename T>
+constexpr size_t cont_split_lds(int nk)   // rows, then u of every level (and what unused slots read)
+{
+    return ((size_t)CX_ROWS * CF + (size_t)(nk + 4) * CX_RL) * sizeof(T);
+}
+// waves per SIMD that the registers of K slots leave room for without a spill
+template <typename T>
+constexpr int cont_split_waves(int K)
+{
+    if (sizeof(T) == 4) return K > 13 ? 3 : K > 10 ? 4 : K > 7 ? 5 : 6;
+    return K > 10 ? 2 : K > 4 ? 3 : 4;
+}
+
+template <typename T, int K, int BASE>
+__device__ __forceinline__ void continuity_x_split(const ContArgsT<T> &a, int monotonic, unsigned bx, unsigned by)
+{
+    extern __shared__ double smem_raw[];
+    constexpr bool F32 = sizeof(T) == 4;
+    constexpr int W = kSplitWaves, NMIN = slot_min(K);
+    // slots go in groups of up to G, straight-line code each (what a few
+    // columns need stands in one branch per group), so that the levels'
+    // dependent chains overlap; the slots that some waves leave unused are one group
+    constexpr int G = 4, NG = (NMIN + G - 1) / G + 1;
+    static_assert(K - NMIN <= G, "a group's arrays hold G slots");
+    auto g_lo = [](int g) __attribute__((always_inline)) { return g < NG - 1 ? g * G : NMIN; };
+    auto g_hi = [](int g) __attribute__((always_inline)) {
+        return g == NG - 1 ? K : g * G + G < NMIN ? g * G + G : NMIN;
+    };
+    const Dims &d = a.d;
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    T *const rows = reinterpret_cast<T *>(smem_raw);
+    auto R = [&](int r) __attribute__((always_inline)) -> T & { return rows[r * CF + lane]; };
+    T(*const U)[CX_RL] = reinterpret_cast<T(*)[CX_RL]>(rows + CX_ROWS * CF);
+    // face (fi, fj) between cells fi and fi+1.  A block advances by 62 faces:
+    // its last lane only lends its cell to the lane below, its first lane's
+    // face feeds the convergence of the second
+    const int f_raw = d.isc - 1 + bx * (CF - 2) + lane;
+    const int fi = f_raw > d.iec ? d.iec : f_raw;           // clamped: evaluated, never written
+    const int fj = d.jsc + (int)by;
+    const bool live = f_raw <= d.iec;
+    const int nk = d.nk;
+    const long long s = d.s2;
+    const int q = nk / W, r = nk % W;
+    const int n = q + (w < r ? 1 : 0);                      // this wave's levels k0+1 .. k0+n
+    const int k0 = w * q + (w < r ? w : r);
+    auto used = [&](int kk) __attribute__((always_inline)) { return kk < NMIN || kk < n; };
+    // a used slot's plane of an array: buffer accesses at the lane's 32-bit byte
+    // offset (flat addresses would be kept in registers over the loops), from a
+    // base every BASE slots
+    auto buf = [&](auto *p, int kk) __attribute__((always_inline)) {
+        return LevelBuf<std::remove_pointer_t<decltype(p)>>(p + (long long)(k0 + kk / BASE * BASE) * s);
+    };
+    auto off = [&](int kk) __attribute__((always_inline)) { return (unsigned)(kk % BASE * s * sizeof(T)); };
+    T(*const Uw)[CX_RL] = U + k0;
+    auto wave_fence = []() __attribute__((always_inline)) {
+        // one wave's LDS operations complete in order: this only keeps the
+        // compiler from moving them across
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+    };
+    // An empty asm on a value keeps its computation where it stands.
+    auto pin = [](T &x) __attribute__((always_inline)) { asm volatile("" : "+v"(x)); };
+
+    ContCols<T, K> col;
+    const long long c2 = IX2(d, fi, fj);
+    // ---- 2D values, ahead of the column's loads (memory answers in order);
+    // those read after the passes are parked in LDS by wave 0 ----
+    double p0 = 0.0, p1 = 0.0, p2 = 0.0, p3 = 0.0;
+    if (w == 0) {
+        p0 = a.IareaT[c2];
+        p1 = a.dxCu[c2];
+        p2 = a.uhbt ? a.uhbt[c2] : 0.0;
+        p3 = a.IareaT[c2 + 1];
+    }
+    const T dxW = (T)a.dxT[c2], dxE = (T)a.dxT[c2 + 1];
+    col.dt = (T)a.dt;
+    col.dy = (T)a.dy_Cu[c2];
+    {   // cell 1's IdxT is the next lane's cell 0's, read at cell min(f_raw, iec+1)
+        const int ci0 = f_raw < d.iec + 1 ? f_raw : d.iec + 1;
+        col.IdxT0 = (T)a.IdxT[IX2(d, ci0, fj)];
+    }
+    const T mCu = (T)a.mask2dCu[c2];
+    // ---- loads: u and the thicknesses of cells lane-2 (and four past the last) ----
+    // a cell index past iec+3 is clamped there: only lanes past iec+1, which
+    // are evaluated and never written, read a clamped cell
+    const int c_lo = f_raw - 2, c_hi = d.iec + 3;
+    const long long rA = IX2(d, c_lo < c_hi ? c_lo : c_hi, fj);
+    const unsigned oA = (unsigned)(rA * sizeof(T)), oF = (unsigned)(c2 * sizeof(T));
+    const int cx = f_raw - lane - 2 + CF + (lane & 3);      // the four cells past the last lane:
+    const long long rX = IX2(d, cx < c_hi ? cx : c_hi, fj); // lane 4*x + y holds cell y of slot x, 16 slots a load
+    T hA[K], us[K], hX[(K + 15) / 16];
+    const T mA = (T)a.mask2dT[rA];
+    const T mB = (T)a.mask2dT[rX];
+#pragma unroll
+    for (int kk = 0; kk < K; ++kk) hA[kk] = used(kk) ? buf(a.hin, kk).load(oA, off(kk)) : T(0.0);
+#pragma unroll
+    for (int x = 0; x < (K + 15) / 16; ++x) {
+        const int kr = k0 + 16 * x + (lane >> 2);
+        hX[x] = a.hin[rX + (kr < nk ? kr : nk - 1) * s];
+    }
+    // u behind the thicknesses: it arrives while the edges are formed
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int kk = 0; kk < K; ++kk) us[kk] = used(kk) ? buf(a.u, kk).load(oF, off(kk)) : T(0.0);
+    __builtin_amdgcn_sched_barrier(0);
+    // ---- PPM edges of the lane's cell (zonal_edge_thickness :185-207): the
+    // rows staged in LDS (where u goes afterwards), 5-cell stencils read back ----
+    col.IdxT1 = __shfl_down(col.IdxT0, 1, CF);
+    if (w == 0) {
+        R(CX_P + 0) = (T)(a.dt * p0);
+        R(CX_P + 1) = (T)p1;
+        R(CX_P + 2) = (T)p2;
+        R(CX_P + 3) = (T)(a.dt * dmin(p0, p3));
+    }
+    T m5[5];
+    Uw[0][lane] = mA;
+    if (lane < 4) Uw[0][CF + lane] = mB;
+    wave_fence();
+#pragma unroll
+    for (int x = 0; x < 5; ++x) m5[x] = Uw[0][lane + x];
+    wave_fence();
+#pragma unroll
+    for (int kk = 0; kk < K; ++kk)
+        if (used(kk)) Uw[kk][lane] = hA[kk];
+#pragma unroll
+    for (int x = 0; x < (K + 15) / 16; ++x)
+        if (16 * x + (lane >> 2) < n) Uw[16 * x + (lane >> 2)][CF + (lane & 3)] = hX[x];
+    wave_fence();
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        if (g == NG - 1 && n <= NMIN) break;
+        T h5[G][5];
+        bool limit = false;
+#pragma unroll
+        for (int kk = g_lo(g); kk < g_hi(g); ++kk)
+#pragma unroll
+            for (int x = 0; x < 5; ++x) h5[kk - g_lo(g)][x] = Uw[kk][lane + x];
+#pragma unroll
+        for (int kk = g_lo(g); kk < g_hi(g); ++kk) {
+            const T *h = h5[kk - g_lo(g)];
+            T sl[3];
+#pragma unroll
+            for (int x = 0; x < 3; ++x) sl[x] = ppm_slope_v(m5[x], m5[x + 1], m5[x + 2], h[x], h[x + 1], h[x + 2]);
+            ppm_edges_v(m5, h, sl, 2, col.hW[kk], col.hE[kk]);
+            limit = limit || ppm_limits(monotonic, h[2], (T)a.h_min, col.hW[kk], col.hE[kk]);
+        }
+        if (__any(limit)) {
+#pragma unroll
+            for (int kk = g_lo(g); kk < g_hi(g); ++kk)
+                ppm_limit(monotonic, h5[kk - g_lo(g)][2], (T)a.h_min, col.hW[kk], col.hE[kk]);
+        }
+#pragma unroll
+        for (int kk = g_lo(g); kk < g_hi(g); ++kk) {
+            col.h0[kk] = h5[kk - g_lo(g)][2];
+            pin(col.hW[kk]);
+            pin(col.hE[kk]);
+            pin(col.h0[kk]);
+        }
+    }
+
+    wave_fence();
+#pragma unroll
+    for (int kk = 0; kk < K; ++kk)
+        if (used(kk)) Uw[kk][lane] = us[kk];
+
+    auto uk = [&](int kk) __attribute__((always_inline)) -> T { return Uw[kk][lane]; };
+    // one pass: every level at u + du.  A face whose du is unchanged gets the
+    // same values again, so all lanes take part.
+    auto eval_group = [&](int g, T du) __attribute__((always_inline)) {
+        bool zero = false;
+#pragma unroll
+        for (int kk = g_lo(g); kk < g_hi(g); ++kk) {
+            const bool z = col.eval(kk, uk(kk) + du, col.f[kk], col.hm[kk]);
+            zero = zero || z;
+        }
+        if (__any(zero)) {
+#pragma unroll
+            for (int kk = g_lo(g); kk < g_hi(g); ++kk)
+                col.eval_zero(kk, uk(kk) + du, col.f[kk], col.hm[kk]);
+        }
+#pragma unroll
+        for (int kk = g_lo(g); kk < g_hi(g); ++kk) {
+            pin(col.f[kk]);
+            pin(col.hm[kk]);
+        }
+    };
+    auto eval_pass = [&](T du) __attribute__((always_inline)) {
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            if (g == NG - 1 && n <= NMIN) break;
+            eval_group(g, du);
+        }
+    };
+    // op on the values handed down so far, wave after wave
+    auto turns = [&](auto op) __attribute__((always_inline)) {
+        for (int t = 0; t < w; ++t) lds_barrier();
+        op();
+        for (int t = w; t < W; ++t) lds_barrier();
+    };
+    // sum + x, or for FP32 terms a Kahan-compensated sum with its correction cmp
+    auto add = [&](T &sum, T &cmp, T x) __attribute__((always_inline)) {
+        if constexpr (F32) {
+            const T y = x - cmp;
+            const T t = sum + y;
+            cmp = (t - sum) - y;
+            sum = t;
+        } else {
+            sum = sum + x;
+        }
+    };
+    // column sums in k order: FIN[0] = x0 + sum f, FIN[1] = sum dy*hm; FIRST also
+    // the scale of the rounding of the flux sum (FP32) and the running minimum
+    // and maximum of the CFL bracket
+    auto sum_pass = [&](T x0, auto first, T hi_w, T lo_w) __attribute__((always_inline)) {
+        constexpr bool FIRST = decltype(first)::value;
+        turns([&]() __attribute__((always_inline)) {
+            T s0 = x0, s1 = T(0.0), e0 = T(0.0), e1 = T(0.0), hi = hi_w, lo = lo_w, sc = T(0.0);
+            if (w > 0) {
+                s0 = R(CX_PAR + 0);
+                s1 = R(CX_PAR + 1);
+                if constexpr (F32) {
+                    e0 = R(CX_PAR + 2);
+                    e1 = R(CX_PAR + 3);
+                }
+                if constexpr (FIRST) {
+                    hi = hmin(hi, R(CX_PAR + 4));
+                    lo = hmax(lo, R(CX_PAR + 5));
+                    if constexpr (F32) sc = R(CX_PAR + 6);
+                }
+            }
+#pragma unroll
+            for (int kk = 0; kk < K; ++kk) {
+                if (!used(kk)) continue;
+                add(s0, e0, col.f[kk]);
+                add(s1, e1, col.dy * col.hm[kk]);
+                if constexpr (FIRST && F32) sc = sc + vabs(col.f[kk]);
+            }
+            T *const o = rows + (w == W - 1 ? CX_FIN : CX_PAR) * CF + lane;   // the same rows of either
+            o[0 * CF] = s0;
+            o[1 * CF] = s1;
+            if constexpr (F32) {
+                o[2 * CF] = e0;
+                o[3 * CF] = e1;
+            }
+            if constexpr (FIRST) {
+                o[4 * CF] = hi;
+                o[5 * CF] = lo;
+                if constexpr (F32) o[6 * CF] = sc;
+            }
+        });
+    };
+
+    // first layer fluxes, their sums and the CFL bracket (zonal_mass_flux
+    // :300-393), a fold over k: hi = (hi > b - u*mask) ? b - u : hi, b = dx*CFL/dt.
+    // With mask = 1 that is the minimum of the b - u (lo: a maximum), in any order
+    eval_pass(T(0.0));
+    const bool plain = __all(mCu == T(1.0));   // the same in every wave
+    {
+        const T CFL_dt = (T)a.CFL_limit_adjust / (T)a.dt;
+        const T dx_W = dxW, dx_E = dxE;
+        const T bW = dx_W * CFL_dt, bE = dx_E * CFL_dt;
+        const T hi0 = T(2.0) * (CFL_dt * dx_W) * T(1.0), lo0 = -(T(2.0) * (CFL_dt * dx_E) * T(1.0));
+        T hi = hi0, lo = lo0;
+#pragma unroll
+        for (int kk = 0; kk < K; ++kk) {
+            if (!used(kk)) continue;
+            const T uu = uk(kk);
+            hi = hmin(hi, bW - uu);
+            lo = hmax(lo, -(bE + uu));
+        }
+        sum_pass(T(0.0), std::true_type{}, hi, lo);
+        if (!plain) {   // in k order
+            if (w == 0)
+                R(CX_FIN + 4) = lds_fold<0>(U, nk, lane, hi0, [&](T x, T uu) {
+                    return (x > bW - uu * mCu) ? (bW - uu) : x;
+                });
+            if (w == 1)
+                R(CX_FIN + 5) = lds_fold<0>(U, nk, lane, lo0, [&](T x, T uu) {
+                    return (x < -bE - uu * mCu) ? -(bE + uu) : x;
+                });
+            lds_barrier();
+        }
+    }
+    const T bt = R(CX_P + 2);
+    const T tol_floor = F32 ? R(CX_P + 3) * (T(4.0f * 1.1920929e-7f) * R(CX_FIN + 6)) : T(0.0);
+    const T tol_eta0 = (T)a.tol_eta0, tol_vel = (T)a.tol_vel;
+    // the Newton iteration's starting point, kept in LDS for the zero-target
+    // iteration of BT_cont.  Every wave stores its own copy (all hold the same
+    // values), so each reads back what it stored whether or not a barrier lies
+    // between
+    {
+        const T s0 = R(CX_FIN + 0), s1 = R(CX_FIN + 1), hi = R(CX_FIN + 4), lo = R(CX_FIN + 5);
+        R(CX_START + 0) = s0;
+        R(CX_START + 1) = s1;
+        R(CX_START + 2) = vmax(hi, T(0.0));
+        R(CX_START + 3) = vmin(lo, T(0.0));
+    }
+
+    // outputs; a face shared with the western neighbour block is written by
+    // that block
+    const bool writes_face = live && (lane > 0 || bx == 0) && lane < CF - 1;
+    const bool writes_cell = live && lane > 0 && lane < CF - 1 && fi >= d.isc;
+    // one slot: uh, continuity_zonal_convergence (:148-176) for cell i (faces
+    // i-1 and i), u_cor, and h_u = marginal thickness hm at u_cor = u + du
+    // (zonal_flux_thickness :602-735)
+    auto store_slot = [&](int kk, T du, T hm) __attribute__((always_inline)) {
+        const T fw = west(col.f[kk]);
+        const T v = vmax(col.h0[kk] - R(CX_P + 0) * (col.f[kk] - fw), T(0.0));
+        if (!used(kk)) return;
+        if (writes_face) {
+            buf(a.uh, kk).store(col.f[kk], oF, off(kk));
+            if (a.u_cor) buf(a.u_cor, kk).store(uk(kk) + du, oF, off(kk));
+            if (a.bt_h_u) buf(a.bt_h_u, kk).store(hm, oF, off(kk));
+        }
+        if (writes_cell) buf(a.h, kk).store(v, oF, off(kk));
+    };
+
+    // zonal_flux_adjust (:739-916), for the barotropic target (keep: uh_3d
+    // present, the fluxes of the last evaluation are the result, evaluated also
+    // at itt = max_itts) and, where some target is not zero, for a zero one
+    // (set_zonal_BT_cont :920-1121; the zero-transport correction equals du
+    // wherever the target is zero: identical iterations).  One loop, so that
+    // its code stands once.
+    const bool bt_any = a.bt_h_u && a.uhbt && block_any(bt != T(0.0));
+    T du_at = T(0.0);   // du of the face's last evaluation
+    // du0 = the (zero-transport) correction, du0_eval = du of the last
+    // evaluation that was summed (NaN if none), FAmt_0 = sum dy*hm at u + du0_eval
+    T du0 = T(0.0), du0_eval = T(0.0), FAmt_0 = T(0.0), du_u = T(0.0);
+    bool stored = false;   // block-uniform
+#pragma nounroll
+    for (int rep = 0; rep < (bt_any ? 2 : 1); ++rep) {
+        const bool keep = rep == 0;
+        const T uhbt = keep ? bt : T(0.0);
+        const int max_itts = 20;
+        const T dtIarea = R(CX_P + 3);
+        T du = T(0.0), du_max = R(CX_START + 2), du_min = R(CX_START + 3);
+        T uh_err = R(CX_START + 0) - uhbt, duhdu_tot = R(CX_START + 1);
+        T uh_err_best = vabs(uh_err), du_eval = T(0.0);   // the first pass evaluated at du = 0
+        // lanes past the last face and the block's last lane (no cell 1 of
+        // its own) take no Newton passes
+        bool do_I = live && lane < CF - 1;
+        for (int itt = 1; itt <= max_itts; ++itt) {
+            if (do_I) {
+                T tol_eta;
+                if (itt <= 1) tol_eta = (T)1e-6f * tol_eta0;
+                else if (itt == 2) tol_eta = (T)1e-4f * tol_eta0;
+                else if (itt == 3) tol_eta = (T)1e-2f * tol_eta0;
+                else tol_eta = tol_eta0;
+                if (F32) tol_eta = vmax(tol_eta, tol_floor);
+                if (uh_err > T(0.0)) du_max = du;
+                else if (uh_err < T(0.0)) du_min = du;
+                else do_I = false;
+                if (do_I) {
+                    const T aerr = vabs(uh_err);
+                    if ((dtIarea * aerr > tol_eta) || ((aerr > tol_vel * duhdu_tot) || (aerr > uh_err_best))) {
+                        const T ddu = -uh_err / duhdu_tot;
+                        const T du_prev = du;
+                        du = du + ddu;
+                        if (vabs(ddu) < (T)1.0e-15f * vabs(du)) {
+                            do_I = false;
+                        } else if (ddu > T(0.0)) {
+                            if (du >= du_max) {
+                                du = T(0.5) * (du_prev + du_max);
+                                if (du_max - du_prev < (T)1.0e-15f * vabs(du)) do_I = false;
+                            }
+                        } else {
+                            if (du <= du_min) {
+                                du = T(0.5) * (du_prev + du_min);
+                                if (du_prev - du_min < (T)1.0e-15f * vabs(du)) do_I = false;
+                            }
+                        }
+                    } else {
+                        do_I = false;
+                    }
+                }
+            }
+            // a finished column keeps its du for the rest of the reference's row loop
+            const bool ev = do_I && ((itt < max_itts) || keep);
+            if (!block_any(ev)) break;
+            if (ev) du_at = du;
+            eval_pass(du_at);
+            const bool summed = ev && itt < max_itts;
+            sum_pass(-uhbt, std::false_type{}, T(0.0), T(0.0));
+            if (summed) {
+                uh_err = R(CX_FIN + 0);
+                duhdu_tot = R(CX_FIN + 1);
+                uh_err_best = vmin(uh_err_best, vabs(uh_err));
+                du_eval = du;
+            } else if (ev) {
+                du_eval = (T)NAN;
+            }
+        }
+        if (keep) {
+            // f and hm hold the last evaluation, which was at u + du where du_eval == du
+            du_u = du;
+            const bool last_at_du = (du_eval == du);
+            const bool again = block_any(!last_at_du);
+            if (a.du_cor && w == 0 && writes_face) a.du_cor[c2] = (double)du;
+            // With the BT_cont outputs the stores go out between the
+            // evaluations of its first pass (all at once, the wave waits for
+            // the memory pipeline to take them), unless f or hm change before
+            if (!a.bt_h_u || bt_any || again) {
+                stored = true;
+#pragma unroll
+                for (int kk = 0; kk < K; ++kk) {
+                    T hm = col.hm[kk];
+                    if (again) {   // h_u evaluated at u + du
+                        T fc, h2;
+                        if (__any(col.eval(kk, uk(kk) + du, fc, h2))) col.eval_zero(kk, uk(kk) + du, fc, h2);
+                        hm = last_at_du ? hm : h2;
+                    }
+                    store_slot(kk, du, hm);
+                }
+            }
+            du0 = du;
+            du0_eval = du_eval;
+            FAmt_0 = duhdu_tot;
+        } else if (bt != T(0.0)) {
+            du0 = du;
+            du0_eval = du_eval;
+            FAmt_0 = duhdu_tot;
+        }
+    }
+    if (!a.bt_h_u) return;   // block-uniform
+
+    // set_zonal_BT_cont: test velocities duR, duL (visc_rem_lim = 1), folds over
+    // k: x = (u + x > -c) ? -(u + c) : x and its mirror image, c = du_CFL.
+    // Except for rounding they are a minimum and a maximum: where x differs from
+    // m = -(u + c) by more than 2^-51 (|u| + c) (FP32: 2^-22), u + x rounds to
+    // the side of -c on which x lies of m (the sum and m are each off by half a
+    // unit in the last place), and at x = m both branches give x.  So every wave
+    // takes the running minimum of its own levels, from the minimum of the
+    // levels above, and votes whether some x came closer than that; only then
+    // waves 0 and 1 fold in k order (75 dependent steps of three operations, 8%
+    // of the kernel).
+    const T Idt = T(1.0) / (T)a.dt;
+    const T CFL_min = (T)1e-6f;
+    const T du_CFL = (CFL_min * Idt) * R(CX_P + 1);
+    const T x0R = vmin(T(0.0), du0 - du_CFL), x0L = vmax(T(0.0), du0 + du_CFL);
+    T duR = x0R, duL = x0L;
+    {
+        T xR = (T)INFINITY, xL = (T)-INFINITY;
+#pragma unroll
+        for (int kk = 0; kk < K; ++kk) {
+            if (!used(kk)) continue;
+            const T uu = uk(kk);
+            xR = hmin(xR, -(uu + du_CFL));
+            xL = hmax(xL, -(uu - du_CFL));
+        }
+        R(CX_BT + 2 * w) = xR;
+        R(CX_BT + 2 * w + 1) = xL;
+        if (w == 0) R(CX_BT + 2 * W) = T(0.0);
+        lds_barrier();
+        bool close = false;
+        const T tiny = F32 ? T(2.384185791015625e-7) : T(4.440892098500626e-16);   // 2^-22, 2^-51
+        for (int t = 0; t < w; ++t) {
+            duR = hmin(duR, R(CX_BT + 2 * t));
+            duL = hmax(duL, R(CX_BT + 2 * t + 1));
+        }
+#pragma unroll
+        for (int kk = 0; kk < K; ++kk) {
+            if (!used(kk)) continue;
+            const T uu = uk(kk);
+            const T mR = -(uu + du_CFL), mL = -(uu - du_CFL), tol = tiny * (vabs(uu) + du_CFL);
+            const T gR = vabs(duR - mR), gL = vabs(duL - mL);
+            close = close || (gR > T(0.0) && gR <= tol) || (gL > T(0.0) && gL <= tol);
+            duR = hmin(duR, mR);
+            duL = hmax(duL, mL);
+        }
+        for (int t = w + 1; t < W; ++t) {
+            duR = hmin(duR, R(CX_BT + 2 * t));
+            duL = hmax(duL, R(CX_BT + 2 * t + 1));
+        }
+        if (__any(close)) R(CX_BT + 2 * W) = T(1.0);
+        lds_barrier();
+        if (block_any(R(CX_BT + 2 * W) != T(0.0))) {
+            if (w == 0)
+                R(CX_BT + 0) = lds_fold<0>(U, nk, lane, x0R, [&](T x, T uu) {
+                    return (uu + x > -du_CFL) ? -(uu + du_CFL) : x;
+                });
+            if (w == 1)
+                R(CX_BT + 1) = lds_fold<0>(U, nk, lane, x0L, [&](T x, T uu) {
+                    return (uu + x < du_CFL) ? -(uu - du_CFL) : x;
+                });
+            lds_barrier();
+            duR = R(CX_BT + 0);
+            duL = R(CX_BT + 1);
+        }
+    }
+    // FAmt_0 = sum dy*hm(u + du0): the sum of the iteration's last evaluation
+    // when that was at du0 (the same terms in the same order), else a pass of
+    // its own; FAmt_L, uhtot_L at u + duL; FAmt_R, uhtot_R at u + duR
+    const bool have0 = (du0_eval == du0);
+    T uhtot_L = T(0.0), FAmt_L = T(0.0), uhtot_R = T(0.0), FAmt_R = T(0.0);
+#pragma nounroll
+    for (int pass = block_any(!have0) ? 0 : 1; pass < 3; ++pass) {
+        const T du = pass == 0 ? du0 : pass == 1 ? duL : duR;
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            if (g == NG - 1 && n <= NMIN) break;
+            if (!stored) {
+#pragma unroll
+                for (int kk = g_lo(g); kk < g_hi(g); ++kk) store_slot(kk, du_u, col.hm[kk]);
+            }
+            eval_group(g, du);
+        }
+        stored = true;
+        sum_pass(T(0.0), std::false_type{}, T(0.0), T(0.0));
+        if (pass == 0) {
+            if (!have0) FAmt_0 = R(CX_FIN + 1);
+        } else if (pass == 1) {
+            uhtot_L = R(CX_FIN + 0);
+            FAmt_L = R(CX_FIN + 1);
+        } else {
+            uhtot_R = R(CX_FIN + 0);
+            FAmt_R = R(CX_FIN + 1);
+        }
+    }
+    if (!writes_face || w != 0) return;
+    bt_cont_store(a, c2, du0, FAmt_0, duL, uhtot_L, FAmt_L, duR, uhtot_R, FAmt_R);
+}
+
+template <typename T, int K, int BASE>
+__global__ void __launch_bounds__(64 * kSplitWaves) __attribute__((amdgpu_waves_per_eu(cont_split_waves<T>(K))))
+k_continuity_split(ContArgsT<T> a, int monotonic)
+{
+    continuity_x_split<T, K, BASE>(a, monotonic, blockIdx.x, blockIdx.y);
+}
+
+template <typename T, int CW, int K, bool EVEN>
 __global__ void __launch_bounds__(64 * CW) __attribute__((amdgpu_waves_per_eu(
-    (sizeof(T) == 4 || FW == 32) ? 4 : (CW + 3) / 4, (CW >= 12 || sizeof(T) == 4 || FW == 32) ? 4 : 2)))
+    sizeof(T) == 4 ? 4 : (CW + 3) / 4, (CW >= 12 || sizeof(T) == 4) ? 4 : 2)))
 k_continuity_blk(ContArgsT<T> a, int monotonic)
 {
-    continuity_body<T, Y, CW, K, FW, EVEN>(a, monotonic, blockIdx.x, blockIdx.y, true);
+    continuity_body<T, CW, K, EVEN>(a, monotonic, blockIdx.x, blockIdx.y);
 }
 
 // the members of an ensemble that one batched launch covers: entry q of its
@@ -1264,14 +1667,25 @@ struct MemberIndex {
 
 // the members of an ensemble whose depth takes the block shape CW x K, in one
 // launch (EVEN: every one of them spreads its levels evenly)
-template <typename T, bool Y, int CW, int K, bool EVEN>
+template <typename T, int CW, int K, bool EVEN>
 __global__ void __launch_bounds__(64 * CW) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 1, (CW >= 16 || sizeof(T) == 4) ? 4 : 2)))
 k_continuity_batch(const ContArgsT<T> *__restrict__ args, BatchMap mp, MemberIndex mi)
 {
     int m, local;
     batch_locate(mp, blockIdx.x, m, local);
     const ContArgsT<T> a = args[mi.v[m]];
-    continuity_body<T, Y, CW, K, CF, EVEN>(a, a.monotonic, local % mp.nbx[m], local / mp.nbx[m]);
+    continuity_body<T, CW, K, EVEN>(a, a.monotonic, local % mp.nbx[m], local / mp.nbx[m]);
+}
+
+// the same for the zonal pass and members of one slot class
+template <typename T, int K>
+__global__ void __launch_bounds__(64 * kSplitWaves) __attribute__((amdgpu_waves_per_eu(cont_split_waves<T>(K))))
+k_continuity_split_batch(const ContArgsT<T> *__restrict__ args, BatchMap mp, MemberIndex mi)
+{
+    int m, local;
+    batch_locate(mp, blockIdx.x, m, local);
+    const ContArgsT<T> a = args[mi.v[m]];
+    continuity_x_split<T, K, CX_BASE>(a, a.monotonic, local % mp.nbx[m], local / mp.nbx[m]);
 }
 
 // the driver's `h = h0` reset for the cells the convergence does not write:
@@ -1376,13 +1790,6 @@ __global__ void k_convergence(Dims d, const double *hin, const double *__restric
     }
 }
 
-// FP64 block shape beyond 32 levels: false = 64 faces x 12 waves of 7 levels
-// (1.21 ms per call at 720x720x75), true = 32 faces x 8 waves x 2 groups of 5
-// levels, two blocks per CU (1.31 ms: 128 VGPRs with spills, and a block's
-// latency chains -- the column folds, the barriers, the loads -- do not
-// shorten with fewer faces)
-constexpr bool kFP64Narrow = false;
-
 // Blocks in x of a pass with FW faces per block (x: blocks overlap by two faces)
 template <bool Y>
 unsigned blk_nbx(const Dims &d, int FW)
@@ -1393,37 +1800,59 @@ unsigned blk_nbx(const Dims &d, int FW)
 // A block shape of CW waves of K level slots (64 faces): levels spread evenly
 // over the waves when CW*(K-1) <= nk (every shape of 1 or 2 slots, 8 x 4 from
 // 24 levels, 12 x 7 and 8 x 10 from 72)
-template <typename T, bool Y, int CW, int K>
+template <typename T, int CW, int K>
 void launch_shape(const ContArgsT<T> &a, int mono, dim3 g, hipStream_t s)
 {
     const dim3 b(64 * CW);
     constexpr size_t lds = sizeof(ContShared<T, CW, K>);
     if constexpr (K <= 2) {
-        k_continuity_blk<T, Y, CW, K, CF, true><<<g, b, lds, s>>>(a, mono);
+        k_continuity_blk<T, CW, K, true><<<g, b, lds, s>>>(a, mono);
     } else {
-        if (a.d.nk >= CW * (K - 1)) k_continuity_blk<T, Y, CW, K, CF, true><<<g, b, lds, s>>>(a, mono);
-        else k_continuity_blk<T, Y, CW, K, CF, false><<<g, b, lds, s>>>(a, mono);
+        if (a.d.nk >= CW * (K - 1)) k_continuity_blk<T, CW, K, true><<<g, b, lds, s>>>(a, mono);
+        else k_continuity_blk<T, CW, K, false><<<g, b, lds, s>>>(a, mono);
     }
 }
 
-// One pass over nby rows of faces; the block shape follows nk and the type
-template <typename T, bool Y>
-int launch_blk(const ContArgsT<T> &a, int mono, unsigned nby, hipStream_t s)
+// The zonal pass over nby rows of faces (columns of up to kSplitMax levels)
+template <typename T, int BASE>
+void launch_x_base(const ContArgsT<T> &a, int mono, dim3 g, hipStream_t s)
+{
+    const dim3 b(64 * kSplitWaves);
+    const size_t lds = cont_split_lds<T>(a.d.nk);
+    switch (slot_class(a.d.nk)) {
+    case 4: k_continuity_split<T, 4, BASE><<<g, b, lds, s>>>(a, mono); break;
+    case 7: k_continuity_split<T, 7, BASE><<<g, b, lds, s>>>(a, mono); break;
+    case 10: k_continuity_split<T, 10, BASE><<<g, b, lds, s>>>(a, mono); break;
+    case 13: k_continuity_split<T, 13, BASE><<<g, b, lds, s>>>(a, mono); break;
+    case 16: k_continuity_split<T, 16, BASE><<<g, b, lds, s>>>(a, mono); break;
+    case 19: k_continuity_split<T, 19, BASE><<<g, b, lds, s>>>(a, mono); break;
+    default: k_continuity_split<T, 20, BASE><<<g, b, lds, s>>>(a, mono); break;
+    }
+}
+
+template <typename T>
+int launch_x(const ContArgsT<T> &a, int mono, hipStream_t s)
+{
+    const dim3 g(blk_nbx<false>(a.d, CF), (unsigned)(a.d.jec - a.d.jsc + 1));
+    if (cont_split_wide<T>(a.d)) launch_x_base<T, 1>(a, mono, g, s);
+    else launch_x_base<T, CX_BASE>(a, mono, g, s);
+    MOM6H_LAUNCH_CHECK();
+    return MOM6H_OK;
+}
+
+// The meridional pass over nby rows of faces; the block shape follows nk and the type
+template <typename T>
+int launch_y(const ContArgsT<T> &a, int mono, unsigned nby, hipStream_t s)
 {
     const int nk = a.d.nk;
-    const dim3 g(blk_nbx<Y>(a.d, CF), nby);
-    if (nk <= 8) launch_shape<T, Y, 8, 1>(a, mono, g, s);
-    else if (nk <= 16) launch_shape<T, Y, 8, 2>(a, mono, g, s);
-    else if (nk <= 32) launch_shape<T, Y, 8, 4>(a, mono, g, s);
+    const dim3 g(blk_nbx<true>(a.d, CF), nby);
+    if (nk <= 8) launch_shape<T, 8, 1>(a, mono, g, s);
+    else if (nk <= 16) launch_shape<T, 8, 2>(a, mono, g, s);
+    else if (nk <= 32) launch_shape<T, 8, 4>(a, mono, g, s);
     // FP64 beyond 32 levels: 12 waves of 7 levels (three waves per SIMD); the
     // FP32 form: 8 waves of 10 levels (two blocks per CU)
-    else if (sizeof(T) == 8 && !kFP64Narrow) launch_shape<T, Y, 12, 7>(a, mono, g, s);
-    // the alternative: blocks of 32 faces, 8 waves x 2 level groups of 5
-    // levels (64 KB of LDS, two blocks per CU)
-    else if (sizeof(T) == 8)
-        k_continuity_blk<T, Y, 8, 5, 32><<<dim3(blk_nbx<Y>(a.d, 32), nby), dim3(64 * 8), sizeof(ContShared<T, 8, 5, 32>),
-                                            s>>>(a, mono);
-    else launch_shape<T, Y, 8, 10>(a, mono, g, s);
+    else if (sizeof(T) == 8) launch_shape<T, 12, 7>(a, mono, g, s);
+    else launch_shape<T, 8, 10>(a, mono, g, s);
     MOM6H_LAUNCH_CHECK();
     return MOM6H_OK;
 }
@@ -1437,31 +1866,19 @@ int set_blk_lds(long long max_lds)
         if (bytes > max_lds) return hipSuccess;
         return hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
     };
-#define MOM6H_BLK_LDS(Y, CW, K)                                                                                    \
-    MOM6H_CHECK(raise((const void *)k_continuity_blk<T, Y, CW, K, CF, true>, sizeof(ContShared<T, CW, K>)));        \
-    MOM6H_CHECK(raise((const void *)k_continuity_blk<T, Y, CW, K, CF, false>, sizeof(ContShared<T, CW, K>)));       \
-    MOM6H_CHECK(raise((const void *)k_continuity_batch<T, Y, CW, K, true>, sizeof(ContShared<T, CW, K>)));
-#define MOM6H_BATCH_PLAIN_LDS(Y, K)                                                                                \
-    MOM6H_CHECK(raise((const void *)k_continuity_batch<T, Y, 8, K, false>, sizeof(ContShared<T, 8, K>)));
-    MOM6H_BLK_LDS(false, 8, 1) MOM6H_BLK_LDS(false, 8, 2) MOM6H_BLK_LDS(false, 8, 4) MOM6H_BLK_LDS(false, 8, 10)
-    MOM6H_BLK_LDS(true, 8, 1) MOM6H_BLK_LDS(true, 8, 2) MOM6H_BLK_LDS(true, 8, 4) MOM6H_BLK_LDS(true, 8, 10)
-    MOM6H_BATCH_PLAIN_LDS(false, 4) MOM6H_BATCH_PLAIN_LDS(false, 7) MOM6H_BATCH_PLAIN_LDS(false, 10)
-    MOM6H_BATCH_PLAIN_LDS(true, 4) MOM6H_BATCH_PLAIN_LDS(true, 7) MOM6H_BATCH_PLAIN_LDS(true, 10)
-    MOM6H_CHECK(raise((const void *)k_continuity_batch<T, false, 8, 7, true>, sizeof(ContShared<T, 8, 7>)));
-    MOM6H_CHECK(raise((const void *)k_continuity_batch<T, true, 8, 7, true>, sizeof(ContShared<T, 8, 7>)));
+#define MOM6H_BLK_LDS(CW, K)                                                                                       \
+    MOM6H_CHECK(raise((const void *)k_continuity_blk<T, CW, K, true>, sizeof(ContShared<T, CW, K>)));        \
+    MOM6H_CHECK(raise((const void *)k_continuity_blk<T, CW, K, false>, sizeof(ContShared<T, CW, K>)));       \
+    MOM6H_CHECK(raise((const void *)k_continuity_batch<T, CW, K, true>, sizeof(ContShared<T, CW, K>)));
+#define MOM6H_BATCH_PLAIN_LDS(K)                                                                                   \
+    MOM6H_CHECK(raise((const void *)k_continuity_batch<T, 8, K, false>, sizeof(ContShared<T, 8, K>)));
+    MOM6H_BLK_LDS(8, 1) MOM6H_BLK_LDS(8, 2) MOM6H_BLK_LDS(8, 4) MOM6H_BLK_LDS(8, 10)
+    MOM6H_BATCH_PLAIN_LDS(4) MOM6H_BATCH_PLAIN_LDS(7) MOM6H_BATCH_PLAIN_LDS(10)
+    MOM6H_CHECK(raise((const void *)k_continuity_batch<T, 8, 7, true>, sizeof(ContShared<T, 8, 7>)));
 #undef MOM6H_BATCH_PLAIN_LDS
 #undef MOM6H_BLK_LDS
-    for (const bool Y : {false, true}) {
-        const void *even = Y ? (const void *)k_continuity_blk<T, true, 12, 7, CF, true>
-                             : (const void *)k_continuity_blk<T, false, 12, 7, CF, true>;
-        const void *plain = Y ? (const void *)k_continuity_blk<T, true, 12, 7, CF, false>
-                              : (const void *)k_continuity_blk<T, false, 12, 7, CF, false>;
-        const void *narrow = Y ? (const void *)k_continuity_blk<T, true, 8, 5, 32>
-                               : (const void *)k_continuity_blk<T, false, 8, 5, 32>;
-        MOM6H_CHECK(raise(even, sizeof(ContShared<T, 12, 7>)));
-        MOM6H_CHECK(raise(plain, sizeof(ContShared<T, 12, 7>)));
-        MOM6H_CHECK(raise(narrow, sizeof(ContShared<T, 8, 5, 32>)));
-    }
+    MOM6H_CHECK(raise((const void *)k_continuity_blk<T, 12, 7, true>, sizeof(ContShared<T, 12, 7>)));
+    MOM6H_CHECK(raise((const void *)k_continuity_blk<T, 12, 7, false>, sizeof(ContShared<T, 12, 7>)));
     return MOM6H_OK;
 }
 
@@ -1478,7 +1895,9 @@ bool blk_fits(const mom6h_continuity_cs *cs)
     constexpr long long bytes = sizeof(ContShared<double, 12, 7>) > sizeof(ContShared<double, 8, 10>)
                                     ? sizeof(ContShared<double, 12, 7>)
                                     : sizeof(ContShared<double, 8, 10>);
-    return cs->d.nk <= 80 && !cs->upwind_1st && !cs->simple_2nd && bytes <= cs->max_lds;
+    // and, for 32-bit byte offsets within a plane, planes below 4 GiB
+    return cs->d.nk <= 80 && !cs->upwind_1st && !cs->simple_2nd && bytes <= cs->max_lds &&
+           cs->d.s2 * (long long)sizeof(double) < (1LL << 32);
 }
 
 // The zonal pass of the block kernel for either type
@@ -1493,7 +1912,7 @@ int continuity_blk_x(mom6h_continuity_cs *cs, const T *u, const T *hin, T *h, T 
                    bt ? bt->FA_u_EE : nullptr, bt ? bt->FA_u_E0 : nullptr, bt ? bt->FA_u_W0 : nullptr,
                    bt ? bt->FA_u_WW : nullptr, bt ? bt->uBT_WW : nullptr, bt ? bt->uBT_EE : nullptr,
                    bt ? bt_h_u : nullptr};
-    int rc = launch_blk<T, false>(a, cs->monotonic, (unsigned)(d.jec - d.jsc + 1), s);
+    int rc = launch_x<T>(a, cs->monotonic, s);
     if (rc) return rc;
     if (hin_halo_to_h) {
         launch_halo_copy(d, hin, h, s);
@@ -1513,7 +1932,7 @@ int continuity_blk_y(mom6h_continuity_cs *cs, const T *v, const T *hin, T *h, T 
                    bt ? bt->FA_u_EE : nullptr, bt ? bt->FA_u_E0 : nullptr, bt ? bt->FA_u_W0 : nullptr,
                    bt ? bt->FA_u_WW : nullptr, bt ? bt->uBT_WW : nullptr, bt ? bt->uBT_EE : nullptr,
                    bt ? bt_h_v : nullptr};
-    int rc = launch_blk<T, true>(a, cs->monotonic, (unsigned)(d.jec - d.jsc + 2), s);
+    int rc = launch_y<T>(a, cs->monotonic, (unsigned)(d.jec - d.jsc + 2), s);
     if (rc) return rc;
     {
         dim3 b(128), gc((d.iec - d.isc + 1 + 127) / 128, d.jec - d.jsc + 1, d.nk);
@@ -1545,13 +1964,51 @@ int continuity_batch(const ContArgsT<T> *d_args, const ContArgsT<T> *h_args, int
         nk_max = d.nk > nk_max ? d.nk : nk_max;
     }
     MOM6H_REQUIRE(nk_max <= 80 && (long long)sizeof(ContShared<T, 8, 10>) <= max_lds, "continuity batch: nk <= 80");
-    // one launch per block shape: 8 waves of K level slots, K from the
-    // member's depth (a member of 25 levels takes 8 x 4 = 32 slots rather than
-    // the 80 of the deepest member's 8 x 10); the levels spread evenly when
-    // every member of the launch has nk >= 8*(K-1)
+    // one launch per block shape, K from the member's depth.  x: the slot class
+    bool wide = false;
+    for (int m = 0; m < n; ++m) wide = wide || cont_split_wide<T>(h_args[m].d);
+    if (!y_pass && wide) {   // member by member
+        for (int m = 0; m < n; ++m) {
+            const int rc = launch_x<T>(h_args[m], h_args[m].monotonic, s);
+            if (rc) return rc;
+        }
+    } else if (!y_pass) {
+        for (const int K : {4, 7, 10, 13, 16, 19, 20}) {
+            BatchMap g{};
+            MemberIndex mi{};
+            int nk_class = 1;
+            for (int m = 0; m < n; ++m) {
+                const int nk = h_args[m].d.nk;
+                if (slot_class(nk) != K) continue;
+                const int q = g.n++;
+                mi.v[q] = m;
+                g.nbx[q] = mp.nbx[m];
+                g.nby[q] = mp.nby[m];
+                g.first[q + 1] = g.first[q] + g.nbx[q] * g.nby[q];
+                nk_class = nk > nk_class ? nk : nk_class;
+            }
+            if (g.n == 0) continue;
+            const dim3 nb((unsigned)g.first[g.n]), b(64 * kSplitWaves);
+            const size_t lds = cont_split_lds<T>(nk_class);
+            switch (K) {
+            case 4: k_continuity_split_batch<T, 4><<<nb, b, lds, s>>>(d_args, g, mi); break;
+            case 7: k_continuity_split_batch<T, 7><<<nb, b, lds, s>>>(d_args, g, mi); break;
+            case 10: k_continuity_split_batch<T, 10><<<nb, b, lds, s>>>(d_args, g, mi); break;
+            case 13: k_continuity_split_batch<T, 13><<<nb, b, lds, s>>>(d_args, g, mi); break;
+            case 16: k_continuity_split_batch<T, 16><<<nb, b, lds, s>>>(d_args, g, mi); break;
+            case 19: k_continuity_split_batch<T, 19><<<nb, b, lds, s>>>(d_args, g, mi); break;
+            default: k_continuity_split_batch<T, 20><<<nb, b, lds, s>>>(d_args, g, mi); break;
+            }
+            MOM6H_LAUNCH_CHECK();
+        }
+    }
+    // y: 8 waves of K level slots (a member of 25 levels takes 8 x 4 = 32 slots
+    // rather than the 80 of the deepest member's 8 x 10); the levels spread
+    // evenly when every member of the launch has nk >= 8*(K-1)
     const int shapes[5] = {1, 2, 4, 7, 10};
     auto shape_of = [](int nk) { return nk <= 8 ? 1 : nk <= 16 ? 2 : nk <= 32 ? 4 : nk <= 56 ? 7 : 10; };
     for (const int K : shapes) {
+        if (!y_pass) break;
         BatchMap g{};
         MemberIndex mi{};
         bool even = true;
@@ -1568,25 +2025,20 @@ int continuity_batch(const ContArgsT<T> *d_args, const ContArgsT<T> *h_args, int
         if (g.n == 0) continue;
         const unsigned nb = (unsigned)g.first[g.n];
         const dim3 b(64 * 8);
-#define CB(Y, KK)                                                                                             \
-    if (even) k_continuity_batch<T, Y, 8, KK, true><<<nb, b, sizeof(ContShared<T, 8, KK>), s>>>(d_args, g, mi); \
-    else k_continuity_batch<T, Y, 8, KK, false><<<nb, b, sizeof(ContShared<T, 8, KK>), s>>>(d_args, g, mi);
-#define CBY(KK) \
-    if (y_pass) { CB(true, KK) } else { CB(false, KK) }
+#define CB(KK)                                                                                                   \
+    if (even) k_continuity_batch<T, 8, KK, true><<<nb, b, sizeof(ContShared<T, 8, KK>), s>>>(d_args, g, mi); \
+    else k_continuity_batch<T, 8, KK, false><<<nb, b, sizeof(ContShared<T, 8, KK>), s>>>(d_args, g, mi);
         if (K == 1) {   // shapes of 1 and 2 slots always spread evenly
-            if (y_pass) k_continuity_batch<T, true, 8, 1, true><<<nb, b, sizeof(ContShared<T, 8, 1>), s>>>(d_args, g, mi);
-            else k_continuity_batch<T, false, 8, 1, true><<<nb, b, sizeof(ContShared<T, 8, 1>), s>>>(d_args, g, mi);
+            k_continuity_batch<T, 8, 1, true><<<nb, b, sizeof(ContShared<T, 8, 1>), s>>>(d_args, g, mi);
         } else if (K == 2) {
-            if (y_pass) k_continuity_batch<T, true, 8, 2, true><<<nb, b, sizeof(ContShared<T, 8, 2>), s>>>(d_args, g, mi);
-            else k_continuity_batch<T, false, 8, 2, true><<<nb, b, sizeof(ContShared<T, 8, 2>), s>>>(d_args, g, mi);
+            k_continuity_batch<T, 8, 2, true><<<nb, b, sizeof(ContShared<T, 8, 2>), s>>>(d_args, g, mi);
         } else if (K == 4) {
-            CBY(4)
+            CB(4)
         } else if (K == 7) {
-            CBY(7)
+            CB(7)
         } else {
-            CBY(10)
+            CB(10)
         }
-#undef CBY
 #undef CB
         MOM6H_LAUNCH_CHECK();
     }

@@ -7,6 +7,7 @@
 // with -ffp-contract=off: no FMA contraction, IEEE division, Fortran's
 // left-to-right association kept by explicit parentheses.
 #pragma once
+#include <type_traits>
 
 #include <hip/hip_runtime.h>
 
@@ -80,6 +81,45 @@ __device__ __forceinline__ void lds_barrier()
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
+
+// Level-split column kernels: a block of kSplitWaves waves owns 64 columns, each
+// wave a quarter of the levels in registers (L slots).  Slot classes: few
+// unused slots at any depth.
+constexpr int kSplitWaves = 4;
+constexpr int kSplitMax = 80;   // kSplitWaves * the largest class
+__host__ __device__ constexpr int slot_class(int nk)
+{
+    return nk <= 16 ? 4 : nk <= 28 ? 7 : nk <= 40 ? 10 : nk <= 52 ? 13 : nk <= 64 ? 16 : nk <= 76 ? 19 : 20;
+}
+// slots in use in every wave of a column of class L
+__host__ __device__ constexpr int slot_min(int L) { return L == 4 ? 0 : L == 20 ? 19 : L - 3; }
+
+// An array from a uniform address on, for accesses at a lane's byte offset plus
+// a uniform one (each below 4 GiB)
+template <typename T>
+struct LevelBuf {
+    __amdgpu_buffer_rsrc_t r;
+    using V = std::remove_const_t<T>;
+    using B = std::conditional_t<sizeof(V) == 8, unsigned __attribute__((ext_vector_type(2))), unsigned>;
+    __device__ __forceinline__ explicit LevelBuf(T *base)
+        : r(__builtin_amdgcn_make_buffer_rsrc((void *)base, 0, 0xffffffffu, 0x00027000))
+    {
+    }
+    __device__ __forceinline__ V load(unsigned lane_off, unsigned off) const
+    {
+        if constexpr (sizeof(V) == 8)
+            return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(r, lane_off, off, 0));
+        else
+            return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(r, lane_off, off, 0));
+    }
+    __device__ __forceinline__ void store(V x, unsigned lane_off, unsigned off) const
+    {
+        if constexpr (sizeof(V) == 8)
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(B, x), r, lane_off, off, 0);
+        else
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(B, x), r, lane_off, off, 0);
+    }
+};
 
 // Several grids (the members of an ensemble) in one launch: the blocks of
 // member m are first[m] .. first[m+1]-1, laid out as that member's own

@@ -546,7 +546,7 @@ __device__ __forceinline__ void vv_body(const VVArgs<T> &p, int bx, int row, VVS
     if (act) *tb_out = t;
 }
 
-// Level-split variant, for columns of up to VV_SPLIT_MAX levels.  A block of
+// Level-split variant, for columns of up to kSplitMax levels.  A block of
 // four waves owns 64 columns of one row; wave w holds a quarter of the levels
 // in registers (L slots, n of them in use) and reads them once, so nothing but
 // the state goes through memory and every division off the tridiagonal
@@ -567,22 +567,13 @@ __device__ __forceinline__ void vv_body(const VVArgs<T> &p, int bx, int row, VVS
 // keeps the deeper columns (more slots would spill) and planes whose level
 // offsets pass 4 GiB.  One spilled value per level made it slower than the
 // chunked kernel (1170 us), hence the pins and fences below.
-constexpr int VV_W = 4;                       // waves (level groups) of a block
-constexpr int VV_SPLIT_MAX = 80;              // VV_W * the largest slot class
 constexpr int VV_HAND = 4;                    // LDS rows of the hand-over between waves
 constexpr int VV_G = 6;                       // levels whose divisions are interleaved (2 and 4 measured 1-3% slower)
-
-// slot classes (L slots, up to VV_W*L levels): few unused slots at any depth
-__host__ __device__ constexpr int vv_class(int nk)
-{
-    return nk <= 16 ? 4 : nk <= 28 ? 7 : nk <= 40 ? 10 : nk <= 52 ? 13 : nk <= 64 ? 16 : nk <= 76 ? 19 : 20;
-}
-constexpr int vv_nmin(int L) { return L == 4 ? 0 : L == 20 ? 19 : L - 3; }   // slots in use in every wave
 
 // columns the level-split kernel takes: its level offsets are 32-bit bytes
 inline bool vv_split_fits(const Dims &d)
 {
-    return d.nk <= VV_SPLIT_MAX && VV_SPLIT_MAX / VV_W * d.s2 * (long long)sizeof(double) < (1LL << 32);
+    return d.nk <= kSplitMax && kSplitMax / kSplitWaves * d.s2 * (long long)sizeof(double) < (1LL << 32);
 }
 
 template <typename T>
@@ -600,39 +591,12 @@ constexpr int vv_waves(int L)
     return L > 13 ? 3 : L > 7 ? 4 : L > 4 ? 6 : 8;
 }
 
-// An array from a uniform address on, for accesses at a lane's byte offset plus
-// a uniform one (each below 4 GiB)
-template <typename T>
-struct LevelBuf {
-    __amdgpu_buffer_rsrc_t r;
-    using V = std::remove_const_t<T>;
-    using B = std::conditional_t<sizeof(V) == 8, unsigned __attribute__((ext_vector_type(2))), unsigned>;
-    __device__ __forceinline__ explicit LevelBuf(T *base)
-        : r(__builtin_amdgcn_make_buffer_rsrc((void *)base, 0, 0xffffffffu, 0x00027000))
-    {
-    }
-    __device__ __forceinline__ V load(unsigned lane_off, unsigned off) const
-    {
-        if constexpr (sizeof(V) == 8)
-            return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(r, lane_off, off, 0));
-        else
-            return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(r, lane_off, off, 0));
-    }
-    __device__ __forceinline__ void store(V x, unsigned lane_off, unsigned off) const
-    {
-        if constexpr (sizeof(V) == 8)
-            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(B, x), r, lane_off, off, 0);
-        else
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(B, x), r, lane_off, off, 0);
-    }
-};
-
 template <typename T, bool KEEP, bool RAY3, int L>
 __device__ __forceinline__ void vv_split(const VVArgs<T> &p, int bx, int row, double *lds)
 {
     using C = T;                 // arithmetic of the coefficients (as in vv_body)
     using ZT = VVSlot<T>;
-    constexpr int NMIN = vv_nmin(L);
+    constexpr int NMIN = slot_min(L);
     const Dims &d = p.d;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -643,7 +607,7 @@ __device__ __forceinline__ void vv_split(const VVArgs<T> &p, int bx, int row, do
     const int j = is_u ? d.jsc + (row - 1) / 2 : d.jsc - 1 + row / 2;
     if (i > d.iec) return;       // the same lanes in every wave
     const long long c2 = IX2(d, i, j);
-    const int q = nk / VV_W, r = nk % VV_W;
+    const int q = nk / kSplitWaves, r = nk % kSplitWaves;
     const int n = q + (w < r ? 1 : 0);                 // this wave's levels k1 .. k1+n-1
     const int k1 = w * q + (w < r ? w : r) + 1;
     double *Hs = lds + lane;                           // hand-over rows
@@ -837,9 +801,9 @@ __device__ __forceinline__ void vv_split(const VVArgs<T> &p, int bx, int row, do
         }
         vbot = vprev;
         abot = a_k;
-        if (w < VV_W - 1) { Hs[0] = d1; Hs[64] = b1; Hs[128] = vprev; Hs[192] = a_k; }
+        if (w < kSplitWaves - 1) { Hs[0] = d1; Hs[64] = b1; Hs[128] = vprev; Hs[192] = a_k; }
     }
-    for (int t = w; t < 2 * (VV_W - 1) - w; ++t) lds_barrier();
+    for (int t = w; t < 2 * (kSplitWaves - 1) - w; ++t) lds_barrier();
     // ---- back substitution, bottom-up (:447-449) ----
     {
         const bool bottom = n > 0 && k1 + n - 1 == nk;
@@ -889,7 +853,7 @@ __device__ __forceinline__ void vv_split(const VVArgs<T> &p, int bx, int row, do
 
 // one grid, tiles renumbered per XCD
 template <typename T, bool KEEP, bool RAY3, int L>
-__global__ void __launch_bounds__(64 * VV_W) __attribute__((amdgpu_waves_per_eu(vv_waves<T, RAY3>(L))))
+__global__ void __launch_bounds__(64 * kSplitWaves) __attribute__((amdgpu_waves_per_eu(vv_waves<T, RAY3>(L))))
 k_vert_visc_split(VVArgs<T> p)
 {
     extern __shared__ double Zs_raw[];
@@ -901,8 +865,8 @@ template <typename T, bool KEEP, bool RAY3>
 void vv_split_launch(const VVArgs<T> &p, dim3 g, hipStream_t s)
 {
     const size_t lds = vv_split_lds<T>(p.d.nk);
-    const dim3 b(64 * VV_W);
-    switch (vv_class(p.d.nk)) {
+    const dim3 b(64 * kSplitWaves);
+    switch (slot_class(p.d.nk)) {
     case 4: k_vert_visc_split<T, KEEP, RAY3, 4><<<g, b, lds, s>>>(p); break;
     case 7: k_vert_visc_split<T, KEEP, RAY3, 7><<<g, b, lds, s>>>(p); break;
     case 10: k_vert_visc_split<T, KEEP, RAY3, 10><<<g, b, lds, s>>>(p); break;
@@ -941,7 +905,7 @@ k_vert_visc_batch(const VVArgs<T> *__restrict__ args, BatchMap mp)
 
 // the same with level-split members only
 template <typename T>
-__global__ void __launch_bounds__(64 * VV_W) __attribute__((amdgpu_waves_per_eu(vv_waves<T, false>(20))))
+__global__ void __launch_bounds__(64 * kSplitWaves) __attribute__((amdgpu_waves_per_eu(vv_waves<T, false>(20))))
 k_vert_visc_split_batch(const VVArgs<T> *__restrict__ args, BatchMap mp)
 {
     extern __shared__ double Zs_raw[];
@@ -949,7 +913,7 @@ k_vert_visc_split_batch(const VVArgs<T> *__restrict__ args, BatchMap mp)
     batch_locate(mp, xcd_tile(blockIdx.x, gridDim.x), m, local);
     const VVArgs<T> p = args[m];
     const int bx = local % mp.nbx[m], row = local / mp.nbx[m];
-    switch (vv_class(p.d.nk)) {
+    switch (slot_class(p.d.nk)) {
     case 4: vv_split<T, false, false, 4>(p, bx, row, Zs_raw); break;
     case 7: vv_split<T, false, false, 7>(p, bx, row, Zs_raw); break;
     case 10: vv_split<T, false, false, 10>(p, bx, row, Zs_raw); break;
@@ -1002,7 +966,7 @@ int vert_visc_batch(const VVArgs<T> *d_args, const VVArgs<T> *h_args, int n, lon
     const size_t lds = (size_t)(nk_max + 1) * 64 * sizeof(VVSlot<T>);
     MOM6H_REQUIRE((long long)lds <= max_lds, "vert_visc batch: nk = %d exceeds the LDS column", nk_max);
     if (split)
-        k_vert_visc_split_batch<T><<<(unsigned)mp.first[n], 64 * VV_W, vv_split_lds<T>(nk_max), s>>>(d_args, mp);
+        k_vert_visc_split_batch<T><<<(unsigned)mp.first[n], 64 * kSplitWaves, vv_split_lds<T>(nk_max), s>>>(d_args, mp);
     else
         k_vert_visc_batch<T><<<(unsigned)mp.first[n], 64, lds, s>>>(d_args, mp);
     MOM6H_LAUNCH_CHECK();
