@@ -549,8 +549,8 @@ __device__ __forceinline__ void vv_body(const VVArgs<T> &p, int bx, int row, VVS
 // Level-split variant, for columns of up to kSplitMax levels.  A block of
 // four waves owns 64 columns; wave w holds a quarter of the levels in registers
 // (L slots, n of them in use) and reads them once, so nothing but the state
-// goes through memory and every division off the tridiagonal
-// recurrence runs in four waves side by side.  The two running sums (z_i from
+// goes through memory and every division off the tridiagonal recurrence runs in
+// four waves side by side.  The two running sums (z_i from
 // the bottom, z_top from the top) go through LDS in the serial order: each wave
 // adds up the levels before its own again (a chain of adds costs less than
 // handing the sum on from wave to wave).  The recurrence passes from wave to
@@ -559,14 +559,15 @@ __device__ __forceinline__ void vv_body(const VVArgs<T> &p, int bx, int row, VVS
 //
 // The chunked kernel (one wave per SIMD, held there by its LDS column, and the
 // eliminated velocity written and read back: 2.8 GB a call) took 756 us per
-// FP64 call at 720x720x75 and 396 us in the FP32 form; this one 450 and 285 us
-// (1.6 GB, 3.5 TB/s, VALU 60% busy; FP32 73%): VALU issue and the recurrence's
-// latency at three waves per SIMD.  180x180x75: 76 -> 43 us, 471x363x50: 180 ->
-// 109, 300x260x25: 52 -> 31, 200x100x12: 21 -> 15; with drag at every level
-// 347x188x75 269 -> 97 (289 -> 122 with the coefficients stored).  Faster at every depth it takes; the chunked kernel
-// keeps the deeper columns (more slots would spill) and planes whose level
-// offsets pass 4 GiB.  One spilled value per level made it slower than the
-// chunked kernel (1170 us), hence the pins and fences below.
+// FP64 call at 720x720x75 and 396 us in the FP32 form; this one 438 and 270 us
+// (1.6 GB, 3.6 TB/s, VALU 61% busy; FP32 73%): VALU issue and the recurrence's
+// latency at three waves per SIMD.  180x180x75: 76 -> 38 us, 471x363x50: 180 ->
+// 107, 300x260x25: 52 -> 30, 200x100x12: 21 -> 12; with drag at every level
+// 347x188x75 269 -> 94 (289 -> 118 with the coefficients stored).  Faster at
+// every depth it takes; the chunked kernel keeps the deeper columns (more slots
+// would spill) and planes whose level offsets pass 4 GiB.  One spilled value per
+// level made it slower than the chunked kernel (1170 us), hence the pins and
+// fences below.
 constexpr int VV_HAND = 4;                    // LDS rows of the hand-over between waves
 constexpr int VV_G = 6;                       // levels whose divisions are interleaved (2 and 4 measured 1-3% slower)
 
