@@ -739,6 +739,13 @@ static HV make_hv(const mom6h_hor_visc_cs *cs)
 
 static bool closures_on(const mom6h_hor_visc_cs *cs) { return cs->smagorinsky || cs->leith || cs->better_bound; }
 
+// every metric that the options in use read is constant
+static bool march_takes(const mom6h_hor_visc_cs *cs)
+{
+    return cs->uniform && (!cs->biharmonic || cs->bih_uniform) && (!closures_on(cs) || cs->area_uniform) &&
+           (!cs->leith || cs->leith_uniform);
+}
+
 // the march's launch over the data domain: chunks of rows that leave about
 // four waves per SIMD, at least 8 (a chunk walks five rows more than it writes)
 template <bool SMAG, bool LEITH, bool BOUND, bool BIH>
@@ -877,7 +884,7 @@ int mom6h_hor_visc(mom6h_hor_visc_cs *cs, const double *u, const double *v, cons
     const Dims &d = cs->d;
     hipStream_t s = (hipStream_t)stream;
     HV p = make_hv(cs);
-    if (cs->uniform && (!cs->biharmonic || cs->bih_uniform) && (!closures_on(cs) || cs->closure_uniform) && !cs->general) {
+    if (march_takes(cs) && !cs->general) {
         const unsigned nring = (unsigned)((ring_points(d) + 63) / 64);
         if (closures_on(cs)) {
             k_hv_ring<<<dim3(nring, d.nk), 64, 0, s>>>(p, u, v, h, cs->ring_q);
@@ -922,26 +929,26 @@ int mom6h_hor_visc_set_closures(mom6h_hor_visc_cs *cs, int smagorinsky, int leit
     MOM6H_REQUIRE(!leith || (dxBu && dyBu && IdxBu && IdyBu), "mom6h_hor_visc_set_closures: Leith needs the q-point metrics");
     const size_t n2 = (size_t)cs->d.s2;
     int rc = 0;
+    // the metrics are the first call's; the march's values are taken with them
+    HVUniform &g = cs->g;
     if (smagorinsky || leith || better_bound) {
-        if (!cs->areaT) rc = dev_upload(&cs->areaT, areaT, n2);
+        if (!cs->areaT) {
+            rc = dev_upload(&cs->areaT, areaT, n2);
+            cs->area_uniform = hv_uniform(cs->d, {{areaT, &g.areaT}});
+        }
         if (!rc && !cs->ring_Kh) rc = dev_alloc(&cs->ring_Kh, n2, true);
         if (!rc && !cs->ring_Ah) rc = dev_alloc(&cs->ring_Ah, n2, true);
         if (!rc && !cs->ring_q) rc = dev_alloc(&cs->ring_q, (size_t)2 * cs->d.nk * ring_points(cs->d), false);
-        HVUniform &g = cs->g;
-        cs->closure_uniform = hv_uniform(cs->d, {{areaT, &g.areaT}});
-        if (leith) {
-            double dx = 0.0, dy = 0.0, idx = 0.0, idy = 0.0;
-            cs->closure_uniform = cs->closure_uniform &&
-                                  hv_uniform(cs->d, {{dxBu, &dx}, {dyBu, &dy}, {IdxBu, &idx}, {IdyBu, &idy}});
-            g.DY_dxBu_v = dy * idx;
-            g.DX_dyBu_v = dx * idy;
-        }
     }
     if (!rc && leith && !cs->dxBu) {
         rc = dev_upload(&cs->dxBu, dxBu, n2);
         rc = rc ? rc : dev_upload(&cs->dyBu, dyBu, n2);
         rc = rc ? rc : dev_upload(&cs->IdxBu, IdxBu, n2);
         rc = rc ? rc : dev_upload(&cs->IdyBu, IdyBu, n2);
+        double dx = 0.0, dy = 0.0, idx = 0.0, idy = 0.0;
+        cs->leith_uniform = hv_uniform(cs->d, {{dxBu, &dx}, {dyBu, &dy}, {IdxBu, &idx}, {IdyBu, &idy}});
+        g.DY_dxBu_v = dy * idx;
+        g.DX_dyBu_v = dx * idy;
     }
     if (rc) return rc;
     cs->smagorinsky = smagorinsky;

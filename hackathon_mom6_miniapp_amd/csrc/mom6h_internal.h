@@ -459,8 +459,8 @@ struct mom6h_hor_visc_cs {
     double *ring_Kh = nullptr, *ring_Ah = nullptr, *ring_q = nullptr;
     // every metric constant over the points the stencil reads (is-2..ie+2 x
     // js-2..je+2): the values, for the march; bih_uniform likewise for the four
-    // biharmonic metrics, closure_uniform for the closures'
-    int uniform = 0, bih_uniform = 0, closure_uniform = 0;
+    // biharmonic metrics, area_uniform and leith_uniform for the closures'
+    int uniform = 0, bih_uniform = 0, area_uniform = 0, leith_uniform = 0;
     int general = 0;         // use the general kernel even on a uniform grid
     mom6h::HVUniform g{};
 };

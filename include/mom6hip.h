@@ -199,7 +199,8 @@ int mom6h_hor_visc_set_options(mom6h_hor_visc_cs *cs, int laplacian, int biharmo
  * (mom6_hor_visc_serial.F90:160-286; Smagorinsky_Kh/_Ah, Leith_Kh/_Ah follow
  * the Laplacian/biharmonic switches; better_bound sets the Kh and Ah bounds)
  * with the grid metrics they need: areaT (the Smagorinsky, Leith and bound
- * constants), dxBu, dyBu, IdxBu, IdyBu (Leith).  Before the first call. */
+ * constants), dxBu, dyBu, IdxBu, IdyBu (Leith).  Before the first call; the
+ * metrics are those of the first call that needs them. */
 int mom6h_hor_visc_set_closures(mom6h_hor_visc_cs *cs, int smagorinsky, int leith, int better_bound,
                                 const double *h_areaT, const double *h_dxBu, const double *h_dyBu,
                                 const double *h_IdxBu, const double *h_IdyBu);
