@@ -64,6 +64,18 @@ int plan_momentum_batch(MomArgsT<T> *h_args, int n, int rows);
 template <typename T>
 int launch_momentum_batch(const MomArgsT<T> *d_args, const MomArgsT<T> *h_args, int n, hipStream_t s);
 
+// MomArgsT::mask from the FP64 masks (2D, n points each) of one or several grids
+struct MaskJob {
+    const double *mask2dT, *mask2dBu;
+    unsigned char *bits;
+    long long n;
+};
+struct MaskJobs {
+    int n;
+    MaskJob j[kMaxMembers];
+};
+int launch_mask_bits(const MaskJobs &jobs, hipStream_t s);
+
 // Rows a wave of the momentum stencil marches through for the options
 // momentum_tile and momentum_splits (0 while neither is set: chosen from the grid)
 inline int march_rows(int tile, int splits)

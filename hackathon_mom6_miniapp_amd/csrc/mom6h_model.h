@@ -41,7 +41,7 @@ struct mom6h_model {
     int fused = 1;           // fused momentum stencil (module-by-module when 0)
     bool uniform = false;    // every metric array constant (fused kernels allowed)
     bool fused_rows = false; // masks 0/1 and Coriolis constant along rows (what the fused stencil reads)
-    unsigned char *mask_bits = nullptr;   // those masks, one byte per point (MomArgsT::mask)
+    unsigned char *mask_bits = nullptr;   // those masks, one byte per point (MomArgsT::mask), from every step call
     UMetrics ug{};
     hipStream_t s0 = nullptr, s1 = nullptr;
     hipEvent_t e_start = nullptr, e_bt = nullptr;
@@ -94,4 +94,6 @@ struct mom6h_model {
 namespace mom6h {
 // the fused stencils apply (uniform metrics, Sadourny Coriolis, Laplacian [+ biharmonic])
 bool fused_ok(const mom6h_model *m);
+// the model's byte masks (allocated by the first call) as a job of launch_mask_bits
+int mask_job(mom6h_model *m, MaskJob *job);
 }  // namespace mom6h

@@ -632,12 +632,6 @@ int mom6h_model_prepare(mom6h_model *m)
         m->uniform = ok;
         m->fused_rows = binary_mask(mT.data(), n) && binary_mask(mBu.data(), n) &&
                         rows_uniform(fq.data(), (size_t)d.n1, (size_t)d.n2);
-        if (m->fused_rows) {
-            std::vector<unsigned char> bits(n);
-            for (size_t q = 0; q < n; ++q) bits[q] = (unsigned char)((mT[q] != 0.0 ? 1 : 0) | (mBu[q] != 0.0 ? 2 : 0));
-            RC(dev_alloc_bytes((void **)&m->mask_bits, n, false));
-            MOM6H_CHECK(hipMemcpy(m->mask_bits, bits.data(), n, hipMemcpyHostToDevice));
-        }
     }
     MOM6H_REQUIRE(!m->mixed || (m->uniform && m->fused_rows),
                   "mom6h_model_prepare: the mixed-precision form needs a grid with uniform metrics, 0/1 masks "
@@ -692,7 +686,13 @@ int mom6h_model_step(mom6h_model *m, int niter)
     // The fused path consumes vert_visc's coupling coefficients on chip; the
     // module path keeps them in the control structure, as the reference does.
     RC(mom6h_vert_visc_keep_coefficients(m->vv, fused_ok(m) ? 0 : 1));
+    // the fused stencil's byte masks follow the mask fields (ahead of a capture,
+    // which holds their address; on s0 behind the fork, so that s1 need not wait)
+    MaskJobs mj{};
+    if (fused_ok(m)) RC(mask_job(m, &mj.j[mj.n++]));
+    auto masks = [&]() -> int { return mj.n ? launch_mask_bits(mj, m->s0) : MOM6H_OK; };
     if (m->c.coupled) {
+        RC(masks());
         // the coupled form: each continuity call waits for its btstep call, so
         // the whole step runs in order on the 3D stream (one graph when captured)
         if (m->use_graph && !m->profile) {
@@ -726,6 +726,7 @@ int mom6h_model_step(mom6h_model *m, int niter)
         }
         MOM6H_CHECK(hipEventRecord(m->e_start, m->s0));
         MOM6H_CHECK(hipStreamWaitEvent(m->s1, m->e_start, 0));
+        RC(masks());
         for (int it = 0; it < niter; ++it) {
             MOM6H_CHECK(hipGraphLaunch(m->gexec_bt, m->s1));
             MOM6H_CHECK(hipGraphLaunch(m->gexec, m->s0));
@@ -735,6 +736,7 @@ int mom6h_model_step(mom6h_model *m, int niter)
         return MOM6H_OK;
     }
     if (m->serialize) {
+        RC(masks());
         for (int it = 0; it < niter; ++it) {
             RC(enqueue_barotropic(m));
             RC(enqueue_step(m));
@@ -751,6 +753,7 @@ int mom6h_model_step(mom6h_model *m, int niter)
     // chains would run one after the other instead of side by side.
     MOM6H_CHECK(hipEventRecord(m->e_start, m->s0));
     MOM6H_CHECK(hipStreamWaitEvent(m->s1, m->e_start, 0));
+    RC(masks());
     for (int it = 0; it < niter; ++it) {
         RC(enqueue_barotropic(m));
         RC(enqueue_step(m));
@@ -897,6 +900,9 @@ int mom6h_model_autotune(mom6h_model *m, int reps, char *report, int nbytes)
     MOM6H_REQUIRE(m->prepared, "mom6h_model_autotune: call mom6h_model_prepare first");
     MOM6H_REQUIRE(fused_ok(m), "mom6h_model_autotune: only the fused stencil has tile shapes to choose");
     MOM6H_CHECK(hipDeviceSynchronize());
+    MaskJobs mj{};
+    RC(mask_job(m, &mj.j[mj.n++]));
+    RC(launch_mask_bits(mj, m->s0));
     const int saved_profile = m->profile;
     m->profile = 0;
     // the predictor's momentum stencil (u, v, h0 -> up, vp): every step rewrites its outputs
@@ -976,5 +982,12 @@ bool fused_ok(const mom6h_model *m)
 {
     return m->fused && m->uniform && m->fused_rows && m->c.laplacian && m->c.coriolis_scheme == 1 &&
            !m->c.smagorinsky && !m->c.leith && !m->c.better_bound;
+}
+
+int mask_job(mom6h_model *m, MaskJob *job)
+{
+    if (!m->mask_bits) RC(dev_alloc_bytes((void **)&m->mask_bits, (size_t)m->d.s2, false));
+    *job = MaskJob{m->mask2dT, m->mask2dBu, m->mask_bits, m->d.s2};
+    return MOM6H_OK;
 }
 }  // namespace mom6h
