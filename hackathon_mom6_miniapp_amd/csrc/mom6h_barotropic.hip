@@ -585,7 +585,6 @@ inline std::vector<int> bt_split(int nstep, bool periodic, int ts)
 // us per call at 4 / 5 / 6 / 8 / 10 / 14 substeps (alone): 28x20, 20 substeps:
 // 82 / 78 / 74 / 74 / 71 / 71; 180x180, 30: 140 / 133 / 125 / 118 / 111 / 105;
 // 720x720, 50: 279 / 264 / 250 / 357 / 364 / 724 (two rounds from 7 on).
-constexpr int kBTMost = 16;
 inline int bt_auto_substeps(const std::vector<Dims> &grids, int nstep, bool periodic)
 {
     double points = 0.0, best = 0.0;
@@ -665,7 +664,7 @@ __global__ void __launch_bounds__(kBTThreads) k_bt_multi_batch(const BTMember *_
 int btstep_batch(const BTMember *d_args, const BTMember *h_args, int n, hipStream_t s, int ty, int per_launch)
 {
     MOM6H_REQUIRE(ty == 4 || ty == 8 || ty == 16, "btstep batch: tile rows must be 4, 8 or 16");
-    MOM6H_REQUIRE(per_launch >= 0 && per_launch <= 5, "btstep batch: 1..5 substeps per launch, or 0");
+    MOM6H_REQUIRE(per_launch >= 0 && per_launch <= kBTMost, "btstep batch: 1..%d substeps per launch, or 0", kBTMost);
     const int BT_TY = ty;
     MOM6H_REQUIRE(n >= 1 && n <= kMaxMembers, "btstep batch: 1..%d members", kMaxMembers);
     const int nstep = h_args[0].p.nstep;

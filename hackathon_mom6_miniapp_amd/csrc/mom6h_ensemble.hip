@@ -413,7 +413,8 @@ int mom6h_ensemble_set_option(mom6h_ensemble *e, const char *key, double value)
         e->use_graph = value != 0.0;
     } else if (k == "momentum_tile") {
         const int ty = (int)value;
-        MOM6H_REQUIRE(ty == 4 || ty == 8 || ty == 16, "mom6h_ensemble_set_option: momentum_tile must be 4, 8 or 16");
+        MOM6H_REQUIRE(value == 0.0 || ty == 4 || ty == 8 || ty == 16,
+                      "mom6h_ensemble_set_option: momentum_tile must be 4, 8 or 16, or 0 (not set)");
         e->momentum_tile = ty;
         if (e->prepared) RC(set_march(e));
         drop_graph(e);
@@ -422,14 +423,15 @@ int mom6h_ensemble_set_option(mom6h_ensemble *e, const char *key, double value)
         e->bt_tile = (int)value;
         drop_graph(e);
     } else if (k == "bt_substeps") {
-        MOM6H_REQUIRE(value >= 1.0 && value <= 5.0 && value == (double)(int)value,
-                      "mom6h_ensemble_set_option: bt_substeps must be 1..5");
+        MOM6H_REQUIRE(value >= 0.0 && value <= kBTMost && value == (double)(int)value,
+                      "mom6h_ensemble_set_option: bt_substeps must be 1..%d, or 0 for the number chosen from the grids",
+                      kBTMost);
         e->bt_substeps = (int)value;
         drop_graph(e);
     } else if (k == "momentum_splits") {
         MOM6H_REQUIRE(e->prepared, "mom6h_ensemble_set_option: momentum_splits after prepare");
         const int v = (int)value;
-        MOM6H_REQUIRE(v >= 1, "mom6h_ensemble_set_option: momentum_splits >= 1");
+        MOM6H_REQUIRE(value == 0.0 || v >= 1, "mom6h_ensemble_set_option: momentum_splits >= 1, or 0 (not set)");
         e->momentum_splits = v;
         RC(set_march(e));
         drop_graph(e);

@@ -395,6 +395,10 @@ struct mom6h_coriolis_cs {
     double u_Area_q = 0;
 };
 
+namespace mom6h {
+constexpr int kBTMost = 16;   // barotropic substeps per launch (an output tile of 64 - 3*16 points a side is left)
+}
+
 struct mom6h_barotropic_cs {
     mom6h::Dims d;
     mom6h::Halo halo;

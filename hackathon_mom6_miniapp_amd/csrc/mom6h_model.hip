@@ -804,18 +804,19 @@ int mom6h_model_set_option(mom6h_model *m, const char *key, double value)
     }
     else if (k == "bt_substeps") {
         MOM6H_REQUIRE(m->bt_cs, "mom6h_model_set_option: bt_substeps after prepare");
-        MOM6H_REQUIRE(value >= 1.0 && value <= 5.0 && value == (double)(int)value,
-                      "mom6h_model_set_option: bt_substeps must be 1..5");
+        MOM6H_REQUIRE(value >= 0.0 && value <= kBTMost && value == (double)(int)value,
+                      "mom6h_model_set_option: bt_substeps must be 1..%d, or 0 for the number chosen from the grid", kBTMost);
         m->bt_cs->substeps = (int)value;
         drop_graphs(m);
     }
     else if (k == "momentum_tile" || k == "momentum_splits") {
         const int v = (int)value;
         if (k == "momentum_tile") {
-            MOM6H_REQUIRE(v == 4 || v == 8 || v == 16, "mom6h_model_set_option: momentum_tile must be 4, 8 or 16");
+            MOM6H_REQUIRE(value == 0.0 || v == 4 || v == 8 || v == 16,
+                          "mom6h_model_set_option: momentum_tile must be 4, 8 or 16, or 0 (not set)");
             m->momentum_tile = v;
         } else {
-            MOM6H_REQUIRE(v >= 1 && v <= m->c.nk, "mom6h_model_set_option: momentum_splits must be 1..nk");
+            MOM6H_REQUIRE(value == 0.0 || v >= 1, "mom6h_model_set_option: momentum_splits >= 1, or 0 (not set)");
             m->momentum_splits = v;
         }
         drop_graphs(m);   // the captured step holds the old launch shape

@@ -319,14 +319,15 @@ int mom6h_model_step(mom6h_model *m, int niter);
 int mom6h_model_synchronize(mom6h_model *m);
 /* Options: "graph" (1 = capture one step as two hipGraphs, the 3D chain on
  * the model's first stream and the barotropic chain on its second, and replay
- * them per step, joined once per call as the eager path is; default 0), "momentum_tile" (4, 8 or 16;
- * default 8) and "momentum_splits" (1..nk; default 1): a wave of the fused
- * momentum stencil marches through 8*tile/splits rows (at least 4), or through
- * a number chosen from the grid while neither is set, "bt_tile" (rows of the barotropic substep tile,
+ * them per step, joined once per call as the eager path is; default 0), "momentum_tile" (4, 8 or 16)
+ * and "momentum_splits" (1 or more): a wave of the fused momentum stencil
+ * marches through 8*tile/splits rows (at least 4; an unset one counts as 8 or
+ * 1), or through a number chosen from the grid while neither is set, the
+ * default and again after both are set to 0, "bt_tile" (rows of the barotropic substep tile,
  * 4, 8 or 16; after prepare; default 4), "bt_substeps" (barotropic substeps per
- * launch: 1 = one launch per substep, 2-5 = the blocked kernel with at most so
- * many; after prepare; by default the blocked kernel with a number chosen from
- * the grid), "bt_rows" (1 = the blocked kernel takes Datv and the Coriolis factor
+ * launch: 1 = one launch per substep, 2-16 = the blocked kernel with at most so
+ * many, 0 = the blocked kernel with a number chosen from the grid; after
+ * prepare; default 0), "bt_rows" (1 = the blocked kernel takes Datv and the Coriolis factor
  * per row when both are constant along the compute rows, 0 = always as 2D
  * fields; after prepare; default 1), "fused" (1 = fused momentum stencil and
  * on-chip vert_visc coefficients where the grid allows, default 1; 0 = the
@@ -369,10 +370,9 @@ int mom6h_ensemble_prepare(mom6h_ensemble *e);
 int mom6h_ensemble_step(mom6h_ensemble *e, int niter);
 int mom6h_ensemble_synchronize(mom6h_ensemble *e);
 /* Options: "graph" (1 = capture one step, replay it per step), "momentum_tile"
- * (4, 8 or 16; default 8) and "momentum_splits" (after prepare; default 1): the
- * rows of the momentum march as for the model, "bt_tile" (4, 8 or 16),
- * "bt_substeps" (barotropic substeps per blocked launch, 1-5; by default chosen
- * from the members' grids). */
+ * and "momentum_splits" (after prepare): the rows of the momentum march as for
+ * the model, "bt_tile" (4, 8 or 16), "bt_substeps" (barotropic substeps per
+ * blocked launch, 1-16; 0, the default: chosen from the members' grids). */
 int mom6h_ensemble_set_option(mom6h_ensemble *e, const char *key, double value);
 /* Times the fused momentum launch of the ensemble (reps launches) for marches
  * of 4 to 128 rows, keeps the fastest and writes the timings into report.  It runs
