@@ -390,6 +390,11 @@ int mom6h_ensemble_step(mom6h_ensemble *e, int niter)
     }
     MOM6H_CHECK(hipEventRecord(e->e_bt, e->s1));
     MOM6H_CHECK(hipStreamWaitEvent(e->s0, e->e_bt, 0));
+    if (niter > 0)
+        for (mom6h_model *m : e->members) {
+            m->fused_last = true;
+            RC(refresh_del2(m, e->s0));
+        }
     return MOM6H_OK;
 }
 

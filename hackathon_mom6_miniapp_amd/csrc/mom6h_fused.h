@@ -64,6 +64,20 @@ int plan_momentum_batch(MomArgsT<T> *h_args, int n, int rows);
 template <typename T>
 int launch_momentum_batch(const MomArgsT<T> *d_args, const MomArgsT<T> *h_args, int n, hipStream_t s);
 
+// Del2u and Del2v of the biharmonic term as fields, for a caller that asks for
+// them (the stencil itself keeps them in registers)
+template <typename T>
+struct Del2Args {
+    Dims d;
+    UMetrics g;
+    int no_slip;
+    const T *u, *v;
+    const double *mask2dBu;
+    T *del2u, *del2v;   // written on their own ranges only, zero elsewhere from allocation
+};
+template <typename T>
+int launch_del2(const Del2Args<T> &a, hipStream_t s);
+
 // MomArgsT::mask from the FP64 masks (2D, n points each) of one or several grids
 struct MaskJob {
     const double *mask2dT, *mask2dBu;

@@ -343,6 +343,52 @@ int launch_momentum_batch(const MomArgsT<T> *d_args, const MomArgsT<T> *h_args, 
     return MOM6H_OK;
 }
 
+// Del2u on u points I = is-1..ie, j = js..je and Del2v on v points i = is..ie,
+// J = js-1..je (mom6_hor_visc_serial.F90:587-607), one thread per point with the
+// march's expressions; runs only for a caller that reads the two fields
+template <typename T>
+__global__ void __launch_bounds__(256) k_del2(Del2Args<T> a)
+{
+    const Dims &d = a.d;
+    const UMetT<T> g(a.g);
+    const int i = d.isc - 1 + (int)blockIdx.x * 64 + (int)(threadIdx.x & 63);
+    const int j = d.jsc - 1 + (int)blockIdx.y * 4 + (int)(threadIdx.x >> 6);
+    const int k = 1 + (int)blockIdx.z;
+    if (i > d.iec || j > d.jec) return;
+    auto U = [&](int ii, int jj) -> T { return a.u[IX3(d, ii, jj, k)]; };
+    auto V = [&](int ii, int jj) -> T { return a.v[IX3(d, ii, jj, k)]; };
+    auto sh_xx = [&](int ii, int jj) -> T {   // h point (:503-510)
+        const T dudx = g.DY_dxT * ((g.IdyCu * U(ii, jj)) - (g.IdyCu * U(ii - 1, jj)));
+        const T dvdy = g.DX_dyT * ((g.IdxCv * V(ii, jj)) - (g.IdxCv * V(ii, jj - 1)));
+        return dudx - dvdy;
+    };
+    auto sh_xy = [&](int I, int J) -> T {     // q point (:513-547)
+        const T dvdx = g.DY_dxBu * ((V(I + 1, J) * g.IdyCv) - (V(I, J) * g.IdyCv));
+        const T dudy = g.DX_dyBu * ((U(I, J + 1) * g.IdxCu) - (U(I, J) * g.IdxCu));
+        const T m = (T)a.mask2dBu[IX2(d, I, J)];
+        return (a.no_slip ? (T(2.0) - m) : m) * (dvdx + dudy);
+    };
+    const long long c = IX3(d, i, j, k);
+    if (j >= d.jsc)
+        a.del2u[c] = g.Idx2dyCu * ((g.dx2q * sh_xy(i, j)) - (g.dx2q * sh_xy(i, j - 1))) +
+                     g.Idxdy2u * ((g.dy2h * sh_xx(i + 1, j)) - (g.dy2h * sh_xx(i, j)));
+    if (i >= d.isc)
+        a.del2v[c] = g.Idxdy2v * ((g.dy2q * sh_xy(i, j)) - (g.dy2q * sh_xy(i - 1, j))) -
+                     g.Idx2dyCv * ((g.dx2h * sh_xx(i, j + 1)) - (g.dx2h * sh_xx(i, j)));
+}
+
+template <typename T>
+int launch_del2(const Del2Args<T> &a, hipStream_t s)
+{
+    const Dims &d = a.d;
+    k_del2<T><<<dim3((d.iec - d.isc + 2 + 63) / 64, (d.jec - d.jsc + 2 + 3) / 4, d.nk), 256, 0, s>>>(a);
+    MOM6H_LAUNCH_CHECK();
+    return MOM6H_OK;
+}
+
+template int launch_del2<double>(const Del2Args<double> &, hipStream_t);
+template int launch_del2<float>(const Del2Args<float> &, hipStream_t);
+
 // The masks as the stencil reads them: formed anew on every step call, since a
 // caller may rewrite the fields between calls (their device addresses are
 // public).  17 bytes per point of one plane, about 3 us at 720x720.

@@ -58,7 +58,13 @@ struct mom6h_model {
     struct {
         float *u, *v, *h, *h0, *htmp, *uh, *vh, *up, *vp, *u_cor, *bt_h_u;
         float *hx, *v_cor, *bt_h_v;   // meridional pass
+        float *del2u, *del2v;         // as below
     } f{};
+    // fields "del2u" and "del2v" of a biharmonic model: Del2 of the last fused
+    // corrector's velocities, formed at the end of a step call once a caller has
+    // asked for either (allocated then)
+    double *del2u = nullptr, *del2v = nullptr;
+    bool fused_last = false;      // the last step call ran the fused stencil
     std::vector<Field> fields;
     // host copies of the uniform metrics (init_ocean_grid)
     std::vector<double> IareaT, areaT, dxT, dyT, IdxT, IdyT, dxCu, dyCu, dy_Cu, IdxCu, IdyCu;
@@ -94,6 +100,8 @@ struct mom6h_model {
 namespace mom6h {
 // the fused stencils apply (uniform metrics, Sadourny Coriolis, Laplacian [+ biharmonic])
 bool fused_ok(const mom6h_model *m);
+// the fields "del2u" and "del2v" brought up to date on stream s, when in use
+int refresh_del2(mom6h_model *m, hipStream_t s);
 // the model's byte masks (allocated by the first call) as a job of launch_mask_bits
 int mask_job(mom6h_model *m, MaskJob *job);
 }  // namespace mom6h

@@ -66,6 +66,20 @@ const Field *find_field(const mom6h_model *m, const char *name)
     return nullptr;
 }
 
+// Allocates the fields del2u and del2v and brings them up to date
+int start_del2(mom6h_model *m)
+{
+    const size_t n3 = (size_t)m->d.s2 * m->c.nk;
+    auto alloc = [&](auto *&p) -> int { return p ? MOM6H_OK : dev_alloc_bytes((void **)&p, n3 * sizeof(*p), true); };
+    int rc = m->mixed ? alloc(m->f.del2u) : alloc(m->del2u);
+    rc = rc ? rc : m->mixed ? alloc(m->f.del2v) : alloc(m->del2v);
+    if (rc) return rc;
+    MOM6H_CHECK(hipDeviceSynchronize());
+    if (m->fused_last) rc = refresh_del2(m, m->s0);
+    if (!rc) MOM6H_CHECK(hipStreamSynchronize(m->s0));
+    return rc;
+}
+
 // init_ocean_grid (src/common/mom6_types.F90:130-258): uniform spacing dx.
 void host_grid(mom6h_model *m)
 {
@@ -410,6 +424,11 @@ int mom6h_model_create(mom6h_model **out, const mom6h_config *c)
         rc = rc ? rc : add_field(m, "dv_cor", &m->dv_cor, n2, true);
         bt_fields(m->bt_v, bt_v_names, &m->f.bt_h_v);
     }
+    if (!rc && c->biharmonic) {   // allocated when first asked for
+        const int bytes = m->mixed ? 4 : 8;
+        m->fields.push_back(Field{"del2u", m->mixed ? (void **)&m->f.del2u : (void **)&m->del2u, n3, bytes, true});
+        m->fields.push_back(Field{"del2v", m->mixed ? (void **)&m->f.del2v : (void **)&m->del2v, n3, bytes, true});
+    }
     if (!rc && hipStreamCreateWithFlags(&m->s0, hipStreamNonBlocking) != hipSuccess)
         rc = set_error(MOM6H_ENOMEM, "stream creation failed");
     if (!rc && hipStreamCreateWithFlags(&m->s1, hipStreamNonBlocking) != hipSuccess)
@@ -440,6 +459,7 @@ int mom6h_model_field(mom6h_model *m, const char *name, void **d_ptr, long *coun
 {
     MOM6H_REQUIRE(m && name, "mom6h_model_field: NULL argument");
     if (const Field *f = find_field(m, name)) {
+        if (d_ptr && !*f->p) RC(start_del2(m));   // the only fields not there from the start
         if (d_ptr) *d_ptr = *f->p;
         if (count) *count = (long)f->n;
         return MOM6H_OK;
@@ -678,11 +698,8 @@ static int capture_on(mom6h_model *m, hipStream_t s, int (*enq)(mom6h_model *), 
     return MOM6H_OK;
 }
 
-int mom6h_model_step(mom6h_model *m, int niter)
+static int run_steps(mom6h_model *m, int niter)
 {
-    MOM6H_REQUIRE(m != nullptr, "mom6h_model_step: NULL model");
-    MOM6H_REQUIRE(m->prepared, "mom6h_model_step: call mom6h_model_prepare first");
-    MOM6H_REQUIRE(niter >= 0, "mom6h_model_step: niter >= 0 required");
     // The fused path consumes vert_visc's coupling coefficients on chip; the
     // module path keeps them in the control structure, as the reference does.
     RC(mom6h_vert_visc_keep_coefficients(m->vv, fused_ok(m) ? 0 : 1));
@@ -761,6 +778,16 @@ int mom6h_model_step(mom6h_model *m, int niter)
     MOM6H_CHECK(hipEventRecord(m->e_bt, m->s1));
     MOM6H_CHECK(hipStreamWaitEvent(m->s0, m->e_bt, 0));
     return MOM6H_OK;
+}
+
+int mom6h_model_step(mom6h_model *m, int niter)
+{
+    MOM6H_REQUIRE(m != nullptr, "mom6h_model_step: NULL model");
+    MOM6H_REQUIRE(m->prepared, "mom6h_model_step: call mom6h_model_prepare first");
+    MOM6H_REQUIRE(niter >= 0, "mom6h_model_step: niter >= 0 required");
+    RC(run_steps(m, niter));
+    if (niter > 0) m->fused_last = fused_ok(m);
+    return niter > 0 && m->fused_last ? refresh_del2(m, m->s0) : MOM6H_OK;
 }
 
 int mom6h_model_synchronize(mom6h_model *m)
@@ -983,6 +1010,15 @@ bool fused_ok(const mom6h_model *m)
 {
     return m->fused && m->uniform && m->fused_rows && m->c.laplacian && m->c.coriolis_scheme == 1 &&
            !m->c.smagorinsky && !m->c.leith && !m->c.better_bound;
+}
+
+int refresh_del2(mom6h_model *m, hipStream_t s)
+{
+    if (m->f.del2u)
+        return launch_del2(Del2Args<float>{m->d, m->ug, m->c.no_slip, m->f.up, m->f.vp, m->mask2dBu, m->f.del2u, m->f.del2v}, s);
+    if (m->del2u)
+        return launch_del2(Del2Args<double>{m->d, m->ug, m->c.no_slip, m->up, m->vp, m->mask2dBu, m->del2u, m->del2v}, s);
+    return MOM6H_OK;
 }
 
 int mask_job(mom6h_model *m, MaskJob *job)

@@ -304,7 +304,10 @@ typedef struct mom6h_model mom6h_model;
 int mom6h_model_create(mom6h_model **m, const mom6h_config *c);
 /* Device address and element count of a field; its element type is FP64,
  * or FP32 for the layer fields of the mixed-precision form
- * (mom6h_model_field_bytes gives 8 or 4). */
+ * (mom6h_model_field_bytes gives 8 or 4).  A biharmonic model's "del2u" and
+ * "del2v" (Del2 of the velocities its last fused corrector started from) are
+ * allocated when first asked for and formed at the end of each step call from
+ * then on. */
 int mom6h_model_field(mom6h_model *m, const char *name, void **d_ptr, long *count);
 int mom6h_model_field_bytes(mom6h_model *m, const char *name, int *elem_bytes);
 /* Host FP64 values in and out (converted for FP32 fields), and a fill from
