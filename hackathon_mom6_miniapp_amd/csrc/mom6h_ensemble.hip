@@ -229,14 +229,19 @@ int capture_on(mom6h_ensemble *e, hipStream_t s, int (*enq)(mom6h_ensemble *), h
     return MOM6H_OK;
 }
 
-// the march of every member's momentum launch, both phases
+// the march of every member's momentum launch (one phase, both phases)
+template <typename T>
+int set_rows(Table<MomArgsT<T>> &x, int rows)
+{
+    RC(plan_momentum_batch<T>(x.h.data(), x.n(), rows));
+    if (x.d) MOM6H_CHECK(hipMemcpy(x.d, x.h.data(), x.h.size() * sizeof(x.h[0]), hipMemcpyHostToDevice));
+    return MOM6H_OK;
+}
+
 template <typename T>
 int set_march(StepTables<T> &t, int rows)
 {
-    for (auto *x : {&t.mom_pred, &t.mom_corr}) {
-        RC(plan_momentum_batch<T>(x->h.data(), x->n(), rows));
-        if (x->d) MOM6H_CHECK(hipMemcpy(x->d, x->h.data(), x->h.size() * sizeof(x->h[0]), hipMemcpyHostToDevice));
-    }
+    for (auto *x : {&t.mom_pred, &t.mom_corr}) RC(set_rows(*x, rows));
     return MOM6H_OK;
 }
 
@@ -258,24 +263,36 @@ void drop_graph(mom6h_ensemble *e)
     e->graph_bt = nullptr;
 }
 
-// mean time (ms) of reps predictor momentum launches
+// tune_march with the predictor's launch (u, v, h0 -> up, vp) and the corrector's
+// with the roles changed, from u, v onto up, vp, which every step rewrites; up, vp
+// hold the predictor's result in the end
 template <typename T>
-int time_momentum(mom6h_ensemble *e, StepTables<T> &t, int reps, float *ms)
+int tune(mom6h_ensemble *e, StepTables<T> &t, int reps, std::string *report)
 {
     const int n = (int)e->members.size();
-    hipEvent_t a, b;
-    MOM6H_CHECK(hipEventCreate(&a));
-    MOM6H_CHECK(hipEventCreate(&b));
-    int rc = launch_momentum_batch<T>(t.mom_pred.d, t.mom_pred.h.data(), n, e->s0);   // warm
-    if (!rc && hipEventRecord(a, e->s0) != hipSuccess) rc = set_error(MOM6H_ESTATE, "event record failed");
-    for (int r = 0; r < reps && !rc; ++r) rc = launch_momentum_batch<T>(t.mom_pred.d, t.mom_pred.h.data(), n, e->s0);
-    if (!rc && hipEventRecord(b, e->s0) != hipSuccess) rc = set_error(MOM6H_ESTATE, "event record failed");
-    if (!rc && hipEventSynchronize(b) != hipSuccess) rc = set_error(MOM6H_ESTATE, "event wait failed");
-    float x = 0.f;
-    if (!rc && hipEventElapsedTime(&x, a, b) != hipSuccess) rc = set_error(MOM6H_ESTATE, "event timing failed");
-    *ms = x / (float)(reps > 0 ? reps : 1);
-    (void)hipEventDestroy(a);
-    (void)hipEventDestroy(b);
+    Table<MomArgsT<T>> corr;
+    for (int m = 0; m < n; ++m) {
+        const MomArgsT<T> &p = t.mom_pred.h[m];
+        MomArgsT<T> a = t.mom_corr.h[m];
+        a.u = p.u; a.v = p.v; a.bu = a.ou = p.ou; a.bv = a.ov = p.ov;
+        corr.h.push_back(a);
+    }
+    auto pred = [&]() -> int { return launch_momentum_batch<T>(t.mom_pred.d, t.mom_pred.h.data(), n, e->s0); };
+    auto both = [&]() -> int {
+        RC(pred());
+        return launch_momentum_batch<T>(corr.d, corr.h.data(), n, e->s0);
+    };
+    auto set = [&](int tile, int splits) -> int {
+        e->momentum_tile = tile;
+        e->momentum_splits = splits;
+        RC(set_march(e));
+        return set_rows(corr, march_rows(tile, splits));
+    };
+    int rc = corr.upload();
+    rc = rc ? rc : tune_march(e->s0, reps, set, both, report);
+    rc = rc ? rc : pred();
+    if (hipStreamSynchronize(e->s0) != hipSuccess && !rc) rc = set_error(MOM6H_ESTATE, "stream wait failed");
+    corr.release();
     return rc;
 }
 
@@ -452,31 +469,10 @@ int mom6h_ensemble_autotune(mom6h_ensemble *e, int reps, char *report, int nbyte
     MOM6H_REQUIRE(e->prepared, "mom6h_ensemble_autotune: call mom6h_ensemble_prepare first");
     MOM6H_CHECK(hipDeviceSynchronize());
     RC(launch_mask_bits(e->masks, e->s0));
-    // marches of 128, 64, 32, 16, 8 and 4 rows
-    const int tiles[6] = {16, 8, 4, 4, 4, 4}, splits[6] = {1, 1, 1, 2, 4, 8};
-    float best = 0.f;
-    int pick = 8, pick_s = 1;
-    std::string rep = "momentum march rows (ms):";
-    for (int q = 0; q < 6; ++q) {
-        float ms = 0.f;
-        e->momentum_tile = tiles[q];
-        e->momentum_splits = splits[q];
-        RC(set_march(e));
-        RC(e->mixed ? time_momentum<float>(e, e->tf, reps, &ms) : time_momentum<double>(e, e->td, reps, &ms));
-        char buf[64];
-        snprintf(buf, sizeof(buf), " %d %.4f;", march_rows(tiles[q], splits[q]), ms);
-        rep += buf;
-        if (q == 0 || ms < best) {
-            best = ms;
-            pick = tiles[q];
-            pick_s = splits[q];
-        }
-    }
-    e->momentum_tile = pick;
-    e->momentum_splits = pick_s;
-    RC(set_march(e));
+    std::string rep;
+    const int rc = e->mixed ? tune<float>(e, e->tf, reps, &rep) : tune<double>(e, e->td, reps, &rep);
     drop_graph(e);
-    rep += " chosen " + std::to_string(march_rows(pick, pick_s));
+    if (rc) return rc;
     if (report && nbytes > 0) snprintf(report, (size_t)nbytes, "%s", rep.c_str());
     return MOM6H_OK;
 }

@@ -1,5 +1,7 @@
 // mom6h_fused.h -- kernels of the fused step for grids with uniform metrics.
 #pragma once
+#include <functional>
+#include <string>
 
 #include "mom6h_internal.h"
 
@@ -98,6 +100,15 @@ inline int march_rows(int tile, int splits)
     const int rows = 8 * (tile ? tile : 8) / (splits ? splits : 1);
     return rows < 4 ? 4 : rows;
 }
+
+// Chooses the options momentum_tile and momentum_splits by timing launch (what a
+// step does with the stencil) on stream s under each candidate, which set puts in
+// force: marches of 128 to 4 rows and the one chosen from the grid (0, 0), which
+// stays unless another is faster by more than 1%.  One round over the candidates
+// warms up, then `reps` rounds in alternating order; the shortest time of each
+// counts.  Leaves the choice set and adds the times to the report.
+int tune_march(hipStream_t s, int reps, const std::function<int(int tile, int splits)> &set,
+               const std::function<int()> &launch, std::string *report);
 
 // true and the common value when every element of a[0..n) is identical
 inline bool uniform_value(const double *a, size_t n, double *v)

@@ -17,6 +17,7 @@
 // them the q values on row js-1 and column is-1 still see the zero hArea the
 // reference reads, exactly as here.
 #include <algorithm>
+#include <cstdio>
 
 #include "mom6h_fused.h"
 
@@ -340,6 +341,59 @@ int launch_momentum_batch(const MomArgsT<T> *d_args, const MomArgsT<T> *h_args, 
         else k_momentum_batch<T, false, false><<<nb, 256, 0, s>>>(d_args, mp);
     }
     MOM6H_LAUNCH_CHECK();
+    return MOM6H_OK;
+}
+
+// One timing of each candidate in a fixed order, predictor only, chose 128 rows at
+// 720x720x75 (0.42 ms, in the first place after a pause) where a step's two
+// launches then took 1.01 ms, against 0.89 ms with 16 rows: the first milliseconds
+// after a pause run faster, and the corrector's extra base rows weigh on long
+// marches.  Hence the warm-up round, the alternating order and both phases: 28 ms
+// with reps = 3 there, and two timings of one length then differ by 1.3% at most.
+int tune_march(hipStream_t s, int reps, const std::function<int(int, int)> &set, const std::function<int()> &launch,
+               std::string *report)
+{
+    constexpr int N = 7;
+    const int tile[N] = {0, 16, 8, 4, 4, 4, 4}, splits[N] = {0, 1, 1, 1, 2, 4, 8};   // auto, 128 .. 4 rows
+    float ms[N] = {};
+    hipEvent_t a = nullptr, b = nullptr;
+    int rc = hipEventCreate(&a) == hipSuccess && hipEventCreate(&b) == hipSuccess
+                 ? MOM6H_OK
+                 : set_error(MOM6H_ENOMEM, "event creation failed");
+    int per = 1;   // launches per timing: about 0.3 ms
+    for (int round = 0; round <= (reps > 1 ? reps : 1) && !rc; ++round) {
+        float slowest = 0.f;
+        for (int c = 0; c < N && !rc; ++c) {
+            const int q = round % 2 ? N - 1 - c : c;
+            rc = set(tile[q], splits[q]);
+            if (!rc && hipEventRecord(a, s) != hipSuccess) rc = set_error(MOM6H_ESTATE, "event record failed");
+            for (int r = 0; r < per && !rc; ++r) rc = launch();
+            if (!rc && hipEventRecord(b, s) != hipSuccess) rc = set_error(MOM6H_ESTATE, "event record failed");
+            if (!rc && hipEventSynchronize(b) != hipSuccess) rc = set_error(MOM6H_ESTATE, "event wait failed");
+            float t = 0.f;
+            if (!rc && hipEventElapsedTime(&t, a, b) != hipSuccess) rc = set_error(MOM6H_ESTATE, "event timing failed");
+            t /= (float)per;
+            slowest = std::max(slowest, t);
+            if (round == 1 || (round > 1 && t < ms[q])) ms[q] = t;
+        }
+        if (round == 0) per = slowest >= 0.3f ? 1 : slowest > 0.02f ? (int)(0.3f / slowest) + 1 : 16;
+    }
+    if (a) (void)hipEventDestroy(a);
+    if (b) (void)hipEventDestroy(b);
+    int pick = 0;
+    for (int q = 1; q < N && !rc; ++q)
+        if (ms[q] < 0.99f * ms[0] && (pick == 0 || ms[q] < ms[pick])) pick = q;
+    const int rs = set(tile[pick], splits[pick]);
+    rc = rc ? rc : rs;
+    if (rc) return rc;
+    auto name = [&](int q) { return q ? std::to_string(march_rows(tile[q], splits[q])) : std::string("auto"); };
+    *report += "momentum march rows (ms, predictor + corrector):";
+    for (int q = 0; q < N; ++q) {
+        char buf[32];
+        snprintf(buf, sizeof(buf), " %.4f;", ms[q]);
+        *report += " " + name(q) + buf;
+    }
+    *report += " chosen " + name(pick);
     return MOM6H_OK;
 }
 

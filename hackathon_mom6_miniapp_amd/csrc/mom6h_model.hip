@@ -203,6 +203,43 @@ int enqueue_barotropic(mom6h_model *m)
 }
 
 
+// the fused stencil's arguments: from u, v, h onto the base bu, bv into ou, ov
+template <typename T>
+MomArgsT<T> mom_args(const mom6h_model *m, const T *u, const T *v, const T *h, const T *bu, const T *bv, T *ou, T *ov,
+                     double fdt)
+{
+    MomArgsT<T> a;
+    a.d = m->d; a.g = m->ug; a.Kh = (T)m->c.Kh; a.h_neglect = (T)1.0e-3; a.fdt = (T)fdt; a.no_slip = m->c.no_slip;
+    a.u = u; a.v = v; a.h = h; a.bu = bu; a.bv = bv; a.ou = ou; a.ov = ov;
+    a.mask = m->mask_bits; a.CoriolisBu = m->CoriolisBu;
+    a.Ah = (T)m->c.Ah; a.bih = m->c.biharmonic; a.march = march_rows(m->momentum_tile, m->momentum_splits);
+    return a;
+}
+
+// tune_march with the predictor's launch (u, v, h0 -> up, vp) and the corrector's
+// with the roles changed, from u, v onto up, vp, which every step rewrites; up, vp
+// hold the predictor's result in the end
+template <typename T>
+int tune_model(mom6h_model *m, const T *u, const T *v, const T *h0, const T *htmp, T *up, T *vp, int reps,
+               std::string *report)
+{
+    const double dt = m->c.dt;
+    auto pred = [&]() -> int { return launch_momentum(mom_args<T>(m, u, v, h0, u, v, up, vp, dt), m->s0); };
+    auto both = [&]() -> int {
+        RC(pred());
+        return launch_momentum(mom_args<T>(m, u, v, htmp, up, vp, up, vp, 0.5 * dt), m->s0);
+    };
+    auto set = [&](int tile, int splits) -> int {
+        m->momentum_tile = tile;
+        m->momentum_splits = splits;
+        return MOM6H_OK;
+    };
+    RC(tune_march(m->s0, reps, set, both, report));
+    RC(pred());
+    MOM6H_CHECK(hipStreamSynchronize(m->s0));
+    return MOM6H_OK;
+}
+
 // transports + hor_visc + CorAdCalc + velocity update of one phase
 int momentum_phase(mom6h_model *m, const double *u, const double *v, const double *h, double *ou,
                    double *ov, double fdt)
@@ -212,12 +249,7 @@ int momentum_phase(mom6h_model *m, const double *u, const double *v, const doubl
     hipStream_t s0 = m->s0;
     if (fused_ok(m)) {
         StageTimer t(m, ST_MOMENTUM, s0);
-        MomArgs a;
-        a.d = d; a.g = m->ug; a.Kh = m->c.Kh; a.h_neglect = 1.0e-3; a.fdt = fdt; a.no_slip = m->c.no_slip;
-        a.u = u; a.v = v; a.h = h; a.bu = m->u; a.bv = m->v; a.ou = ou; a.ov = ov;
-        a.mask = m->mask_bits; a.CoriolisBu = m->CoriolisBu;
-        a.Ah = m->c.Ah; a.bih = m->c.biharmonic; a.march = march_rows(m->momentum_tile, m->momentum_splits);
-        return launch_momentum(a, s0);
+        return launch_momentum(mom_args<double>(m, u, v, h, m->u, m->v, ou, ov, fdt), s0);
     }
     { StageTimer t(m, ST_TRANSPORTS, s0);
       RC(mom6h_transports(d.isd, d.ied, d.jsd, d.jed, nk, u, v, h, m->cor->dyCu, m->cor->dxCv, m->uh, m->vh, s0)); }
@@ -253,13 +285,7 @@ int momentum_phase_f32(mom6h_model *m, const float *u, const float *v, const flo
                        double fdt)
 {
     StageTimer t(m, ST_MOMENTUM, m->s0);
-    MomArgsT<float> a;
-    a.d = m->d; a.g = m->ug; a.Kh = (float)m->c.Kh; a.h_neglect = 1.0e-3f; a.fdt = (float)fdt;
-    a.no_slip = m->c.no_slip;
-    a.u = u; a.v = v; a.h = h; a.bu = m->f.u; a.bv = m->f.v; a.ou = ou; a.ov = ov;
-    a.mask = m->mask_bits; a.CoriolisBu = m->CoriolisBu;
-    a.Ah = (float)m->c.Ah; a.bih = m->c.biharmonic; a.march = march_rows(m->momentum_tile, m->momentum_splits);
-    return launch_momentum(a, m->s0);
+    return launch_momentum(mom_args<float>(m, u, v, h, m->f.u, m->f.v, ou, ov, fdt), m->s0);
 }
 
 int continuity_phase_f32(mom6h_model *m, const float *u, const float *v, const float *hin, float *hout, double dt)
@@ -931,49 +957,11 @@ int mom6h_model_autotune(mom6h_model *m, int reps, char *report, int nbytes)
     MaskJobs mj{};
     RC(mask_job(m, &mj.j[mj.n++]));
     RC(launch_mask_bits(mj, m->s0));
-    const int saved_profile = m->profile;
-    m->profile = 0;
-    // the predictor's momentum stencil (u, v, h0 -> up, vp): every step rewrites its outputs
-    auto launch = [&]() -> int {
-        return m->mixed ? momentum_phase_f32(m, m->f.u, m->f.v, m->f.h0, m->f.up, m->f.vp, m->c.dt)
-                        : momentum_phase(m, m->u, m->v, m->h0, m->up, m->vp, m->c.dt);
-    };
-    hipEvent_t a, b;
-    MOM6H_CHECK(hipEventCreate(&a));
-    MOM6H_CHECK(hipEventCreate(&b));
-    // marches of 128, 64, 32, 16, 8 and 4 rows
-    const int tiles[6] = {16, 8, 4, 4, 4, 4}, splits[6] = {1, 1, 1, 2, 4, 8};
-    float best = 0.f;
-    int pick = 8, pick_s = 1, rc = 0;
-    std::string rep = "momentum march rows (ms):";
-    for (int q = 0; q < 6 && !rc; ++q) {
-        m->momentum_tile = tiles[q];
-        m->momentum_splits = splits[q];
-        rc = launch();   // warm
-        if (!rc && hipEventRecord(a, m->s0) != hipSuccess) rc = set_error(MOM6H_ESTATE, "event record failed");
-        for (int r = 0; r < reps && !rc; ++r) rc = launch();
-        if (!rc && hipEventRecord(b, m->s0) != hipSuccess) rc = set_error(MOM6H_ESTATE, "event record failed");
-        if (!rc && hipEventSynchronize(b) != hipSuccess) rc = set_error(MOM6H_ESTATE, "event wait failed");
-        float ms = 0.f;
-        if (!rc && hipEventElapsedTime(&ms, a, b) != hipSuccess) rc = set_error(MOM6H_ESTATE, "event timing failed");
-        ms /= (float)(reps > 0 ? reps : 1);
-        char buf[64];
-        snprintf(buf, sizeof(buf), " %d %.4f;", march_rows(m->momentum_tile, m->momentum_splits), ms);
-        rep += buf;
-        if (q == 0 || ms < best) {
-            best = ms;
-            pick = m->momentum_tile;
-            pick_s = m->momentum_splits;
-        }
-    }
-    (void)hipEventDestroy(a);
-    (void)hipEventDestroy(b);
-    m->profile = saved_profile;
-    m->momentum_tile = pick;
-    m->momentum_splits = pick_s;
+    std::string rep;
+    const int rc = m->mixed ? tune_model(m, m->f.u, m->f.v, m->f.h0, m->f.htmp, m->f.up, m->f.vp, reps, &rep)
+                            : tune_model(m, m->u, m->v, m->h0, m->htmp, m->up, m->vp, reps, &rep);
     drop_graphs(m);
     if (rc) return rc;
-    rep += " chosen " + std::to_string(march_rows(pick, pick_s));
     if (report && nbytes > 0) snprintf(report, (size_t)nbytes, "%s", rep.c_str());
     return MOM6H_OK;
 }

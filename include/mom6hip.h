@@ -343,10 +343,12 @@ int mom6h_model_set_option(mom6h_model *m, const char *key, double value);
  * written comma-separated into names (size nbytes). Returns the stage count. */
 int mom6h_model_stage_times(mom6h_model *m, double *ms, int max_stages, char *names, int nbytes);
 int mom6h_model_main_stream(mom6h_model *m, void **stream);
-/* Times the fused momentum stencil (reps launches of the predictor's, whose
- * outputs every step rewrites) for marches of 4 to 128 rows, keeps the fastest
- * as options "momentum_tile" and "momentum_splits" and writes the timings into
- * report. */
+/* Times the fused momentum stencil (a predictor's and a corrector's launch, onto
+ * outputs that every step rewrites) for marches of 4 to 128 rows and for the
+ * number chosen from the grid: one round to warm up, then reps rounds (at least
+ * one) over all of them.  Keeps the fastest as options "momentum_tile" and
+ * "momentum_splits" (both 0 unless one beats the grid's number by more than 1%)
+ * and writes the shortest times into report. */
 int mom6h_model_autotune(mom6h_model *m, int reps, char *report, int nbytes);
 /* With option "diag" = 1 (FP64 form) every step posts the predictor's
  * diffu_sum and diffv_sum statistics; this call adds KE and mass of the
@@ -377,10 +379,7 @@ int mom6h_ensemble_synchronize(mom6h_ensemble *e);
  * the model, "bt_tile" (4, 8 or 16), "bt_substeps" (barotropic substeps per
  * blocked launch, 1-16; 0, the default: chosen from the members' grids). */
 int mom6h_ensemble_set_option(mom6h_ensemble *e, const char *key, double value);
-/* Times the fused momentum launch of the ensemble (reps launches) for marches
- * of 4 to 128 rows, keeps the fastest and writes the timings into report.  It runs
- * only the predictor's momentum stencil, whose outputs every step rewrites,
- * so the state is unchanged. */
+/* The same for the ensemble's launches; the state is unchanged. */
 int mom6h_ensemble_autotune(mom6h_ensemble *e, int reps, char *report, int nbytes);
 int mom6h_ensemble_destroy(mom6h_ensemble *e);
 
