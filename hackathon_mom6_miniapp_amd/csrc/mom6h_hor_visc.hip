@@ -746,6 +746,15 @@ static bool march_takes(const mom6h_hor_visc_cs *cs)
            (!cs->leith || cs->leith_uniform);
 }
 
+int hor_visc_scratch(mom6h_hor_visc_cs *cs)
+{
+    if (!cs->biharmonic || (march_takes(cs) && !cs->general)) return MOM6H_OK;
+    const size_t n3 = (size_t)cs->d.s2 * cs->d.nk;
+    int rc = cs->Del2u ? MOM6H_OK : dev_alloc(&cs->Del2u, n3, true);
+    if (!rc && !cs->Del2v) rc = dev_alloc(&cs->Del2v, n3, true);
+    return rc;
+}
+
 // the march's launch over the data domain: chunks of rows that leave about
 // four waves per SIMD, at least 8 (a chunk walks five rows more than it writes)
 template <bool SMAG, bool LEITH, bool BOUND, bool BIH>
@@ -859,21 +868,19 @@ int mom6h_hor_visc_set_options(mom6h_hor_visc_cs *cs, int laplacian, int biharmo
     cs->no_slip = no_slip;
     cs->Ah = Ah;
     if (biharmonic && !cs->biharmonic) {
-        const size_t n2 = (size_t)cs->d.s2, n3 = n2 * cs->d.nk;
+        const size_t n2 = (size_t)cs->d.s2;
         int rc = 0;
         rc = rc ? rc : dev_upload(&cs->Idx2dyCu, Idx2dyCu, n2);
         rc = rc ? rc : dev_upload(&cs->Idxdy2u, Idxdy2u, n2);
         rc = rc ? rc : dev_upload(&cs->Idx2dyCv, Idx2dyCv, n2);
         rc = rc ? rc : dev_upload(&cs->Idxdy2v, Idxdy2v, n2);
-        rc = rc ? rc : dev_alloc(&cs->Del2u, n3, true);
-        rc = rc ? rc : dev_alloc(&cs->Del2v, n3, true);
         if (rc) return rc;
         HVUniform &g = cs->g;
         cs->bih_uniform = hv_uniform(cs->d, {{Idx2dyCu, &g.Idx2dyCu}, {Idxdy2u, &g.Idxdy2u},
                                              {Idx2dyCv, &g.Idx2dyCv}, {Idxdy2v, &g.Idxdy2v}});
     }
     cs->biharmonic = biharmonic;
-    return MOM6H_OK;
+    return hor_visc_scratch(cs);
 }
 
 int mom6h_hor_visc(mom6h_hor_visc_cs *cs, const double *u, const double *v, const double *h,
@@ -954,7 +961,7 @@ int mom6h_hor_visc_set_closures(mom6h_hor_visc_cs *cs, int smagorinsky, int leit
     cs->smagorinsky = smagorinsky;
     cs->leith = leith;
     cs->better_bound = better_bound;
-    return MOM6H_OK;
+    return hor_visc_scratch(cs);
 }
 
 int mom6h_hor_visc_end(mom6h_hor_visc_cs *cs)

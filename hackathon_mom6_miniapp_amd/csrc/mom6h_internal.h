@@ -452,7 +452,9 @@ struct mom6h_hor_visc_cs {
     double *IareaCu, *IareaCv, *mask2dT, *mask2dBu, *reduction_xx, *reduction_xy;
     double *dy2h, *dx2h, *dy2q, *dx2q;
     double *Idx2dyCu, *Idxdy2u, *Idx2dyCv, *Idxdy2v;
-    double *Del2u, *Del2v;   // biharmonic scratch (3D, zero outside their ranges)
+    // biharmonic scratch of the general kernels (3D, zero outside their ranges);
+    // not there while the march runs
+    double *Del2u, *Del2v;
     // Smagorinsky / Leith viscosities and the thickness-aware bounds
     // (hor_visc_init Smagorinsky=, Leith=, better_bound=)
     int smagorinsky = 0, leith = 0, better_bound = 0;
@@ -468,3 +470,8 @@ struct mom6h_hor_visc_cs {
     int general = 0;         // use the general kernel even on a uniform grid
     mom6h::HVUniform g{};
 };
+
+namespace mom6h {
+// allocates what the kernels of the options in use need, whenever those change
+int hor_visc_scratch(mom6h_hor_visc_cs *cs);
+}

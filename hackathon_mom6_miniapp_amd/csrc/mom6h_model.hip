@@ -875,7 +875,10 @@ int mom6h_model_set_option(mom6h_model *m, const char *key, double value)
         drop_graphs(m);   // the captured step holds the old launch shape
     }
     else if (k == "general") {   // module hor_visc and CorAdCalc: the general kernels on any grid
-        if (m->hv) m->hv->general = value != 0.0;
+        if (m->hv) {
+            m->hv->general = value != 0.0;
+            RC(hor_visc_scratch(m->hv));
+        }
         if (m->cor) m->cor->general = value != 0.0;
         drop_graphs(m);
     }
