@@ -16,6 +16,10 @@
 //                   bracket, Newton to the barotropic transport, BT_cont and
 //                   h_u, u_cor/du_cor                       zonal_mass_flux
 //   k_convergence   (i,j,k) threads  -> h                  continuity_zonal_convergence
+// are the general forms (columns too deep for the two below); k_continuity_split
+// (zonal) and k_continuity_blk do a whole pass in one launch.
+#include <algorithm>
+
 #include "mom6h_internal.h"
 
 namespace mom6h {
@@ -330,7 +334,8 @@ __global__ void k_mass_flux(Dims d, const double *__restrict__ u, const double *
 }
 
 // ----------------------------------------------------- block column path ---
-// The meridional pass.  A block of CW wavefronts owns CF = 64 consecutive faces
+// The meridional pass, and the zonal one where few blocks make it the faster
+// kernel (cont_blk_faster) or planes of 4 GiB leave no other.  A block of CW wavefronts owns CF = 64 consecutive faces
 // of a row (one face per lane, the same face in every wavefront) and all their levels:
 // wavefront w holds levels w*K+1 .. w*K+K of its lane's face in registers (u,
 // the PPM edges and thickness of both neighbouring cells, the layer transport
@@ -341,7 +346,8 @@ __global__ void k_mass_flux(Dims d, const double *__restrict__ u, const double *
 // one lane per face -- a sequential sum costs 64 faces one add per level.
 // The Newton logic of a face runs redundantly in every wavefront on the same
 // values, so all copies agree; the block keeps iterating while any face
-// needs another evaluation.
+// needs another evaluation.  Zonal blocks overlap by two faces: the convergence
+// of a cell needs the transport at the face to the west (the neighbouring lane).
 constexpr int CF = 64;
 
 
@@ -551,7 +557,8 @@ struct ContShared {
     static constexpr int L = CW * K, FW = CF;
     T U[L][FW], S0[L][FW], S1[L][FW], R[9][FW];
     // per-face 2D values, loaded with the block's set-up loads and parked here
-    // until they are used rather than held in registers: P[1] = dxCu of its face, P[2] = its barotropic
+    // until they are used rather than held in registers: P[0] = dt*IareaT of
+    // the lane's cell (x), P[1] = dxCu of its face, P[2] = its barotropic
     // transport target, P[3] = dt*min(IareaT) of its two cells, P[4], P[5] =
     // dxT of cells 0 and 1; P[6], P[7] = du_eval and sum_dyhm of the face's
     // Newton iteration, kept over the output stores for BT_cont
@@ -679,17 +686,18 @@ __device__ __forceinline__ void bt_cont_store(const ContArgsT<T> &a, long long c
                                 : (T(1.5) * (duR - du0)) * ((FAmt_R - FA_avg) / (FAmt_R - FA_0)));
 }
 
-// The meridional pass: a block covers the faces (i, J), i = i0 .. i0+63, of one
-// face row J (lanes run along i, so every load stays coalesced); its
-// convergence is a separate kernel (the faces J-1 belong to another block).
-// The cell across the face is another row's, so each lane keeps both cells'
-// terms of every level, and the levels spread over 8 or 12 waves.
+// Y = false: the zonal pass.  A block covers the faces I0-1 .. I0+62 of row j
+// and also updates the thickness of cells I0 .. I0+62 (the convergence needs
+// the neighbouring lane's transport).  Y = true: the meridional pass, the same
+// algorithm across the rows: a block covers the faces (i, J), i = i0 .. i0+63,
+// of one face row J (lanes still run along i, so every load stays coalesced);
+// its convergence is a separate kernel (the faces J-1 belong to another block).
 //
 // FP32 form: the Newton stopping test of zonal_flux_adjust also accepts a
 // residual at the rounding level of the layer fluxes (4 ulp of sum |uh_k| of
 // the first pass); the FP64 tolerance of 1e-12 m lies below what FP32 sums
 // resolve, and the iteration would otherwise run to its 20-pass limit.
-template <typename T, int CW, int K, bool EVEN>
+template <typename T, bool Y, int CW, int K, bool EVEN>
 __device__ __forceinline__ void continuity_body(const ContArgsT<T> &a, int monotonic, unsigned bx, unsigned by)
 {
     extern __shared__ double smem_raw[];
@@ -700,15 +708,18 @@ __device__ __forceinline__ void continuity_body(const ContArgsT<T> &a, int monot
     const Dims &d = a.d;
     const int w = threadIdx.x >> 6;
     const int lane = threadIdx.x & (FW - 1);                  // the face of the block this thread works on
-    // face (fi, fj) between cell 0 = (fi, fj) and cell 1 = (fi, fj+1)
-    const int f_raw = d.isc + bx * FW + lane;
+    // face (fi, fj) between cell 0 = (fi, fj) and cell 1 = (fi+1, fj) [x] or (fi, fj+1) [y]
+    // x: a block advances by FW-2 faces (its last face lane only lends its cell
+    // to the lane below; its first lane's face feeds the convergence of the second)
+    const int f_raw = Y ? d.isc + bx * FW + lane : d.isc - 1 + bx * (FW - 2) + lane;
     const int f_max = d.iec;
     const int fi = f_raw > f_max ? f_max : f_raw;           // clamped: evaluated, never written
-    const int fj = d.jsc - 1 + (int)by;
+    const int fj = Y ? d.jsc - 1 + (int)by : d.jsc + (int)by;
     const bool live = f_raw <= f_max;
     auto cell = [&](int q) __attribute__((always_inline)) -> long long {   // q-th cell of the stencil, q = 2: cell 0
-        return IX2(d, fi, fj - 2 + q);
+        return Y ? IX2(d, fi, fj - 2 + q) : IX2(d, fi - 2 + q, fj);
     };
+    const int i = fi, j = fj;
     const int nk = d.nk;
     const long long s = d.s2;
     // my levels.  EVEN = false: k0+1 .. k0+K, every slot evaluated (a slot
@@ -741,8 +752,17 @@ __device__ __forceinline__ void continuity_body(const ContArgsT<T> &a, int monot
     col.dt = (T)a.dt;
     const long long c2 = IX2(d, fi, fj);
     col.dy = (T)a.dy_Cu[c2];
-    col.IdxT0 = (T)a.IdxT[cell(2)];
-    col.IdxT1 = (T)a.IdxT[cell(3)];
+    if constexpr (!Y) {
+        // cell 1's IdxT is the next lane's cell 0's, read at cell
+        // min(f_raw, iec+1): the lane after the last live one holds cell
+        // iec+1 (a lane past iec evaluates values that are never written)
+        const int ci0 = f_raw < d.iec + 1 ? f_raw : d.iec + 1;
+        col.IdxT0 = (T)a.IdxT[IX2(d, ci0, fj)];
+        col.IdxT1 = __shfl_down(col.IdxT0, 1, FW);
+    } else {
+        col.IdxT0 = (T)a.IdxT[cell(2)];
+        col.IdxT1 = (T)a.IdxT[cell(3)];
+    }
     T mCu = T(0.0);   // read by the CFL folds of waves 2 and 3 only
     if (w == 2 || w == 3) mCu = (T)a.mask2dCu[c2];
     const long long cu = IX3(d, fi, fj, 1);
@@ -761,6 +781,7 @@ __device__ __forceinline__ void continuity_body(const ContArgsT<T> &a, int monot
     }
     auto park = [&]() __attribute__((always_inline)) {
         if (w == 0) {
+            if (!Y) S.P[0][lane] = (T)(a.dt * IareaT0);
             S.P[1][lane] = (T)dxCu_f;
             S.P[2][lane] = (T)uhbt_f;
             S.P[3][lane] = (T)(a.dt * dmin(IareaT0, IareaT1));
@@ -768,10 +789,133 @@ __device__ __forceinline__ void continuity_body(const ContArgsT<T> &a, int monot
             S.P[5][lane] = (T)dxT1;
         }
     };
-    // PPM edges of cells 0 and 1 (zonal_edge_thickness :185-207), both from the
-    // 6-cell stencil along j; the loads of a slot past the lane's levels read
-    // level min(k, nk) (in bounds) and nothing is formed from them
-    {
+    // PPM edges of cells 0 and 1 (zonal_edge_thickness :185-207); the loads
+    // of a slot past the lane's levels read level min(k, nk) (in bounds) and
+    // nothing is formed from them.  x: each lane reconstructs its own cell 0 from the
+    // 5-cell stencil and takes cell 1 from the next lane (whose cell 0 it is),
+    // so every cell is reconstructed once.  y: both cells from the 6-cell
+    // stencil along j.
+    if (!Y) {
+        const int ci = f_raw < d.iec + 1 ? f_raw : d.iec + 1;   // this lane's cell (in bounds)
+        auto ccell = [&](int q) __attribute__((always_inline)) -> long long { return IX2(d, ci - 2 + q, fj); };
+        // STAGE: each level's row of thicknesses is loaded once, the lanes'
+        // own cells (position t = lane holds cell f_raw(lane 0) - 2 + t) and
+        // the four beyond the last lane (t = 64..67, those of all the wave's
+        // levels in one load), and each lane reads its 5-cell stencil t =
+        // lane .. lane+4 back from LDS: one load per level and lane instead
+        // of five (a load with few active lanes costs about what a full one
+        // does, so the extensions share one).  The rows are
+        // staged in the wave's own rows of S0 (levels 0..KA-1) and S1 (the
+        // rest), which no other wave touches before the first pass's barrier
+        // and this wave's first pass overwrites only after these reads.  A
+        // cell index past iec+3 (the last one the lanes of the unstaged form
+        // read) is clamped there: only lanes past iec+1, which are evaluated
+        // and never written, read a clamped cell.  STAGE_M: the row of masks
+        // likewise, after the thickness rows in S1 where they fit.
+        constexpr bool STAGE = K >= 3;
+        constexpr int KA = K / 2, RL = FW + 4;
+        static_assert(!STAGE || (KA * RL <= (K - 1) * FW && (K - KA) * RL <= K * FW &&
+                                 (K - 1 - KA) * RL <= (K - 1) * FW),
+                      "staged rows exceed the wave's own rows");
+        constexpr bool STAGE_M = STAGE && (K - KA + 1) * RL <= (K - 1) * FW;
+        T m5[5], hs[K][5], us[K];
+        if constexpr (!STAGE_M) {
+#pragma unroll
+            for (int q = 0; q < 5; ++q) m5[q] = (T)a.mask2dT[ccell(q)];
+        }
+        if constexpr (STAGE) {
+            const int c_lo = f_raw - 2, c_hi = d.iec + 3;
+            const long long rA = IX2(d, c_lo < c_hi ? c_lo : c_hi, fj);
+            const long long rB = IX2(d, c_lo + FW < c_hi ? c_lo + FW : c_hi, fj);
+            T mA = T(0.0), mB = T(0.0);
+            if constexpr (STAGE_M) {
+                mA = (T)a.mask2dT[rA];
+                if (lane < 4) mB = (T)a.mask2dT[rB];
+            }
+            T hA[K], hX = T(0.0);
+            // the four cells past the last lane of every level in one load:
+            // lane 4*kk + x holds cell 64 + x of slot kk
+            const int xk = lane >> 2;
+            const int cx = f_raw - lane - 2 + FW + (lane & 3);
+            const long long rX = IX2(d, cx < c_hi ? cx : c_hi, fj);
+#pragma unroll
+            for (int kk = 0; kk < K; ++kk) {
+                const int kr = k0 + kk + 1;
+                const int k = kr < nk ? kr : nk;
+                const long long o = (long long)(k - 1) * s;
+                us[kk] = a.u[cu + o];
+                if (!formed(kk)) continue;
+                hA[kk] = a.hin[rA + o];
+            }
+            if (lane < 4 * K) {
+                const int kr = k0 + xk + 1;
+                hX = a.hin[rX + (long long)((kr < nk ? kr : nk) - 1) * s];
+            }
+            park();
+            auto row = [&](int kk) __attribute__((always_inline)) -> T * {
+                return kk < KA ? &S.S0[k0][0] + kk * RL : &S.S1[k0][0] + (kk - KA) * RL;
+            };
+            T *const mrow = &S.S1[k0][0] + (K - KA) * RL;
+            if constexpr (STAGE_M) {
+                mrow[lane] = mA;
+                if (lane < 4) mrow[FW + lane] = mB;
+            }
+#pragma unroll
+            for (int kk = 0; kk < K; ++kk) {
+                if (!formed(kk)) continue;
+                row(kk)[lane] = hA[kk];
+            }
+            if (lane < 4 * K && formed(xk)) {
+                T *const r = xk < KA ? &S.S0[k0][0] + xk * RL : &S.S1[k0][0] + (xk - KA) * RL;
+                r[FW + (lane & 3)] = hX;
+            }
+            // one wave's LDS operations complete in order: the fences only
+            // keep the compiler from moving the reads above the stores
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+            if constexpr (STAGE_M) {
+#pragma unroll
+                for (int q = 0; q < 5; ++q) m5[q] = mrow[lane + q];
+            }
+#pragma unroll
+            for (int kk = 0; kk < K; ++kk) {
+                if (!formed(kk)) continue;
+#pragma unroll
+                for (int q = 0; q < 5; ++q) hs[kk][q] = row(kk)[lane + q];
+            }
+        } else {
+#pragma unroll
+            for (int kk = 0; kk < K; ++kk) {
+                const int kr = k0 + kk + 1;
+                const int k = kr < nk ? kr : nk;
+                const long long o = (long long)(k - 1) * s;
+                us[kk] = a.u[cu + o];
+#pragma unroll
+                for (int q = 0; q < 5; ++q) hs[kk][q] = a.hin[ccell(q) + o];
+            }
+            park();
+        }
+        T wW[K], wE[K], w0[K];
+#pragma unroll
+        for (int kk = 0; kk < K; ++kk) {
+            if (!formed(kk)) continue;
+            S.U[k0 + kk][lane] = us[kk];
+            const T *h5 = hs[kk];
+            T sl[3];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) sl[q] = ppm_slope_v(m5[q], m5[q + 1], m5[q + 2], h5[q], h5[q + 1], h5[q + 2]);
+            ppm_edges_v(m5, h5, sl, 2, wW[kk], wE[kk]);
+            w0[kk] = h5[2];
+        }
+#pragma unroll
+        for (int kk = 0; kk < K; ++kk) {
+            if (!formed(kk)) continue;
+            ppm_limit(monotonic, w0[kk], (T)a.h_min, wW[kk], wE[kk]);
+            col.set(kk, wW[kk], wE[kk], w0[kk], __shfl_down(wW[kk], 1, FW), __shfl_down(wE[kk], 1, FW),
+                    __shfl_down(w0[kk], 1, FW));
+        }
+    } else {
         T m6[6], hs[K][6], us[K];
 #pragma unroll
         for (int q = 0; q < 6; ++q) m6[q] = (T)a.mask2dT[cell(q)];
@@ -891,7 +1035,9 @@ __device__ __forceinline__ void continuity_body(const ContArgsT<T> &a, int monot
         T du = T(0.0), du_max = st.du_max_CFL, du_min = st.du_min_CFL;
         T uh_err = st.uh_tot_0 - uhbt, duhdu_tot = st.duhdu_tot_0;
         T uh_err_best = vabs(uh_err);
-        bool do_I = true;
+        // x: lanes past the last face and the block's last lane (no cell 1 of
+        // its own) take no Newton passes
+        bool do_I = Y || (live && lane < FW - 1);
         *du_eval = T(0.0);   // the first pass evaluated at du = 0
         for (int itt = 1; itt <= max_itts; ++itt) {
             if (do_I) {
@@ -955,11 +1101,24 @@ __device__ __forceinline__ void continuity_body(const ContArgsT<T> &a, int monot
     // reads back what it stored whether or not a barrier lies between
     S.P[6][lane] = du_eval;
     S.P[7][lane] = sum_dyhm;
-    // outputs at the face: uh, u_cor, du_cor.  u_cor = u + du needs only u
+    // the convergence's cell thicknesses (cell I = I0 + lane, every level of
+    // the lane's group; clamped levels repeat nk), issued before the face
+    // stores so that one round trip covers all levels
+    T hc[K];
+    if (!Y) {
+#pragma unroll
+        for (int kk = 0; kk < K; ++kk) {
+            const int kr = k0 + kk + 1;
+            hc[kk] = a.hin[IX3(d, i, j, kr < nk ? kr : nk)];
+        }
+    }
+
+    // outputs at the face: uh, u_cor, du_cor; a face shared with the western
+    // neighbour block is written by that block.  u_cor = u + du needs only u
     // (in LDS to the end) and du: with the BT_cont outputs its stores wait for
     // the CFL folds of BT_cont, where the other waves are idle, instead of
     // joining the burst of the other outputs (1.8% of the kernel)
-    const bool writes_face = live;
+    const bool writes_face = live && (Y || ((lane > 0 || bx == 0) && lane < FW - 1));
     auto store_u_cor = [&]() __attribute__((always_inline)) {
         if (a.u_cor && writes_face) {
 #pragma unroll
@@ -975,6 +1134,20 @@ __device__ __forceinline__ void continuity_body(const ContArgsT<T> &a, int monot
         if (a.du_cor && w == 0) a.du_cor[c2] = (double)du;
     }
     if (!a.bt_h_u) store_u_cor();
+    // continuity_zonal_convergence (:148-176) for cell i = I (faces I-1 and I)
+    if (!Y) {
+        const T dtIareaT = S.P[0][lane];   // dt*IareaT(i, j): cell 0 of the face
+        const bool writes_cell = live && lane > 0 && lane < FW - 1 && i >= d.isc;
+#pragma unroll
+        for (int kk = 0; kk < K; ++kk) {
+            if (writes_cell && valid(kk)) {
+                const long long c3 = IX3(d, i, j, k0 + kk + 1);
+                const T fw = S.S0[k0 + kk][lane - 1];   // face I-1 (the lane to the west), same level
+                const T v = hc[kk] - dtIareaT * (S.S0[k0 + kk][lane] - fw);
+                a.h[c3] = vmax(v, T(0.0));
+            }
+        }
+    }
     if (!a.bt_h_u) return;   // block-uniform
 
     // h_u = marginal thickness at u_cor = u + du (zonal_flux_thickness :602-735):
@@ -1071,8 +1244,8 @@ __device__ __forceinline__ void continuity_body(const ContArgsT<T> &a, int monot
 // two blocks share a CU at 75 levels in FP64, three in FP32.  Per call at
 // 720x720x75, FP64: 976 -> 705 us (reads 1.9 -> 0.9 GB: the convergence keeps
 // its thicknesses), FP32 465 -> 393; 471x363x50 352 -> 187 and 154 -> 94;
-// 140x100x40 57 -> 31; 300x260x25 72 -> 48; 180x180x75 88 -> 78.  Faster at
-// every depth, so it replaced the zonal form.  What bounds it: VALU issue (55%
+// 140x100x40 57 -> 31; 300x260x25 72 -> 48; 180x180x75 88 -> 78; grids with fewer
+// blocks than the chip holds at once keep the block kernel (cont_blk_faster).  What bounds it: VALU issue (55%
 // busy at 75 levels FP64) and, at two waves per SIMD, the latency of dependent
 // FP64 operations.  Groups of 3 levels measured the same as 4.
 template <typename T, int K>
@@ -1651,12 +1824,12 @@ k_continuity_split(ContArgsT<T> a, int monotonic)
     continuity_x_split<T, K, BASE>(a, monotonic, blockIdx.x, blockIdx.y);
 }
 
-template <typename T, int CW, int K, bool EVEN>
+template <typename T, bool Y, int CW, int K, bool EVEN>
 __global__ void __launch_bounds__(64 * CW) __attribute__((amdgpu_waves_per_eu(
     sizeof(T) == 4 ? 4 : (CW + 3) / 4, (CW >= 12 || sizeof(T) == 4) ? 4 : 2)))
 k_continuity_blk(ContArgsT<T> a, int monotonic)
 {
-    continuity_body<T, CW, K, EVEN>(a, monotonic, blockIdx.x, blockIdx.y);
+    continuity_body<T, Y, CW, K, EVEN>(a, monotonic, blockIdx.x, blockIdx.y);
 }
 
 // the members of an ensemble that one batched launch covers: entry q of its
@@ -1667,14 +1840,14 @@ struct MemberIndex {
 
 // the members of an ensemble whose depth takes the block shape CW x K, in one
 // launch (EVEN: every one of them spreads its levels evenly)
-template <typename T, int CW, int K, bool EVEN>
+template <typename T, bool Y, int CW, int K, bool EVEN>
 __global__ void __launch_bounds__(64 * CW) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 1, (CW >= 16 || sizeof(T) == 4) ? 4 : 2)))
 k_continuity_batch(const ContArgsT<T> *__restrict__ args, BatchMap mp, MemberIndex mi)
 {
     int m, local;
     batch_locate(mp, blockIdx.x, m, local);
     const ContArgsT<T> a = args[mi.v[m]];
-    continuity_body<T, CW, K, EVEN>(a, a.monotonic, local % mp.nbx[m], local / mp.nbx[m]);
+    continuity_body<T, Y, CW, K, EVEN>(a, a.monotonic, local % mp.nbx[m], local / mp.nbx[m]);
 }
 
 // the same for the zonal pass and members of one slot class
@@ -1800,16 +1973,16 @@ unsigned blk_nbx(const Dims &d, int FW)
 // A block shape of CW waves of K level slots (64 faces): levels spread evenly
 // over the waves when CW*(K-1) <= nk (every shape of 1 or 2 slots, 8 x 4 from
 // 24 levels, 12 x 7 and 8 x 10 from 72)
-template <typename T, int CW, int K>
+template <typename T, bool Y, int CW, int K>
 void launch_shape(const ContArgsT<T> &a, int mono, dim3 g, hipStream_t s)
 {
     const dim3 b(64 * CW);
     constexpr size_t lds = sizeof(ContShared<T, CW, K>);
     if constexpr (K <= 2) {
-        k_continuity_blk<T, CW, K, true><<<g, b, lds, s>>>(a, mono);
+        k_continuity_blk<T, Y, CW, K, true><<<g, b, lds, s>>>(a, mono);
     } else {
-        if (a.d.nk >= CW * (K - 1)) k_continuity_blk<T, CW, K, true><<<g, b, lds, s>>>(a, mono);
-        else k_continuity_blk<T, CW, K, false><<<g, b, lds, s>>>(a, mono);
+        if (a.d.nk >= CW * (K - 1)) k_continuity_blk<T, Y, CW, K, true><<<g, b, lds, s>>>(a, mono);
+        else k_continuity_blk<T, Y, CW, K, false><<<g, b, lds, s>>>(a, mono);
     }
 }
 
@@ -1830,29 +2003,57 @@ void launch_x_base(const ContArgsT<T> &a, int mono, dim3 g, hipStream_t s)
     }
 }
 
-template <typename T>
-int launch_x(const ContArgsT<T> &a, int mono, hipStream_t s)
+// One pass over nby rows of faces by the block kernel; the block shape follows nk and the type
+template <typename T, bool Y>
+int launch_blk(const ContArgsT<T> &a, int mono, unsigned nby, hipStream_t s)
 {
-    const dim3 g(blk_nbx<false>(a.d, CF), (unsigned)(a.d.jec - a.d.jsc + 1));
-    if (cont_split_wide<T>(a.d)) launch_x_base<T, 1>(a, mono, g, s);
-    else launch_x_base<T, CX_BASE>(a, mono, g, s);
+    const int nk = a.d.nk;
+    const dim3 g(blk_nbx<Y>(a.d, CF), nby);
+    if (nk <= 8) launch_shape<T, Y, 8, 1>(a, mono, g, s);
+    else if (nk <= 16) launch_shape<T, Y, 8, 2>(a, mono, g, s);
+    else if (nk <= 32) launch_shape<T, Y, 8, 4>(a, mono, g, s);
+    // FP64 beyond 32 levels: 12 waves of 7 levels (three waves per SIMD); the
+    // FP32 form: 8 waves of 10 levels (two blocks per CU)
+    else if (sizeof(T) == 8) launch_shape<T, Y, 12, 7>(a, mono, g, s);
+    else launch_shape<T, Y, 8, 10>(a, mono, g, s);
     MOM6H_LAUNCH_CHECK();
     return MOM6H_OK;
 }
 
-// The meridional pass over nby rows of faces; the block shape follows nk and the type
-template <typename T>
-int launch_y(const ContArgsT<T> &a, int mono, unsigned nby, hipStream_t s)
+// Columns the split zonal kernel takes: its offsets within a plane are 32-bit bytes
+inline bool cont_split_fits(const Dims &d)
 {
-    const int nk = a.d.nk;
-    const dim3 g(blk_nbx<true>(a.d, CF), nby);
-    if (nk <= 8) launch_shape<T, 8, 1>(a, mono, g, s);
-    else if (nk <= 16) launch_shape<T, 8, 2>(a, mono, g, s);
-    else if (nk <= 32) launch_shape<T, 8, 4>(a, mono, g, s);
-    // FP64 beyond 32 levels: 12 waves of 7 levels (three waves per SIMD); the
-    // FP32 form: 8 waves of 10 levels (two blocks per CU)
-    else if (sizeof(T) == 8) launch_shape<T, 12, 7>(a, mono, g, s);
-    else launch_shape<T, 8, 10>(a, mono, g, s);
+    return d.nk <= kSplitMax && d.s2 * (long long)sizeof(double) < (1LL << 32);
+}
+
+// Whether the block kernel is the faster one for a zonal launch of so many blocks.
+// Where all its blocks run at once (one per CU in FP64, two in FP32; two also of
+// up to 4 levels in FP64) its 8 or 12 waves of few levels each get through a
+// column's chain of passes sooner than four waves that hand every sum on; beyond
+// that the split kernel, of which twice as many blocks are resident, is faster.
+// At 33 to 64 levels (FP32: 52) the block's 84 (80) slots are mostly empty and
+// the split kernel is never slower.  us per call, block / split kernel, with a
+// transport target in FP64: 60x45x8 12.1 / 16.5, 60x45x40 32.4 / 25.8, 60x45x75
+// 33.6 / 40.0, 100x80x24 18.2 / 21.3, 100x80x75 35.2 / 42.9; 140x100 (288 blocks)
+// x3 19.8 / 19.6, x24 34.8 / 26.7, x75 68.7 / 53.3; FP32: 60x45x8 11.8 / 15.4,
+// 100x80x40 24.7 / 24.1, 140x100x24 18.0 / 20.8, 180x140x75 (408 blocks) 33.7 /
+// 38.4, 180x180x75 (528 blocks) 46.7 / 41.0.
+template <typename T>
+bool cont_blk_faster(long long blocks, int nk)
+{
+    constexpr bool F32 = sizeof(T) == 4;
+    if (nk > 32 && nk <= (F32 ? 52 : 64)) return false;
+    return blocks <= (F32 || nk <= 4 ? 512 : 256);
+}
+
+template <typename T>
+int launch_x(const ContArgsT<T> &a, int mono, hipStream_t s)
+{
+    const dim3 g(blk_nbx<false>(a.d, CF), (unsigned)(a.d.jec - a.d.jsc + 1));
+    if (!cont_split_fits(a.d) || cont_blk_faster<T>((long long)g.x * g.y, a.d.nk))
+        return launch_blk<T, false>(a, mono, g.y, s);
+    if (cont_split_wide<T>(a.d)) launch_x_base<T, 1>(a, mono, g, s);
+    else launch_x_base<T, CX_BASE>(a, mono, g, s);
     MOM6H_LAUNCH_CHECK();
     return MOM6H_OK;
 }
@@ -1866,19 +2067,23 @@ int set_blk_lds(long long max_lds)
         if (bytes > max_lds) return hipSuccess;
         return hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
     };
-#define MOM6H_BLK_LDS(CW, K)                                                                                       \
-    MOM6H_CHECK(raise((const void *)k_continuity_blk<T, CW, K, true>, sizeof(ContShared<T, CW, K>)));        \
-    MOM6H_CHECK(raise((const void *)k_continuity_blk<T, CW, K, false>, sizeof(ContShared<T, CW, K>)));       \
-    MOM6H_CHECK(raise((const void *)k_continuity_batch<T, CW, K, true>, sizeof(ContShared<T, CW, K>)));
-#define MOM6H_BATCH_PLAIN_LDS(K)                                                                                   \
-    MOM6H_CHECK(raise((const void *)k_continuity_batch<T, 8, K, false>, sizeof(ContShared<T, 8, K>)));
-    MOM6H_BLK_LDS(8, 1) MOM6H_BLK_LDS(8, 2) MOM6H_BLK_LDS(8, 4) MOM6H_BLK_LDS(8, 10)
-    MOM6H_BATCH_PLAIN_LDS(4) MOM6H_BATCH_PLAIN_LDS(7) MOM6H_BATCH_PLAIN_LDS(10)
-    MOM6H_CHECK(raise((const void *)k_continuity_batch<T, 8, 7, true>, sizeof(ContShared<T, 8, 7>)));
-#undef MOM6H_BATCH_PLAIN_LDS
+#define MOM6H_BLK_LDS(Y, CW, K)                                                                                   \
+    MOM6H_CHECK(raise((const void *)k_continuity_blk<T, Y, CW, K, true>, sizeof(ContShared<T, CW, K>)));        \
+    MOM6H_CHECK(raise((const void *)k_continuity_blk<T, Y, CW, K, false>, sizeof(ContShared<T, CW, K>)));
+#define MOM6H_BATCH_LDS(Y, K)                                                                                     \
+    MOM6H_CHECK(raise((const void *)k_continuity_batch<T, Y, 8, K, true>, sizeof(ContShared<T, 8, K>)));        \
+    MOM6H_CHECK(raise((const void *)k_continuity_batch<T, Y, 8, K, false>, sizeof(ContShared<T, 8, K>)));
+#define MOM6H_PASS_LDS(Y)                                                                                         \
+    MOM6H_BLK_LDS(Y, 8, 1) MOM6H_BLK_LDS(Y, 8, 2) MOM6H_BLK_LDS(Y, 8, 4) MOM6H_BLK_LDS(Y, 8, 10)                 \
+    MOM6H_BLK_LDS(Y, 12, 7)                                                                                      \
+    MOM6H_BATCH_LDS(Y, 4) MOM6H_BATCH_LDS(Y, 7) MOM6H_BATCH_LDS(Y, 10)                                            \
+    MOM6H_CHECK(raise((const void *)k_continuity_batch<T, Y, 8, 1, true>, sizeof(ContShared<T, 8, 1>)));        \
+    MOM6H_CHECK(raise((const void *)k_continuity_batch<T, Y, 8, 2, true>, sizeof(ContShared<T, 8, 2>)));
+    MOM6H_PASS_LDS(false)
+    MOM6H_PASS_LDS(true)
+#undef MOM6H_PASS_LDS
+#undef MOM6H_BATCH_LDS
 #undef MOM6H_BLK_LDS
-    MOM6H_CHECK(raise((const void *)k_continuity_blk<T, 12, 7, true>, sizeof(ContShared<T, 12, 7>)));
-    MOM6H_CHECK(raise((const void *)k_continuity_blk<T, 12, 7, false>, sizeof(ContShared<T, 12, 7>)));
     return MOM6H_OK;
 }
 
@@ -1895,9 +2100,7 @@ bool blk_fits(const mom6h_continuity_cs *cs)
     constexpr long long bytes = sizeof(ContShared<double, 12, 7>) > sizeof(ContShared<double, 8, 10>)
                                     ? sizeof(ContShared<double, 12, 7>)
                                     : sizeof(ContShared<double, 8, 10>);
-    // and, for 32-bit byte offsets within a plane, planes below 4 GiB
-    return cs->d.nk <= 80 && !cs->upwind_1st && !cs->simple_2nd && bytes <= cs->max_lds &&
-           cs->d.s2 * (long long)sizeof(double) < (1LL << 32);
+    return cs->d.nk <= 80 && !cs->upwind_1st && !cs->simple_2nd && bytes <= cs->max_lds;
 }
 
 // The zonal pass of the block kernel for either type
@@ -1932,7 +2135,7 @@ int continuity_blk_y(mom6h_continuity_cs *cs, const T *v, const T *hin, T *h, T 
                    bt ? bt->FA_u_EE : nullptr, bt ? bt->FA_u_E0 : nullptr, bt ? bt->FA_u_W0 : nullptr,
                    bt ? bt->FA_u_WW : nullptr, bt ? bt->uBT_WW : nullptr, bt ? bt->uBT_EE : nullptr,
                    bt ? bt_h_v : nullptr};
-    int rc = launch_y<T>(a, cs->monotonic, (unsigned)(d.jec - d.jsc + 2), s);
+    int rc = launch_blk<T, true>(a, cs->monotonic, (unsigned)(d.jec - d.jsc + 2), s);
     if (rc) return rc;
     {
         dim3 b(128), gc((d.iec - d.isc + 1 + 127) / 128, d.jec - d.jsc + 1, d.nk);
@@ -1964,14 +2167,19 @@ int continuity_batch(const ContArgsT<T> *d_args, const ContArgsT<T> *h_args, int
         nk_max = d.nk > nk_max ? d.nk : nk_max;
     }
     MOM6H_REQUIRE(nk_max <= 80 && (long long)sizeof(ContShared<T, 8, 10>) <= max_lds, "continuity batch: nk <= 80");
-    // one launch per block shape, K from the member's depth.  x: the slot class
-    bool wide = false;
-    for (int m = 0; m < n; ++m) wide = wide || cont_split_wide<T>(h_args[m].d);
+    // x: the members whose depth favours the split kernel (given the blocks of all
+    // members), one launch per slot class
+    bool wide = false, blk[kMaxMembers] = {};
+    for (int m = 0; m < n; ++m) {
+        wide = wide || cont_split_wide<T>(h_args[m].d);
+        blk[m] = y_pass || cont_blk_faster<T>(mp.first[n], h_args[m].d.nk);
+    }
     if (!y_pass && wide) {   // member by member
         for (int m = 0; m < n; ++m) {
             const int rc = launch_x<T>(h_args[m], h_args[m].monotonic, s);
             if (rc) return rc;
         }
+        std::fill(blk, blk + n, false);
     } else if (!y_pass) {
         for (const int K : {4, 7, 10, 13, 16, 19, 20}) {
             BatchMap g{};
@@ -1979,7 +2187,7 @@ int continuity_batch(const ContArgsT<T> *d_args, const ContArgsT<T> *h_args, int
             int nk_class = 1;
             for (int m = 0; m < n; ++m) {
                 const int nk = h_args[m].d.nk;
-                if (slot_class(nk) != K) continue;
+                if (blk[m] || slot_class(nk) != K) continue;
                 const int q = g.n++;
                 mi.v[q] = m;
                 g.nbx[q] = mp.nbx[m];
@@ -2002,19 +2210,18 @@ int continuity_batch(const ContArgsT<T> *d_args, const ContArgsT<T> *h_args, int
             MOM6H_LAUNCH_CHECK();
         }
     }
-    // y: 8 waves of K level slots (a member of 25 levels takes 8 x 4 = 32 slots
-    // rather than the 80 of the deepest member's 8 x 10); the levels spread
-    // evenly when every member of the launch has nk >= 8*(K-1)
+    // the block kernel: one launch per shape, 8 waves of K level slots (a member of
+    // 25 levels takes 8 x 4 = 32 slots rather than the 80 of the deepest member's
+    // 8 x 10); the levels spread evenly when every member of the launch has nk >= 8*(K-1)
     const int shapes[5] = {1, 2, 4, 7, 10};
     auto shape_of = [](int nk) { return nk <= 8 ? 1 : nk <= 16 ? 2 : nk <= 32 ? 4 : nk <= 56 ? 7 : 10; };
     for (const int K : shapes) {
-        if (!y_pass) break;
         BatchMap g{};
         MemberIndex mi{};
         bool even = true;
         for (int m = 0; m < n; ++m) {
             const int nk = h_args[m].d.nk;
-            if (shape_of(nk) != K) continue;
+            if (!blk[m] || shape_of(nk) != K) continue;
             const int q = g.n++;
             mi.v[q] = m;
             g.nbx[q] = mp.nbx[m];
@@ -2025,20 +2232,21 @@ int continuity_batch(const ContArgsT<T> *d_args, const ContArgsT<T> *h_args, int
         if (g.n == 0) continue;
         const unsigned nb = (unsigned)g.first[g.n];
         const dim3 b(64 * 8);
-#define CB(KK)                                                                                                   \
-    if (even) k_continuity_batch<T, 8, KK, true><<<nb, b, sizeof(ContShared<T, 8, KK>), s>>>(d_args, g, mi); \
-    else k_continuity_batch<T, 8, KK, false><<<nb, b, sizeof(ContShared<T, 8, KK>), s>>>(d_args, g, mi);
-        if (K == 1) {   // shapes of 1 and 2 slots always spread evenly
-            k_continuity_batch<T, 8, 1, true><<<nb, b, sizeof(ContShared<T, 8, 1>), s>>>(d_args, g, mi);
-        } else if (K == 2) {
-            k_continuity_batch<T, 8, 2, true><<<nb, b, sizeof(ContShared<T, 8, 2>), s>>>(d_args, g, mi);
-        } else if (K == 4) {
-            CB(4)
-        } else if (K == 7) {
-            CB(7)
-        } else {
-            CB(10)
-        }
+#define CB(Y, KK, EVEN) k_continuity_batch<T, Y, 8, KK, EVEN><<<nb, b, sizeof(ContShared<T, 8, KK>), s>>>(d_args, g, mi)
+#define CBY(KK, EVEN)                  \
+    do {                               \
+        if (y_pass) CB(true, KK, EVEN); \
+        else CB(false, KK, EVEN);      \
+    } while (0)
+        if (K == 1) CBY(1, true);   // shapes of 1 and 2 slots always spread evenly
+        else if (K == 2) CBY(2, true);
+        else if (K == 4 && even) CBY(4, true);
+        else if (K == 4) CBY(4, false);
+        else if (K == 7 && even) CBY(7, true);
+        else if (K == 7) CBY(7, false);
+        else if (even) CBY(10, true);
+        else CBY(10, false);
+#undef CBY
 #undef CB
         MOM6H_LAUNCH_CHECK();
     }

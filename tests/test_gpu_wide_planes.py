@@ -84,6 +84,47 @@ def test_zonal_continuity(target):
             assert bool((got == s[k]).all()), (f, k)
 
 
+def test_planes_of_4_gib():
+    """Zonal and meridional pass of one layer whose plane alone passes 32-bit offsets."""
+    import torch
+
+    from hackathon_mom6_miniapp_amd._lib import check, lib
+
+    n1, n2 = 23176, 23176
+    assert n1 * n2 * 8 >= 2 ** 32
+    g = torch.Generator(device="cuda").manual_seed(7)
+    rnd = lambda *s: torch.randn(*s, generator=g, dtype=torch.float64, device="cuda")  # noqa: E731
+    base = dict(u=0.05 * rnd(8, n1), h=4000.0 + 0.5 * rnd(8, n1))
+
+    def run(n2):
+        rows = torch.as_tensor(_at(n2, 8), device="cuda")
+        u, h = (base[f][rows].contiguous() for f in ("u", "h"))
+        L, cs = lib(), C.c_void_p()
+        keep, one = _host(n1, n2, 1.0)   # every metric 1
+        check(L.mom6h_continuity_init(C.byref(cs), *_bounds(n1, n2), 1, *[one] * 4, 0, *[one] * 3))
+        check(L.mom6h_continuity_set_meridional(cs, *[one] * 5))
+        out = {f: torch.zeros(n2, n1, dtype=torch.float64, device="cuda") for f in ("hx", "uh", "hy", "vh")}
+        torch.cuda.synchronize()
+        for fn, x, t in ((L.mom6h_continuity_ppm, "hx", "uh"), (L.mom6h_continuity_ppm_y, "hy", "vh")):
+            check(fn(cs, _ptr(u), _ptr(h), _ptr(out[x]), _ptr(out[t]), C.c_double(0.5), C.c_void_p(), C.c_void_p(),
+                     C.c_void_p(), C.c_void_p(), 0, C.c_void_p()))
+        check(L.mom6h_device_synchronize())
+        check(L.mom6h_continuity_end(cs))
+        return out
+
+    small = run(14)
+    print(f"[gpu wide] continuity {n1}x{n2}x1", flush=True)
+    wide = run(n2)
+    reps = (n2 - 6) // 8
+    for f, w in wide.items():
+        s = small[f][3:11, 3:n1 - 3]
+        assert s.abs().max() > 0.0, f
+        got = w[3:3 + 8 * reps, 3:n1 - 3]
+        for q in range(0, reps, 64):
+            part = got[8 * q:8 * (q + 64)]
+            assert bool((part.reshape(part.shape[0] // 8, 8, -1) == s).all()), (f, q)
+
+
 # --------------------------------------------------------------- vert_visc --
 def _vert_visc(n, nk, base, ray3d, keep):
     """u, v and the kept coefficients of a call on an n x n grid that repeats the 8 x 8 pattern of base."""
