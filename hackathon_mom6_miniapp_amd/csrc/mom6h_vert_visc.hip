@@ -167,8 +167,8 @@ __global__ void k_vert_visc(Dims d, double *__restrict__ u, double *__restrict__
 }
 
 
-// Chunked variant (columns the level-split variant below does not take).  One
-// thread per column; the only per-column scratch is one
+// Chunked variant (columns the level-split variant below does not take: a few
+// levels, or more than 80).  One thread per column; the only per-column scratch is one
 // LDS slot per level, holding z_i(k) after sweep A and c1(k) after sweep B
 // (slot nk+1 holds z_i(nk+1) = 0).  Sweep B re-derives hvel from h and the input
 // velocity (reloaded) and leaves the forward-eliminated velocity in the
@@ -185,9 +185,8 @@ __global__ void k_vert_visc(Dims d, double *__restrict__ u, double *__restrict__
 // level measured slower: the guards split the body and stop the interleaving).
 // The LDS column holds the kernel at one wave per SIMD, so the registers of
 // the prefetch are free: the FP64 bodies use AGPRs beyond 256 VGPRs rather
-// than scratch.  At nk = 75 these chunk sizes leave a tail of 1-3 levels per
-// sweep; 8 / 16 measured 7-10% slower (an 11-level unprefetched tail in
-// sweeps A and C), 16 / 32 and larger slower again.
+// than scratch.  The chunk sizes were measured at 75 levels, before the split
+// variant: 8 / 16 7-10% slower, 16 / 32 and larger slower again.
 
 constexpr int VV_C = 12;   // levels per chunk of sweep B (heavy bodies)
 constexpr int VV_A = 24;   // levels per chunk of sweeps A and C (light bodies, latency-bound loads)
@@ -563,9 +562,9 @@ __device__ __forceinline__ void vv_body(const VVArgs<T> &p, int bx, int row, VVS
 // (1.6 GB, 3.6 TB/s, VALU 61% busy; FP32 73%): VALU issue and the recurrence's
 // latency at three waves per SIMD.  180x180x75: 76 -> 38 us, 471x363x50: 180 ->
 // 107, 300x260x25: 52 -> 30, 200x100x12: 21 -> 12; with drag at every level
-// 347x188x75 269 -> 94 (289 -> 118 with the coefficients stored).  Faster at
-// every depth it takes; the chunked kernel keeps the deeper columns (more slots
-// would spill) and planes whose level offsets pass 4 GiB.  One spilled value per
+// 347x188x75 269 -> 94 (289 -> 118 with the coefficients stored).  The
+// chunked kernel keeps the shallow columns (vv_chunk_faster), the deeper ones (more
+// slots would spill) and planes whose level offsets pass 4 GiB.  One spilled value per
 // level made it slower than the chunked kernel (1170 us), hence the pins and
 // fences below.
 constexpr int VV_HAND = 4;                    // LDS rows of the hand-over between waves
@@ -575,6 +574,39 @@ constexpr int VV_G = 6;                       // levels whose divisions are inte
 inline bool vv_split_fits(const Dims &d)
 {
     return d.nk <= kSplitMax && kSplitMax / kSplitWaves * d.s2 * (long long)sizeof(double) < (1LL << 32);
+}
+
+// Whether the chunked kernel is the faster one for this grid (cols: of all grids
+// of a launch): with no more levels than waves the split kernel's blocks cost
+// their four waves and six barriers whatever the depth.  us per call, chunked /
+// split: FP64 300x200x2 8.0 / 11.0; 720x720x1 29 / 52, x3 56 / 59, x4 67 / 61, x8
+// 119 / 70; with drag at every level 300x200x3 9.8 / 14.0, 720x720x3 74 / 71; FP32
+// 300x200x6 10.2 / 11.9, 600x600x5 32.2 / 34.1, x6 37.4 / 35.4, 1000x1000x4 75 / 81,
+// x5 91 / 84.  A chunked wave ends with its row: from 4 levels on it needs full rows
+// or few waves (300x200x4 8.7 / 11.6; 200x200x4, rows 77% full, 11.7 / 9.5; 900x24x6
+// 8.3 / 9.7; 300x200x5 10.2 / 11.8; 180x180x5 9.3 / 8.5).
+template <typename T>
+bool vv_chunk_faster(const Dims &d, bool ray3d, long long cols)
+{
+    const int nk = d.nk, row = d.iec - d.isc + 2, per_row = (row + 63) / 64;
+    const long long waves = (long long)per_row * (2 * (d.jec - d.jsc) + 3);
+    auto rows_full = [&](int percent) { return 100 * row >= percent * 64 * per_row; };
+    if (nk <= 3) return !(ray3d && nk == 3 && cols > 250000);
+    if (sizeof(T) == 4) return nk <= (cols <= 110000 ? 6 : cols <= 550000 ? 5 : 4);
+    if (waves <= 900) return nk <= 6;
+    if (nk == 4) return cols <= 110000 && (waves <= 1100 || rows_full(80));
+    return nk == 5 && cols <= 90000 && waves > 1100 && rows_full(90);
+}
+
+inline long long vv_columns(const Dims &d)
+{
+    return (long long)(d.iec - d.isc + 1) * (d.jec - d.jsc + 1);
+}
+
+template <typename T>
+bool vv_takes_split(const Dims &d, bool ray3d)
+{
+    return vv_split_fits(d) && !vv_chunk_faster<T>(d, ray3d, vv_columns(d));
 }
 
 template <typename T>
@@ -953,7 +985,7 @@ int vert_visc_f32(mom6h_vert_visc_cs *cs, float *u, float *v, const float *h, do
     VVArgs<float> p{d, u, v, h, dt, taux, tauy, ray_u_bot, ray_v_bot, cs->mask2dCu, cs->mask2dCv,
                     cs->a_u, cs->a_v, cs->h_u, cs->h_v, cs->taux_bot, cs->tauy_bot, cs->Kv, cs->Kv_ml,
                     cs->Kv_extra_bbl, cs->Hmix, cs->Hbbl};
-    if (vv_split_fits(d))
+    if (vv_takes_split<float>(d, false))
         vv_split_launch<float, false, false>(p, stream);
     else
         k_vert_visc_chunked<float, false><<<g, dim3(64), lds, stream>>>(p);
@@ -968,15 +1000,21 @@ int vert_visc_batch(const VVArgs<T> *d_args, const VVArgs<T> *h_args, int n, lon
     BatchMap mp{};
     mp.n = n;
     int nk_max = 1;
-    bool split = true;
+    // the split kernel unless some plane is too large for it or every member
+    // favours the chunked one
+    bool split = true, shallow = true;
+    long long cols = 0;
+    for (int m = 0; m < n; ++m) cols += vv_columns(h_args[m].d);
     for (int m = 0; m < n; ++m) {
         const Dims &d = h_args[m].d;
         split = split && vv_split_fits(d);
+        shallow = shallow && vv_chunk_faster<T>(d, false, cols);
         mp.nbx[m] = (d.iec - d.isc + 2 + 63) / 64;
         mp.nby[m] = (d.jec - d.jsc + 1) + (d.jec - d.jsc + 2);
         mp.first[m + 1] = mp.first[m] + mp.nbx[m] * mp.nby[m];
         nk_max = d.nk > nk_max ? d.nk : nk_max;
     }
+    split = split && !shallow;
     if (split)
         for (int m = 0; m < n; ++m) mp.first[m + 1] = mp.first[m] + (int)vv_split_blocks(h_args[m].d);
     const size_t lds = (size_t)(nk_max + 1) * 64 * sizeof(VVSlot<T>);
@@ -1051,9 +1089,10 @@ int mom6h_vert_visc(mom6h_vert_visc_cs *cs, double *u, double *v, const double *
                  cs->a_u, cs->a_v, cs->h_u, cs->h_v, cs->taux_bot, cs->tauy_bot, cs->Kv, cs->Kv_ml,
                  cs->Kv_extra_bbl, cs->Hmix, cs->Hbbl};
         const dim3 g((ni + 63) / 64, rows);
-        if (vv_split_fits(d) && cs->keep_coefs)
+        const bool split = vv_takes_split<double>(d, false);
+        if (split && cs->keep_coefs)
             vv_split_launch<double, true, false>(p, (hipStream_t)stream);
-        else if (vv_split_fits(d))
+        else if (split)
             vv_split_launch<double, false, false>(p, (hipStream_t)stream);
         else if (cs->keep_coefs)
             k_vert_visc_chunked<double, true><<<g, dim3(64), lds, (hipStream_t)stream>>>(p);
@@ -1089,9 +1128,10 @@ int mom6h_vert_visc_ray3d(mom6h_vert_visc_cs *cs, double *u, double *v, const do
                      cs->a_u, cs->a_v, cs->h_u, cs->h_v, cs->taux_bot, cs->tauy_bot, cs->Kv, cs->Kv_ml,
                      cs->Kv_extra_bbl, cs->Hmix, cs->Hbbl, ray_u, ray_v};
     const dim3 g((ni + 63) / 64, rows);
-    if (vv_split_fits(d) && cs->keep_coefs)
+    const bool split = vv_takes_split<double>(d, true);
+    if (split && cs->keep_coefs)
         vv_split_launch<double, true, true>(p, (hipStream_t)stream);
-    else if (vv_split_fits(d))
+    else if (split)
         vv_split_launch<double, false, true>(p, (hipStream_t)stream);
     else if (cs->keep_coefs)
         k_vert_visc_chunked<double, true, true><<<g, dim3(64), lds, (hipStream_t)stream>>>(p);
