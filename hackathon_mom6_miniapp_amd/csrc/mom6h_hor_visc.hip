@@ -17,7 +17,7 @@
 // only formed on their own ranges (:587-607) and read as zero outside.  Those
 // values only reach diffu on column is-1 and ie and diffv on rows js-1 and je
 // (biharmonic: also the first interior column/row), and are reproduced here.
-#include "mom6h_internal.h"
+#include "mom6h_fused.h"
 
 #include <algorithm>
 #include <initializer_list>
@@ -33,6 +33,7 @@ struct HV {
     const double *IareaCu, *IareaCv, *mask2dT, *mask2dBu, *reduction_xx, *reduction_xy;
     const double *dy2h, *dx2h, *dy2q, *dx2q;
     const double *Idx2dyCu, *Idxdy2u, *Idx2dyCv, *Idxdy2v;
+    const unsigned char *mask_bits;   // 0/1 masks, one byte per point (MomArgsT::mask)
     double *Del2u, *Del2v;
     // closures (the general kernel): Smagorinsky_Kh/_Ah, Leith_Kh/_Ah,
     // better_bound_Kh/_Ah = bound_Kh/_Ah (hor_visc_init :179-193)
@@ -470,14 +471,19 @@ __global__ void k_hv_keep_ring(HV p, const double *__restrict__ u, const double 
 // Smagorinsky, the bounds and the biharmonic term: 116 us per call (march 98, ring
 // 11) against 3240 us when one thread per point evaluated every work value it
 // needed from u, v and h (and Del2 in a launch of its own, 214 us of them).
-// 471x363x50 Laplacian: 107 us, the time of the 64 x 8 tile staged in LDS that it
-// replaces (108 us); with the biharmonic term it saves the Del2 launch and arrays.
+// Laplacian, against the 64 x 8 tile staged in LDS that it replaces: 28x20x7 8 us
+// (18), 300x260x25 20 (38), 471x363x50 83 (94), 500x500x75 178 (180), 720x720x75 346
+// (379), 1440x1440x20 381 (392).  With FP64 masks and five rows walked beyond a chunk
+// it was slower than the tile from 500x500 on (199, 395 and 436 us): memory bounds it.
+// With the biharmonic term it saves the Del2 launch and arrays: 720x720x75 374 (2600).
 template <bool SMAG, bool LEITH, bool BOUND, bool BIH>
 struct HVMarch {
     static constexpr bool CL = SMAG || LEITH || BOUND;
     static constexpr int LM = CL || BIH ? 2 : 1;                       // lanes that only lend, west
     static constexpr int RM = LEITH ? 3 : CL || BIH ? 2 : 1;           // and east
     static constexpr int OUT = 64 - LM - RM;
+    // rows read before the first and after the last row written
+    static constexpr int BEFORE = CL || BIH ? 2 : 1, AFTER = CL ? 3 : BIH ? 2 : 1;
 };
 
 // compact index of a ring point: (is-1, js-1..je), then (is..ie, js-1)
@@ -516,7 +522,10 @@ __global__ void __launch_bounds__(64) k_hv_keep_last(HV p, const double *__restr
     p.ring_Ah[c] = ring_q[(long long)(2 * d.nk - 1) * n + q];
 }
 
-template <bool SMAG, bool LEITH, bool BOUND, bool BIH>
+// BITS: the masks from one byte per point (the constant-coefficient operators on
+// 0/1 masks: their FP64 planes, read again in every layer, were 0.6 of the 1.74 GB
+// a call read at 720x720x75)
+template <bool SMAG, bool LEITH, bool BOUND, bool BIH, bool BITS>
 __global__ void __launch_bounds__(256) k_hv_march(HV p, HVUniform g, const double *__restrict__ u,
                                                   const double *__restrict__ v, const double *__restrict__ h,
                                                   const double *__restrict__ ring_q, double *__restrict__ diffu,
@@ -548,14 +557,19 @@ __global__ void __launch_bounds__(256) k_hv_march(HV p, HVUniform g, const doubl
     const bool lap = p.laplacian;
     const double smag_K = p.smag_Kh ? 0.15 * 0.15 * area : 0.0, smag_A = 0.06 * 0.06 * (area * area);
 
-    double nu, nv, nh, nmT, nmB, nrK = 0.0, nrA = 0.0;   // the newest row, in flight until its step
+    double nu, nv, nh, nmT = 0.0, nmB = 0.0, nrK = 0.0, nrA = 0.0;   // the newest row, in flight until its step
+    unsigned nm = 0;
     auto load = [&](int r) __attribute__((always_inline)) {
         const long long row = row_of(r), o = layer + row;
         nu = (u + o)[col];
         nv = (v + o)[col];
         nh = (h + o)[col];
-        nmT = (p.mask2dT + row)[col];
-        nmB = (p.mask2dBu + row)[col];
+        if (BITS) {
+            nm = (p.mask_bits + row)[col];
+        } else {
+            nmT = (p.mask2dT + row)[col];
+            nmB = (p.mask2dBu + row)[col];
+        }
         if (M::CL) {   // the ring's Kh and Ah for the stress of h row r - 2
             const int J = r - 2;
             if (in_J(J) && (ring_strip || J == js - 1)) {
@@ -580,12 +594,14 @@ __global__ void __launch_bounds__(256) k_hv_march(HV p, HVUniform g, const doubl
     double hrat2 = 1.0;                                                                           // BOUND
     double d2u2 = 0.0, d2v2 = 0.0, d2v3 = 0.0;                                                    // BIH
     double tx3 = 0.0, ty3 = 0.0;                                               // stresses of row r - 3
-    load(ja - 2);
-    u1 = nu; v1 = nv; h1 = nh; ve1 = east(nv); he1 = east(nh); mh1 = nmT * nh; mB1 = nmB;
-    load(ja - 1);
-    for (int r = ja - 1; r <= jb + 3; ++r) {
-        const double u0 = nu, v0 = nv, h0 = nh, mT0 = nmT, mB0 = nmB, rK = nrK, rA = nrA;
-        if (r < jb + 3) load(r + 1);
+    auto mask_T = [&]() { return BITS ? (double)(nm & 1u) : nmT; };
+    auto mask_B = [&]() { return BITS ? (double)((nm >> 1) & 1u) : nmB; };
+    load(ja - M::BEFORE);
+    u1 = nu; v1 = nv; h1 = nh; ve1 = east(nv); he1 = east(nh); mh1 = mask_T() * nh; mB1 = mask_B();
+    load(ja - M::BEFORE + 1);
+    for (int r = ja - M::BEFORE + 1; r <= jb + 3; ++r) {
+        const double u0 = nu, v0 = nv, h0 = nh, mT0 = mask_T(), mB0 = mask_B(), rK = nrK, rA = nrA;
+        if (r < jb + M::AFTER) load(r + 1);   // later rows reach no output
         const double ve0 = east(v0), he0 = east(h0), mh0 = mT0 * h0;
         // tension at the h points of row r (:503-530)
         const double dudx = g.DY_dxT * ((g.IdyCu * u0) - (g.IdyCu * west(u0)));
@@ -726,6 +742,7 @@ static HV make_hv(const mom6h_hor_visc_cs *cs)
     p.reduction_xx = cs->reduction_xx; p.reduction_xy = cs->reduction_xy;
     p.dy2h = cs->dy2h; p.dx2h = cs->dx2h; p.dy2q = cs->dy2q; p.dx2q = cs->dx2q;
     p.Idx2dyCu = cs->Idx2dyCu; p.Idxdy2u = cs->Idxdy2u; p.Idx2dyCv = cs->Idx2dyCv; p.Idxdy2v = cs->Idxdy2v;
+    p.mask_bits = cs->mask_bits;
     p.Del2u = cs->Del2u; p.Del2v = cs->Del2v;
     p.smag_Kh = cs->smagorinsky && cs->laplacian;
     p.smag_Ah = cs->smagorinsky && cs->biharmonic;
@@ -756,7 +773,10 @@ int hor_visc_scratch(mom6h_hor_visc_cs *cs)
 }
 
 // the march's launch over the data domain: chunks of rows that leave about
-// four waves per SIMD, at least 8 (a chunk walks five rows more than it writes)
+// four waves per SIMD, at least 8, at most 48 with the closures (a chunk then walks
+// five rows more than it writes) and 40 without (Laplacian, us per call at 32 / 40 /
+// 48 / 56 / 64: 500x500x75 179 / 178 / 185 / 175 / 184, 720x720x75 347 / 346 / 355 /
+// 358 / 362, 1440x1440x20 377 / 381 / 391 / 394 / 388)
 template <bool SMAG, bool LEITH, bool BOUND, bool BIH>
 static void launch_march(const mom6h_hor_visc_cs *cs, const HV &p, const double *u, const double *v, const double *h,
                          double *diffu, double *diffv, hipStream_t s)
@@ -764,13 +784,19 @@ static void launch_march(const mom6h_hor_visc_cs *cs, const HV &p, const double 
     const Dims &d = cs->d;
     constexpr int OUT = HVMarch<SMAG, LEITH, BOUND, BIH>::OUT;
     const int strips = (d.n1 + OUT - 1) / OUT;
-    int rows = (int)std::min(48LL, std::max(8LL, (long long)strips * d.n2 * d.nk / 4096));
+    int rows = (int)std::min(HVMarch<SMAG, LEITH, BOUND, BIH>::CL ? 48LL : 40LL, std::max(8LL, (long long)strips * d.n2 * d.nk / 4096));
     int chunks = (d.n2 + rows - 1) / rows;
     rows = (d.n2 + chunks - 1) / chunks;
     chunks = (d.n2 + rows - 1) / rows;
     const long long tasks = (long long)strips * chunks * d.nk;
-    k_hv_march<SMAG, LEITH, BOUND, BIH><<<(unsigned)((tasks + 3) / 4), 256, 0, s>>>(
-        p, cs->g, u, v, h, cs->ring_q, diffu, diffv, strips, chunks, rows);
+    const unsigned blocks = (unsigned)((tasks + 3) / 4);
+    constexpr bool CL = HVMarch<SMAG, LEITH, BOUND, BIH>::CL;
+    if (!CL && cs->mask_bits)
+        k_hv_march<SMAG, LEITH, BOUND, BIH, !CL><<<blocks, 256, 0, s>>>(p, cs->g, u, v, h, cs->ring_q, diffu, diffv,
+                                                                      strips, chunks, rows);
+    else
+        k_hv_march<SMAG, LEITH, BOUND, BIH, false><<<blocks, 256, 0, s>>>(p, cs->g, u, v, h, cs->ring_q, diffu, diffv,
+                                                                        strips, chunks, rows);
 }
 
 template <bool SMAG, bool LEITH, bool BOUND>
@@ -853,6 +879,15 @@ int mom6h_hor_visc_init(mom6h_hor_visc_cs **out, int isd, int ied, int jsd, int 
                                      {IareaCv, &g.IareaCv}, {reduction_xx, &g.red_xx},
                                      {reduction_xy, &g.red_xy}, {dy2h, &g.dy2h}, {dx2h, &g.dx2h},
                                      {dy2q, &g.dy2q}, {dx2q, &g.dx2q}});
+    if (cs->uniform && binary_mask(mask2dT, n2) && binary_mask(mask2dBu, n2)) {
+        rc = dev_alloc_bytes((void **)&cs->mask_bits, n2, false);
+        if (!rc) rc = launch_mask_bits(MaskJobs{1, {{cs->mask2dT, cs->mask2dBu, cs->mask_bits, (long long)n2}}}, nullptr);
+        if (!rc && hipStreamSynchronize(nullptr) != hipSuccess) rc = set_error(MOM6H_ESTATE, "mask conversion failed");
+        if (rc) {
+            mom6h_hor_visc_end(cs);
+            return rc;
+        }
+    }
     *out = cs;
     return MOM6H_OK;
 }
@@ -973,6 +1008,7 @@ int mom6h_hor_visc_end(mom6h_hor_visc_cs *cs)
                       cs->Idx2dyCu, cs->Idxdy2u, cs->Idx2dyCv, cs->Idxdy2v, cs->Del2u, cs->Del2v,
                       cs->areaT, cs->dxBu, cs->dyBu, cs->IdxBu, cs->IdyBu, cs->ring_Kh, cs->ring_Ah, cs->ring_q})
         dev_free(p);
+    if (cs->mask_bits) (void)hipFree(cs->mask_bits);
     delete cs;
     return MOM6H_OK;
 }

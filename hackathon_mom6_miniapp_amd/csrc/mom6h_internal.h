@@ -467,6 +467,7 @@ struct mom6h_hor_visc_cs {
     // js-2..je+2): the values, for the march; bih_uniform likewise for the four
     // biharmonic metrics, area_uniform and leith_uniform for the closures'
     int uniform = 0, bih_uniform = 0, area_uniform = 0, leith_uniform = 0;
+    unsigned char *mask_bits = nullptr;   // uniform grids with 0/1 masks: one byte per point, for the march
     int general = 0;         // use the general kernel even on a uniform grid
     mom6h::HVUniform g{};
 };
