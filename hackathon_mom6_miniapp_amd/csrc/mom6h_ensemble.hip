@@ -88,7 +88,6 @@ struct mom6h_ensemble {
     int bt_tile = 4;         // rows of the barotropic substep tile (4, 8 or 16)
     int bt_substeps = 0;     // barotropic substeps per blocked launch (1 = one launch per substep, 0 = chosen from the grids)
     long long max_lds = 0;
-    MaskJobs masks{};        // the members' byte masks
     StepTables<float> tf;
     StepTables<double> td;
     Table<BTMember> bt_pred, bt_corr;
@@ -166,6 +165,14 @@ template <typename T>
 int halo(const Table<HaloJob<T>> &t, hipStream_t s)
 {
     return t.n() ? halo_batch<T>(t.d, t.h.data(), t.n(), s) : MOM6H_OK;
+}
+
+// the members' byte masks that may be out of date, on s0
+int refresh_masks(mom6h_ensemble *e)
+{
+    MaskJobs jobs{};
+    for (mom6h_model *m : e->members) RC(stale_masks(m, &jobs));
+    return jobs.n ? launch_mask_bits(jobs, e->s0) : MOM6H_OK;
 }
 
 // the 3D chain of one step for all members (stream s0)
@@ -361,7 +368,7 @@ int mom6h_ensemble_prepare(mom6h_ensemble *e)
         MOM6H_REQUIRE(m->bt_cs->uniform, "mom6h_ensemble_prepare: members need uniform barotropic coefficients");
         e->max_lds = m->vv->max_lds;
     }
-    for (mom6h_model *m : e->members) RC(mask_job(m, &e->masks.j[e->masks.n++]));
+    RC(refresh_masks(e));   // allocated here: the tables hold their addresses
     RC(e->mixed ? build_tables<float>(e, e->tf, layers_f32) : build_tables<double>(e, e->td, layers_f64));
     for (mom6h_model *m : e->members) {
         BTMember p{}, c{};
@@ -397,7 +404,7 @@ int mom6h_ensemble_step(mom6h_ensemble *e, int niter)
     }
     MOM6H_CHECK(hipEventRecord(e->e_start, e->s0));
     MOM6H_CHECK(hipStreamWaitEvent(e->s1, e->e_start, 0));
-    RC(launch_mask_bits(e->masks, e->s0));
+    RC(refresh_masks(e));
     // enqueued in turn, so that s0 has work while the host still enqueues s1's
     for (int it = 0; it < niter; ++it) {
         if (e->use_graph) MOM6H_CHECK(hipGraphLaunch(e->gexec_bt, e->s1));
@@ -468,7 +475,7 @@ int mom6h_ensemble_autotune(mom6h_ensemble *e, int reps, char *report, int nbyte
     MOM6H_REQUIRE(e != nullptr, "mom6h_ensemble_autotune: NULL ensemble");
     MOM6H_REQUIRE(e->prepared, "mom6h_ensemble_autotune: call mom6h_ensemble_prepare first");
     MOM6H_CHECK(hipDeviceSynchronize());
-    RC(launch_mask_bits(e->masks, e->s0));
+    RC(refresh_masks(e));
     std::string rep;
     const int rc = e->mixed ? tune<float>(e, e->tf, reps, &rep) : tune<double>(e, e->td, reps, &rep);
     drop_graph(e);

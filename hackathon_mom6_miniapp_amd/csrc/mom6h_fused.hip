@@ -443,9 +443,9 @@ int launch_del2(const Del2Args<T> &a, hipStream_t s)
 template int launch_del2<double>(const Del2Args<double> &, hipStream_t);
 template int launch_del2<float>(const Del2Args<float> &, hipStream_t);
 
-// The masks as the stencil reads them: formed anew on every step call, since a
-// caller may rewrite the fields between calls (their device addresses are
-// public).  17 bytes per point of one plane, about 3 us at 720x720.
+// The masks as the stencil reads them, formed ahead of a step call when the fields
+// were uploaded since, or when a caller holds the address of one and may have
+// written it: 17 bytes per point of one plane, about 3 us at 720x720.
 __global__ void __launch_bounds__(256) k_mask_bits(MaskJobs jobs)
 {
     const MaskJob a = jobs.j[blockIdx.y];

@@ -41,7 +41,9 @@ struct mom6h_model {
     int fused = 1;           // fused momentum stencil (module-by-module when 0)
     bool uniform = false;    // every metric array constant (fused kernels allowed)
     bool fused_rows = false; // masks 0/1 and Coriolis constant along rows (what the fused stencil reads)
-    unsigned char *mask_bits = nullptr;   // those masks, one byte per point (MomArgsT::mask), from every step call
+    unsigned char *mask_bits = nullptr;   // those masks, one byte per point (MomArgsT::mask)
+    bool masks_stale = true;              // the mask fields were written since mask_bits were formed
+    bool masks_shared = false;            // a caller holds a mask field's device address
     UMetrics ug{};
     hipStream_t s0 = nullptr, s1 = nullptr;
     hipEvent_t e_start = nullptr, e_bt = nullptr;
@@ -102,6 +104,7 @@ namespace mom6h {
 bool fused_ok(const mom6h_model *m);
 // the fields "del2u" and "del2v" brought up to date on stream s, when in use
 int refresh_del2(mom6h_model *m, hipStream_t s);
-// the model's byte masks (allocated by the first call) as a job of launch_mask_bits
-int mask_job(mom6h_model *m, MaskJob *job);
+// Adds the model's byte masks (allocated by the first call) to what the caller is
+// to form with launch_mask_bits ahead of the stencil, if they may be out of date
+int stale_masks(mom6h_model *m, MaskJobs *jobs);
 }  // namespace mom6h

@@ -481,7 +481,7 @@ int mom6h_model_create(mom6h_model **out, const mom6h_config *c)
     return MOM6H_OK;
 }
 
-int mom6h_model_field(mom6h_model *m, const char *name, void **d_ptr, long *count)
+static int field_of(mom6h_model *m, const char *name, void **d_ptr, long *count)
 {
     MOM6H_REQUIRE(m && name, "mom6h_model_field: NULL argument");
     if (const Field *f = find_field(m, name)) {
@@ -506,12 +506,24 @@ int mom6h_model_field(mom6h_model *m, const char *name, void **d_ptr, long *coun
     return set_error(MOM6H_EINVAL, "mom6h_model_field: unknown field '%s'", name);
 }
 
+static bool stencil_mask(const char *name)
+{
+    return !strcmp(name, "mask2dT") || !strcmp(name, "mask2dBu");
+}
+
+int mom6h_model_field(mom6h_model *m, const char *name, void **d_ptr, long *count)
+{
+    RC(field_of(m, name, d_ptr, count));
+    if (d_ptr && stencil_mask(name)) m->masks_shared = true;   // the caller may write it at any time
+    return MOM6H_OK;
+}
+
 int mom6h_model_field_bytes(mom6h_model *m, const char *name, int *elem_bytes)
 {
     MOM6H_REQUIRE(m && name && elem_bytes, "mom6h_model_field_bytes: NULL argument");
     const Field *f = find_field(m, name);
     long n = 0;
-    if (!f) RC(mom6h_model_field(m, name, nullptr, &n));   // the vert_visc arrays: FP64
+    if (!f) RC(field_of(m, name, nullptr, &n));   // the vert_visc arrays: FP64
     *elem_bytes = f ? f->bytes : 8;
     return MOM6H_OK;
 }
@@ -521,9 +533,10 @@ int mom6h_model_upload(mom6h_model *m, const char *name, const double *src, long
     void *p = nullptr;
     long n = 0;
     int bytes = 8;
-    RC(mom6h_model_field(m, name, &p, &n));
+    RC(field_of(m, name, &p, &n));
     RC(mom6h_model_field_bytes(m, name, &bytes));
     MOM6H_REQUIRE(src && count == n, "mom6h_model_upload(%s): expected %ld values, got %ld", name, n, count);
+    if (stencil_mask(name)) m->masks_stale = true;
     MOM6H_CHECK(hipDeviceSynchronize());
     if (bytes == 8) {
         MOM6H_CHECK(hipMemcpy(p, src, (size_t)n * sizeof(double), hipMemcpyHostToDevice));
@@ -540,9 +553,10 @@ int mom6h_model_fill(mom6h_model *m, const char *name, const double *d_src, long
     void *p = nullptr;
     long n = 0;
     int bytes = 8;
-    RC(mom6h_model_field(m, name, &p, &n));
+    RC(field_of(m, name, &p, &n));
     RC(mom6h_model_field_bytes(m, name, &bytes));
     MOM6H_REQUIRE(d_src && count == n, "mom6h_model_fill(%s): expected %ld values, got %ld", name, n, count);
+    if (stencil_mask(name)) m->masks_stale = true;
     MOM6H_CHECK(hipDeviceSynchronize());
     if (bytes == 8) MOM6H_CHECK(hipMemcpy(p, d_src, (size_t)n * sizeof(double), hipMemcpyDeviceToDevice));
     else RC(narrow_to_f32(d_src, (float *)p, n, m->s0));
@@ -555,7 +569,7 @@ int mom6h_model_download(mom6h_model *m, const char *name, double *dst, long cou
     void *p = nullptr;
     long n = 0;
     int bytes = 8;
-    RC(mom6h_model_field(m, name, &p, &n));
+    RC(field_of(m, name, &p, &n));
     RC(mom6h_model_field_bytes(m, name, &bytes));
     MOM6H_REQUIRE(dst && count == n, "mom6h_model_download(%s): expected %ld values, got %ld", name, n, count);
     MOM6H_CHECK(hipDeviceSynchronize());
@@ -729,10 +743,10 @@ static int run_steps(mom6h_model *m, int niter)
     // The fused path consumes vert_visc's coupling coefficients on chip; the
     // module path keeps them in the control structure, as the reference does.
     RC(mom6h_vert_visc_keep_coefficients(m->vv, fused_ok(m) ? 0 : 1));
-    // the fused stencil's byte masks follow the mask fields (ahead of a capture,
-    // which holds their address; on s0 behind the fork, so that s1 need not wait)
+    // the fused stencil's byte masks follow the mask fields (allocated ahead of a
+    // capture, which holds their address; formed behind the fork, so that s1 need not wait)
     MaskJobs mj{};
-    if (fused_ok(m)) RC(mask_job(m, &mj.j[mj.n++]));
+    if (fused_ok(m)) RC(stale_masks(m, &mj));
     auto masks = [&]() -> int { return mj.n ? launch_mask_bits(mj, m->s0) : MOM6H_OK; };
     if (m->c.coupled) {
         RC(masks());
@@ -958,8 +972,8 @@ int mom6h_model_autotune(mom6h_model *m, int reps, char *report, int nbytes)
     MOM6H_REQUIRE(fused_ok(m), "mom6h_model_autotune: only the fused stencil has tile shapes to choose");
     MOM6H_CHECK(hipDeviceSynchronize());
     MaskJobs mj{};
-    RC(mask_job(m, &mj.j[mj.n++]));
-    RC(launch_mask_bits(mj, m->s0));
+    RC(stale_masks(m, &mj));
+    if (mj.n) RC(launch_mask_bits(mj, m->s0));
     std::string rep;
     const int rc = m->mixed ? tune_model(m, m->f.u, m->f.v, m->f.h0, m->f.htmp, m->f.up, m->f.vp, reps, &rep)
                             : tune_model(m, m->u, m->v, m->h0, m->htmp, m->up, m->vp, reps, &rep);
@@ -1012,10 +1026,12 @@ int refresh_del2(mom6h_model *m, hipStream_t s)
     return MOM6H_OK;
 }
 
-int mask_job(mom6h_model *m, MaskJob *job)
+int stale_masks(mom6h_model *m, MaskJobs *jobs)
 {
     if (!m->mask_bits) RC(dev_alloc_bytes((void **)&m->mask_bits, (size_t)m->d.s2, false));
-    *job = MaskJob{m->mask2dT, m->mask2dBu, m->mask_bits, m->d.s2};
+    if (m->masks_stale || m->masks_shared)
+        jobs->j[jobs->n++] = MaskJob{m->mask2dT, m->mask2dBu, m->mask_bits, m->d.s2};
+    m->masks_stale = false;
     return MOM6H_OK;
 }
 }  // namespace mom6h

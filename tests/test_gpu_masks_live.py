@@ -77,3 +77,29 @@ def test_masks_rewritten_between_replays():
         m.close()
     for a, b in zip(*got):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_address_held_over_steps(graph):
+    """A mask written several times through an address taken once."""
+    from hackathon_mom6_miniapp_amd._lib import check
+    from hackathon_mom6_miniapp_amd.model import Ensemble, Model
+
+    case = make_case(CFG, init="seeded", seed=4)
+    masks = [np.asfortranarray(case["mask2dBu"]), _land(case, "mask2dBu")]
+    want, late, ens = Model(CFG, case), Model(CFG, case, graph=graph), Ensemble([CFG, CFG], [case, case], graph=graph)
+    runs = [(late, late.device_ptr("mask2dBu")), (ens, ens.members[1].device_ptr("mask2dBu"))]
+    for q in range(5):
+        mask = masks[q in (1, 2, 4)]
+        want.upload("mask2dBu", mask)
+        want.step(1)
+        want.synchronize()
+        for m, ptr in runs:
+            check(late.L.mom6h_memcpy_h2d(ptr, mask.ctypes.data, mask.nbytes))
+            m.step(1)
+            m.synchronize()
+        for f in ("u", "v", "h"):
+            assert np.array_equal(late.get(f), want.get(f)), (q, f)
+            assert np.array_equal(ens.members[1].get(f), want.get(f)), (q, f)
+    for m in (want, late, ens):
+        m.close()
