@@ -584,11 +584,14 @@ inline std::vector<int> bt_split(int nstep, bool periodic, int ts)
 // launches mean fewer of the first, smaller tiles and so more of the others.
 // us per call at 4 / 5 / 6 / 8 / 10 / 14 substeps (alone): 28x20, 20 substeps:
 // 82 / 78 / 74 / 74 / 71 / 71; 180x180, 30: 140 / 133 / 125 / 118 / 111 / 105;
-// 720x720, 50: 279 / 264 / 250 / 357 / 364 / 724 (two rounds from 7 on).
+// 720x720, 50: 279 / 264 / 250 / 357 / 364 / 724 (two rounds from 7 on).  A call of
+// two substeps takes two blocked launches in any case, against a copy-in and two
+// one-substep launches: 180x180 19 / 14, 400x400 20 / 20, 720x720 22 / 35.
 inline int bt_auto_substeps(const std::vector<Dims> &grids, int nstep, bool periodic)
 {
     double points = 0.0, best = 0.0;
     for (const Dims &d : grids) points += (double)d.s2;
+    if (nstep == 2 && points < 160000.0) return 1;
     int pick = 5;
     for (int ts = 2; ts <= kBTMost; ++ts) {
         double cost = 0.0;
@@ -668,7 +671,7 @@ int btstep_batch(const BTMember *d_args, const BTMember *h_args, int n, hipStrea
     const int BT_TY = ty;
     MOM6H_REQUIRE(n >= 1 && n <= kMaxMembers, "btstep batch: 1..%d members", kMaxMembers);
     const int nstep = h_args[0].p.nstep;
-    bool blocked = per_launch != 1 && nstep >= 2, rowwise = true, periodic = false;
+    bool blocked = nstep >= 2, rowwise = true, periodic = false;
     std::vector<Dims> grids;
     for (int m = 0; m < n; ++m) {
         MOM6H_REQUIRE(h_args[m].p.nstep == nstep, "btstep batch: members differ in bt_nsteps");
@@ -677,8 +680,8 @@ int btstep_batch(const BTMember *d_args, const BTMember *h_args, int n, hipStrea
         rowwise = rowwise && h_args[m].m.Datv_row != nullptr;
         periodic = periodic || h_args[m].p.px || h_args[m].p.py;
     }
-    if (blocked) {
-        const int ts = per_launch ? per_launch : bt_auto_substeps(grids, nstep, periodic);
+    const int ts = per_launch ? per_launch : bt_auto_substeps(grids, nstep, periodic);
+    if (blocked && ts != 1) {
         int n0 = 1, src = 0;
         for (int ns : bt_split(nstep, periodic, ts)) {
             BatchMap mm{};
@@ -901,7 +904,8 @@ static int btstep_run(mom6h_barotropic_cs *cs, double *const w[8], bool zero_b, 
     p.ubt_av = w[6]; p.vbt_av = w[7];
     const Dims &d = cs->d;
     double *A[3] = {w[0], w[1], w[2]}, *B[3] = {w[3], w[4], w[5]};
-    if (cs->substeps != 1 && cs->blocked_ok && cs->nstep >= 2) {   // blocked launches
+    const int ts = cs->substeps ? cs->substeps : cs->auto_substeps;
+    if (ts != 1 && cs->blocked_ok && cs->nstep >= 2) {   // blocked launches
         BTUniform m{cs->u_Datu, cs->u_gtot, cs->u_rem_u, cs->u_rem_v, cs->u_IareaT, cs->u_IdxCu, cs->u_IdyCv,
                     cs->Datv, cs->f4};
         const bool periodic = p.px || p.py, rows = cs->Datv_row && cs->use_rows;
@@ -909,7 +913,6 @@ static int btstep_run(mom6h_barotropic_cs *cs, double *const w[8], bool zero_b, 
             m.Datv_row = cs->Datv_row;
             m.f4_row = cs->f4_row;
         }
-        const int ts = cs->substeps ? cs->substeps : cs->auto_substeps;
         BTMulti st;
         st.eta_o = eta_in; st.ubt_o = ubt_in; st.vbt_o = vbt_in;
         st.out_u = u_av; st.out_v = v_av; st.out_eta = eta_av;
