@@ -103,10 +103,11 @@ inline int march_rows(int tile, int splits)
 
 // Chooses the options momentum_tile and momentum_splits by timing launch (what a
 // step does with the stencil) on stream s under each candidate, which set puts in
-// force: marches of 128 to 4 rows and the one chosen from the grid (0, 0), which
-// stays unless another is faster by more than 1%.  One round over the candidates
-// warms up, then `reps` rounds in alternating order; the shortest time of each
-// counts.  Leaves the choice set and adds the times to the report.
+// force: marches of 64 to 4 rows and the one chosen from the grid (0, 0), which
+// stays unless another is faster by more than 1%.  After a warm-up one round over the
+// candidates, then up to `reps` in all over those within 5% of the best, in
+// alternating order; the shortest time of each counts.  Leaves the choice set and
+// adds the times to the report.
 int tune_march(hipStream_t s, int reps, const std::function<int(int tile, int splits)> &set,
                const std::function<int()> &launch, std::string *report);
 
@@ -123,8 +124,12 @@ inline bool uniform_value(const double *a, size_t n, double *v)
 // momentum stencil can read as a bit)
 inline bool binary_mask(const double *a, size_t n)
 {
-    for (size_t q = 0; q < n; ++q)
-        if (!(a[q] == 0.0 || a[q] == 1.0)) return false;
+    for (size_t q0 = 0; q0 < n; q0 += 4096) {   // whole blocks without a branch: vector compares
+        const size_t q1 = q0 + 4096 < n ? q0 + 4096 : n;
+        bool ok = true;
+        for (size_t q = q0; q < q1; ++q) ok &= (a[q] == 0.0) | (a[q] == 1.0);
+        if (!ok) return false;
+    }
     return true;
 }
 

@@ -346,37 +346,43 @@ int launch_momentum_batch(const MomArgsT<T> *d_args, const MomArgsT<T> *h_args, 
 
 // One timing of each candidate in a fixed order, predictor only, chose 128 rows at
 // 720x720x75 (0.42 ms, in the first place after a pause) where a step's two
-// launches then took 1.01 ms, against 0.89 ms with 16 rows: the first milliseconds
-// after a pause run faster, and the corrector's extra base rows weigh on long
-// marches.  Hence the warm-up round, the alternating order and both phases: 28 ms
-// with reps = 3 there, and two timings of one length then differ by 1.3% at most.
+// launches then took 1.01 ms, against 0.89 ms with 16 rows: the clock moves for
+// some milliseconds after a pause, and the corrector's extra base rows weigh on long
+// marches.  Hence the warm-up, the alternating order and both phases: 20 ms with reps
+// = 3 there.
 int tune_march(hipStream_t s, int reps, const std::function<int(int, int)> &set, const std::function<int()> &launch,
                std::string *report)
 {
-    constexpr int N = 7;
-    const int tile[N] = {0, 16, 8, 4, 4, 4, 4}, splits[N] = {0, 1, 1, 1, 2, 4, 8};   // auto, 128 .. 4 rows
-    float ms[N] = {};
+    constexpr int N = 6;
+    const int tile[N] = {0, 8, 4, 4, 4, 4}, splits[N] = {0, 1, 1, 2, 4, 8};   // auto, 64 .. 4 rows
     hipEvent_t a = nullptr, b = nullptr;
     int rc = hipEventCreate(&a) == hipSuccess && hipEventCreate(&b) == hipSuccess
                  ? MOM6H_OK
                  : set_error(MOM6H_ENOMEM, "event creation failed");
-    int per = 1;   // launches per timing: about 0.3 ms
-    for (int round = 0; round <= (reps > 1 ? reps : 1) && !rc; ++round) {
-        float slowest = 0.f;
-        for (int c = 0; c < N && !rc; ++c) {
+    // ms per launch of candidate q, over n launches
+    auto time = [&](int q, int n) -> float {
+        float t = 0.f;
+        if (!rc) rc = set(tile[q], splits[q]);
+        if (!rc && hipEventRecord(a, s) != hipSuccess) rc = set_error(MOM6H_ESTATE, "event record failed");
+        for (int r = 0; r < n && !rc; ++r) rc = launch();
+        if (!rc && hipEventRecord(b, s) != hipSuccess) rc = set_error(MOM6H_ESTATE, "event record failed");
+        if (!rc && hipEventSynchronize(b) != hipSuccess) rc = set_error(MOM6H_ESTATE, "event wait failed");
+        if (!rc && hipEventElapsedTime(&t, a, b) != hipSuccess) rc = set_error(MOM6H_ESTATE, "event timing failed");
+        return t / (float)n;
+    };
+    // warm-up: about 6 ms; then timings of about 0.3 ms each
+    const float first = std::max(time(0, 1), 1.0e-3f);
+    const int warm = std::min(200, (int)(6.f / first)), per = first >= 0.3f ? 1 : std::min(16, (int)(0.3f / first) + 1);
+    if (warm > 0) time(0, warm);
+    float ms[N] = {}, best = 0.f;
+    for (int round = 0; round < (reps > 1 ? reps : 1); ++round) {
+        for (int c = 0; c < N; ++c) {
             const int q = round % 2 ? N - 1 - c : c;
-            rc = set(tile[q], splits[q]);
-            if (!rc && hipEventRecord(a, s) != hipSuccess) rc = set_error(MOM6H_ESTATE, "event record failed");
-            for (int r = 0; r < per && !rc; ++r) rc = launch();
-            if (!rc && hipEventRecord(b, s) != hipSuccess) rc = set_error(MOM6H_ESTATE, "event record failed");
-            if (!rc && hipEventSynchronize(b) != hipSuccess) rc = set_error(MOM6H_ESTATE, "event wait failed");
-            float t = 0.f;
-            if (!rc && hipEventElapsedTime(&t, a, b) != hipSuccess) rc = set_error(MOM6H_ESTATE, "event timing failed");
-            t /= (float)per;
-            slowest = std::max(slowest, t);
-            if (round == 1 || (round > 1 && t < ms[q])) ms[q] = t;
+            if (round > 0 && q != 0 && ms[q] > 1.05f * best) continue;   // out of the running
+            const float t = time(q, per);
+            if (round == 0 || t < ms[q]) ms[q] = t;
         }
-        if (round == 0) per = slowest >= 0.3f ? 1 : slowest > 0.02f ? (int)(0.3f / slowest) + 1 : 16;
+        best = *std::min_element(ms, ms + N);
     }
     if (a) (void)hipEventDestroy(a);
     if (b) (void)hipEventDestroy(b);

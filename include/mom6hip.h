@@ -344,11 +344,11 @@ int mom6h_model_set_option(mom6h_model *m, const char *key, double value);
 int mom6h_model_stage_times(mom6h_model *m, double *ms, int max_stages, char *names, int nbytes);
 int mom6h_model_main_stream(mom6h_model *m, void **stream);
 /* Times the fused momentum stencil (a predictor's and a corrector's launch, onto
- * outputs that every step rewrites) for marches of 4 to 128 rows and for the
- * number chosen from the grid: one round to warm up, then reps rounds (at least
- * one) over all of them.  Keeps the fastest as options "momentum_tile" and
- * "momentum_splits" (both 0 unless one beats the grid's number by more than 1%)
- * and writes the shortest times into report. */
+ * outputs that every step rewrites) for marches of 4 to 64 rows and for the
+ * number chosen from the grid: a warm-up, one round over all of them, then up to
+ * reps rounds in all over the fastest.  Keeps the best as options "momentum_tile"
+ * and "momentum_splits" (both 0 unless one beats the grid's number by more than
+ * 1%) and writes the shortest times into report. */
 int mom6h_model_autotune(mom6h_model *m, int reps, char *report, int nbytes);
 /* With option "diag" = 1 (FP64 form) every step posts the predictor's
  * diffu_sum and diffv_sum statistics; this call adds KE and mass of the
