@@ -75,9 +75,9 @@ STAGE_ARRAYS = {            # (3D, 2D) per call
 STAGE_CALLS = {"transports": 2, "hor_visc": 2, "coriolis": 2, "vel_update": 2, "vert_visc": 2,
                "continuity": 2, "btstep": 2, "halo": 1, "momentum": 2}
 # Stages that are ONE kernel launch per call on the 3D stream (the fused path),
-# and that kernel.  The barotropic stage brackets bt_nsteps+1 launches on the
-# second stream, so its events do not time a single kernel; it is reported in
-# "stages" only.
+# and that kernel.  The barotropic stage brackets some ten launches of several
+# substeps on the second stream, so its events do not time a single kernel; it is
+# reported in "stages" only.
 ROOFLINE_KERNELS = {"momentum": "k_momentum", "vert_visc": "k_vert_visc_split",
                     "continuity": "k_continuity_split"}
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic_720x720x75.md")
@@ -87,7 +87,8 @@ FP64_PEAK_TFLOPS = 78.6   # MI355X FP64 vector
 ROOFLINE_LIMIT = {
     "k_continuity_split": "VALU issue and, at two waves per SIMD, the latency of dependent FP64 "
                           "operations (k-order column sums handed from wave to wave)",
-    "k_momentum": "VALU issue (bit-exact FP64 divisions)",
+    "k_momentum": "VALU issue (81-87% busy: bit-exact FP64 divisions) and HBM (4.8 of 5.4 TB/s of a "
+                  "plain copy) about equally",
     "k_vert_visc_split": "VALU issue (four exact divisions per level) and the tridiagonal recurrence's "
                          "latency at three waves per SIMD",
 }

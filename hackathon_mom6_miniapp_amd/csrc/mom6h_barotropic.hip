@@ -5,10 +5,11 @@
 // transport ranges (btstep_do_step, :379-474) with a refill of the ubt, vbt and
 // eta halos after every substep but the last (app/rk2_mpi_serial_driver.F90:
 // 297-306).  The reference CUDA-C path issues ~9 dependent launches per
-// substep from the host; here each substep is ONE launch of an LDS-tiled
-// kernel that runs the whole substep (eta predictor, pressure forces, both
-// Coriolis/velocity updates in the alternating order, transports, free
-// surface, time averages, periodic refill) on its tile.  Transports that the
+// substep from the host; here a launch runs whole substeps (eta predictor,
+// pressure forces, both Coriolis/velocity updates in the alternating order,
+// transports, free surface, time averages, periodic refill) on its tile: one in
+// LDS on grids whose coefficients vary, several in registers (k_bt_multi) on
+// uniform grids.  Transports that the
 // reference never writes (uhbt on I = is-1 and ie, vhbt on J = js-1 and je
 // with the narrow ranges) read as zero, as they do there.
 #include <algorithm>
@@ -296,8 +297,9 @@ struct BTMulti {
 // read by a valid point.  ts substeps leave a tile of 64 - 3 ts in each
 // direction.
 //
-// What bounds it: VALU issue, 65 instructions per position and substep (76 in
-// waves that need the range selects), and about 8 us per launch for the launch
+// What bounds it: the latency of the dependent FP64 operations of a substep (65
+// instructions per position, 76 in waves that need the range selects) at two waves
+// per SIMD, VALU 34% busy over a launch, and some 6 to 8 us per launch for the launch
 // and the state's way in and out.  At 720x720 a launch of 6 substeps takes 26.7
 // us and a call of 100 substeps 413 us.  The form before kept the state in LDS,
 // mapped threads to the positions of a shrinking rectangle in each of four

@@ -48,11 +48,11 @@ __device__ __forceinline__ T sdiv(T num, T den)
 // What bounds it: 225 VALU instructions per row of 62 points (FP64, Laplacian)
 // against the 370 of a 64 x 8 tile staged in LDS with its recomputed ring, 38
 // KB of LDS and two barriers per layer, which was VALU-bound.  At 720x720x75
-// the predictor now takes 0.40 ms and the corrector 0.49 ms (0.61-0.69 ms
-// before): 1.68 and 2.35 GB of memory traffic at 4.2 and 4.8 TB/s, the rate of
-// a plain copy.  FP32: 0.22 ms (0.34), its memory and VALU time about equal; with
-// the biharmonic term 0.26 ms, which took 0.70 ms with Del2 formed by a launch
-// of its own (0.30 ms) and read back.
+// predictor and corrector now take 0.84 ms together at 16 rows (1.30 ms before):
+// 1.69 and 2.32 GB of memory traffic at 4.8 TB/s, near the 5.4 of a plain copy, with
+// the VALU 87% and 81% busy: both about equal.  FP32: 0.44 ms (0.68), VALU issue; with
+// the biharmonic term 0.53 ms, which took 1.40 ms with Del2 formed by a launch of its
+// own and read back.
 template <typename T, bool BIH>
 struct March {
     static constexpr int LM = BIH ? 2 : 1;          // lent lanes on either side
@@ -269,12 +269,14 @@ void march_launch(const MomArgsT<T> &a, const MarchPlan &m, hipStream_t s)
 }
 
 // Rows of a march when the caller sets none: a long march repeats less (each
-// starts LAG + 1 rows early), a short one gives more waves.  Four waves per SIMD
-// (4096) are worth shorter marches, down to 4 rows; beyond that 32 rows serve
-// every size.  FP64, us per launch at 128 / 64 / 32 / 16 / 8 / 4 rows:
-// 140x100x40: 67 / 36 / 26 / 15 / 13 / 11; 180x180x75: 79 / 56 / 39 / 31 / 27 /
-// 30; 720x720x75: 495 / 432 / 400 / 397 / 414 / 456; 1440x1440x75: 1702 / 1513 /
-// 1504 / 1534 / 1631 / 1775.
+// starts LAG rows early and walks LAG rows beyond its last), a short one gives more
+// waves.  Four waves per SIMD (4096) are worth shorter marches, down to 4 rows;
+// beyond that 32 rows serve every size within 4%.  us per step (predictor and
+// corrector, among a step's other kernels) at 128 / 64 / 32 / 16 / 8 / 4 rows, FP64:
+// 140x100x40: 185 / 99 / 71 / 43 / 33 / 28; 180x180x75: 174 / 124 / 84 / 67 / 63 /
+// 65; 720x720x75: 955 / 879 / 860 / 841 / 851 / 909; 1440x1440x75: 3288 / 3150 /
+// 3128 / 3089 / 3179 / 3562; FP32 720x720x75: 564 / 487 / 456 / 443 / 465 / 526, with
+// the biharmonic term 627 / 533 / 530 / 546 / 611 / 759.
 constexpr long long kMarchWaves = 4096;
 inline int auto_rows(long long wave_rows)
 {

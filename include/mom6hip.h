@@ -115,11 +115,10 @@ int mom6h_coriolis_end(mom6h_coriolis_cs *cs);
 /* ------------------------------------------------------------ barotropic --
  * barotropic_init_cuda_c (src/cuda_c/mom6_barotropic_cuda_c.F90:226-300),
  * btstep_cuda_c (:305-433), barotropic_end_cuda_c (:629-669); arithmetic of
- * src/serial/mom6_barotropic_serial.F90:178-356.  Each substep is ONE launch
- * of an LDS-tiled kernel (eta predictor, pressure forces, both velocity
- * updates, transports, free surface, time averages on a tile plus its halo)
- * instead of ~9 dependent launches; grids whose coefficients are uniform run
- * several substeps per launch in registers.  periodic_x/periodic_y select the
+ * src/serial/mom6_barotropic_serial.F90:178-356.  A launch runs a whole substep
+ * (eta predictor, pressure forces, both velocity updates, transports, free
+ * surface, time averages on a tile plus its halo) instead of ~9 dependent
+ * launches, and several substeps where the coefficients are uniform.  periodic_x/periodic_y select the
  * split-API ranges (btstep_do_step, :379-474) with a halo refill of
  * ubt, vbt, eta after every substep but the last. */
 typedef struct mom6h_barotropic_cs mom6h_barotropic_cs;
