@@ -182,9 +182,11 @@ int set_error(int code, const char *fmt, ...);
 #define MOM6H_CHECK(expr)                                                          \
     do {                                                                           \
         hipError_t e_ = (expr);                                                    \
-        if (e_ != hipSuccess)                                                      \
+        if (e_ != hipSuccess) {                                                    \
+            (void)hipGetLastError(); /* the next launch check has its own to see */ \
             return ::mom6h::set_error((int)e_, "%s:%d %s: %s", __FILE__, __LINE__, \
                                       #expr, hipGetErrorString(e_));               \
+        }                                                                          \
     } while (0)
 #define MOM6H_LAUNCH_CHECK() MOM6H_CHECK(hipGetLastError())
 #define MOM6H_REQUIRE(cond, ...)                                                   \

@@ -20,11 +20,19 @@ int set_error(int code, const char *fmt, ...)
     return code;
 }
 
+// hipMalloc; a failure is reported here alone, not again by the next launch's check
+static hipError_t try_malloc(void **p, size_t bytes)
+{
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
+
 int dev_alloc(double **p, size_t count, bool zero)
 {
     *p = nullptr;
     if (count == 0) count = 1;
-    hipError_t e = hipMalloc((void **)p, count * sizeof(double));
+    const hipError_t e = try_malloc((void **)p, count * sizeof(double));
     if (e != hipSuccess)
         return set_error(MOM6H_ENOMEM, "hipMalloc(%zu doubles): %s", count, hipGetErrorString(e));
     if (zero) MOM6H_CHECK(hipMemset(*p, 0, count * sizeof(double)));
@@ -196,7 +204,7 @@ int dev_alloc_bytes(void **p, size_t bytes, bool zero)
 {
     *p = nullptr;
     if (bytes == 0) bytes = 8;
-    hipError_t e = hipMalloc(p, bytes);
+    const hipError_t e = try_malloc(p, bytes);
     if (e != hipSuccess) return set_error(MOM6H_ENOMEM, "hipMalloc(%zu bytes): %s", bytes, hipGetErrorString(e));
     if (zero) MOM6H_CHECK(hipMemset(*p, 0, bytes));
     return MOM6H_OK;
@@ -318,7 +326,7 @@ int mom6h_device_synchronize(void)
 int mom6h_malloc(void **p, size_t bytes)
 {
     MOM6H_REQUIRE(p != nullptr, "mom6h_malloc: NULL out pointer");
-    hipError_t e = hipMalloc(p, bytes ? bytes : 1);
+    const hipError_t e = try_malloc(p, bytes ? bytes : 1);
     if (e != hipSuccess)
         return set_error(MOM6H_ENOMEM, "hipMalloc(%zu bytes): %s", bytes, hipGetErrorString(e));
     return MOM6H_OK;
