@@ -899,9 +899,6 @@ int mom6h_hor_visc_set_options(mom6h_hor_visc_cs *cs, int laplacian, int biharmo
     MOM6H_REQUIRE(cs != nullptr, "mom6h_hor_visc_set_options: NULL cs");
     MOM6H_REQUIRE(!biharmonic || (Idx2dyCu && Idxdy2u && Idx2dyCv && Idxdy2v),
                   "mom6h_hor_visc_set_options: biharmonic needs its four metrics");
-    cs->laplacian = laplacian;
-    cs->no_slip = no_slip;
-    cs->Ah = Ah;
     if (biharmonic && !cs->biharmonic) {
         const size_t n2 = (size_t)cs->d.s2;
         int rc = 0;
@@ -914,8 +911,17 @@ int mom6h_hor_visc_set_options(mom6h_hor_visc_cs *cs, int laplacian, int biharmo
         cs->bih_uniform = hv_uniform(cs->d, {{Idx2dyCu, &g.Idx2dyCu}, {Idxdy2u, &g.Idxdy2u},
                                              {Idx2dyCv, &g.Idx2dyCv}, {Idxdy2v, &g.Idxdy2v}});
     }
+    const int was = cs->biharmonic;
     cs->biharmonic = biharmonic;
-    return hor_visc_scratch(cs);
+    const int rc = hor_visc_scratch(cs);
+    if (rc) {
+        cs->biharmonic = was;   // never on without its work fields
+        return rc;
+    }
+    cs->laplacian = laplacian;
+    cs->no_slip = no_slip;
+    cs->Ah = Ah;
+    return MOM6H_OK;
 }
 
 int mom6h_hor_visc(mom6h_hor_visc_cs *cs, const double *u, const double *v, const double *h,
@@ -993,10 +999,17 @@ int mom6h_hor_visc_set_closures(mom6h_hor_visc_cs *cs, int smagorinsky, int leit
         g.DX_dyBu_v = dx * idy;
     }
     if (rc) return rc;
+    const int was[3] = {cs->smagorinsky, cs->leith, cs->better_bound};
     cs->smagorinsky = smagorinsky;
     cs->leith = leith;
     cs->better_bound = better_bound;
-    return hor_visc_scratch(cs);
+    rc = hor_visc_scratch(cs);
+    if (rc) {
+        cs->smagorinsky = was[0];
+        cs->leith = was[1];
+        cs->better_bound = was[2];
+    }
+    return rc;
 }
 
 int mom6h_hor_visc_end(mom6h_hor_visc_cs *cs)

@@ -890,8 +890,13 @@ int mom6h_model_set_option(mom6h_model *m, const char *key, double value)
     }
     else if (k == "general") {   // module hor_visc and CorAdCalc: the general kernels on any grid
         if (m->hv) {
+            const int was = m->hv->general;
             m->hv->general = value != 0.0;
-            RC(hor_visc_scratch(m->hv));
+            const int rc = hor_visc_scratch(m->hv);
+            if (rc) {
+                m->hv->general = was;
+                return rc;
+            }
         }
         if (m->cor) m->cor->general = value != 0.0;
         drop_graphs(m);
@@ -1019,9 +1024,9 @@ bool fused_ok(const mom6h_model *m)
 
 int refresh_del2(mom6h_model *m, hipStream_t s)
 {
-    if (m->f.del2u)
+    if (m->f.del2u && m->f.del2v)
         return launch_del2(Del2Args<float>{m->d, m->ug, m->c.no_slip, m->f.up, m->f.vp, m->mask2dBu, m->f.del2u, m->f.del2v}, s);
-    if (m->del2u)
+    if (m->del2u && m->del2v)
         return launch_del2(Del2Args<double>{m->d, m->ug, m->c.no_slip, m->up, m->vp, m->mask2dBu, m->del2u, m->del2v}, s);
     return MOM6H_OK;
 }
